@@ -50,3 +50,88 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
   if (chunk_offsets_out) chunk_offsets_out[n_seqs] = row;
   return FLA_OK;
 }
+
+// Where a sequence is cut.  A scan's time is its longest workgroup's chunks times the chunk period once every workgroup
+// has a CU of its own, so the segments are as short as 256 CUs allow (GLA forward of 16 heads x 8192 tokens, K = V = 128:
+// 4, 8, 16 and 32 segments 112, 80, 86 and 111 us, uncut 293).  The first pass gets about as many workgroups as there are
+// CUs: 1, 2 and 4 sub-blocks per segment of that forward 94, 80 and 84 us, of one of 64 pairs in two segments 169, 136 and
+// 125 us (uncut 155).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands: the
+// caller says how many chunk periods it has to save.
+extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
+                              int64_t min_saved, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
+  constexpr int64_t kCUs = 256, kChunk = 64, kMinSeg = 4, kPassWorkgroups = 256;
+  if (!out || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
+  auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
+  int64_t longest = 0, total = 0;
+  for (int64_t n = 0; n < N; ++n) {
+    const int64_t c = chunks_of(n);
+    longest = c > longest ? c : longest;
+    total += c;
+  }
+  const int64_t room = kCUs / (H * slabs);   // segments the chip holds at once
+  if (room < 2 || N > room || longest > 0x7fffffff / kChunk) return 0;
+  // the shortest segment with which all of them fit
+  auto segments = [&](int64_t len) {
+    int64_t s = 0;
+    for (int64_t n = 0; n < N; ++n) {
+      const int64_t c = fla_cdiv(chunks_of(n), len);
+      s += c > 0 ? c : 1;
+    }
+    return s;
+  };
+  int64_t seg = fla_cdiv(total, room);
+  seg = seg < kMinSeg ? kMinSeg : seg;
+  while (segments(seg) > room) ++seg;
+  if (longest - seg < min_saved) return 0;
+  const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
+  int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;
+  ratio = ratio < 1 ? 1 : ratio > seg / 2 ? seg / 2 : ratio;
+  const int64_t sub = fla_cdiv(seg, ratio);
+  ratio = fla_cdiv(seg, sub);
+  out->sub_chunks = (int32_t)sub;
+  out->ratio = (int32_t)ratio;
+  out->reserved = 0;
+  out->seg_table = out->sub_table = out->sub_base = nullptr;
+  auto subs_of = [&](int64_t n) {
+    const int64_t s = fla_cdiv(chunks_of(n), sub);
+    return s > 0 ? s : 1;
+  };
+  if (!offsets) {
+    out->nsub = (int32_t)subs_of(0);
+    out->nseg = (int32_t)fla_cdiv(out->nsub, ratio);
+    out->slots = (int32_t)(out->nsub * N);
+    return out->nseg > 1;
+  }
+  // packed batch: the tables list the segments in rounds, so that those of the longest sequences come first
+  int64_t nseg = 0, nsub = 0, base = 0, most = 0;
+  for (int64_t n = 0; n < N; ++n) {
+    const int64_t s = subs_of(n), g = fla_cdiv(s, ratio);
+    if (sub_base) sub_base[n] = (int32_t)base;
+    base += s;
+    nseg += g;
+    most = g > most ? g : most;
+    const int64_t lo = reverse ? ratio : 0, hi = reverse ? s : (g - 1) * ratio;
+    for (int64_t j = lo; j < hi; ++j, ++nsub)
+      if (sub_table) {
+        sub_table[2 * nsub] = (int32_t)n;
+        sub_table[2 * nsub + 1] = (int32_t)j;
+      }
+  }
+  if (sub_base) sub_base[N] = (int32_t)base;
+  if (seg_table) {
+    int64_t row = 0;
+    // whole segments before the shorter last pieces of the sequences
+    for (int pass = 0; pass < 2; ++pass)
+      for (int64_t n = 0; n < N; ++n) {
+        const int64_t g = fla_cdiv(subs_of(n), ratio);
+        for (int64_t s = pass ? g - 1 : 0; s < (pass ? g : g - 1); ++s, ++row) {
+          seg_table[2 * row] = (int32_t)n;
+          seg_table[2 * row + 1] = (int32_t)s;
+        }
+      }
+  }
+  out->nseg = (int32_t)nseg;
+  out->nsub = (int32_t)nsub;
+  out->slots = (int32_t)base;
+  return most > 1;
+}

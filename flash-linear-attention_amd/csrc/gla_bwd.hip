@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "chunk_common.h"
+#include "seq_split.h"
 
 namespace {
 
@@ -222,6 +223,7 @@ struct BDhvParams {
   int64_t T;
   int H, V, N;
   float scale;
+  SplitView split;      // sequences cut into segments (ratio 0: not)
 };
 
 template <typename T, int K>
@@ -253,12 +255,17 @@ __global__ __launch_bounds__(512) void gla_bwd_dhv_kernel(BDhvParams p) {
   const int nvt = V / BV;
   int64_t id = xcd_remap(blockIdx.x, gridDim.x);
   const int vt = (int)(id % nvt);
-  const int nh = (int)(id / nvt);
-  const int n = nh / H, hh = nh % H;
+  const int item = (int)(id / nvt);
+  const int hh = item % H;
   const int vbase = vt * BV;
-  SeqSpan sp = seq_span(p.offsets, n, p.T);
-  const int64_t nchunks = (sp.len + BT - 1) / BT;
-  const int64_t chunk0 = p.chunk_offsets ? p.chunk_offsets[n] : (int64_t)n * ((p.T + BT - 1) / BT);
+  const ScanSpan span = scan_span<true>(p.split, item / H, nullptr, p.offsets, p.chunk_offsets, p.T);
+  const int nh = span.n * H + hh;
+  const SeqSpan sp = span.sp;
+  const int64_t nchunks = span.nchunks, chunk0 = span.chunk0;
+  // the gradient of the state leaving this workgroup's chunks
+  const float* dht = p.split.ratio ? p.split.states + (span.slot * H + hh) * (int64_t)K * V
+                     : p.dht       ? p.dht + (int64_t)nh * K * V
+                                   : nullptr;
   auto chunk_len = [&](int64_t c) {
     int64_t rem = sp.len - c * BT;
     return (int)(rem < BT ? rem : BT);
@@ -391,12 +398,11 @@ __global__ __launch_bounds__(512) void gla_bwd_dhv_kernel(BDhvParams p) {
     // =========================== matrix waves ===========================
     const int kt = wave;   // this wave's 32 key rows of the state gradient
     f32x16 acc = zero16(), acct = zero16();   // dH / s: rows k x columns v, and transposed
-    if (p.dht && kt < KT32) {
-      const float* d0 = p.dht + (int64_t)nh * K * V;
+    if (dht && kt < KT32) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        acc[r] = d0[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + (lane & 31)] * inv_scale;
-        acct[r] = d0[(int64_t)(kt * 32 + (lane & 31)) * V + vbase + c32_row(r, lane)] * inv_scale;
+        acc[r] = dht[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + (lane & 31)] * inv_scale;
+        acct[r] = dht[(int64_t)(kt * 32 + (lane & 31)) * V + vbase + c32_row(r, lane)] * inv_scale;
       }
     }
     // gradient w.r.t. the state leaving chunk c: 16-bit transpose in LDS, FRAGMENT_T copy in memory
@@ -469,7 +475,7 @@ __global__ __launch_bounds__(512) void gla_bwd_dhv_kernel(BDhvParams p) {
       }
       if (c > 0) publish(c - 1);
     }
-    if (p.dh0 && kt < KT32) {
+    if (p.dh0 && span.first && kt < KT32) {
       float* o = p.dh0 + (int64_t)nh * K * V;
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + (lane & 31)] = acc[r] * scale;
@@ -1521,7 +1527,7 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* g, const
                float* dg_head, float* dh0, const int* wide,
                const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT, int64_t B,
                int64_t T_, int64_t H, int64_t K, int64_t V, int64_t N, float scale, hipStream_t st,
-               const void* kh_t = nullptr, const void* scores = nullptr) {
+               const void* kh_t = nullptr, const void* scores = nullptr, const fla_split* split = nullptr) {
   dim3 grid;
   int ntfix;
   int rc = chunk_grid(offsets, indices, B, T_, H, NT, &grid, &ntfix);
@@ -1531,8 +1537,16 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* g, const
   const bool fused_dv = qg && kh_t && scores;   // the reverse state scan also forms dv
   if (fused_dv) {
     BDhvParams p{qg, kh_t, scores, decay, dout, dht, wide, dhtf, dv, dh0, offsets, chunk_offsets, T_, (int)H, (int)V, (int)N,
-                 scale};
-    const int64_t total = (V / 32) * N * H;
+                 scale, split_view(split)};
+    int64_t seqs = N;
+    if (split) {
+      // the gradient leaving every segment: dH <- decay dH + scale (q e^{G})^T do over the sub-blocks
+      rc = gla_split_states(qg, dout, decay, dht, split, false, true, false, 1.f, 0.f, scale, offsets, chunk_offsets,
+                            std::is_same<T, bf16>::value ? FLA_BF16 : FLA_F16, FLA_F32, T_, H, K, V, N, st);
+      if (rc) return rc;
+      seqs = offsets ? split->nseg : split->nseg * N;
+    }
+    const int64_t total = (V / 32) * seqs * H;
     FLA_REQUIRE(total <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
     if (K == 64) hipLaunchKernelGGL((gla_bwd_dhv_kernel<T, 64>), dim3((unsigned)total), dim3(512), 0, st, p);
     else if (K == 128) hipLaunchKernelGGL((gla_bwd_dhv_kernel<T, 128>), dim3((unsigned)total), dim3(512), 0, st, p);
@@ -1597,7 +1611,8 @@ static int gla_bwd_impl(const void* q, const void* k, const void* v, const void*
                         const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT,
                         int qkv_dtype, int gate_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V,
                         int64_t N, float scale, fla_stream_t stream, bool head_gates = false,
-                        const void* kh_t = nullptr, const void* scores = nullptr) {
+                        const void* kh_t = nullptr, const void* scores = nullptr, const fla_split* split = nullptr) {
+  if (split) FLA_REQUIRE(kh_t && scores, FLA_E_INVALID);
   FLA_REQUIRE(q && k && v && gates && dout && hT && dh_frag_t && dq && dk && dv && (dg || dg_head),
               FLA_E_INVALID);
   if (head_gates) FLA_REQUIRE(q_gated && dg_head, FLA_E_INVALID);
@@ -1616,7 +1631,7 @@ static int gla_bwd_impl(const void* q, const void* k, const void* v, const void*
   hipStream_t st = (hipStream_t)stream;
 #define FLA_BWD(TT, GG)                                                                                           \
   return launch_bwd<TT, GG>(q, k, v, gates, dout, dht, hT, q_gated, chunk_decay, dh_frag_t, dq, dk, dv, dg, dg_head, dh0, wide,   \
-                            offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st, kh_t, scores)
+                            offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st, kh_t, scores, split)
   if (head_gates && qkv_dtype == FLA_BF16) FLA_BWD(bf16, HeadGate);
   if (head_gates && qkv_dtype == FLA_F16) FLA_BWD(f16, HeadGate);
   if (head_gates) return FLA_E_UNSUPPORTED;
@@ -1664,4 +1679,19 @@ extern "C" int fla_chunk_simple_gla_bwd(const void* q, const void* k, const void
   return gla_bwd_impl(q, k, v, g, dout, dht, hT, q_gated, chunk_decay, dh_frag_t, dq, dk, dv, nullptr, dg, dh0, wide,
                       offsets, indices, chunk_offsets, NT, qkv_dtype, FLA_F32, B, T, H, K, V, N, scale, stream, true,
                       khat_t, scores);
+}
+
+extern "C" int fla_chunk_gla_bwd_split(const void* q, const void* k, const void* v, const void* gates, const void* dout,
+                                       const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,
+                                       const void* khat_t, const void* scores, void* dh_frag_t, void* dq, void* dk,
+                                       void* dv, float* dg, float* dh0, const int* wide, const int64_t* offsets,
+                                       const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split,
+                                       int64_t NT, int qkv_dtype, int gate_dtype, int64_t B, int64_t T, int64_t H,
+                                       int64_t K, int64_t V, int64_t N, float scale, int head_gates,
+                                       fla_stream_t stream) {
+  FLA_REQUIRE(q_gated && chunk_decay && split && dg, FLA_E_INVALID);
+  return gla_bwd_impl(q, k, v, gates, dout, dht, hT, q_gated, chunk_decay, dh_frag_t, dq, dk, dv, head_gates ? nullptr : dg,
+                      head_gates ? dg : nullptr, dh0, wide, offsets, indices, chunk_offsets, NT, qkv_dtype,
+                      head_gates ? FLA_F32 : gate_dtype, B, T, H, K, V, N, scale, stream, head_gates != 0, khat_t, scores,
+                      split);
 }

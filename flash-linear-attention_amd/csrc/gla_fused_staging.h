@@ -2,6 +2,7 @@
 // tiles, and the work of the staging waves (loads, prefix sums of the log-gates, gated operand tiles).
 #pragma once
 #include "chunk_common.h"
+#include "seq_split.h"
 
 namespace {
 
@@ -33,6 +34,7 @@ struct FusedParams {
   // the workgroup redoes the output rows of its own flagged chunks after its last chunk (the 64- and 32-column
   // kernels; otherwise a second launch does)
   int exact_tail;
+  SplitView split;        // sequences cut into segments (ratio 0: not)
 };
 
 // log2(sigmoid(x)) * inv_norm, clamped from below at clamp2 (both in the log2 domain): two transcendental

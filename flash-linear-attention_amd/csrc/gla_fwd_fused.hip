@@ -269,12 +269,15 @@ __global__ __launch_bounds__(256 + 64 * NSTG) void gla_fwd_fused_kernel(FusedPar
   const ScanItem wi = scan_item(nvb);
   const int vb = wi.slab;
   const int hh = (int)(wi.item % H);
-  const int n = p.seq_order ? (int)p.seq_order[wi.item / H] : (int)(wi.item / H);
-  const int nh = n * H + hh;
   const int vbase = vb * BV;
-  SeqSpan sp = seq_span(p.offsets, n, p.T);
-  const int64_t nchunks = (sp.len + BT - 1) / BT;
-  const int64_t chunk0 = p.chunk_offsets ? p.chunk_offsets[n] : (int64_t)n * ((p.T + BT - 1) / BT);
+  const ScanSpan span = scan_span<false>(p.split, wi.item / H, p.seq_order, p.offsets, p.chunk_offsets, p.T);
+  const int nh = span.n * H + hh;
+  const SeqSpan sp = span.sp;
+  const int64_t nchunks = span.nchunks, chunk0 = span.chunk0;
+  // the state entering this workgroup's chunks
+  const float* hin = p.split.ratio ? p.split.states + (span.slot * H + hh) * (int64_t)K * V
+                     : p.h0        ? p.h0 + (int64_t)nh * K * V
+                                   : nullptr;
   auto chunk_len = [&](int64_t c) {
     int64_t rem = sp.len - c * BT;
     return (int)(rem < BT ? rem : BT);
@@ -326,11 +329,10 @@ __global__ __launch_bounds__(256 + 64 * NSTG) void gla_fwd_fused_kernel(FusedPar
       for (int vt = 0; vt < NVT; ++vt) {
         acc[a][vt] = zero16();
         int kt = wave + 4 * a;
-        if (p.h0 && kt < KT32) {
-          const float* h0p = p.h0 + (int64_t)nh * K * V;
+        if (hin && kt < KT32) {
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            acc[a][vt][r] = h0p[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + vt * 32 + (lane & 31)];
+            acc[a][vt][r] = hin[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + vt * 32 + (lane & 31)];
         }
       }
     // HT: the state entering chunk c in transposed fragment order (rows v, columns k: what the backward kernels
@@ -577,7 +579,7 @@ __global__ __launch_bounds__(256 + 64 * NSTG) void gla_fwd_fused_kernel(FusedPar
       publish_state();
     }
     if (nchunks > 0) lds_barrier();  // hands the last output tile to the staging waves
-    if (p.ht) {
+    if (p.ht && span.last) {
       float* htp = p.ht + (int64_t)nh * K * V;
 #pragma unroll
       for (int a = 0; a < NKT; ++a) {
@@ -667,12 +669,14 @@ int launch_exact(const ExactParams& p, int K, int V, dim3 grid, hipStream_t st) 
 // against 238 us at 128 heads).
 constexpr int64_t kWideMinHeads = 128;
 inline bool use_wide_kernel(const FusedParams& p, int K) {
-  return K == 128 && p.V == 128 && !p.hT && (int64_t)p.N * p.H > kWideMinHeads;
+  return K == 128 && p.V == 128 && !p.hT && !p.split.ratio && (int64_t)p.N * p.H > kWideMinHeads;
 }
 
 template <typename T, typename GT, bool SG = false>
 int launch_fused(const FusedParams& p, int K, hipStream_t st, bool logits = false) {
-  int64_t total = (int64_t)(p.V / 64) * p.N * p.H;
+  // (sequence, head) pairs, or (segment, head) pairs of sequences cut into segments
+  const int64_t seqs = !p.split.ratio ? p.N : p.split.seg_table ? p.split.nseg : (int64_t)p.split.nseg * p.N;
+  int64_t total = (int64_t)(p.V / 64) * seqs * p.H;
   if (total == 0) return FLA_OK;
   FLA_REQUIRE(total <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
   if constexpr (!SG) {
@@ -723,7 +727,8 @@ static int gla_fwd_fused_impl(const void* q, const void* k, const void* v, const
                               int qkv_dtype, int gate_dtype, int64_t B, int64_t T, int64_t H, int64_t K,
                               int64_t V, int64_t N, float scale, fla_stream_t stream, bool head_gates = false,
                               bool exact_pass = true, void* kh_t = nullptr, void* scores = nullptr,
-                              bool logits = false, float gate_inv_norm = 1.f, float gate_clamp_min = -INFINITY) {
+                              bool logits = false, float gate_inv_norm = 1.f, float gate_clamp_min = -INFINITY,
+                              const fla_split* split = nullptr) {
   FLA_REQUIRE(q && k && v && gates && o, FLA_E_INVALID);
   if (logits) FLA_REQUIRE(!head_gates && !h_frag_t, FLA_E_UNSUPPORTED);
   if (head_gates) FLA_REQUIRE(gate_dtype == FLA_F32, FLA_E_UNSUPPORTED);
@@ -753,8 +758,15 @@ static int gla_fwd_fused_impl(const void* q, const void* k, const void* v, const
     FLA_REQUIRE(((uintptr_t)kh_t | (uintptr_t)scores) % 16 == 0, FLA_E_ALIGNMENT);
   }
   FusedParams p{q, k, v, gates, h0, o, ht, offsets, chunk_offsets, seq_order, ws_wide, ws_hwide,
-                T, (int)H, (int)V, (int)N, scale, h_frag_t, qg, decay, kh_t, scores, gate_inv_norm, gate_clamp_min, 0};
+                T, (int)H, (int)V, (int)N, scale, h_frag_t, qg, decay, kh_t, scores, gate_inv_norm, gate_clamp_min, 0,
+                split_view(split)};
   hipStream_t st = (hipStream_t)stream;
+  if (split) {
+    FLA_REQUIRE(!offsets || chunk_offsets, FLA_E_INVALID);
+    int rc = gla_split_states(k, v, gates, h0, split, head_gates, false, logits, gate_inv_norm, gate_clamp_min, 1.f, offsets,
+                              chunk_offsets, qkv_dtype, gate_dtype, T, H, K, V, N, st);
+    if (rc) return rc;
+  }
   dim3 grid;
   int ntfix = 0;
   if (ws_wide) {
@@ -862,4 +874,20 @@ extern "C" int fla_chunk_gla_fwd_fused_logits(const void* q, const void* k, cons
                             indices, chunk_offsets, seq_order, NT, qkv_dtype, gate_dtype, B, T, H, K, V, N, scale,
                             stream, false, true, nullptr, nullptr, true, 1.f / normalizer,
                             has_clamp ? clamp_min : -INFINITY);
+}
+
+extern "C" int fla_chunk_gla_fwd_fused_split(const void* q, const void* k, const void* v, const void* gates, const float* h0,
+                                             void* o, float* ht, int* ws_wide, void* ws_hwide, void* h_frag_t,
+                                             void* q_gated, float* chunk_decay, void* khat_t, void* scores,
+                                             const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets,
+                                             const fla_split* split, int64_t NT, int qkv_dtype, int gate_dtype, int64_t B,
+                                             int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale,
+                                             int gate_form, float normalizer, int has_clamp, float clamp_min,
+                                             fla_stream_t stream) {
+  FLA_REQUIRE(split && gate_form >= 0 && gate_form <= 2 && normalizer != 0.f, FLA_E_INVALID);
+  const bool logits = gate_form == 2;
+  return gla_fwd_fused_impl(q, k, v, gates, h0, o, ht, ws_wide, ws_hwide, h_frag_t, q_gated, chunk_decay, offsets, indices,
+                            chunk_offsets, nullptr, NT, qkv_dtype, gate_dtype, B, T, H, K, V, N, scale, stream,
+                            gate_form == 1, true, khat_t, scores, logits, logits ? 1.f / normalizer : 1.f,
+                            logits && has_clamp ? clamp_min : -INFINITY, split);
 }

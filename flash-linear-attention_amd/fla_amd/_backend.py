@@ -16,11 +16,18 @@ _lib = None
 
 FLA_F32, FLA_BF16, FLA_F16 = 0, 1, 2
 FLA_H_ROW_MAJOR, FLA_H_FRAGMENT, FLA_H_FRAGMENT_T = 0, 1, 2
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _DTYPES = {torch.float32: FLA_F32, torch.bfloat16: FLA_BF16, torch.float16: FLA_F16}
 
 P, I64, I, F = c_void_p, c_int64, c_int, c_float
+
+
+class Split(ctypes.Structure):
+    """``fla_split`` of include/fla_hip.h: how a scan cuts its sequences into segments."""
+    _fields_ = [(n, ctypes.c_int32) for n in ("sub_chunks", "ratio", "nseg", "nsub", "slots", "reserved")] + \
+               [(n, c_void_p) for n in ("seg_table", "sub_table", "sub_base", "states", "decays")]
+
 
 # name -> (restype, argtypes); mirrors include/fla_hip.h declaration by declaration
 SIGNATURES = {
@@ -28,6 +35,7 @@ SIGNATURES = {
     "fla_error_string": (c_char_p, [c_int]),
     "fla_count_chunks": (c_int64, [P, I64, I64]),
     "fla_prepare_chunk_indices": (c_int, [P, I64, I64, P, P]),
+    "fla_scan_split": (c_int, [P, I64, I64, I64, I, I, I64, P, P, P, P]),
     "fla_chunk_local_cumsum": (c_int, [P, P, I, I64, I64, I64, I64, I64, I, P, P, I64, P]),
     "fla_chunk_local_cumsum_inverse": (c_int, [P, P, I64, I64, I64, I64, I64, I, P, P, I64, P]),
     "fla_chunk_global_cumsum": (c_int, [P, P, P, I, I, I64, I64, I64, I64, I64, I, P, P, I64, P]),
@@ -49,6 +57,7 @@ SIGNATURES = {
     "fla_chunk_gla_fwd_fused_states": (c_int, [P] * 14 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gla_fwd_fused_kept": (c_int, [P] * 18 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_simple_gla_fwd_fused": (c_int, [P] * 18 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
+    "fla_chunk_gla_fwd_fused_split": (c_int, [P] * 18 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, I, F, I, F, P]),
     "fla_gdr_fwd_wy": (c_int, [P, P, P, P, P, P, P, P, P, P, I64, I, I64, I64, I64, I64, I64, P]),
     "fla_chunk_gated_delta_rule_fwd_h": (c_int, [P, P, P, P, P, P, P, P, P, P, I, I, I,
                                                  I64, I64, I64, I64, I64, I64, P]),
@@ -61,6 +70,7 @@ SIGNATURES = {
     "fla_chunk_gated_delta_rule_fwd_onepass": (c_int, [P] * 11 + [I, I64, I64, I64, I64, I64, I64, F, I, F, P]),
     "fla_chunk_fwd_o": (c_int, [P, P, P, P, P, P, P, P, I64, I, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gla_bwd": (c_int, [P] * 17 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, P]),
+    "fla_chunk_gla_bwd_split": (c_int, [P] * 22 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, I, P]),
     "fla_chunk_gla_bwd_kept": (c_int, [P] * 21 + [I64, I, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_simple_gla_bwd": (c_int, [P] * 21 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gla_fwd_o_gk": (c_int, [P] * 8 + [I64, I, I, I, I64, I64, I64, I64, I64, F, P]),

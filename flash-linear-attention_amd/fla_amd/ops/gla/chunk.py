@@ -7,6 +7,7 @@ output rows recomputed exactly by the same launch after its last chunk).  The tw
 ``fla_chunk_gla_fwd_o``) serves the reference-shaped internal entry points ``chunk_gla_fwd`` /
 ``chunk_fwd_h`` / ``chunk_gla_fwd_o_gk``.
 """
+import ctypes
 import os
 import threading
 import warnings
@@ -16,7 +17,8 @@ import torch
 import torch.nn.functional as F
 
 from ... import _backend as be
-from ...utils import VarlenPlan, check_varlen_args, contiguous, empty_batch_result, resolve_offsets
+from ...utils import (MIN_SAVED_CHUNKS, VarlenPlan, check_varlen_args, contiguous, empty_batch_result, resolve_offsets,
+                      scan_split)
 from ..common.chunk_h import chunk_fwd_h
 from ..utils.cumsum import chunk_local_cumsum, chunk_local_cumsum_inverse
 
@@ -31,6 +33,10 @@ KEEP_STATES_FOR_BACKWARD = os.environ.get("FLA_AMD_RECOMPUTE_STATES", "0") in ("
 # With the states, a differentiated forward (per-key gates, V <= 128) also keeps k^ = k e^{G_last - G} and the score tile
 # of every chunk (1.5 more tensors of k's size), from which the backward's reverse state scan forms dv on its way.
 KEEP_KHAT_AND_SCORES = os.environ.get("FLA_AMD_GLA_FUSED_DV", "1") not in ("", "0")
+# A differentiated pass waits for its host code longer than for the device until the scans are long: it cuts its
+# sequences only where that takes this many chunks off a scan (557 -> 537 us at 32 chunks saved, B=4, T=4096, H=16,
+# K=V=128; 178 -> 212 us at 24, B=2, T=2000, H=32, K=V=64).
+_MIN_SAVED_CHUNKS_TRAINING = 28
 # fp32 q/k/v run through the fp16 chunk kernels, as the reference runs them through its chunk kernels with fp32 operands
 # on the matrix pipe at reduced precision (tests/ops/test_gla.py:149-201): q, k and v are divided by a power of two >= their
 # largest magnitude (exact; found on the device, no synchronisation) and rounded to fp16, gates and states stay fp32, and
@@ -308,7 +314,30 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
             0 if plan is None else plan.NT,
             be.dt(q), be.dt(g), B, T, H, K, V, N, float(scale), be.stream_of(q))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(h0), be.ptr(o), be.ptr(ht), be.ptr(wide), be.ptr(hwide))
-    if gate_logits is not None:
+    split = None
+    if V <= 128 and not first_launch_only:
+        split = scan_split(plan, N, T, H, V // 64,
+                           min_saved=MIN_SAVED_CHUNKS if states_out is None else _MIN_SAVED_CHUNKS_TRAINING)
+    if split is not None:
+        if head_gates and (g.dtype != torch.float32 or g.shape != q.shape[:3]):
+            raise ValueError("head gates must be fp32 [B, T, H]")
+        kept = [None] * 5
+        if states_out is not None:
+            nt = plan.NT if plan is not None else -(-T // BT)
+            kept[:3] = (q.new_empty(B, nt, H, K, V), torch.empty_like(q), q.new_empty(B, nt, H, K, dtype=torch.float32))
+            if KEEP_KHAT_AND_SCORES:
+                kept[3:] = q.new_empty(B, nt, H, K, BT), q.new_empty(B, nt, H, BT, BT)
+            states_out.extend(x for x in kept if x is not None)
+        st = q.new_empty(split.slots, H, K, V, dtype=torch.float32)
+        dec = q.new_empty(split.slots, H, K, dtype=torch.float32)
+        form, normalizer, clamp_min = (1, 1.0, None) if head_gates else (0, 1.0, None)
+        if gate_logits is not None:
+            form, (normalizer, clamp_min) = 2, gate_logits
+        be.check(be.lib().fla_chunk_gla_fwd_fused_split(
+            *head, *(be.ptr(x) for x in kept), *tail[:3], ctypes.byref(split.bind(st, dec)), *tail[4:-1], form,
+            float(normalizer), int(clamp_min is not None), float(clamp_min or 0.0), tail[-1]),
+            "fla_chunk_gla_fwd_fused_split")
+    elif gate_logits is not None:
         if head_gates or states_out is not None or first_launch_only:
             raise ValueError("gate logits: per-key gates, forward without kept states")
         normalizer, clamp_min = gate_logits
@@ -489,7 +518,16 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
             be.ptr(idx), be.ptr(co), NT, be.dt(q), be.dt(g), B, T, H, K, V, N, float(scale), be.stream_of(q))
     outs = (be.ptr(dhtf), be.ptr(dq), be.ptr(dk), be.ptr(dv), be.ptr(dg))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(do), be.ptr(dht), be.ptr(hT))
-    if kept and head_gates:
+    split = None
+    if kept and kh is not None:
+        split = scan_split(plan, N, T, H, V // 32, True, _MIN_SAVED_CHUNKS_TRAINING)
+    if split is not None:
+        st = q.new_empty(split.slots, H, K, V, dtype=torch.float32)
+        dec = q.new_empty(split.slots, H, K, dtype=torch.float32)
+        be.check(be.lib().fla_chunk_gla_bwd_split(
+            *head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs, *tail[:5],
+            ctypes.byref(split.bind(st, dec)), *tail[5:-1], int(head_gates), tail[-1]), "fla_chunk_gla_bwd_split")
+    elif kept and head_gates:
         be.check(be.lib().fla_chunk_simple_gla_bwd(*head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs,
                                                    *tail[:7], *tail[8:]),
                  "fla_chunk_simple_gla_bwd")

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FLA_ABI_VERSION 14
+#define FLA_ABI_VERSION 15
 
 enum fla_dtype { FLA_F32 = 0, FLA_BF16 = 1, FLA_F16 = 2 };
 
@@ -55,6 +55,31 @@ int64_t fla_count_chunks(const int64_t* offsets_host, int64_t n_seqs, int64_t ch
  * = exclusive prefix sum of per-sequence chunk counts.  Either may be NULL. */
 int fla_prepare_chunk_indices(const int64_t* offsets_host, int64_t n_seqs, int64_t chunk_size,
                               int64_t* indices_out, int64_t* chunk_offsets_out);
+
+/* How a serial scan cuts its sequences into segments that are scanned side by side (no counterpart in the reference):
+ * a scan gives one workgroup to a (sequence, head, value slab), so a launch of few pairs and long sequences leaves most of
+ * the chip idle.  A sub-block is `sub_chunks` chunks, a segment `ratio` sub-blocks; what a sub-block adds to a zero state
+ * and its transition are formed first, folded into the state entering every segment, and the scan then starts there.
+ * Equal-length sequences: nseg segments and nsub sub-blocks each, no tables.  Packed batches: nseg rows of seg_table
+ * (sequence, segment), nsub rows of sub_table (sequence, sub-block: those the first pass forms), sub_base [N+1] the first
+ * slot of a sequence.  states [slots, H, K, V] and decays [slots, H, K] (GLA) or [slots, H, K, K] (delta rule) are fp32
+ * workspaces. */
+typedef struct fla_split {
+  int32_t sub_chunks, ratio, nseg, nsub, slots, reserved;
+  const int32_t* seg_table;
+  const int32_t* sub_table;
+  const int32_t* sub_base;
+  float* states;
+  float* decays;
+} fla_split;
+
+/* The plan for N sequences of T tokens (or, with offsets_host [N+1], of a packed batch) and H heads in `slabs` workgroups
+ * per (sequence, head), where cutting makes the scan at least min_saved chunks shorter; reverse: for a scan from right
+ * to left.  Fills the integer fields and returns 1, or returns 0 where
+ * cutting would not pay (host arithmetic, host pointers).  A packed batch's tables are written on a second call with
+ * seg_table / sub_table / sub_base given (2 x nseg, 2 x nsub and N+1 words). */
+int fla_scan_split(const int64_t* offsets_host, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
+                   int64_t min_saved, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base);
 
 /* ------------------------------------------------------------------------
  * chunk_local_cumsum (fla/ops/utils/cumsum.py:389-407; scalar kernel :24-57,
@@ -268,6 +293,18 @@ int fla_chunk_gla_fwd_fused_kept(const void* q, const void* k, const void* v, co
                                  int64_t NT, int qkv_dtype, int gate_dtype, int64_t B, int64_t T, int64_t H,
                                  int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
 
+/* The three entry points above on sequences cut into segments (fla_scan_split with V / 64 slabs): two launches form the
+ * state entering every segment, then the same scan runs over the segments.  The outputs past ws_hwide may be NULL as in the
+ * entry points without `split`; gate_form 0: per-key log-gates, 1: one fp32 log-gate per (token, head), 2: gate logits
+ * (normalizer, has_clamp and clamp_min as in fla_chunk_gla_fwd_fused_logits). */
+int fla_chunk_gla_fwd_fused_split(const void* q, const void* k, const void* v, const void* gates, const float* h0,
+                                  void* o, float* ht, int* ws_wide, void* ws_hwide, void* h_frag_t, void* q_gated,
+                                  float* chunk_decay, void* khat_t, void* scores, const int64_t* offsets,
+                                  const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split,
+                                  int64_t NT, int qkv_dtype, int gate_dtype, int64_t B, int64_t T, int64_t H, int64_t K,
+                                  int64_t V, int64_t N, float scale, int gate_form, float normalizer, int has_clamp,
+                                  float clamp_min, fla_stream_t stream);
+
 /* The fused forward for one log-gate per (token, head), g fp32 [B,T,H]: chunk_simple_gla
  * (fla/ops/simple_gla/chunk.py:16-131: h_t = e^{g_t} h_{t-1} + k_t v_t^T, o_t = scale q_t^T h_t) without
  * the [B,T,H,K] gate tensor a call through fla_chunk_gla_fwd_fused would need.  Same kernel, the staging
@@ -466,6 +503,17 @@ int fla_chunk_simple_gla_bwd(const void* q, const void* k, const void* v, const 
                              const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT,
                              int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N,
                              float scale, fla_stream_t stream);
+
+/* fla_chunk_gla_bwd_kept (head_gates: fla_chunk_simple_gla_bwd) with khat_t and scores on sequences cut into segments
+ * (fla_scan_split with V / 32 slabs, reverse): the state gradient leaving every segment is formed first and the reverse
+ * state scan runs over the segments. */
+int fla_chunk_gla_bwd_split(const void* q, const void* k, const void* v, const void* gates, const void* dout,
+                            const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,
+                            const void* khat_t, const void* scores, void* dh_frag_t, void* dq, void* dk, void* dv, float* dg,
+                            float* dh0, const int* wide, const int64_t* offsets, const int64_t* indices,
+                            const int64_t* chunk_offsets, const fla_split* split, int64_t NT, int qkv_dtype, int gate_dtype,
+                            int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, int head_gates,
+                            fla_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * The chunk-parallel stages of GLA under the operand layouts of the reference's internal

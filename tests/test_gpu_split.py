@@ -1,0 +1,79 @@
+"""GPU: scans over sequences cut into segments (few (sequence, head) pairs, long time axis) against the fp32
+recurrences.  The gates are weak, so that the state entering a segment decides its output, and the lengths leave short
+last chunks, short last segments and, in packed batches, sequences shorter than a segment.  Tolerances are those of the
+uncut operators (16-bit operands, fp32 sums): 1e-2 on o, 5e-3 on the final state, 2e-2 on the gradients."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from helpers import assert_close, gdr_inputs, gla_inputs
+from oracle.recurrent import naive_recurrent_gated_delta_rule, naive_recurrent_gla
+
+pytestmark = pytest.mark.gpu
+
+
+def _cut(B, T, H, slabs, reverse, offsets, device):
+    from fla_amd.utils import VarlenPlan, scan_split
+    plan = None if offsets is None else VarlenPlan(offsets, 64)
+    return scan_split(plan, B if plan is None else plan.N, T, H, slabs, reverse)
+
+
+CASES = [
+    # B, T, H, K, V, boundaries of a packed batch, dtype
+    (1, 833, 1, 64, 64, None, torch.bfloat16),        # 14 chunks, the last of one token
+    (2, 1087, 2, 128, 128, None, torch.bfloat16),     # 17 chunks, the last of 63 tokens
+    (1, 1024, 3, 128, 64, None, torch.float16),
+    (1, 1500, 2, 64, 128, [0, 1, 1, 900, 964, 1500], torch.bfloat16),
+    (1, 2200, 1, 128, 128, [0, 1290, 1354, 2200], torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", CASES)
+@pytest.mark.parametrize("heads", [False, True])
+def test_gla_cut_sequences(device, monkeypatch, B, T, H, K, V, bounds, dtype, heads):
+    import fla_amd.ops.gla.chunk as gla_mod
+    from fla_amd.ops.gla import chunk_gla
+    monkeypatch.setattr(gla_mod, "_MIN_SAVED_CHUNKS_TRAINING", 8)
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    N = B if bounds is None else len(bounds) - 1
+    offs = None if bounds is None else torch.tensor(bounds, device=device)
+    assert _cut(B, T, H, V // 64, False, offs, device) is not None
+    assert _cut(B, T, H, V // 32, True, offs, device) is not None
+    print("cut", B, T, H, K, V, bounds, dtype, heads, flush=True)
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
+    if heads:
+        g = g[..., 0].contiguous()
+    do, dht = torch.randn(B, T, H, V).to(dtype), torch.randn(N, H, K, V) * 0.1
+    op = chunk_simple_gla if heads else chunk_gla
+    dev = [x.to(device) for x in (q, k, v, g, h0)]
+    with torch.no_grad():
+        o1, ht1 = op(*dev[:4], initial_state=dev[4], output_final_state=True, cu_seqlens=offs, head_first=False)
+    leaves = [x.requires_grad_() for x in dev]
+    o, ht = op(*leaves[:4], initial_state=leaves[4], output_final_state=True, cu_seqlens=offs, head_first=False)
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    refs = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*refs[:3], None if heads else refs[3], initial_state=refs[4], output_final_state=True,
+                                  offsets=bounds, g=refs[3] if heads else None)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for a, b in ((o1, ht1), (o, ht)):
+        assert_close("o", ro, a, 1e-2)
+        assert_close("ht", rht, b, 5e-3)
+    for name, r, d in zip(("dq", "dk", "dv", "dg", "dh0"), refs, leaves):
+        assert_close(name, r.grad, d.grad, 2e-2)
+
+
+def test_gla_cut_gate_logits_and_strong_gates(device):
+    """Gates formed from pre-activations, some of them far outside the range of the chunk's single reference point."""
+    from fla_amd.ops.gla import chunk_gla
+    q, k, v, _, h0 = gla_inputs(1, 1100, 2, 128, 128, seed=5)
+    x = torch.randn(1, 1100, 2, 128)
+    x[:, 300:330] -= 40.0
+    offs = None
+    assert _cut(1, 1100, 2, 2, False, offs, device) is not None
+    print("cut, gate logits", flush=True)
+    with torch.no_grad():
+        o, ht = chunk_gla(*(t.to(device) for t in (q, k, v, x)), initial_state=h0.to(device), output_final_state=True,
+                          head_first=False, gate_logit_normalizer=8.0)
+    ro, rht = naive_recurrent_gla(q, k, v, F.logsigmoid(x) / 8.0, initial_state=h0, output_final_state=True)
+    assert_close("o", ro, o, 1e-2)
+    assert_close("ht", rht, ht, 5e-3)
