@@ -1,4 +1,5 @@
-"""Build libfla_hip.so (gfx950) from csrc/*.hip with hipcc, in-tree.
+"""Build libfla_hip.so (gfx950) from csrc/*.hip with hipcc, and the host extension _fla_host.so from csrc/torch_host.cpp
+with g++, in-tree.
 
     python flash-linear-attention_amd/build.py [--force] [-j N]
 
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_DIR = os.path.join(HERE, "fla_amd", "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libfla_hip.so")
+HOST_SRC, HOST_PATH = os.path.join(CSRC, "torch_host.cpp"), os.path.join(LIB_DIR, "_fla_host.so")
 
 HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 FLAGS = [
@@ -59,6 +62,32 @@ def _compile(src, force):
     return obj, log
 
 
+def _build_host(force):
+    """The CPython extension over libfla_hip.so (host code only; torch is asked for its include and library folders)."""
+    header = os.path.join(HERE, "..", "include", "fla_hip.h")
+    if (not force and os.path.exists(HOST_PATH)
+            and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(HOST_SRC), os.path.getmtime(header))):
+        return ""
+    from torch.utils import cpp_extension as ext
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    includes = [p for p in ext.include_paths() if os.path.isdir(p)] + [os.path.join(rocm, "include"), "/opt/rocm/include",
+                                                                       sysconfig.get_path("include")]
+    import torch
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for p in includes:
+        cmd += ["-isystem", p]
+    cmd += [HOST_SRC, "-o", HOST_PATH]
+    for p in ext.library_paths():
+        cmd += ["-L" + p]
+    cmd += ["-L" + LIB_DIR, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-lfla_hip",
+            "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on torch_host.cpp:\n" + r.stdout + r.stderr)
+    return r.stderr
+
+
 def build(force=False, jobs=None, verbose=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -73,8 +102,9 @@ def build(force=False, jobs=None, verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
+    _build_host(force)
     if verbose:
-        print(f"built {LIB_PATH} from {len(objs)} objects")
+        print(f"built {LIB_PATH} from {len(objs)} objects, and {HOST_PATH}")
     return LIB_PATH
 
 

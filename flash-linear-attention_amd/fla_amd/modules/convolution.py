@@ -7,6 +7,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import _backend as be
+from .._native import host
 
 
 def _act_flag(activation: Optional[str]) -> int:
@@ -60,12 +61,16 @@ class CausalConv1dFunction(torch.autograd.Function):
 def causal_conv1d(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                   activation: Optional[str] = None) -> torch.Tensor:
     """``x`` [B,T,D], ``weight`` [D,W] (or the ``nn.Conv1d`` layout [D,1,W]) -> [B,T,D]."""
-    return CausalConv1dFunction.apply(x, weight, bias, activation)
+    y = host().causal_conv1d(x, weight, bias, _act_flag(activation))
+    return y if y is not None else CausalConv1dFunction.apply(x, weight, bias, activation)
 
 
 def causal_conv1d_update(x: torch.Tensor, cache: torch.Tensor, weight: torch.Tensor,
                          bias: Optional[torch.Tensor] = None, activation: Optional[str] = None) -> torch.Tensor:
     """Single-token step: ``x`` [B,D]; ``cache`` [B,D,W] is shifted and updated in place."""
+    y = host().causal_conv1d_update(x, cache, weight, bias, _act_flag(activation))
+    if y is not None:
+        return y
     be.require_gpu(x, cache)
     B, D = x.shape
     W = weight.shape[-1]

@@ -6,6 +6,7 @@ import torch
 import torch.nn as nn
 
 from .. import _backend as be
+from .._native import host
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -109,10 +110,18 @@ class LayerNormSwishGateFn(torch.autograd.Function):
 
 
 def layer_norm_swish_gate_fn(x, o, weight, bias, residual=None, prenorm=False, residual_in_fp32=False, eps=1e-6):
+    if residual is None and not prenorm and not residual_in_fp32:
+        y = host().norm_swish_gate(x, o, weight, bias, eps, False)
+        if y is not None:
+            return y
     return LayerNormSwishGateFn.apply(x, o, weight, bias, residual, eps, prenorm, residual_in_fp32, False)
 
 
 def rms_norm_swish_gate_fn(x, o, weight, bias, residual=None, prenorm=False, residual_in_fp32=False, eps=1e-6):
+    if residual is None and not prenorm and not residual_in_fp32:
+        y = host().norm_swish_gate(x, o, weight, bias, eps, True)
+        if y is not None:
+            return y
     return LayerNormSwishGateFn.apply(x, o, weight, bias, residual, eps, prenorm, residual_in_fp32, True)
 
 

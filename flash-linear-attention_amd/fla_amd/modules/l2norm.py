@@ -4,6 +4,7 @@ from typing import Optional
 import torch
 
 from .. import _backend as be
+from .._native import host
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -58,4 +59,8 @@ class L2NormFunction(torch.autograd.Function):
 
 
 def l2_norm(x: torch.Tensor, eps: float = 1e-6, output_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+    if output_dtype is None or output_dtype == x.dtype:
+        y = host().l2_norm(x, eps)
+        if y is not None:
+            return y
     return L2NormFunction.apply(x, eps, output_dtype)

@@ -6,6 +6,7 @@ from typing import Optional, Tuple
 import torch
 
 from ... import _backend as be
+from ..._native import host
 from ...utils import autocast_custom_bwd, autocast_custom_fwd, contiguous
 
 
@@ -191,5 +192,9 @@ def fused_recurrent(
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     if scale is None:
         scale = k.shape[-1] ** -0.5
+    if offsets is None and not head_first:
+        res = host().recurrent_gla(q, k, v, g, gk, gv, scale, initial_state, output_final_state, reverse, inplace_state)
+        if res is not None:
+            return res
     return FusedRecurrentFunction.apply(q, k, v, g, gk, gv, scale, initial_state, output_final_state,
                                         reverse, offsets, head_first, inplace_state)

@@ -17,8 +17,9 @@ import torch
 import torch.nn.functional as F
 
 from ... import _backend as be
+from ..._native import host
 from ...utils import (VarlenPlan, autocast_custom_bwd, autocast_custom_fwd, check_varlen_args, contiguous,
-                      empty_batch_result, resolve_offsets)
+                      empty_batch_result, native_plan, resolve_offsets)
 from ..common.chunk_delta_h import (chunk_gated_delta_rule_fwd_h, chunk_gated_delta_rule_fwd_h_both,
                                     chunk_gated_delta_rule_fwd_onepass, chunk_gated_delta_rule_fwd_scan)
 from ..common.chunk_o import chunk_fwd_o
@@ -27,6 +28,7 @@ from .wy_fast import fwd_prepare_scan_operands, fwd_prepare_wy_repr
 
 BT = 64
 _SUPPORTED_KV = {(64, 64), (128, 128), (64, 128), (128, 64), (256, 64), (256, 128)}
+L2NORM_EPS = 1e-6   # the eps of fla.modules.l2norm
 _FUSED_MAX_K = 128  # the one-pass forward kernel holds at most 128 key channels of the state
 
 # A forward pass that will be differentiated keeps w, Aw, v_new and the per-chunk states for its
@@ -247,28 +249,42 @@ class ChunkGatedDeltaRuleFunction(torch.autograd.Function):
                 None, None, None)
 
 
-def _direct_launch_ok(q, k, v, g, beta, initial_state, head_first) -> bool:
-    """True when a call can go straight to the two forward launches: no operand takes part in autograd and every
-    operand already has the layout, dtype and head dims the kernels read.  Anything else takes the autograd
-    function, which converts and pads."""
-    if head_first or q.dtype not in (torch.bfloat16, torch.float16):
-        return False
-    K, V = q.shape[-1], v.shape[-1]
-    if K > _FUSED_MAX_K or (K, V) not in _SUPPORTED_KV:
-        return False
-    if torch.is_autocast_enabled():
-        return False
-    ts = (q, k, v, beta) if g is None else (q, k, v, beta, g)
-    if torch.is_grad_enabled() and (any(t.requires_grad for t in ts) or
-                                    (initial_state is not None and initial_state.requires_grad)):
-        return False
-    if not all(t.is_cuda and t.is_contiguous() for t in ts):
-        return False
-    return initial_state is None or (initial_state.dtype == torch.float32 and initial_state.is_contiguous())
+def _launch(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, l2norm_eps=None):
+    """Seq-first operands as the kernels read them through the host extension; ``None`` if they need a conversion."""
+    if ONEPASS_FORWARD:
+        return None
+    return host().chunk_gdr(q, k, v, g, beta, scale, initial_state, output_final_state, native_plan(offsets),
+                            KEEP_STATES_FOR_BACKWARD, l2norm_eps)
+
+
+def _apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first):
+    """One slab of at most 128 value columns.  Key dims up to 128: converted to what the host extension takes (seq-first,
+    head dims 64 or 128, fp32 state) by differentiable torch operations; K = 256, passes that recompute in the backward
+    and the one-launch forward go through the autograd function."""
+    K, V = k.shape[-1], v.shape[-1]
+    KP, VP = _round_k(K), _round64(V)
+    grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (q, k, v, g, beta, initial_state))
+    if KP <= _FUSED_MAX_K and not ONEPASS_FORWARD and not (grad and not KEEP_STATES_FOR_BACKWARD):
+        be.require_gpu(q, k, v, beta)
+        x, h0 = (q, k, v, g, beta), initial_state
+        if head_first:
+            x = tuple(None if t is None else t.transpose(1, 2) for t in x)
+        if (KP, VP) != (K, V):
+            x = tuple(F.pad(t, (0, p - t.shape[-1])) for t, p in zip(x, (KP, KP, VP))) + x[3:]
+            h0 = None if h0 is None else F.pad(h0, (0, VP - V, 0, KP - K))
+        res = _launch(*x, scale, None if h0 is None else h0.float(), output_final_state, offsets)
+        if res is not None:
+            o, ht = res
+            if VP != V:
+                o = o[..., :V]
+            if ht is not None and (KP, VP) != (K, V):
+                ht = ht[..., :K, :V].contiguous()
+            return (o.transpose(1, 2).contiguous() if head_first else o), ht
+    return ChunkGatedDeltaRuleFunction.apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first)
 
 
 def apply_in_value_slabs(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first):
-    """The autograd function on heads of any supported width (``g`` may be None: un-gated rule)."""
+    """The operator on heads of any supported width (``g`` may be None: un-gated rule)."""
     K, V = k.shape[-1], v.shape[-1]
     if K > 256:
         raise NotImplementedError(f"fla_amd chunk_gated_delta_rule: key head dims up to 256 are covered (got {K}), "
@@ -279,13 +295,11 @@ def apply_in_value_slabs(q, k, v, g, beta, scale, initial_state, output_final_st
         outs, states = [], []
         for v0 in range(0, V, 128):
             h0 = None if initial_state is None else initial_state[..., v0:v0 + 128]
-            o, ht = ChunkGatedDeltaRuleFunction.apply(q, k, v[..., v0:v0 + 128], g, beta, scale, h0, output_final_state,
-                                                      offsets, head_first)
+            o, ht = _apply(q, k, v[..., v0:v0 + 128], g, beta, scale, h0, output_final_state, offsets, head_first)
             outs.append(o)
             states.append(ht)
         return torch.cat(outs, dim=-1), (torch.cat(states, dim=-1) if output_final_state else None)
-    return ChunkGatedDeltaRuleFunction.apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets,
-                                             head_first)
+    return _apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first)
 
 
 def chunk_gated_delta_rule(
@@ -329,15 +343,12 @@ def chunk_gated_delta_rule(
         assert scale > 0, "Scale must be positive."
     if q.numel() == 0:
         return empty_batch_result(q.transpose(1, 2) if head_first else q, v, offsets, initial_state, output_final_state)
-    direct = _direct_launch_ok(q, k, v, g, beta, initial_state, head_first)
-    if use_qk_l2norm_in_kernel and not direct:
+    if not head_first:
+        res = _launch(q, k, v, g, beta, scale, initial_state, output_final_state, offsets,
+                      L2NORM_EPS if use_qk_l2norm_in_kernel else None)
+        if res is not None:
+            return res
+    if use_qk_l2norm_in_kernel:
         from ...modules.l2norm import l2_norm
         q, k = l2_norm(q), l2_norm(k)
-    if direct:
-        # nothing to differentiate and nothing to convert: no autograd node, no copies
-        _, o, _, _, ht = chunk_gated_delta_rule_fwd(q, k, v, g, beta, scale, initial_state, output_final_state,
-                                                    offsets=offsets, head_first=False, chunk_size=BT, store_A=False,
-                                                    l2norm_eps=1e-6 if use_qk_l2norm_in_kernel else None,
-                                                    want_g_cumsum=False)
-        return o, ht
     return apply_in_value_slabs(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first)

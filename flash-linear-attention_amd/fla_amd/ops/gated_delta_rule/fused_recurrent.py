@@ -6,6 +6,7 @@ from typing import Optional, Tuple
 import torch
 
 from ... import _backend as be
+from ..._native import host
 from ...utils import check_varlen_args, contiguous, resolve_offsets
 
 L2NORM_EPS = 1e-6   # the eps of fla.modules.l2norm
@@ -107,7 +108,8 @@ def fused_recurrent_gated_delta_rule(
     launches fewer per decode step).
     """
     offsets = resolve_offsets(offsets, cu_seqlens)
-    check_varlen_args(q, offsets, head_first, initial_state)
+    if offsets is not None:
+        check_varlen_args(q, offsets, head_first, initial_state)
     if scale is None:
         scale = k.shape[-1] ** -0.5
     else:
@@ -115,6 +117,10 @@ def fused_recurrent_gated_delta_rule(
     if beta is None:
         beta = torch.ones_like(q[..., 0])
     l2norm_eps = L2NORM_EPS if use_qk_l2norm_in_kernel else None
+    if offsets is None and not head_first:
+        res = host().recurrent_gdr(q, k, v, g, beta, scale, initial_state, output_final_state, inplace_state, l2norm_eps)
+        if res is not None:
+            return res
     if not (torch.is_grad_enabled() and any(t is not None and t.requires_grad
                                             for t in (q, k, v, g, beta, initial_state))):
         # decode loops: no autograd node to build, and the host time of a step is of the order of its device time

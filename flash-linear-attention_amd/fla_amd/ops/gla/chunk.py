@@ -7,7 +7,6 @@ output rows recomputed exactly by the same launch after its last chunk).  The tw
 ``fla_chunk_gla_fwd_o``) serves the reference-shaped internal entry points ``chunk_gla_fwd`` /
 ``chunk_fwd_h`` / ``chunk_gla_fwd_o_gk``.
 """
-import ctypes
 import os
 import threading
 import warnings
@@ -17,8 +16,9 @@ import torch
 import torch.nn.functional as F
 
 from ... import _backend as be
-from ...utils import (MIN_SAVED_CHUNKS, VarlenPlan, check_varlen_args, contiguous, empty_batch_result, resolve_offsets,
-                      scan_split)
+from ..._native import host
+from ...utils import (VarlenPlan, check_varlen_args, contiguous, empty_batch_result, native_plan,
+                      resolve_offsets)
 from ..common.chunk_h import chunk_fwd_h
 from ..utils.cumsum import chunk_local_cumsum, chunk_local_cumsum_inverse
 
@@ -33,10 +33,6 @@ KEEP_STATES_FOR_BACKWARD = os.environ.get("FLA_AMD_RECOMPUTE_STATES", "0") in ("
 # With the states, a differentiated forward (per-key gates, V <= 128) also keeps k^ = k e^{G_last - G} and the score tile
 # of every chunk (1.5 more tensors of k's size), from which the backward's reverse state scan forms dv on its way.
 KEEP_KHAT_AND_SCORES = os.environ.get("FLA_AMD_GLA_FUSED_DV", "1") not in ("", "0")
-# A differentiated pass waits for its host code longer than for the device until the scans are long: it cuts its
-# sequences only where that takes this many chunks off a scan (557 -> 537 us at 32 chunks saved, B=4, T=4096, H=16,
-# K=V=128; 178 -> 212 us at 24, B=2, T=2000, H=32, K=V=64).
-_MIN_SAVED_CHUNKS_TRAINING = 28
 # fp32 q/k/v run through the fp16 chunk kernels, as the reference runs them through its chunk kernels with fp32 operands
 # on the matrix pipe at reduced precision (tests/ops/test_gla.py:149-201): q, k and v are divided by a power of two >= their
 # largest magnitude (exact; found on the device, no synchronisation) and rounded to fp16, gates and states stay fp32, and
@@ -314,30 +310,7 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
             0 if plan is None else plan.NT,
             be.dt(q), be.dt(g), B, T, H, K, V, N, float(scale), be.stream_of(q))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(h0), be.ptr(o), be.ptr(ht), be.ptr(wide), be.ptr(hwide))
-    split = None
-    if V <= 128 and not first_launch_only:
-        split = scan_split(plan, N, T, H, V // 64,
-                           min_saved=MIN_SAVED_CHUNKS if states_out is None else _MIN_SAVED_CHUNKS_TRAINING)
-    if split is not None:
-        if head_gates and (g.dtype != torch.float32 or g.shape != q.shape[:3]):
-            raise ValueError("head gates must be fp32 [B, T, H]")
-        kept = [None] * 5
-        if states_out is not None:
-            nt = plan.NT if plan is not None else -(-T // BT)
-            kept[:3] = (q.new_empty(B, nt, H, K, V), torch.empty_like(q), q.new_empty(B, nt, H, K, dtype=torch.float32))
-            if KEEP_KHAT_AND_SCORES:
-                kept[3:] = q.new_empty(B, nt, H, K, BT), q.new_empty(B, nt, H, BT, BT)
-            states_out.extend(x for x in kept if x is not None)
-        st = q.new_empty(split.slots, H, K, V, dtype=torch.float32)
-        dec = q.new_empty(split.slots, H, K, dtype=torch.float32)
-        form, normalizer, clamp_min = (1, 1.0, None) if head_gates else (0, 1.0, None)
-        if gate_logits is not None:
-            form, (normalizer, clamp_min) = 2, gate_logits
-        be.check(be.lib().fla_chunk_gla_fwd_fused_split(
-            *head, *(be.ptr(x) for x in kept), *tail[:3], ctypes.byref(split.bind(st, dec)), *tail[4:-1], form,
-            float(normalizer), int(clamp_min is not None), float(clamp_min or 0.0), tail[-1]),
-            "fla_chunk_gla_fwd_fused_split")
-    elif gate_logits is not None:
+    if gate_logits is not None:
         if head_gates or states_out is not None or first_launch_only:
             raise ValueError("gate logits: per-key gates, forward without kept states")
         normalizer, clamp_min = gate_logits
@@ -518,16 +491,7 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
             be.ptr(idx), be.ptr(co), NT, be.dt(q), be.dt(g), B, T, H, K, V, N, float(scale), be.stream_of(q))
     outs = (be.ptr(dhtf), be.ptr(dq), be.ptr(dk), be.ptr(dv), be.ptr(dg))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(do), be.ptr(dht), be.ptr(hT))
-    split = None
-    if kept and kh is not None:
-        split = scan_split(plan, N, T, H, V // 32, True, _MIN_SAVED_CHUNKS_TRAINING)
-    if split is not None:
-        st = q.new_empty(split.slots, H, K, V, dtype=torch.float32)
-        dec = q.new_empty(split.slots, H, K, dtype=torch.float32)
-        be.check(be.lib().fla_chunk_gla_bwd_split(
-            *head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs, *tail[:5],
-            ctypes.byref(split.bind(st, dec)), *tail[5:-1], int(head_gates), tail[-1]), "fla_chunk_gla_bwd_split")
-    elif kept and head_gates:
+    if kept and head_gates:
         be.check(be.lib().fla_chunk_simple_gla_bwd(*head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs,
                                                    *tail[:7], *tail[8:]),
                  "fla_chunk_simple_gla_bwd")
@@ -599,6 +563,8 @@ def chunk_gla_bwd(q, k, v, g, g_cumsum, scale, initial_state, h, A, do, dht,
 
 
 class ChunkGLAFunction(torch.autograd.Function):
+    """A differentiated pass that keeps nothing but its inputs (``KEEP_STATES_FOR_BACKWARD = False``): the backward starts
+    by recomputing the per-chunk states like the reference."""
 
     @staticmethod
     @contiguous
@@ -625,13 +591,9 @@ class ChunkGLAFunction(torch.autograd.Function):
                 h0 = F.pad(h0, (0, VP - V, 0, KP - K))
         needs_grad = any(ctx.needs_input_grad)
         flags = [] if needs_grad else None   # the backward pass reads the guard's flags
-        states = [] if KEEP_STATES_FOR_BACKWARD and needs_grad else None
-        o, ht, _ = _gla_forward(q, k, v, g, scale, h0, output_final_state, offsets, flags_out=flags,
-                                states_out=states)
-        # the inputs, the small table of chunks whose gates need the exact intra-chunk arithmetic, and
-        # (unless recomputation is asked for) the per-chunk states the fused launch wrote on its way
-        kept = tuple(states) + (None,) * (5 - len(states)) if states else (None,) * 5
-        ctx.save_for_backward(q, k, v, g, h0, offsets, flags[0] if flags else None, *kept)
+        o, ht, _ = _gla_forward(q, k, v, g, scale, h0, output_final_state, offsets, flags_out=flags)
+        # the inputs and the small table of chunks whose gates need the exact intra-chunk arithmetic
+        ctx.save_for_backward(q, k, v, g, h0, offsets, flags[0] if flags else None)
         ctx.scale, ctx.head_first, ctx.dims, ctx.in_dtypes = scale, head_first, (K, V, KP, VP), in_dtypes
         ctx.h0_dtype = None if initial_state is None else initial_state.dtype
         if (KP, VP) != (K, V):
@@ -646,7 +608,7 @@ class ChunkGLAFunction(torch.autograd.Function):
     @staticmethod
     @contiguous
     def backward(ctx, do, dht):
-        q, k, v, g, h0, offsets, wide, hT, qg, decay, kh, scores = ctx.saved_tensors
+        q, k, v, g, h0, offsets, wide = ctx.saved_tensors
         K, V, KP, VP = ctx.dims
         if ctx.head_first:
             do = do.transpose(1, 2)
@@ -656,8 +618,7 @@ class ChunkGLAFunction(torch.autograd.Function):
         do = do.contiguous()
         if dht is not None and (KP, VP) != (K, V):
             dht = F.pad(dht, (0, VP - V, 0, KP - K))
-        dq, dk, dv, dg, dh0 = chunk_gla_bwd_device(q, k, v, g, ctx.scale, h0, do, dht, offsets, wide, hT=hT, qg=qg,
-                                                   decay=decay, kh=kh, scores=scores)
+        dq, dk, dv, dg, dh0 = chunk_gla_bwd_device(q, k, v, g, ctx.scale, h0, do, dht, offsets, wide)
         if (KP, VP) != (K, V):
             dq, dk, dg, dv = dq[..., :K], dk[..., :K], dg[..., :K], dv[..., :V]
             if dh0 is not None:
@@ -670,24 +631,41 @@ class ChunkGLAFunction(torch.autograd.Function):
         return dq.to(qd), dk.to(kd), dv.to(vd), dg.to(gd), None, dh0, None, None, None
 
 
-def _direct_launch_ok(q, k, v, g, initial_state, head_first) -> bool:
-    """True when a call can go straight to the fused launch: no operand takes part in autograd, and every
-    operand already has the layout, dtype and head dims the kernel reads (seq-first, contiguous, one 16-bit
-    dtype, fp32 or 16-bit gates, fp32 state, built tile sizes).  Anything else takes the autograd function,
-    which converts and pads."""
-    if head_first or q.dtype not in (torch.bfloat16, torch.float16) or k.dtype != q.dtype or v.dtype != q.dtype:
-        return False
-    if g.dtype != torch.float32 and g.dtype != q.dtype:
-        return False
-    if (q.shape[-1], v.shape[-1]) not in _SUPPORTED_KV:
-        return False
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad or g.requires_grad or
-                                    (initial_state is not None and initial_state.requires_grad)):
-        return False
-    if not (q.is_cuda and k.is_cuda and v.is_cuda and g.is_cuda and q.is_contiguous() and k.is_contiguous()
-            and v.is_contiguous() and g.is_contiguous()):
-        return False
-    return initial_state is None or (initial_state.dtype == torch.float32 and initial_state.is_contiguous())
+def _needs_grad(*tensors) -> bool:
+    return torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors)
+
+
+def _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first):
+    """16-bit q with K, V <= 128 in any layout: converted to what the host extension takes (seq-first, one dtype, head
+    dims 64 or 128, fp32 state) by differentiable torch operations, and the results back."""
+    be.require_gpu(q, k, v, g)
+    K, V, v_dtype = q.shape[-1], v.shape[-1], v.dtype
+    KP, VP = _round64(K), _round64(V)
+    if (KP, VP) not in _SUPPORTED_KV:
+        raise NotImplementedError(f"fla_amd chunk_gla: head dims K={K}, V={V} are outside the built tiles "
+                                  f"{sorted(_SUPPORTED_KV)} (after rounding up to multiples of 64)")
+    if q.dtype not in (torch.bfloat16, torch.float16):
+        raise NotImplementedError(f"fla_amd chunk_gla kernels: q must be bf16 or fp16, got {q.dtype}")
+    if head_first:
+        q, k, v, g = (x.transpose(1, 2) for x in (q, k, v, g))
+    k, v = k.to(q.dtype), v.to(q.dtype)
+    g = g if g.dtype in (torch.float32, q.dtype) else g.float()
+    h0 = None if initial_state is None else initial_state.float()
+    q, k, g, v = _pad_dim(q, KP), _pad_dim(k, KP), _pad_dim(g, KP), _pad_dim(v, VP)
+    if h0 is not None and (KP, VP) != (K, V):
+        h0 = F.pad(h0, (0, VP - V, 0, KP - K))
+    res = host().chunk_gla(q, k, v, g, scale, h0, output_final_state, native_plan(offsets), True, KEEP_KHAT_AND_SCORES,
+                           None, None)
+    if res is None:
+        raise ValueError(f"fla_amd chunk_gla: inconsistent operands q {tuple(q.shape)}, k {tuple(k.shape)}, "
+                         f"v {tuple(v.shape)}, g {tuple(g.shape)}")
+    o, ht = res
+    if VP != V:
+        o = o[..., :V]
+    if ht is not None and (KP, VP) != (K, V):
+        ht = ht[..., :K, :V].contiguous()
+    o = o.to(v_dtype)
+    return (o.transpose(1, 2).contiguous() if head_first else o), ht
 
 
 def _chunk_gla_fp32(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first):
@@ -754,17 +732,20 @@ def chunk_gla(
     Returns ``(o, final_state)``.
     """
     offsets = resolve_offsets(offsets, cu_seqlens)
+    if offsets is not None:
+        check_varlen_args(q, offsets, head_first, initial_state)
+    if not head_first:
+        # seq-first operands as the kernels read them: nothing left to do in Python
+        res = host().chunk_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
+                               KEEP_STATES_FOR_BACKWARD, KEEP_KHAT_AND_SCORES, gate_logit_normalizer, gate_clamp_min)
+        if res is not None:
+            return res
     if gate_logit_normalizer is not None:
         from ...modules.gate_activations import gla_gate
-        if (q.numel() and q.dtype != torch.float32 and q.shape[-1] in (64, 128) and v.shape[-1] <= 128
-                and _direct_launch_ok(q, k, v, g, initial_state, head_first)):
-            check_varlen_args(q, offsets, head_first, initial_state)
-            return chunk_gla_fwd_fused(q, k, v, g, q.shape[-1] ** -0.5 if scale is None else scale, initial_state,
-                                       output_final_state, offsets,
-                                       gate_logits=(gate_logit_normalizer, gate_clamp_min))
         g = gla_gate(g, gate_logit_normalizer, gate_clamp_min,
                      output_dtype=torch.float32 if q.dtype != torch.float32 else None)
-    check_varlen_args(q, offsets, head_first, initial_state)
+        return chunk_gla(q, k, v, g, scale=scale, initial_state=initial_state, output_final_state=output_final_state,
+                         offsets=offsets, head_first=head_first)
     if scale is None:
         scale = q.shape[-1] ** -0.5
     if q.numel() == 0:
@@ -792,13 +773,11 @@ def chunk_gla(
         outs, states = [], []
         for v0 in range(0, V, 128):
             h0 = None if initial_state is None else initial_state[..., v0:v0 + 128]
-            o, ht = ChunkGLAFunction.apply(q, k, v[..., v0:v0 + 128], g, scale, h0, output_final_state, offsets,
-                                           head_first)
+            o, ht = chunk_gla(q, k, v[..., v0:v0 + 128], g, scale=scale, initial_state=h0,
+                              output_final_state=output_final_state, offsets=offsets, head_first=head_first)
             outs.append(o)
             states.append(ht)
         return torch.cat(outs, dim=-1), (torch.cat(states, dim=-1) if output_final_state else None)
-    if _direct_launch_ok(q, k, v, g, initial_state, head_first):
-        # nothing to differentiate and nothing to convert: no autograd node, no copies
-        return chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets)
-    o, final_state = ChunkGLAFunction.apply(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first)
-    return o, final_state
+    if _needs_grad(q, k, v, g, initial_state) and (not KEEP_STATES_FOR_BACKWARD or float(scale) == 0.0):
+        return ChunkGLAFunction.apply(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first)
+    return _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first)

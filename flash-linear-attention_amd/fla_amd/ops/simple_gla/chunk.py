@@ -13,7 +13,8 @@ import torch
 import os
 
 from ... import _backend as be
-from ...utils import VarlenPlan, check_varlen_args, contiguous, resolve_offsets
+from ..._native import host
+from ...utils import VarlenPlan, check_varlen_args, contiguous, native_plan, resolve_offsets
 from ..gla import chunk as gla_chunk
 from ..gla.chunk import chunk_gla, chunk_gla_bwd_device, chunk_gla_fwd_fused
 
@@ -109,7 +110,13 @@ def chunk_simple_gla(
     Returns ``(o, final_state)``.
     """
     offsets = resolve_offsets(offsets, cu_seqlens)
-    check_varlen_args(q, offsets, head_first, initial_state)
+    if offsets is not None:
+        check_varlen_args(q, offsets, head_first, initial_state)
+    if SCAN_FORWARD and not head_first:
+        res = host().chunk_simple_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
+                                      gla_chunk.KEEP_STATES_FOR_BACKWARD, gla_chunk.KEEP_KHAT_AND_SCORES)
+        if res is not None:
+            return res
     if scale is None:
         scale = k.shape[-1] ** -0.5
     K = k.shape[-1]

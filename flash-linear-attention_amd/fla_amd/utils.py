@@ -114,8 +114,7 @@ class VarlenPlan:
         self.indices = idx.to(dev, non_blocking=True)
         self.chunk_offsets = co.to(dev, non_blocking=True)
         self.N = len(host) - 1
-        self.host = host
-        self._splits = {}
+        self._host, self._native = host, None
         self.NT = idx.shape[0]
         # sequence ids, longest first: the order in which the serial scan kernels start sequences
         lens = [host[i + 1] - host[i] for i in range(self.N)]
@@ -123,57 +122,18 @@ class VarlenPlan:
         self.seq_order = torch.tensor(order, dtype=torch.int64).to(dev, non_blocking=True)
 
 
-    def split(self, H: int, slabs: int, reverse: bool, min_saved: int):
-        """The segments a scan over this batch is cut into (:func:`scan_split`), with their device tables."""
-        key = (H, slabs, reverse, min_saved)
-        if key not in self._splits:
-            self._splits[key] = self._build_split(*key)
-        return self._splits[key]
-
-    def _build_split(self, H, slabs, reverse, min_saved):
-        arr = (ctypes.c_int64 * (self.N + 1))(*self.host)
-        sp = be.Split()
-        args = (arr, self.N, 0, H, slabs, int(reverse), min_saved, ctypes.byref(sp))
-        if self.N == 0 or not be.lib().fla_scan_split(*args, None, None, None):
-            return None
-        tables = [torch.empty(2 * sp.nseg, dtype=torch.int32), torch.empty(2 * sp.nsub, dtype=torch.int32),
-                  torch.empty(self.N + 1, dtype=torch.int32)]
-        be.lib().fla_scan_split(*args, *(ctypes.c_void_p(t.data_ptr()) for t in tables))
-        dev = self.offsets.device
-        return ScanSplit(sp, [t.to(dev, non_blocking=True) for t in tables])
+    @property
+    def native(self):
+        """The plan as the host extension takes it."""
+        if self._native is None:
+            from ._native import host
+            self._native = host().plan(self.offsets, self.indices, self.chunk_offsets, self.seq_order,
+                                       torch.tensor(self._host, dtype=torch.int64))
+        return self._native
 
 
-class ScanSplit:
-    """Integers (and, for a packed batch, device tables) of ``fla_split``; :meth:`bind` adds one call's workspaces."""
-
-    def __init__(self, sp, tables=()):
-        self.ints = (sp.sub_chunks, sp.ratio, sp.nseg, sp.nsub, sp.slots, 0)
-        self.slots = sp.slots
-        self.tables = tables
-        self.table_ptrs = tuple(t.data_ptr() for t in tables) or (None, None, None)
-
-    def bind(self, states, transitions):
-        return be.Split(*self.ints, *self.table_ptrs, states.data_ptr(), transitions.data_ptr())
-
-
-@functools.lru_cache(maxsize=256)
-def _uniform_split(N: int, T: int, H: int, slabs: int, reverse: bool, min_saved: int):
-    sp = be.Split()
-    if not be.lib().fla_scan_split(None, N, T, H, slabs, int(reverse), min_saved, ctypes.byref(sp), None, None, None):
-        return None
-    return ScanSplit(sp)
-
-
-# Chunk periods (1.5 - 3 us each) that cutting has to take off a scan: the two launches ahead of it and its two workspaces
-# are 12 us on the device and the host (42 -> 33 us for a forward of 16 chunks cut into 4, B=1, H=16, K=V=128).
-MIN_SAVED_CHUNKS = 8
-
-
-def scan_split(plan, N: int, T: int, H: int, slabs: int, reverse: bool = False, min_saved: int = MIN_SAVED_CHUNKS):
-    """How a scan of ``slabs`` workgroups per (sequence, head) cuts its sequences, or ``None`` where it does not."""
-    if plan is None:
-        return _uniform_split(N, T, H, slabs, reverse, min_saved)
-    return plan.split(H, slabs, reverse, min_saved)
+def native_plan(offsets: Optional[torch.Tensor], chunk_size: int = 64):
+    return None if offsets is None else VarlenPlan(offsets, chunk_size).native
 
 
 def resolve_offsets(offsets: Optional[torch.Tensor], cu_seqlens: Optional[torch.Tensor]):

@@ -2,6 +2,8 @@
 recurrences.  The gates are weak, so that the state entering a segment decides its output, and the lengths leave short
 last chunks, short last segments and, in packed batches, sequences shorter than a segment.  Tolerances are those of the
 uncut operators (16-bit operands, fp32 sums): 1e-2 on o, 5e-3 on the final state, 2e-2 on the gradients."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -12,10 +14,12 @@ from oracle.recurrent import naive_recurrent_gated_delta_rule, naive_recurrent_g
 pytestmark = pytest.mark.gpu
 
 
-def _cut(B, T, H, slabs, reverse, offsets, device):
-    from fla_amd.utils import VarlenPlan, scan_split
-    plan = None if offsets is None else VarlenPlan(offsets, 64)
-    return scan_split(plan, B if plan is None else plan.N, T, H, slabs, reverse)
+def _cut(N, T, H, slabs, reverse, bounds):
+    """Whether the launches cut this batch."""
+    from fla_amd import _backend as be
+    sp = be.Split()
+    arr = None if bounds is None else (ctypes.c_int64 * len(bounds))(*bounds)
+    return be.lib().fla_scan_split(arr, N, T, H, slabs, int(reverse), 8, ctypes.byref(sp), None, None, None)
 
 
 CASES = [
@@ -30,15 +34,12 @@ CASES = [
 
 @pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", CASES)
 @pytest.mark.parametrize("heads", [False, True])
-def test_gla_cut_sequences(device, monkeypatch, B, T, H, K, V, bounds, dtype, heads):
-    import fla_amd.ops.gla.chunk as gla_mod
+def test_gla_cut_sequences(device, B, T, H, K, V, bounds, dtype, heads):
     from fla_amd.ops.gla import chunk_gla
-    monkeypatch.setattr(gla_mod, "_MIN_SAVED_CHUNKS_TRAINING", 8)
     from fla_amd.ops.simple_gla import chunk_simple_gla
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(B, T, H, V // 64, False, offs, device) is not None
-    assert _cut(B, T, H, V // 32, True, offs, device) is not None
+    assert _cut(N, T, H, V // 64, False, bounds) and _cut(N, T, H, V // 32, True, bounds)
     print("cut", B, T, H, K, V, bounds, dtype, heads, flush=True)
     q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
     if heads:
@@ -68,8 +69,7 @@ def test_gla_cut_gate_logits_and_strong_gates(device):
     q, k, v, _, h0 = gla_inputs(1, 1100, 2, 128, 128, seed=5)
     x = torch.randn(1, 1100, 2, 128)
     x[:, 300:330] -= 40.0
-    offs = None
-    assert _cut(1, 1100, 2, 2, False, offs, device) is not None
+    assert _cut(1, 1100, 2, 2, False, None)
     print("cut, gate logits", flush=True)
     with torch.no_grad():
         o, ht = chunk_gla(*(t.to(device) for t in (q, k, v, x)), initial_state=h0.to(device), output_final_state=True,
