@@ -55,12 +55,20 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // has a CU of its own, so the segments are as short as 256 CUs allow (GLA forward of 16 heads x 8192 tokens, K = V = 128:
 // 4, 8, 16 and 32 segments 112, 80, 86 and 111 us, uncut 293).  The first pass gets about as many workgroups as there are
 // CUs: 1, 2 and 4 sub-blocks per segment of that forward 94, 80 and 84 us, of one of 64 pairs in two segments 169, 136 and
-// 125 us (uncut 155).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands: the
-// caller says how many chunk periods it has to save.
+// 125 us (uncut 155).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands,
+// which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us).
+//
+// The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 1.2 us per
+// segment, so it takes longer segments and only batches that fall into at least kMinSegments of them (forward of K = V = 128,
+// 16 heads, uncut against cut in us: one sequence of 5003 tokens in 8 segments 119 / 74, of 16384 in 8 359 / 163, of 8192
+// with 4 heads in 32, 16 and 8 segments 175 / 76, 63 and 74; two of 4096 in 4 segments 105 / 94, four in 2 127 / 158).  A
+// forward that keeps its intermediates is longer by the stores and gains less: two sequences of 2048 in 4 segments 58 / 60.
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
-                              int64_t min_saved, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
-  constexpr int64_t kCUs = 256, kChunk = 64, kMinSeg = 4, kPassWorkgroups = 256;
-  if (!out || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
+                              int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
+  constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
+  const bool delta = kind != FLA_SCAN_GLA;
+  const int64_t kMinSeg = delta ? 8 : 4, kMinSaved = delta ? 16 : 8, kMinSegments = kind == FLA_SCAN_DELTA_KEPT ? 6 : delta ? 3 : 2;
+  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_DELTA_KEPT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
   int64_t longest = 0, total = 0;
   for (int64_t n = 0; n < N; ++n) {
@@ -82,10 +90,12 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   int64_t seg = fla_cdiv(total, room);
   seg = seg < kMinSeg ? kMinSeg : seg;
   while (segments(seg) > room) ++seg;
-  if (longest - seg < min_saved) return 0;
+  if (longest - seg < kMinSaved || longest < (kMinSegments - 1) * seg + 1) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;
-  ratio = ratio < 1 ? 1 : ratio > seg / 2 ? seg / 2 : ratio;
+  ratio = ratio > seg / 2 ? seg / 2 : ratio;
+  if (delta) ratio = 1;
+  ratio = ratio < 1 ? 1 : ratio;
   const int64_t sub = fla_cdiv(seg, ratio);
   ratio = fla_cdiv(seg, sub);
   out->sub_chunks = (int32_t)sub;

@@ -35,7 +35,7 @@
 // the halves (state) or neighbouring rows of 16 lanes (v_new) pairs them up into 16-byte stores (a store
 // instruction costs the CU's memory pipeline the same whatever its width, and that pipeline is what bounds
 // the scan).
-#include "chunk_common.h"
+#include "seq_split.h"
 
 namespace {
 
@@ -62,6 +62,7 @@ struct GdrScanParams {
   float scale;
   float l2_eps;     // L2N: q and k are un-normalised; the launch works with x / sqrt(sum x^2 + l2_eps) ...
   const float* rk;  //      ... the factors of k, fp32 [rows, H], come from fla_gdr_fwd_prep_l2norm
+  SplitView split;  // sequences cut into segments (ratio 0: not)
 };
 
 // Two 4-element results per lane (16-bit after conversion) -> one 8-element vector per lane: lanes 0-31 keep
@@ -146,12 +147,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const ScanItem wi = scan_item(nvb);
   const int vb = wi.slab;
   const int hh = (int)(wi.item % H);
-  const int n = p.seq_order ? (int)p.seq_order[wi.item / H] : (int)(wi.item / H);
-  const int nh = n * H + hh;
   const int vbase = vb * BV;
-  SeqSpan sp = seq_span(p.offsets, n, p.T);
-  const int nchunks = (int)((sp.len + BT - 1) / BT);
-  const int64_t chunk0 = p.chunk_offsets ? p.chunk_offsets[n] : (int64_t)n * ((p.T + BT - 1) / BT);
+  const ScanSpan span = scan_span<false>(p.split, wi.item / H, p.seq_order, p.offsets, p.chunk_offsets, p.T);
+  const int nh = span.n * H + hh;
+  const SeqSpan sp = span.sp;
+  const int nchunks = (int)span.nchunks;
+  const int64_t chunk0 = span.chunk0;
+  // the state entering this workgroup's chunks
+  const float* hin = p.split.ratio ? p.split.states + (span.slot * H + hh) * (int64_t)K * V
+                     : p.h0        ? p.h0 + (int64_t)nh * K * V
+                                   : nullptr;
 
   // Aqk = scale tril(q k^T * Gamma) of the chunk whose tiles are in buffer b, shared out over waves 0-3 by 16x16
   // block: a block is computed transposed (k rows against q rows), which leaves every lane with four
@@ -473,8 +478,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       acc[kt] = zero4();
-      if (p.h0) {
-        const float* h0p = p.h0 + (int64_t)nh * K * V + vbase + cb + c;
+      if (hin) {
+        const float* h0p = hin + vbase + cb + c;
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[kt][r] = h0p[(int64_t)(16 * kt + 4 * g + r) * V];
       }
@@ -692,7 +697,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         b3 = n3;
       }
     }
-    if (p.ht) {
+    if (p.ht && span.last) {
       float* htp = p.ht + (int64_t)nh * K * V + vbase + cb + c;
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
@@ -704,7 +709,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 template <typename T>
 int launch_scan(const GdrScanParams& p, int K, hipStream_t st) {
-  int64_t nblk = (int64_t)p.N * p.H * (p.V / 64);
+  // (sequence, head) pairs, or (segment, head) pairs of sequences cut into segments
+  const int64_t seqs = !p.split.ratio ? p.N : p.split.seg_table ? p.split.nseg : (int64_t)p.split.nseg * p.N;
+  int64_t nblk = seqs * p.H * (p.V / 64);
   FLA_REQUIRE(nblk <= 0x7fffffffLL / 2, FLA_E_UNSUPPORTED);
   if (nblk == 0) return FLA_OK;
   // 32-column slabs while they still give every workgroup a CU of its own
@@ -754,7 +761,8 @@ static int gdr_fwd_scan_impl(const void* q, const void* k, const void* v, const 
                              const float* h0, void* o, float* ht, void* v_new, void* h_frag_t, void* Aqk_out,
                              const int64_t* offsets, const int64_t* chunk_offsets, const int64_t* seq_order,
                              int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N,
-                             float scale, float l2_eps, fla_stream_t stream, const float* k_rstd = nullptr) {
+                             float scale, float l2_eps, fla_stream_t stream, const float* k_rstd = nullptr,
+                             const fla_split* split = nullptr) {
   FLA_REQUIRE(q && k && v && o, FLA_E_INVALID);   // AT == NULL: the plain scan (fla_chunk_simple_gla_fwd_scan)
   FLA_REQUIRE((l2_eps >= 0.f) == (k_rstd != nullptr), FLA_E_INVALID);
   FLA_REQUIRE(B >= 0 && T >= 0 && H > 0 && K > 0 && V > 0 && N >= 0, FLA_E_INVALID);
@@ -765,7 +773,14 @@ static int gdr_fwd_scan_impl(const void* q, const void* k, const void* v, const 
   FLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)AT | (uintptr_t)o | (uintptr_t)v_new |
                (uintptr_t)h_frag_t | (uintptr_t)Aqk_out) % 16 == 0, FLA_E_ALIGNMENT);
   GdrScanParams p{q, k, v, AT, g_cumsum, h0, o, ht, v_new, h_frag_t, Aqk_out, offsets, chunk_offsets, seq_order, T,
-                  (int)H, (int)V, (int)N, scale, l2_eps, k_rstd};
+                  (int)H, (int)V, (int)N, scale, l2_eps, k_rstd, split_view(split)};
+  if (split) {
+    const int rc = AT ? gdr_split_states(k, v, AT, g_cumsum, k_rstd, h0, split, offsets, chunk_offsets, qkv_dtype, T, H, K, V, N,
+                                         (hipStream_t)stream)
+                      : gla_split_states(k, v, g_cumsum, h0, split, true, false, false, 1.f, 0.f, 1.f, offsets, chunk_offsets,
+                                         qkv_dtype, FLA_F32, T, H, K, V, N, (hipStream_t)stream);
+    if (rc) return rc;
+  }
   if (qkv_dtype == FLA_BF16) return launch_scan<bf16>(p, (int)K, (hipStream_t)stream);
   if (qkv_dtype == FLA_F16) return launch_scan<f16>(p, (int)K, (hipStream_t)stream);
   return FLA_E_UNSUPPORTED;
@@ -801,4 +816,17 @@ extern "C" int fla_chunk_simple_gla_fwd_scan(const void* q, const void* k, const
                                              float scale, fla_stream_t stream) {
   return gdr_fwd_scan_impl(q, k, v, nullptr, g, h0, o, ht, nullptr, nullptr, nullptr, offsets, chunk_offsets,
                            seq_order, qkv_dtype, B, T, H, K, V, N, scale, -1.f, stream);
+}
+
+extern "C" int fla_chunk_gated_delta_rule_fwd_scan_split(const void* q, const void* k, const void* v, const void* AT,
+                                                         const float* gates, const float* k_rstd, const float* h0, void* o,
+                                                         float* ht, void* v_new, void* h_frag_t, void* Aqk_out,
+                                                         const int64_t* offsets, const int64_t* chunk_offsets,
+                                                         const fla_split* split, int qkv_dtype, int64_t B, int64_t T,
+                                                         int64_t H, int64_t K, int64_t V, int64_t N, float scale, float eps,
+                                                         fla_stream_t stream) {
+  FLA_REQUIRE(split && (AT || gates), FLA_E_INVALID);
+  FLA_REQUIRE(K <= 128 && V <= 128, FLA_E_UNSUPPORTED);
+  return gdr_fwd_scan_impl(q, k, v, AT, gates, h0, o, ht, v_new, h_frag_t, Aqk_out, offsets, chunk_offsets, nullptr, qkv_dtype, B,
+                           T, H, K, V, N, scale, k_rstd ? eps : -1.f, stream, k_rstd, split);
 }

@@ -113,3 +113,8 @@ int gla_split_states(const void* a, const void* b, const void* g, const float* i
                      bool reverse, bool logits, float gate_inv_norm, float gate_clamp_min, float scale,
                      const int64_t* offsets, const int64_t* chunk_offsets, int qkv_dtype, int gate_dtype, int64_t T,
                      int64_t H, int64_t K, int64_t V, int64_t N, hipStream_t st);
+
+// gdr_split.hip: the two launches ahead of a delta-rule scan over cut sequences (segments of one sub-block).
+int gdr_split_states(const void* k, const void* v, const void* AT, const float* g_cumsum, const float* k_rstd, const float* init,
+                     const fla_split* split, const int64_t* offsets, const int64_t* chunk_offsets, int qkv_dtype, int64_t T,
+                     int64_t H, int64_t K, int64_t V, int64_t N, hipStream_t st);

@@ -29,9 +29,6 @@ using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 constexpr int64_t BT = 64;
-// Chunk periods (1.5 - 3 us each) that cutting its sequences has to take off a scan: the two launches ahead of the scan and
-// its workspaces are about 12 us on the device (42 -> 33 us for a GLA forward of 16 chunks cut into 4, B=1, H=16, K=V=128).
-constexpr int64_t kMinSavedChunks = 8;
 
 // ---------------------------------------------------------------------------------------------------- helpers
 void check(int code, const char* what) {
@@ -102,17 +99,17 @@ struct Plan : torch::CustomClassHolder {
   std::vector<int64_t> host;
   int64_t N = 0, NT = 0;
   std::mutex mu;
-  std::map<std::tuple<int64_t, int, bool>, SplitTables> splits;
+  std::map<std::tuple<int64_t, int, bool, int>, SplitTables> splits;
 
   // The tables of a cut are used by later calls on any stream: the copies to the device are synchronous.
-  SplitTables split(int64_t H, int slabs, bool reverse) {
+  SplitTables split(int64_t H, int slabs, bool reverse, int kind) {
     std::lock_guard<std::mutex> lock(mu);
-    auto [it, fresh] = splits.try_emplace({H, slabs, reverse});
+    auto [it, fresh] = splits.try_emplace({H, slabs, reverse, kind});
     SplitTables& s = it->second;
     if (fresh && N > 0) {
       fla_split sp{};
       auto plan = [&](int32_t* a, int32_t* b, int32_t* c) {
-        return fla_scan_split(host.data(), N, 0, H, slabs, reverse, kMinSavedChunks, &sp, a, b, c);
+        return fla_scan_split(host.data(), N, 0, H, slabs, reverse, kind, &sp, a, b, c);
       };
       if (plan(nullptr, nullptr, nullptr)) {
         auto opts = at::TensorOptions().dtype(at::kInt);
@@ -145,13 +142,13 @@ struct Cut {
   Tensor states, transitions;
 };
 std::optional<Cut> cut_scan(const PlanPtr& plan, int64_t N, int64_t T, int64_t H, int slabs, bool reverse, const Tensor& like,
-                            int64_t state_elems, int64_t transition_elems) {
+                            int64_t state_elems, int64_t transition_elems, int kind = FLA_SCAN_GLA) {
   Cut c;
   if (plan) {
-    c.tables = plan->split(H, slabs, reverse);
+    c.tables = plan->split(H, slabs, reverse, kind);
     if (!c.tables.cut) return std::nullopt;
     c.s = c.tables.ints;
-  } else if (!fla_scan_split(nullptr, N, T, H, slabs, reverse, kMinSavedChunks, &c.s, nullptr, nullptr, nullptr)) {
+  } else if (!fla_scan_split(nullptr, N, T, H, slabs, reverse, kind, &c.s, nullptr, nullptr, nullptr)) {
     return std::nullopt;
   }
   c.states = fresh({c.s.slots * H * state_elems}, like, at::kFloat);
@@ -319,6 +316,13 @@ Tensor simple_gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const 
   const Dims& d = a.d;
   Tensor o = fresh_like(v);
   if (a.want_ht) *ht = fresh({d.N, d.H, d.K, d.V}, q, at::kFloat);
+  if (auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K)) {
+    check(fla_chunk_gated_delta_rule_fwd_scan_split(ptr(q), ptr(k), ptr(v), nullptr, fptr(g), nullptr, fptr(h0), ptr(o),
+                                                    fptr(*ht), nullptr, nullptr, nullptr, offs(a.plan), coff(a.plan), &c->s,
+                                                    dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale, 0.f, stream_of(q)),
+          "fla_chunk_gated_delta_rule_fwd_scan_split");
+    return o;
+  }
   check(fla_chunk_simple_gla_fwd_scan(ptr(q), ptr(k), ptr(v), fptr(g), fptr(h0), ptr(o), fptr(*ht), offs(a.plan),
                                       coff(a.plan), order(a.plan), dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale,
                                       stream_of(q)),
@@ -346,11 +350,25 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   Tensor gc = g.defined() ? fresh_like(g) : Tensor();
   Tensor o = fresh_like(v);
   if (a.want_ht) *ht = fresh({d.N, d.H, d.K, d.V}, q, at::kFloat);
+  // sequences cut into segments: their K x K transitions take the place of the decays
+  const auto cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K * d.K,
+                            kept ? FLA_SCAN_DELTA_KEPT : FLA_SCAN_DELTA);
+  auto scan_cut = [&](const Tensor& rstd, const GdrKept& x) {
+    check(fla_chunk_gated_delta_rule_fwd_scan_split(ptr(q), ptr(k), ptr(v), ptr(AT), fptr(gc), fptr(rstd), fptr(h0), ptr(o),
+                                                    fptr(*ht), ptr(x.v_new), ptr(x.hT), ptr(x.Aqk), offs(a.plan), coff(a.plan),
+                                                    &cut->s, dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale,
+                                                    (float)a.l2norm_eps.value_or(0.0), st),
+          "fla_chunk_gated_delta_rule_fwd_scan_split");
+  };
   if (a.l2norm_eps) {
     Tensor rstd = fresh({d.B, d.T, d.H}, q, at::kFloat);
     check(fla_gdr_fwd_prep_l2norm(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), fptr(rstd), offs(a.plan), idx(a.plan),
                                   d.NT, dt(q), d.B, d.T, d.H, d.K, (float)*a.l2norm_eps, st),
           "fla_gdr_fwd_prep_l2norm");
+    if (cut) {
+      scan_cut(rstd, {});
+      return o;
+    }
     check(fla_chunk_gated_delta_rule_fwd_scan_l2norm(ptr(q), ptr(k), ptr(v), ptr(AT), fptr(gc), fptr(rstd), fptr(h0), ptr(o),
                                                      fptr(*ht), offs(a.plan), coff(a.plan), order(a.plan), dt(q), d.B, d.T,
                                                      d.H, d.K, d.V, d.N, (float)a.scale, (float)*a.l2norm_eps, st),
@@ -369,6 +387,10 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   check(fla_gdr_fwd_prep(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), ptr(x.w), ptr(x.Aw), offs(a.plan), idx(a.plan),
                          d.NT, dt(q), d.B, d.T, d.H, d.K, st),
         "fla_gdr_fwd_prep");
+  if (cut) {
+    scan_cut({}, x);
+    return o;
+  }
   check(fla_chunk_gated_delta_rule_fwd_scan(ptr(q), ptr(k), ptr(v), ptr(AT), fptr(gc), fptr(h0), ptr(o), fptr(*ht),
                                             ptr(x.v_new), ptr(x.hT), ptr(x.Aqk), offs(a.plan), coff(a.plan), order(a.plan),
                                             dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale, st),

@@ -35,7 +35,7 @@ SIGNATURES = {
     "fla_error_string": (c_char_p, [c_int]),
     "fla_count_chunks": (c_int64, [P, I64, I64]),
     "fla_prepare_chunk_indices": (c_int, [P, I64, I64, P, P]),
-    "fla_scan_split": (c_int, [P, I64, I64, I64, I, I, I64, P, P, P, P]),
+    "fla_scan_split": (c_int, [P, I64, I64, I64, I, I, I, P, P, P, P]),
     "fla_chunk_local_cumsum": (c_int, [P, P, I, I64, I64, I64, I64, I64, I, P, P, I64, P]),
     "fla_chunk_local_cumsum_inverse": (c_int, [P, P, I64, I64, I64, I64, I64, I, P, P, I64, P]),
     "fla_chunk_global_cumsum": (c_int, [P, P, P, I, I, I64, I64, I64, I64, I64, I, P, P, I64, P]),
@@ -62,6 +62,7 @@ SIGNATURES = {
     "fla_chunk_gated_delta_rule_fwd_h": (c_int, [P, P, P, P, P, P, P, P, P, P, I, I, I,
                                                  I64, I64, I64, I64, I64, I64, P]),
     "fla_chunk_gated_delta_rule_fwd_h_both": (c_int, [P] * 11 + [I, I64, I64, I64, I64, I64, I64, P]),
+    "fla_chunk_gated_delta_rule_fwd_scan_split": (c_int, [P] * 15 + [I, I64, I64, I64, I64, I64, I64, F, F, P]),
     "fla_gdr_fwd_prep": (c_int, [P, P, P, I, P, P, P, P, P, P, I64, I, I64, I64, I64, I64, P]),
     "fla_chunk_gated_delta_rule_fwd_scan": (c_int, [P] * 14 + [I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_simple_gla_fwd_scan": (c_int, [P] * 10 + [I, I64, I64, I64, I64, I64, I64, F, P]),

@@ -62,8 +62,8 @@ int fla_prepare_chunk_indices(const int64_t* offsets_host, int64_t n_seqs, int64
  * and its transition are formed first, folded into the state entering every segment, and the scan then starts there.
  * Equal-length sequences: nseg segments and nsub sub-blocks each, no tables.  Packed batches: nseg rows of seg_table
  * (sequence, segment), nsub rows of sub_table (sequence, sub-block: those the first pass forms), sub_base [N+1] the first
- * slot of a sequence.  states [slots, H, K, V] and decays [slots, H, K] (GLA) or [slots, H, K, K] (delta rule) are fp32
- * workspaces. */
+ * slot of a sequence.  states [slots, H, K, V] and decays [slots, H, K] (GLA) or its transitions, [slots, H, K, K] words
+ * (delta rule), are workspaces. */
 typedef struct fla_split {
   int32_t sub_chunks, ratio, nseg, nsub, slots, reserved;
   const int32_t* seg_table;
@@ -73,13 +73,15 @@ typedef struct fla_split {
   float* decays;
 } fla_split;
 
+enum fla_scan_kind { FLA_SCAN_GLA = 0, FLA_SCAN_DELTA = 1, FLA_SCAN_DELTA_KEPT = 2 /* keeps its intermediates */ };
+
 /* The plan for N sequences of T tokens (or, with offsets_host [N+1], of a packed batch) and H heads in `slabs` workgroups
- * per (sequence, head), where cutting makes the scan at least min_saved chunks shorter; reverse: for a scan from right
- * to left.  Fills the integer fields and returns 1, or returns 0 where
+ * per (sequence, head); reverse: for a scan from right to left; kind: the recurrence (the delta rule: segments of one
+ * sub-block).  Fills the integer fields and returns 1, or returns 0 where
  * cutting would not pay (host arithmetic, host pointers).  A packed batch's tables are written on a second call with
  * seg_table / sub_table / sub_base given (2 x nseg, 2 x nsub and N+1 words). */
 int fla_scan_split(const int64_t* offsets_host, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
-                   int64_t min_saved, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base);
+                   int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base);
 
 /* ------------------------------------------------------------------------
  * chunk_local_cumsum (fla/ops/utils/cumsum.py:389-407; scalar kernel :24-57,
@@ -329,6 +331,15 @@ int fla_chunk_simple_gla_fwd_scan(const void* q, const void* k, const void* v, c
                                   void* o, float* ht, const int64_t* offsets, const int64_t* chunk_offsets,
                                   const int64_t* seq_order, int qkv_dtype, int64_t B, int64_t T, int64_t H,
                                   int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
+
+/* fla_chunk_gated_delta_rule_fwd_scan (with k_rstd and eps its _l2norm form; with AT == NULL and raw gates
+ * fla_chunk_simple_gla_fwd_scan) on sequences cut into segments (fla_scan_split with V / 64 slabs). */
+int fla_chunk_gated_delta_rule_fwd_scan_split(const void* q, const void* k, const void* v, const void* AT,
+                                              const float* gates, const float* k_rstd, const float* h0, void* o, float* ht,
+                                              void* v_new, void* h_frag_t, void* Aqk_out, const int64_t* offsets,
+                                              const int64_t* chunk_offsets, const fla_split* split, int qkv_dtype, int64_t B,
+                                              int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, float eps,
+                                              fla_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Chunked gated delta rule forward (chunk size 64).  g_cumsum is the fp32

@@ -14,12 +14,12 @@ from oracle.recurrent import naive_recurrent_gated_delta_rule, naive_recurrent_g
 pytestmark = pytest.mark.gpu
 
 
-def _cut(N, T, H, slabs, reverse, bounds):
+def _cut(N, T, H, slabs, reverse, bounds, kind=0):
     """Whether the launches cut this batch."""
     from fla_amd import _backend as be
     sp = be.Split()
     arr = None if bounds is None else (ctypes.c_int64 * len(bounds))(*bounds)
-    return be.lib().fla_scan_split(arr, N, T, H, slabs, int(reverse), 8, ctypes.byref(sp), None, None, None)
+    return be.lib().fla_scan_split(arr, N, T, H, slabs, int(reverse), kind, ctypes.byref(sp), None, None, None)
 
 
 CASES = [
@@ -75,5 +75,67 @@ def test_gla_cut_gate_logits_and_strong_gates(device):
         o, ht = chunk_gla(*(t.to(device) for t in (q, k, v, x)), initial_state=h0.to(device), output_final_state=True,
                           head_first=False, gate_logit_normalizer=8.0)
     ro, rht = naive_recurrent_gla(q, k, v, F.logsigmoid(x) / 8.0, initial_state=h0, output_final_state=True)
+    assert_close("o", ro, o, 1e-2)
+    assert_close("ht", rht, ht, 5e-3)
+
+
+GDR_CASES = [
+    (1, 1601, 1, 64, 64, None, torch.bfloat16),      # 26 chunks, the last of one token
+    (2, 1727, 2, 128, 128, None, torch.bfloat16),    # the last chunk of 63 tokens
+    (1, 1600, 3, 128, 64, None, torch.float16),
+    (1, 2500, 2, 64, 128, [0, 1, 1, 1900, 1964, 2500], torch.bfloat16),
+    (1, 3200, 1, 128, 128, [0, 1790, 1854, 3200], torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", GDR_CASES)
+@pytest.mark.parametrize("gated", [True, False])
+def test_gdr_cut_sequences(device, B, T, H, K, V, bounds, dtype, gated):
+    """A quarter of the keys' corrections and almost no decay: the transition of a segment is far from zero."""
+    from fla_amd.ops.delta_rule import chunk_delta_rule
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    N = B if bounds is None else len(bounds) - 1
+    offs = None if bounds is None else torch.tensor(bounds, device=device)
+    assert _cut(N, T, H, V // 64, False, bounds, 1)
+    print("cut delta rule", B, T, H, K, V, bounds, dtype, gated, flush=True)
+    q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=2000.0, N=N)
+    beta = beta * 0.02
+    dev = [x.to(device) for x in (q, k, v, g, beta, h0)]
+
+    def op(q, k, v, g, beta, h0, **kw):
+        kw.update(initial_state=h0, output_final_state=True, cu_seqlens=offs, head_first=False)
+        return chunk_gated_delta_rule(q, k, v, g, beta, **kw) if gated else chunk_delta_rule(q, k, v, beta, **kw)
+
+    with torch.no_grad():
+        o1, ht1 = op(*dev)
+    leaves = [x.requires_grad_() for x in dev]
+    o, ht = op(*leaves)
+    do, dht = torch.randn(B, T, H, V).to(dtype), torch.randn(N, H, K, V) * 0.1
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    refs = [x.float().requires_grad_() for x in (q, k, v, g, beta, h0)]
+    ro, rht = naive_recurrent_gated_delta_rule(*refs[:3], refs[3] if gated else torch.zeros_like(refs[3]), refs[4],
+                                               initial_state=refs[5], output_final_state=True, offsets=bounds)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for a, b in ((o1, ht1), (o, ht)):
+        assert_close("o", ro, a, 1e-2)
+        assert_close("ht", rht, b, 5e-3)
+    for name, r, d in zip(("dq", "dk", "dv", "dg", "dbeta", "dh0"), refs, leaves):
+        if name != "dg" or gated:
+            assert_close(name, r.grad, d.grad, 2e-2)
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128)])
+def test_gdr_cut_l2norm_in_kernel(device, K, V):
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from oracle.modules import l2norm
+    q, k, v, g, beta, h0 = gdr_inputs(1, 1700, 2, K, V, seed=3, normalizer=2000.0)
+    k = torch.randn(k.shape).to(k.dtype) * 3
+    beta = beta * 0.02
+    assert _cut(1, 1700, 2, V // 64, False, None, 1)
+    print("cut delta rule, raw q and k", K, V, flush=True)
+    with torch.no_grad():
+        o, ht = chunk_gated_delta_rule(*(t.to(device) for t in (q, k, v, g, beta)), initial_state=h0.to(device),
+                                       output_final_state=True, head_first=False, use_qk_l2norm_in_kernel=True)
+    ro, rht = naive_recurrent_gated_delta_rule(l2norm(q), l2norm(k), v, g, beta, initial_state=h0, output_final_state=True)
     assert_close("o", ro, o, 1e-2)
     assert_close("ht", rht, ht, 5e-3)
