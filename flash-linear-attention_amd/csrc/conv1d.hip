@@ -3,8 +3,8 @@
 // Replaces the external causal_conv1d package the reference's ShortConvolution needs
 // (fla/modules/convolution.py:79-211; forward :171-186, single-token step :188-211).
 //
-// HBM-streaming kernels: a lane owns 8 (backward: 4) adjacent channels (one 16-byte access per
-// row for 16-bit storage) and walks a tile of consecutive time steps with the last W inputs (and, in
+// HBM-streaming kernels: a lane owns 8 (backward: 4; half of that where little work has to fill the chip) adjacent
+// channels (one 16-byte access per row for 16-bit storage) and walks a tile of consecutive time steps with the last W inputs (and, in
 // backward, the last W pre-activation gradients) in registers, so every input row is read
 // once per tile plus a (W-1)-row halo that the neighbouring tile has just pulled into L2.
 // The weight/bias gradients are accumulated in registers over all tiles a lane visits, summed
@@ -14,7 +14,11 @@
 
 namespace {
 
-constexpr int TT = 16;   // time steps per tile
+// Time steps per tile.  All rows of a tile are in flight at once, so the tile sets the registers and with them the waves
+// that hide each other's latency: tiles of 16 steps take 210 registers, two waves per SIMD, tiles of 8 three waves for
+// three more rows of halo out of the L2 (forward of 2048 channels in bf16, B=8, T=4096: 62 -> 54 us).  A short forward
+// takes tiles of 4, which fill the chip with half the rows: see launch_conv.
+constexpr int kTileFwd = 8, kTileFwdShort = 4, kTileBwd = 8;
 
 // A lane's slice of one row: N adjacent channels, kept in storage precision until use so that
 // a whole tile of rows can be in flight at once.
@@ -59,23 +63,36 @@ FLA_DEVICE float silu_grad(float z) {
   return s * (1.f + z * (1.f - s));
 }
 
+// The taps w[i][j] and bias of CV adjacent channels: W CV consecutive floats, four at a time
+template <int W, int CV>
+FLA_DEVICE void load_weights(const ConvParams& p, int d0, float (*w)[CV], float* bias) {
+  const float* src = p.w + (int64_t)d0 * W;
+  if constexpr (W * CV % 4 == 0) {
+#pragma unroll
+    for (int e = 0; e < W * CV; e += 4) {
+      const f32x4 x = *(const f32x4_any*)(src + e);
+#pragma unroll
+      for (int z = 0; z < 4; ++z) w[(e + z) % W][(e + z) / W] = x[z];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < W * CV; ++e) w[e % W][e / W] = src[e];
+  }
+#pragma unroll
+  for (int j = 0; j < CV; ++j) bias[j] = p.bias ? p.bias[d0 + j] : 0.f;
+}
+
 // block (64, 4): x = channel vector, y = tile slot; grid (channel blocks, tile groups): the
 // workgroups that share rows of x are adjacent in dispatch order
-template <typename T, int W>
+template <typename T, int W, int TT, int CV>
 __global__ __launch_bounds__(256) void conv_fwd_kernel(ConvParams p) {
-  constexpr int CV = 8;
   typedef Chan<T, CV> C;
   const int dv = blockIdx.x * 64 + threadIdx.x;
   const int D = p.D;
   if (dv * CV >= D) return;
   const int d0 = dv * CV;
   float w[W][CV], bias[CV];
-#pragma unroll
-  for (int j = 0; j < CV; ++j) {
-#pragma unroll
-    for (int i = 0; i < W; ++i) w[i][j] = p.w[(int64_t)(d0 + j) * W + i];
-    bias[j] = p.bias ? p.bias[d0 + j] : 0.f;
-  }
+  load_weights<W, CV>(p, d0, w, bias);
   const int64_t tiles_per_seq = (p.T + TT - 1) / TT, ntiles = p.B * tiles_per_seq;
   for (int64_t tile = (int64_t)blockIdx.y * 4 + threadIdx.y; tile < ntiles; tile += (int64_t)gridDim.y * 4) {
     const int64_t b = tile / tiles_per_seq, t0 = (tile % tiles_per_seq) * TT;
@@ -113,10 +130,10 @@ __global__ __launch_bounds__(256) void conv_fwd_kernel(ConvParams p) {
   }
 }
 
-// Backward: a lane owns 4 channels (the running state is four times the forward's).
-template <typename T, int W>
+// Backward: a lane owns 4 or 2 channels (the running state is four times the forward's).
+template <typename T, int W, int CV>
 __global__ __launch_bounds__(256) void conv_bwd_kernel(ConvParams p) {
-  constexpr int CV = 4;
+  constexpr int TT = kTileBwd;
   typedef Chan<T, CV> C;
   __shared__ float sred[4][64][(W + 1) * CV + 1];
   const int dv = blockIdx.x * 64 + threadIdx.x;
@@ -124,14 +141,11 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(ConvParams p) {
   const bool active = dv * CV < D;   // idle lanes still take part in the reduction barrier
   const int d0 = active ? dv * CV : 0;
   float w[W][CV], bias[CV], dw[W][CV], db[CV];
+  load_weights<W, CV>(p, d0, w, bias);
 #pragma unroll
   for (int j = 0; j < CV; ++j) {
 #pragma unroll
-    for (int i = 0; i < W; ++i) {
-      w[i][j] = p.w[(int64_t)(d0 + j) * W + i];
-      dw[i][j] = 0.f;
-    }
-    bias[j] = p.bias ? p.bias[d0 + j] : 0.f;
+    for (int i = 0; i < W; ++i) dw[i][j] = 0.f;
     db[j] = 0.f;
   }
   const int64_t tiles_per_seq = (p.T + TT - 1) / TT, ntiles = active ? p.B * tiles_per_seq : 0;
@@ -238,9 +252,9 @@ __global__ __launch_bounds__(256) void conv_bwd_kernel(ConvParams p) {
 }
 
 // single-token step: shift the cache [B,D,W] left by one, append x, y = act(bias + sum cache * w)
-template <typename T, int W>
+template <typename T, typename WT, int W>
 __global__ __launch_bounds__(256) void conv_update_kernel(const T* __restrict__ x, T* __restrict__ cache,
-                                                          const float* __restrict__ w, const float* __restrict__ bias,
+                                                          const WT* __restrict__ w, const float* __restrict__ bias,
                                                           T* __restrict__ y, int64_t BD, int D, int silu) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= BD) return;
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(256) void conv_update_kernel(const T* __restrict__ 
   float acc = bias ? bias[d] : 0.f;
 #pragma unroll
   for (int k = 0; k < W; ++k) {
-    acc = fmaf((float)c[k], w[(int64_t)d * W + k], acc);
+    acc = fmaf((float)c[k], (float)w[(int64_t)d * W + k], acc);
     cache[i * W + k] = c[k];
   }
   y[i] = (T)(silu ? silu_f(acc) : acc);
@@ -262,22 +276,32 @@ __global__ __launch_bounds__(256) void conv_update_kernel(const T* __restrict__ 
 
 // backward: few enough workgroups that the partial sums stay small, enough to fill the chip
 int64_t conv_bwd_parts(int64_t B, int64_t T) {
-  const int64_t g = fla_cdiv(B * fla_cdiv(T, TT), 4);
+  const int64_t g = fla_cdiv(B * fla_cdiv(T, kTileBwd), 4);
   return g < 1 ? 1 : (g > 128 ? 128 : g);
 }
 
 template <typename T, int W>
 int launch_conv(const ConvParams& p, bool bwd, hipStream_t st) {
-  const int64_t ntiles = p.B * fla_cdiv(p.T, TT);
-  const int64_t cblocks = fla_cdiv(p.D / (bwd ? 4 : 8), 64);
-  int64_t gy = fla_cdiv(ntiles, 4);
-  if (bwd) gy = conv_bwd_parts(p.B, p.T);
-  else if (gy * cblocks > 4096) gy = fla_cdiv(4096, cblocks);   // a few tiles per lane: weights are loaded once
-  if (gy < 1) gy = 1;
-  if (gy > 65535) gy = 65535;
-  dim3 grid((unsigned)cblocks, (unsigned)gy), block(64, 4);
-  if (bwd) hipLaunchKernelGGL((conv_bwd_kernel<T, W>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((conv_fwd_kernel<T, W>), grid, block, 0, st, p);
+  const dim3 block(64, 4);
+  auto cblocks = [&](int cv) { return fla_cdiv(p.D / cv, 64); };
+  if (bwd) {
+    // two channels per lane while four leave fewer than eight waves per SIMD (B=2, T=2048, 2048 channels in bf16:
+    // 16.9 -> 15.0 us, B=1, T=300, 512 channels 6.5 -> 4.8; B=8, T=4096, 2048 channels 94 -> 99)
+    const bool narrow = p.B * fla_cdiv(p.T, kTileBwd) * cblocks(4) < 8 * 1024;
+    const dim3 grid((unsigned)cblocks(narrow ? 2 : 4), (unsigned)conv_bwd_parts(p.B, p.T));
+    if (narrow) hipLaunchKernelGGL((conv_bwd_kernel<T, W, 2>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((conv_bwd_kernel<T, W, 4>), grid, block, 0, st, p);
+  } else {
+    // tiles of 4 steps x 4 channels while those of 8 x 8 leave fewer than one wave per SIMD (B=1, T=300, 512 channels:
+    // 5.5 -> 3.7 us; at two waves, B=2, T=2048, 2048 channels, 11.6 -> 13 us)
+    const bool brief = p.B * fla_cdiv(p.T, kTileFwd) * cblocks(8) < 1024;
+    const int64_t cb = cblocks(brief ? 4 : 8);
+    int64_t gy = fla_cdiv(p.B * fla_cdiv(p.T, brief ? kTileFwdShort : kTileFwd), 4);
+    if (gy * cb > 4096) gy = fla_cdiv(4096, cb);   // a few tiles per lane: weights are loaded once
+    const dim3 grid((unsigned)cb, (unsigned)(gy < 1 ? 1 : gy > 65535 ? 65535 : gy));
+    if (brief) hipLaunchKernelGGL((conv_fwd_kernel<T, W, kTileFwdShort, 4>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((conv_fwd_kernel<T, W, kTileFwd, 8>), grid, block, 0, st, p);
+  }
   FLA_CHECK_LAUNCH();
   return FLA_OK;
 }
@@ -290,13 +314,13 @@ int dispatch_conv(const ConvParams& p, int W, bool bwd, hipStream_t st) {
   return FLA_E_UNSUPPORTED;
 }
 
-template <typename T>
-int dispatch_update(const void* x, void* cache, const float* w, const float* bias, void* y, int64_t BD, int D, int W,
+template <typename T, typename WT>
+int dispatch_update(const void* x, void* cache, const void* w, const float* bias, void* y, int64_t BD, int D, int W,
                     int silu, hipStream_t st) {
   dim3 grid((unsigned)fla_cdiv(BD, 256));
 #define U(WW)                                                                                                    \
   if (W == WW) {                                                                                                 \
-    hipLaunchKernelGGL((conv_update_kernel<T, WW>), grid, dim3(256), 0, st, (const T*)x, (T*)cache, w, bias, (T*)y, \
+    hipLaunchKernelGGL((conv_update_kernel<T, WT, WW>), grid, dim3(256), 0, st, (const T*)x, (T*)cache, (const WT*)w, bias, (T*)y, \
                        BD, D, silu);                                                                             \
     FLA_CHECK_LAUNCH();                                                                                          \
     return FLA_OK;                                                                                               \
@@ -341,14 +365,20 @@ extern "C" int fla_causal_conv1d_bwd(const void* x, const float* weight, const f
   return FLA_E_UNSUPPORTED;
 }
 
-extern "C" int fla_causal_conv1d_update(const void* x, void* cache, const float* weight, const float* bias, void* y,
-                                        int64_t B, int64_t D, int64_t W, int silu, int dtype, fla_stream_t stream) {
+extern "C" int fla_causal_conv1d_update(const void* x, void* cache, const void* weight, const float* bias, void* y,
+                                        int64_t B, int64_t D, int64_t W, int silu, int dtype, int weight_dtype,
+                                        fla_stream_t stream) {
   FLA_REQUIRE(x && cache && weight && y && B >= 0 && D > 0, FLA_E_INVALID);
   FLA_REQUIRE(W >= 2 && W <= 4, FLA_E_UNSUPPORTED);
   if (B == 0) return FLA_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == FLA_BF16) return dispatch_update<bf16>(x, cache, weight, bias, y, B * D, (int)D, (int)W, silu, st);
-  if (dtype == FLA_F16) return dispatch_update<f16>(x, cache, weight, bias, y, B * D, (int)D, (int)W, silu, st);
-  if (dtype == FLA_F32) return dispatch_update<float>(x, cache, weight, bias, y, B * D, (int)D, (int)W, silu, st);
+#define U(E, T, WE, WT) \
+  if (dtype == E && weight_dtype == WE) return dispatch_update<T, WT>(x, cache, weight, bias, y, B * D, (int)D, (int)W, silu, st);
+  U(FLA_BF16, bf16, FLA_BF16, bf16)
+  U(FLA_BF16, bf16, FLA_F32, float)
+  U(FLA_F16, f16, FLA_F16, f16)
+  U(FLA_F16, f16, FLA_F32, float)
+  U(FLA_F32, float, FLA_F32, float)
+#undef U
   return FLA_E_UNSUPPORTED;
 }

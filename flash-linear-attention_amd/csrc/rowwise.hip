@@ -206,6 +206,21 @@ FLA_DEVICE void store8_as(void* base, int f32, int64_t idx, const float* v) {
   else Row8<T>::store((T*)base + idx, v);
 }
 
+// A lane's eight weights (or biases) in two loads: as eight single ones they were half of the memory instructions of a
+// workgroup that handles 16 rows of 128 columns (forward of 65536 rows: 20 us, with four rows per lane 13.5)
+FLA_DEVICE void load_affine(const float* base, int col, float otherwise, float* o) {
+  f32x4 a = {otherwise, otherwise, otherwise, otherwise}, c = a;
+  if (base) {   // uniform
+    a = *(const f32x4_any*)(base + col);
+    c = *(const f32x4_any*)(base + col + 4);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    o[i] = a[i];
+    o[4 + i] = c[i];
+  }
+}
+
 template <typename T, bool RMS, int LPR, int NP>
 __global__ __launch_bounds__(256) void norm_gate_fwd_kernel(NormGateParams p) {
   constexpr int RPW = 256 / LPR;
@@ -215,38 +230,37 @@ __global__ __launch_bounds__(256) void norm_gate_fwd_kernel(NormGateParams p) {
 #pragma unroll
   for (int pss = 0; pss < NP; ++pss) {
     const int col = (pss * LPR + sub) * VEC;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      w[pss][i] = (p.w && col < N) ? p.w[col + i] : 1.f;
-      b[pss][i] = (p.b && col < N) ? p.b[col + i] : 0.f;
-    }
+    load_affine(p.w, col < N ? col : 0, 1.f, w[pss]);
+    load_affine(p.b, col < N ? col : 0, 0.f, b[pss]);
   }
   const float invN = 1.f / (float)N;
-  // The rows of the next pass are fetched (in storage precision) before this pass computes, so
-  // that a lane always has two passes of loads in flight; past the last row the fetch repeats it.
+  // A lane's R rows are fetched together (in storage precision); past the last row the fetch repeats it.
   typedef typename Row8<T>::raw raw_t;
-  const int64_t step = (int64_t)gridDim.x * RPW;
-  const int64_t first = (int64_t)blockIdx.x * RPW + rl;
-  raw_t nx[NP], ng[NP];
-  auto fetch = [&](int64_t row) {
-    const int64_t r = row < p.M ? row : p.M - 1;
+  constexpr int R = 1;
+  const int64_t first = (int64_t)blockIdx.x * (RPW * R) + rl;
+  raw_t nx[R][NP], ng[R][NP];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int64_t r = first + q * RPW < p.M ? first + q * RPW : p.M - 1;
 #pragma unroll
     for (int pss = 0; pss < NP; ++pss) {
       const int col = (pss * LPR + sub) * VEC;
       const int c = col < N ? col : 0;
-      nx[pss] = Row8<T>::load_raw((const T*)p.x + r * N + c);
-      ng[pss] = Row8<T>::load_raw((const T*)p.gate + r * N + c);
+      nx[q][pss] = Row8<T>::load_raw((const T*)p.x + r * N + c);
+      ng[q][pss] = Row8<T>::load_raw((const T*)p.gate + r * N + c);
     }
-  };
-  fetch(first);
-  for (int64_t row = first; row < p.M; row += step) {
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int64_t row = first + q * RPW;
+    if (row >= p.M) break;
     float v[NP][VEC], g[NP][VEC];
     float s1 = 0.f;
 #pragma unroll
     for (int pss = 0; pss < NP; ++pss) {
       const int col = (pss * LPR + sub) * VEC;
-      Row8<T>::unpack(nx[pss], v[pss]);
-      Row8<T>::unpack(ng[pss], g[pss]);
+      Row8<T>::unpack(nx[q][pss], v[pss]);
+      Row8<T>::unpack(ng[q][pss], g[pss]);
       if (col < N) {
         if (p.res) {
           float r8[VEC];
@@ -262,7 +276,6 @@ __global__ __launch_bounds__(256) void norm_gate_fwd_kernel(NormGateParams p) {
         for (int i = 0; i < VEC; ++i) v[pss][i] = g[pss][i] = 0.f;
       }
     }
-    fetch(row + step);
     float mean = 0.f;
     if (!RMS) mean = group_sum<LPR>(s1) * invN;
     float ss = 0.f;
@@ -308,26 +321,49 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(NormGateParams p) {
 #pragma unroll
   for (int pss = 0; pss < NP; ++pss) {
     const int col = (pss * LPR + sub) * VEC;
+    load_affine(p.w, col < N ? col : 0, 1.f, w[pss]);
+    load_affine(p.b, col < N ? col : 0, 0.f, b[pss]);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      w[pss][i] = (p.w && col < N) ? p.w[col + i] : 1.f;
-      b[pss][i] = (p.b && col < N) ? p.b[col + i] : 0.f;
-      dw[pss][i] = db[pss][i] = 0.f;
-    }
+    for (int i = 0; i < VEC; ++i) dw[pss][i] = db[pss][i] = 0.f;
   }
   const float invN = 1.f / (float)N;
-  for (int64_t row = (int64_t)blockIdx.x * RPW + rl; row < p.M; row += (int64_t)gridDim.x * RPW) {
+  // The operands of the next row are fetched (in storage precision) before this one is worked on, so that a lane always
+  // has a row in flight; past the last row the fetch repeats it.
+  typedef typename Row8<T>::raw raw_t;
+  const int64_t step = (int64_t)gridDim.x * RPW;
+  raw_t nx[NP], ng[NP], nd[NP];
+  float nrstd, nmean = 0.f;
+  auto fetch = [&](int64_t row) {
+    const int64_t r = row < p.M ? row : p.M - 1;
+#pragma unroll
+    for (int pss = 0; pss < NP; ++pss) {
+      const int col = (pss * LPR + sub) * VEC;
+      const int c = col < N ? col : 0;
+      if (!p.x_f32) nx[pss] = Row8<T>::load_raw((const T*)p.x + r * N + c);
+      ng[pss] = Row8<T>::load_raw((const T*)p.gate + r * N + c);
+      nd[pss] = Row8<T>::load_raw((const T*)p.dy + r * N + c);
+    }
+    nrstd = p.rstd[r];
+    if (!RMS) nmean = p.mean[r];
+  };
+  fetch((int64_t)blockIdx.x * RPW + rl);
+  for (int64_t row = (int64_t)blockIdx.x * RPW + rl; row < p.M; row += step) {
     float xh[NP][VEC], g[NP][VEC], d[NP][VEC];
-    const float rstd = p.rstd[row];
-    const float mean = RMS ? 0.f : p.mean[row];
+    const float rstd = nrstd, mean = nmean;
+#pragma unroll
+    for (int pss = 0; pss < NP; ++pss) {
+      const int col = (pss * LPR + sub) * VEC;
+      if (!p.x_f32) Row8<T>::unpack(nx[pss], xh[pss]);
+      else if (col < N) load8_as<T>(p.x, 1, row * N + col, xh[pss]);
+      Row8<T>::unpack(ng[pss], g[pss]);
+      Row8<T>::unpack(nd[pss], d[pss]);
+    }
+    fetch(row + step);
     float c1 = 0.f, c2 = 0.f;
 #pragma unroll
     for (int pss = 0; pss < NP; ++pss) {
       const int col = (pss * LPR + sub) * VEC;
       if (col < N) {
-        load8_as<T>(p.x, p.x_f32, row * N + col, xh[pss]);
-        Row8<T>::load((const T*)p.gate + row * N + col, g[pss]);
-        Row8<T>::load((const T*)p.dy + row * N + col, d[pss]);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) {
           const float xhat = (xh[pss][i] - mean) * rstd;
@@ -437,6 +473,47 @@ int launch_ng(const NormGateParams& p, bool bwd, int grid, hipStream_t st) {
   return FLA_OK;
 }
 
+// out[c] = sum over the rows of part [parts, n], in a fixed order: CW columns x 256 / CW slices of the rows per workgroup,
+// eight rows in flight per lane, the slices added up in LDS.  What the weight gradients of a layer leave per workgroup are
+// a few hundred to two thousand rows; torch's reduction takes 6 - 9 us for any of these shapes.
+template <typename T, int CW>
+__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, T* __restrict__ out, int parts, int n) {
+  constexpr int SL = 256 / CW;
+  __shared__ float s[SL][CW];
+  const int c = threadIdx.x % CW, sl = threadIdx.x / CW;
+  const int col = (int)blockIdx.x * CW + c;
+  float acc = 0.f;
+  if (col < n) {
+    for (int r0 = sl; r0 < parts; r0 += SL * 8) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int r = r0 + SL * u;
+        x[u] = part[(int64_t)(r < parts ? r : sl) * n + col];
+        if (r >= parts) x[u] = 0.f;
+      }
+      acc += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    }
+  }
+  s[sl][c] = acc;
+  __syncthreads();
+  if (sl == 0 && col < n) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < SL; ++q) t += s[q][c];
+    out[col] = (T)t;
+  }
+}
+
+template <typename T>
+int launch_sum_partials(const float* part, void* out, int parts, int n, hipStream_t st) {
+  // narrow workgroups while wide ones would leave CUs without one
+  if (n >= 32 * 64) hipLaunchKernelGGL((sum_partials_kernel<T, 32>), dim3((unsigned)fla_cdiv(n, 32)), dim3(256), 0, st, part, (T*)out, parts, n);
+  else hipLaunchKernelGGL((sum_partials_kernel<T, 4>), dim3((unsigned)fla_cdiv(n, 4)), dim3(256), 0, st, part, (T*)out, parts, n);
+  FLA_CHECK_LAUNCH();
+  return FLA_OK;
+}
+
 int rpw_of(int N) { return N <= 64 ? 32 : N <= 128 ? 16 : N <= 256 ? 8 : 4; }
 
 }  // namespace
@@ -483,7 +560,7 @@ extern "C" int fla_l2norm_bwd(const void* x, const void* dy, void* dx, int64_t M
 
 extern "C" int fla_norm_swish_gate_workgroups(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 1;
-  return rows_grid(M, rpw_of((int)N), 2048);
+  return rows_grid(M, rpw_of((int)N), 1024);
 }
 
 extern "C" int fla_norm_swish_gate_residual_fwd(const void* x, const void* gate, const float* weight, const float* bias,
@@ -501,7 +578,9 @@ extern "C" int fla_norm_swish_gate_residual_fwd(const void* x, const void* gate,
   NormGateParams p{x, gate, weight, bias, y, mean, rstd, nullptr, nullptr, nullptr, nullptr, nullptr, M, (int)N, eps,
                    residual, residual_out, nullptr, nullptr,
                    residual && residual_dtype == FLA_F32, residual_out && residual_out_dtype == FLA_F32, 0};
-  const int grid = rows_grid(M, rpw_of((int)N), 4096);   // grid-stride: weights are loaded once per lane
+  const int rpw = rpw_of((int)N);   // rows per workgroup: norm_gate_fwd_kernel
+  FLA_REQUIRE(fla_cdiv(M, rpw) <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
+  const int grid = (int)fla_cdiv(M, rpw);
   hipStream_t st = (hipStream_t)stream;
 #define D(E, TT)                                                         \
   if (dtype == E) {                                                      \
@@ -557,4 +636,13 @@ extern "C" int fla_norm_swish_gate_bwd(const void* dy, const void* x, const void
                                        int is_rms_norm, int dtype, fla_stream_t stream) {
   return fla_norm_swish_gate_residual_bwd(dy, x, dtype, gate, weight, bias, mean, rstd, nullptr, dx, dgate, nullptr,
                                           dw_partial, db_partial, M, N, eps, is_rms_norm, dtype, stream);
+}
+
+extern "C" int fla_sum_partials(const float* partials, void* out, int64_t parts, int64_t n, int out_dtype, fla_stream_t stream) {
+  FLA_REQUIRE(partials && out && parts > 0 && n > 0 && parts <= 0x7ffffff && n <= 0x7fffffff, FLA_E_INVALID);
+  hipStream_t st = (hipStream_t)stream;
+  if (out_dtype == FLA_F32) return launch_sum_partials<float>(partials, out, (int)parts, (int)n, st);
+  if (out_dtype == FLA_BF16) return launch_sum_partials<bf16>(partials, out, (int)parts, (int)n, st);
+  if (out_dtype == FLA_F16) return launch_sum_partials<f16>(partials, out, (int)parts, (int)n, st);
+  return FLA_E_UNSUPPORTED;
 }

@@ -452,6 +452,15 @@ bool rows_ok(const Tensor& x) {
          (is16(x) || x.scalar_type() == at::kFloat);
 }
 
+// The column sums of per-workgroup partial sums [parts, ...], in the dtype and shape of the weight they belong to
+Tensor sum_partials(const Tensor& part, at::IntArrayRef shape, at::ScalarType type) {
+  const bool direct = type == at::kFloat || type == at::kBFloat16 || type == at::kHalf;
+  Tensor out = fresh(shape, part, direct ? type : at::kFloat);
+  check(fla_sum_partials(fptr(part), ptr(out), part.size(0), part.numel() / part.size(0), dt(out), stream_of(part)),
+        "fla_sum_partials");
+  return as(out, type);
+}
+
 struct L2NormNode : torch::autograd::Function<L2NormNode> {
   static Tensor run(const Tensor& x, double eps) {
     Tensor y = fresh_like(x);
@@ -513,7 +522,7 @@ struct ConvNode : torch::autograd::Function<ConvNode> {
     check(fla_causal_conv1d_bwd(ptr(x), fptr(w), fptr(b), ptr(dy), ptr(dx), fptr(dw), fptr(db), B, T, D, W, r.silu, dt(x),
                                 stream_of(x)),
           "fla_causal_conv1d_bwd");
-    return {dx, as(dw.sum(0).reshape(r.w_shape), r.w_type), b.defined() ? as(db.sum(0), *r.b_type) : Tensor(), Tensor()};
+    return {dx, sum_partials(dw, r.w_shape, r.w_type), b.defined() ? sum_partials(db, {D}, *r.b_type) : Tensor(), Tensor()};
   }
 };
 
@@ -559,8 +568,8 @@ struct NormGateNode : torch::autograd::Function<NormGateNode> {
     check(fla_norm_swish_gate_bwd(ptr(dy), ptr(x), ptr(o), fptr(w32), fptr(b32), fptr(mean), fptr(rstd), ptr(dx), ptr(dgate),
                                   fptr(dw), fptr(db), M, D, (float)r.eps, r.rms, dt(x), stream_of(x)),
           "fla_norm_swish_gate_bwd");
-    return {dx, dgate, w.defined() ? as(dw.sum(0), w.scalar_type()) : Tensor(),
-            b.defined() ? as(db.sum(0), b.scalar_type()) : Tensor(), Tensor(), Tensor()};
+    return {dx, dgate, w.defined() ? sum_partials(dw, w.sizes(), w.scalar_type()) : Tensor(),
+            b.defined() ? sum_partials(db, b.sizes(), b.scalar_type()) : Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -852,9 +861,10 @@ PyObject* py_conv_update(PyObject*, PyObject* const* p, Py_ssize_t n) {
       cache.scalar_type() != x.scalar_type())
     return none();
   at::AutoDispatchBelowADInplaceOrView guard;
-  const Tensor xc = x.contiguous(), w32 = f32(w), b32 = f32(b);
+  const Tensor xc = x.contiguous(), b32 = f32(b);
+  const Tensor wc = w.scalar_type() == x.scalar_type() ? w.contiguous() : f32(w);
   Tensor y = fresh_like(xc);
-  check(fla_causal_conv1d_update(ptr(xc), ptr(cache), fptr(w32), fptr(b32), ptr(y), B, D, W, arg_bool(p[4]), dt(xc),
+  check(fla_causal_conv1d_update(ptr(xc), ptr(cache), ptr(wc), fptr(b32), ptr(y), B, D, W, arg_bool(p[4]), dt(xc), dt(wc),
                                  stream_of(xc)),
         "fla_causal_conv1d_update");
   return THPVariable_Wrap(y);

@@ -96,7 +96,8 @@ SIGNATURES = {
     "fla_causal_conv1d_fwd": (c_int, [P, P, P, P, I64, I64, I64, I64, I, I, P]),
     "fla_causal_conv1d_bwd_partials": (c_int, [I64, I64]),
     "fla_causal_conv1d_bwd": (c_int, [P] * 7 + [I64, I64, I64, I64, I, I, P]),
-    "fla_causal_conv1d_update": (c_int, [P] * 5 + [I64, I64, I64, I, I, P]),
+    "fla_sum_partials": (c_int, [P, P, I64, I64, I, P]),
+    "fla_causal_conv1d_update": (c_int, [P] * 5 + [I64, I64, I64, I, I, I, P]),
     "fla_gate_logsigmoid_fwd": (c_int, [P, P, I64, F, I, F, I, I, P]),
     "fla_gate_logsigmoid_bwd": (c_int, [P, P, P, I64, F, I, F, I, I, P]),
     "fla_gdn_gate_workgroups": (c_int, [I64, I64]),

@@ -82,7 +82,7 @@ def causal_conv1d_update(x: torch.Tensor, cache: torch.Tensor, weight: torch.Ten
     b32 = None if bias is None else bias.detach().float().contiguous()
     y = torch.empty_like(x)
     be.check(be.lib().fla_causal_conv1d_update(be.ptr(x), be.ptr(cache), be.ptr(w32), be.ptr(b32), be.ptr(y), B, D, W,
-                                               _act_flag(activation), be.dt(x), be.stream_of(x)),
+                                               _act_flag(activation), be.dt(x), be.FLA_F32, be.stream_of(x)),
              "fla_causal_conv1d_update")
     return y
 

@@ -729,8 +729,14 @@ int fla_causal_conv1d_bwd_partials(int64_t B, int64_t T);
 int fla_causal_conv1d_bwd(const void* x, const float* weight, const float* bias, const void* dy, void* dx,
                           float* dw_partial, float* db_partial, int64_t B, int64_t T, int64_t D, int64_t W, int silu,
                           int dtype, fla_stream_t stream);
-int fla_causal_conv1d_update(const void* x, void* cache, const float* weight, const float* bias, void* y,
-                             int64_t B, int64_t D, int64_t W, int silu, int dtype, fla_stream_t stream);
+int fla_causal_conv1d_update(const void* x, void* cache, const void* weight, const float* bias, void* y,
+                             int64_t B, int64_t D, int64_t W, int silu, int dtype, int weight_dtype,
+                             fla_stream_t stream);
+
+/* out[c] = sum over the rows of partials [parts, n] (fp32, added in a fixed order), in out_dtype: the per-workgroup partial
+ * sums of the weight gradients above (the reference's dw.sum(0), fla/modules/fused_norm_gate.py:393-396). */
+int fla_sum_partials(const float* partials, void* out, int64_t parts, int64_t n, int out_dtype, fla_stream_t stream);
+
 
 /* ------------------------------------------------------------------------
  * Gate pre-activations of the layers that call the chunk operators.
