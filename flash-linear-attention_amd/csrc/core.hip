@@ -59,15 +59,18 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us).
 //
 // The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 1.2 us per
-// segment, so it takes longer segments and only batches that fall into at least kMinSegments of them (forward of K = V = 128,
-// 16 heads, uncut against cut in us: one sequence of 5003 tokens in 8 segments 119 / 74, of 16384 in 8 359 / 163, of 8192
-// with 4 heads in 32, 16 and 8 segments 175 / 76, 63 and 74; two of 4096 in 4 segments 105 / 94, four in 2 127 / 158).  A
-// forward that keeps its intermediates is longer by the stores and gains less: two sequences of 2048 in 4 segments 58 / 60.
+// segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16 chunks 76, 63
+// and 74 us, uncut 175; training step of 64 chunks, 8 heads, in 4 and 8 172 and 158 us, uncut 251), twenty chunks to save
+// (16 chunks: 32 us uncut, 38 cut; training step of 24 chunks 94 / 87) and at least three of them (forward of K = V = 128, 16
+// heads, uncut against cut in us: one sequence of 5003 tokens in 8 119 / 74, of 16384 in 8 359 / 163, two of 4096 in 4
+// 105 / 94, four in 2 127 / 158).  A forward that keeps its intermediates and its backward gain from five on (training
+// step: three sequences of 4096, 8 heads, in 5 377 / 352, two of 16 heads in 4 462 / 468).
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
   const bool delta = kind != FLA_SCAN_GLA;
-  const int64_t kMinSeg = delta ? 8 : 4, kMinSaved = delta ? 16 : 8, kMinSegments = kind == FLA_SCAN_DELTA_KEPT ? 6 : delta ? 3 : 2;
+  const int64_t kMinSaved = delta ? 20 : 8, kMinSegments = kind == FLA_SCAN_DELTA_KEPT ? 5 : delta ? 3 : 2;
+  int64_t min_seg = 4;
   if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_DELTA_KEPT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
   int64_t longest = 0, total = 0;
@@ -76,6 +79,8 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
     longest = c > longest ? c : longest;
     total += c;
   }
+  if (delta)
+    while (100 * min_seg * min_seg < 49 * longest) ++min_seg;
   const int64_t room = kCUs / (H * slabs);   // segments the chip holds at once
   if (room < 2 || N > room || longest > 0x7fffffff / kChunk) return 0;
   // the shortest segment with which all of them fit
@@ -88,7 +93,7 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
     return s;
   };
   int64_t seg = fla_cdiv(total, room);
-  seg = seg < kMinSeg ? kMinSeg : seg;
+  seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
   if (longest - seg < kMinSaved || longest < (kMinSegments - 1) * seg + 1) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
@@ -120,7 +125,8 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
     base += s;
     nseg += g;
     most = g > most ? g : most;
-    const int64_t lo = reverse ? ratio : 0, hi = reverse ? s : (g - 1) * ratio;
+    // (a forward that keeps its intermediates forms the last segment's transition too, for its backward)
+    const int64_t lo = reverse ? ratio : 0, hi = reverse || kind == FLA_SCAN_DELTA_KEPT ? s : (g - 1) * ratio;
     for (int64_t j = lo; j < hi; ++j, ++nsub)
       if (sub_table) {
         sub_table[2 * nsub] = (int32_t)n;

@@ -30,7 +30,7 @@
 //                            (wy_fast.py:440-562, written for the single inverse Aw).
 #include <type_traits>
 
-#include "chunk_common.h"
+#include "seq_split.h"
 
 namespace {
 
@@ -223,6 +223,9 @@ struct DhuParams {
   int64_t T;
   int H, V, N;
   float scale;
+  SplitView split;   // sequences cut into segments (ratio 0: not)
+  float* local;      // PASS: what the segments add to a zero gradient, [slots, H, K, V]
+  int per_seq;       // PASS, equal-length sequences: segments of the pass per sequence
 };
 
 // One workgroup of eight waves: all K rows x 32 value columns of one (sequence, head).
@@ -245,7 +248,9 @@ struct DhuParams {
 // FROMP: dv_loc = Aqk^T do is not read from memory but formed here from the packed score tile Aqk the forward
 // kept (5 KB per chunk and head) and the raw do rows, which then travel with the k group: four more small
 // matrix products per wave and chunk instead of a launch that reads q, k, do and writes dv_loc.
-template <typename T, int K, bool FROMP>
+// PASS: the first pass over sequences cut into segments (seq_split.h): every segment but a sequence's first, from a zero
+// gradient, without outputs but the gradient it ends with.
+template <typename T, int K, bool FROMP, bool PASS = false>
 __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
   typedef typename Elem<T>::v8 v8;
   typedef typename Elem<T>::v4 v4;
@@ -275,12 +280,19 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
   const int nvt = V / BV;
   int64_t id = xcd_remap(blockIdx.x, gridDim.x);
   const int vt = (int)(id % nvt);
-  const int nh = (int)(id / nvt);
-  const int n = nh / H, hh = nh % H;
+  const int item = (int)(id / nvt);
+  const int hh = item % H;
   const int vbase = vt * BV;
-  SeqSpan sp = seq_span(p.offsets, n, p.T);
-  const int64_t nchunks = (sp.len + BT - 1) / BT;
-  const int64_t chunk0 = p.chunk_offsets ? p.chunk_offsets[n] : (int64_t)n * ((p.T + BT - 1) / BT);
+  const ScanSpan span = PASS ? pass_span(p.split, item / H, p.per_seq, p.offsets, p.chunk_offsets, p.T)
+                             : scan_span<true>(p.split, item / H, nullptr, p.offsets, p.chunk_offsets, p.T);
+  const int nh = span.n * H + hh;
+  const SeqSpan sp = span.sp;
+  const int64_t nchunks = span.nchunks, chunk0 = span.chunk0;
+  // the gradient of the state leaving this workgroup's chunks
+  const float* dht = PASS            ? nullptr
+                     : p.split.ratio ? p.split.states + (span.slot * H + hh) * (int64_t)K * V
+                     : p.dht         ? p.dht + (int64_t)nh * K * V
+                                     : nullptr;
   auto chunk_len = [&](int64_t c) {
     int64_t rem = sp.len - c * BT;
     return (int)(rem < BT ? rem : BT);
@@ -398,6 +410,7 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
     const int dgrp = st >> 4, dtb = dgrp >> 2, dvb = dgrp & 3, dj = st & 15;
     const int dsrc = (8 * dvb + (dj >> 2)) * LDT + 16 * dtb + 4 * (dj & 3);
     auto store_dv2 = [&](int64_t c, auto maybe_short) __attribute__((always_inline)) {
+      if constexpr (PASS) return;
       typedef short s4 __attribute__((ext_vector_type(4)));
       typedef __attribute__((address_space(3))) s4 lds_s4;
       s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)&sDv2T[dsrc]);
@@ -449,12 +462,11 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
       acc[a] = zero16();
       acct[a] = zero16();
       int kt = wave + 4 * a;
-      if (p.dht && kt < KT32) {
-        const float* d0 = p.dht + (int64_t)nh * K * V;
+      if (dht && kt < KT32) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          acc[a][r] = d0[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + (lane & 31)];
-          acct[a][r] = d0[(int64_t)(kt * 32 + (lane & 31)) * V + vbase + c32_row(r, lane)];
+          acc[a][r] = dht[(int64_t)(kt * 32 + c32_row(r, lane)) * V + vbase + (lane & 31)];
+          acct[a][r] = dht[(int64_t)(kt * 32 + (lane & 31)) * V + vbase + c32_row(r, lane)];
         }
       }
     }
@@ -471,6 +483,7 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
             for (int b = 0; b < 4; ++b) x[b] = (T)acc[a][4 * q4 + b];
             *(v4*)&sDHt[(lane & 31) * LDK + kt * 32 + 8 * q4 + 4 * (lane >> 5)] = x;
           }
+          if constexpr (PASS) continue;
           v8 lo, hi;
 #pragma unroll
           for (int r = 0; r < 8; ++r) {
@@ -542,7 +555,7 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             acc[a][r] *= dec_c;
-            acct[a][r] *= dec_c;
+            if constexpr (!PASS) acct[a][r] *= dec_c;
           }
 #pragma unroll
           for (int s = 0; s < BT; s += 16) {
@@ -552,15 +565,17 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
             v8 f2 = lds_frag32<T>(sDv2s, LDT, 0, s, lane);
             acc[a] = Elem<T>::mfma32(fq, fd, acc[a]);
             acc[a] = Elem<T>::mfma32(fw, f2, acc[a]);
-            acct[a] = Elem<T>::mfma32(fd, fq, acct[a]);
-            acct[a] = Elem<T>::mfma32(f2, fw, acct[a]);
+            if constexpr (!PASS) {
+              acct[a] = Elem<T>::mfma32(fd, fq, acct[a]);
+              acct[a] = Elem<T>::mfma32(f2, fw, acct[a]);
+            }
           }
         }
       }
       if (c > 0) publish(c - 1);
     }
-    if (p.dh0) {
-      float* o = p.dh0 + (int64_t)nh * K * V;
+    if (PASS || (p.dh0 && span.first)) {
+      float* o = PASS ? p.local + (span.slot * H + hh) * (int64_t)K * V : p.dh0 + (int64_t)nh * K * V;
 #pragma unroll
       for (int a = 0; a < NKT; ++a) {
         int kt = wave + 4 * a;
@@ -1443,7 +1458,8 @@ int launch_dv_local(const DvlParams& p, int64_t K, int64_t V, dim3 grid, hipStre
 // reverse state scan: one workgroup per (sequence, head, 32 value columns)
 template <typename T>
 int launch_dhu(const DhuParams& p, int64_t K, hipStream_t st) {
-  const int64_t total = (int64_t)(p.V / 32) * p.N * p.H;
+  const int64_t seqs = !p.split.ratio ? p.N : p.split.seg_table ? p.split.nseg : (int64_t)p.split.nseg * p.N;
+  const int64_t total = (int64_t)(p.V / 32) * seqs * p.H;
   FLA_REQUIRE(total <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
   if (total == 0) return FLA_OK;
   if (p.Aqk) {
@@ -1456,6 +1472,23 @@ int launch_dhu(const DhuParams& p, int64_t K, hipStream_t st) {
   else return FLA_E_UNSUPPORTED;
   FLA_CHECK_LAUNCH();
   return FLA_OK;
+}
+
+// The gradient leaving every segment: the first pass, then the fold with the transitions the forward left.
+template <typename T>
+int dhu_split(DhuParams p, const fla_split* split, int64_t K, hipStream_t st) {
+  p.local = split->states;
+  p.per_seq = split->nseg - 1;
+  const int64_t segs = p.offsets ? split->nsub : (int64_t)p.per_seq * p.N;
+  const int64_t total = (int64_t)(p.V / 32) * segs * p.H;
+  FLA_REQUIRE(total <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
+  if (total > 0) {
+    if (K == 64) hipLaunchKernelGGL((gdr_bwd_dhu_kernel<T, 64, true, true>), dim3((unsigned)total), dim3(512), 0, st, p);
+    else if (K == 128) hipLaunchKernelGGL((gdr_bwd_dhu_kernel<T, 128, true, true>), dim3((unsigned)total), dim3(512), 0, st, p);
+    else return FLA_E_UNSUPPORTED;
+    FLA_CHECK_LAUNCH();
+  }
+  return gdr_split_fold_reverse(p.dht, split, p.offsets, p.T, p.H, K, p.V, p.N, st);
 }
 
 // one workgroup per (chunk, head, 64 key channels)
@@ -1496,7 +1529,7 @@ int launch_gdr_bwd(const void* q, const void* k, const void* v, const void* w, c
                    const void* Aqk, void* dvl, void* dv2, void* dhtf, void* dw, void* dkp, float* dgam_part, void* dq, void* dk, void* dv,
                    float* dbeta, float* dgam2, float* dh0, const int64_t* offsets, const int64_t* indices,
                    const int64_t* chunk_offsets, int64_t NT, int64_t B, int64_t T_, int64_t H, int64_t K, int64_t V,
-                   int64_t N, float scale, hipStream_t st) {
+                   int64_t N, float scale, hipStream_t st, const fla_split* split) {
   dim3 grid;
   int ntfix;
   int rc = chunk_grid(offsets, indices, B, T_, H, NT, &grid, &ntfix);
@@ -1506,7 +1539,9 @@ int launch_gdr_bwd(const void* q, const void* k, const void* v, const void* w, c
     DvlParams p1{q, k, dout, gam, dvl, offsets, indices, T_, (int)H, ntfix, scale};
     if ((rc = launch_dv_local<T>(p1, K, V, grid, st))) return rc;
   }
-  DhuParams p2{q, k, w, dout, dvl, Aqk, gam, dht, dv2, dhtf, dh0, offsets, chunk_offsets, T_, (int)H, (int)V, (int)N, scale};
+  DhuParams p2{q, k, w, dout, dvl, Aqk, gam, dht, dv2, dhtf, dh0, offsets, chunk_offsets, T_, (int)H, (int)V, (int)N, scale,
+               split_view(split), nullptr, 0};
+  if (split && (rc = dhu_split<T>(p2, split, K, st))) return rc;
   if ((rc = launch_dhu<T>(p2, K, st))) return rc;
   DqkwgParams p3{q, k, vnew, w, dout, dv2, gam, hT, dhtf, dq, dkp, dw, dgam_part, offsets, indices, T_,
                  B * T_, (int)H, (int)K, ntfix, scale};
@@ -1536,13 +1571,14 @@ extern "C" int fla_chunk_bwd_dv_local(const void* q, const void* k, const float*
   return FLA_E_UNSUPPORTED;
 }
 
-extern "C" int fla_chunk_gated_delta_rule_bwd(
+static int gdr_bwd_impl(
     const void* q, const void* k, const void* v, const void* w, const void* v_new, const float* beta,
     const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
     void* ws_dv_local, void* ws_dv2, void* ws_dh_frag_t, void* ws_dw, void* ws_dk_partial, float* ws_dgam_partial,
     void* dq, void* dk, void* dv, float* dbeta, float* dgam2, float* dh0,
     const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT, int qkv_dtype,
-    int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream) {
+    int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream,
+    const fla_split* split) {
   FLA_REQUIRE(q && k && v && w && v_new && beta && Aw && dout && hT && (ws_dv_local || Aqk) && ws_dv2 && ws_dh_frag_t &&
                   ws_dw && ws_dk_partial && ws_dgam_partial && dq && dk && dv && dbeta && dgam2,
               FLA_E_INVALID);
@@ -1551,16 +1587,46 @@ extern "C" int fla_chunk_gated_delta_rule_bwd(
   if (Aqk) FLA_REQUIRE(K <= 128 && (uintptr_t)Aqk % 16 == 0, FLA_E_UNSUPPORTED);
   if (offsets) FLA_REQUIRE(indices && chunk_offsets && B == 1, FLA_E_INVALID);
   else FLA_REQUIRE(N == B, FLA_E_INVALID);
+  if (split) {
+    const int rc = check_split(split, offsets);
+    if (rc) return rc;
+    FLA_REQUIRE(Aqk && split->decays && split->ratio == 1, FLA_E_INVALID);
+  }
   hipStream_t st = (hipStream_t)stream;
   if (qkv_dtype == FLA_BF16)
     return launch_gdr_bwd<bf16>(q, k, v, w, v_new, beta, g_cumsum, Aw, dout, dht, hT, Aqk, ws_dv_local, ws_dv2,
                                 ws_dh_frag_t, ws_dw, ws_dk_partial, ws_dgam_partial, dq, dk, dv, dbeta, dgam2, dh0,
-                                offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st);
+                                offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st, split);
   if (qkv_dtype == FLA_F16)
     return launch_gdr_bwd<f16>(q, k, v, w, v_new, beta, g_cumsum, Aw, dout, dht, hT, Aqk, ws_dv_local, ws_dv2,
                                ws_dh_frag_t, ws_dw, ws_dk_partial, ws_dgam_partial, dq, dk, dv, dbeta, dgam2, dh0,
-                               offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st);
+                               offsets, indices, chunk_offsets, NT, B, T, H, K, V, N, scale, st, split);
   return FLA_E_UNSUPPORTED;
+}
+
+extern "C" int fla_chunk_gated_delta_rule_bwd(
+    const void* q, const void* k, const void* v, const void* w, const void* v_new, const float* beta,
+    const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
+    void* ws_dv_local, void* ws_dv2, void* ws_dh_frag_t, void* ws_dw, void* ws_dk_partial, float* ws_dgam_partial,
+    void* dq, void* dk, void* dv, float* dbeta, float* dgam2, float* dh0,
+    const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT, int qkv_dtype,
+    int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream) {
+  return gdr_bwd_impl(q, k, v, w, v_new, beta, g_cumsum, Aw, dout, dht, hT, Aqk, ws_dv_local, ws_dv2, ws_dh_frag_t, ws_dw,
+                      ws_dk_partial, ws_dgam_partial, dq, dk, dv, dbeta, dgam2, dh0, offsets, indices, chunk_offsets, NT, qkv_dtype,
+                      B, T, H, K, V, N, scale, stream, nullptr);
+}
+
+extern "C" int fla_chunk_gated_delta_rule_bwd_split(
+    const void* q, const void* k, const void* v, const void* w, const void* v_new, const float* beta,
+    const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
+    void* ws_dv2, void* ws_dh_frag_t, void* ws_dw, void* ws_dk_partial, float* ws_dgam_partial,
+    void* dq, void* dk, void* dv, float* dbeta, float* dgam2, float* dh0,
+    const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split, int64_t NT,
+    int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream) {
+  FLA_REQUIRE(split, FLA_E_INVALID);
+  return gdr_bwd_impl(q, k, v, w, v_new, beta, g_cumsum, Aw, dout, dht, hT, Aqk, nullptr, ws_dv2, ws_dh_frag_t, ws_dw,
+                      ws_dk_partial, ws_dgam_partial, dq, dk, dv, dbeta, dgam2, dh0, offsets, indices, chunk_offsets, NT, qkv_dtype,
+                      B, T, H, K, V, N, scale, stream, split);
 }
 
 extern "C" int fla_chunk_gated_delta_rule_bwd_dhu(const void* q, const void* k, const void* w, const float* g_cumsum,
@@ -1578,7 +1644,7 @@ extern "C" int fla_chunk_gated_delta_rule_bwd_dhu(const void* q, const void* k, 
   hipStream_t st = (hipStream_t)stream;
   if (N == 0 || T == 0) return copy_or_zero(dht, dh0, N * H * K * V, st);
   DhuParams p{q, k, w, dout, dv, nullptr, g_cumsum, dht, dv2, dh_frag_t, dh0, offsets, chunk_offsets, T, (int)H, (int)V, (int)N,
-              scale};
+              scale, SplitView(), nullptr, 0};
   if (qkv_dtype == FLA_BF16) return launch_dhu<bf16>(p, K, st);
   if (qkv_dtype == FLA_F16) return launch_dhu<f16>(p, K, st);
   return FLA_E_UNSUPPORTED;

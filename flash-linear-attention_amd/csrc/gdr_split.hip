@@ -29,6 +29,7 @@ struct GdrPassParams {
   const float* rk;      // L2N: 1 / |k|, [rows, H]
   float* states;        // out: S, [slots, H, K, V]
   bf16* trans;          // out: M, [slots, H, 2 (high, low part), K/32 slices, K/16 row tiles, 64 lanes, 8]
+  bf16* trans_t;        // out, or NULL: M^T in the same order
   const int64_t* offsets;
   const int64_t* chunk_offsets;
   SplitView split;
@@ -362,11 +363,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           }
           *(b8*)(out + part * K * K + (2 * ks + half) * 64 * 8) = y;
         }
+      if (p.trans_t) {   // a column of M is a row of M^T: the accumulators are the operand as they are
+        bf16* ot = p.trans_t + (slot * H + hh) * (int64_t)(2 * K * K) + ((ks * KT + (col - V) / 16) * 64 + lane) * 8;
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) {
+          *(b8*)(ot + jb * 64 * 8) = hi[jb];
+          *(b8*)(ot + K * K + jb * 64 * 8) = lo[jb];
+        }
+      }
     }
   }
 }
 
-template <int K>
+template <int K, bool REVERSE>
 __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* states, const bf16* trans, const float* init,
                                                                        SplitView split, const int64_t* offsets, int64_t T,
                                                                        int H, int V) {
@@ -393,7 +402,8 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
     f32x4 s;
   } A, B;
   auto load = [&](Regs& R, int seg) __attribute__((always_inline)) {
-    const int x = seg < nseg - 1 ? seg : nseg - 2;   // (the last segment has neither)
+    // `seg` counts in the order of the walk: backwards the segments come from the last to the second
+    const int y = seg < nseg - 1 ? seg : nseg - 2, x = REVERSE ? nseg - 1 - y : y;
 #pragma unroll
     for (int part = 0; part < 2; ++part)
 #pragma unroll
@@ -413,7 +423,7 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
     // the state entering this segment takes the place of its S, which this lane has read
     f32x4 a0 = R.s, a1 = zero4(), a2 = zero4();
 #pragma unroll
-    for (int r = 0; r < 4; ++r) S[seg * sstr + (int64_t)r * V] = h[r];
+    for (int r = 0; r < 4; ++r) S[(REVERSE ? nseg - 1 - seg : seg) * sstr + (int64_t)r * V] = h[r];
     lds_barrier();
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -443,7 +453,7 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
     }
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) S[(nseg - 1) * sstr + (int64_t)r * V] = h[r];
+  for (int r = 0; r < 4; ++r) S[(REVERSE ? 0 : nseg - 1) * sstr + (int64_t)r * V] = h[r];
 }
 
 template <typename T, bool L2N>
@@ -462,6 +472,20 @@ int launch_gdr_pass(const GdrPassParams& p, int K, int V, unsigned grid, hipStre
   return FLA_E_UNSUPPORTED;
 }
 
+template <bool REVERSE>
+int launch_gdr_fold(const float* init, const fla_split* split, const int64_t* offsets, int64_t T, int64_t H, int64_t K, int64_t V,
+                    int64_t N, hipStream_t st) {
+  const dim3 grid((unsigned)(N * H), (unsigned)(V / 16));
+  if (K == 128)
+    hipLaunchKernelGGL((gdr_split_fold_kernel<128, REVERSE>), grid, dim3(512), 0, st, split->states, (const bf16*)split->decays,
+                       init, split_view(split), offsets, T, (int)H, (int)V);
+  else
+    hipLaunchKernelGGL((gdr_split_fold_kernel<64, REVERSE>), grid, dim3(256), 0, st, split->states, (const bf16*)split->decays,
+                       init, split_view(split), offsets, T, (int)H, (int)V);
+  FLA_CHECK_LAUNCH();
+  return FLA_OK;
+}
+
 }  // namespace
 
 int gdr_split_states(const void* k, const void* v, const void* AT, const float* g_cumsum, const float* k_rstd, const float* init,
@@ -471,8 +495,9 @@ int gdr_split_states(const void* k, const void* v, const void* AT, const float* 
   if (rc) return rc;
   FLA_REQUIRE(split->decays && split->ratio == 1, FLA_E_INVALID);
   FLA_REQUIRE(BT * H * K * 2 <= 0x7fffffffLL && BT * H * V * 2 <= 0x7fffffffLL, FLA_E_UNSUPPORTED);   // 32-bit offsets in a chunk
-  GdrPassParams p{k, v, AT, g_cumsum, k_rstd, split->states, (bf16*)split->decays, offsets, chunk_offsets, split_view(split), T, (int)H,
-                  split->nseg - 1, (int)((V + K + 127) / 128)};
+  GdrPassParams p{k, v, AT, g_cumsum, k_rstd, split->states, (bf16*)split->decays, (bf16*)split->transitions_t, offsets,
+                  chunk_offsets, split_view(split), T, (int)H, split->nseg - (split->transitions_t ? 0 : 1),
+                  (int)((V + K + 127) / 128)};
   const int64_t subs = offsets ? split->nsub : (int64_t)p.per_seq * N;
   FLA_REQUIRE(subs * H * p.col_wgs <= 0x7fffffffLL && N * H <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
   if (subs > 0) {
@@ -485,13 +510,10 @@ int gdr_split_states(const void* k, const void* v, const void* AT, const float* 
       rc = FLA_E_UNSUPPORTED;
     if (rc) return rc;
   }
-  const dim3 fgrid((unsigned)(N * H), (unsigned)(V / 16));
-  if (K == 128)
-    hipLaunchKernelGGL(gdr_split_fold_kernel<128>, fgrid, dim3(512), 0, st, split->states, (const bf16*)split->decays, init, p.split, offsets,
-                       T, (int)H, (int)V);
-  else
-    hipLaunchKernelGGL(gdr_split_fold_kernel<64>, fgrid, dim3(256), 0, st, split->states, (const bf16*)split->decays, init, p.split, offsets,
-                       T, (int)H, (int)V);
-  FLA_CHECK_LAUNCH();
-  return FLA_OK;
+  return launch_gdr_fold<false>(init, split, offsets, T, H, K, V, N, st);
+}
+
+int gdr_split_fold_reverse(const float* init, const fla_split* split, const int64_t* offsets, int64_t T, int64_t H, int64_t K,
+                           int64_t V, int64_t N, hipStream_t st) {
+  return launch_gdr_fold<true>(init, split, offsets, T, H, K, V, N, st);
 }

@@ -105,6 +105,30 @@ FLA_DEVICE ScanSpan scan_span(const SplitView& v, int64_t i, const int64_t* seq_
   return r;
 }
 
+// Item i of a first pass from right to left over segments of one sub-block: every segment but a sequence's first.
+FLA_DEVICE ScanSpan pass_span(const SplitView& v, int64_t i, int per_seq, const int64_t* offsets, const int64_t* chunk_offsets,
+                              int64_t T) {
+  ScanSpan r;
+  int s;
+  if (v.sub_table) {
+    r.n = v.sub_table[2 * i];
+    s = v.sub_table[2 * i + 1];
+  } else {
+    r.n = (int)((uint32_t)i / (uint32_t)per_seq);
+    s = (int)((uint32_t)i % (uint32_t)per_seq) + 1;
+  }
+  const SeqSpan whole = seq_span(offsets, r.n, T);
+  const int64_t all = (whole.len + BT - 1) / BT, c0 = (int64_t)s * v.sub_chunks;
+  r.first = false;
+  r.last = c0 + v.sub_chunks >= all;
+  r.nchunks = r.last ? all - c0 : v.sub_chunks;
+  r.sp.bos = whole.bos + c0 * BT;
+  r.sp.len = r.last ? whole.len - c0 * BT : (int64_t)v.sub_chunks * BT;
+  r.chunk0 = (chunk_offsets ? chunk_offsets[r.n] : (int64_t)r.n * ((T + BT - 1) / BT)) + c0;
+  r.slot = (v.sub_base ? v.sub_base[r.n] : (int64_t)r.n * v.nsub) + s;
+  return r;
+}
+
 }  // namespace
 
 // gla_split.hip: the two launches ahead of a GLA scan over cut sequences.  Forward: a = k, b = v, g = the gates, init the
@@ -118,3 +142,7 @@ int gla_split_states(const void* a, const void* b, const void* g, const float* i
 int gdr_split_states(const void* k, const void* v, const void* AT, const float* g_cumsum, const float* k_rstd, const float* init,
                      const fla_split* split, const int64_t* offsets, const int64_t* chunk_offsets, int qkv_dtype, int64_t T,
                      int64_t H, int64_t K, int64_t V, int64_t N, hipStream_t st);
+// ... and, backwards, the fold alone: `states` holds what every segment adds to a zero gradient, split->decays the transposed
+// transitions the forward left, init the gradients of the final states.
+int gdr_split_fold_reverse(const float* init, const fla_split* split, const int64_t* offsets, int64_t T, int64_t H, int64_t K,
+                           int64_t V, int64_t N, hipStream_t st);

@@ -339,7 +339,7 @@ struct GdrArgs {
   std::optional<double> l2norm_eps;
 };
 struct GdrKept {
-  Tensor gc, w, Aw, v_new, hT, Aqk;
+  Tensor gc, w, Aw, v_new, hT, Aqk, Mt;   // Mt: the segments' transposed transitions where the forward was cut
 };
 
 Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& h0,
@@ -351,7 +351,7 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   Tensor o = fresh_like(v);
   if (a.want_ht) *ht = fresh({d.N, d.H, d.K, d.V}, q, at::kFloat);
   // sequences cut into segments: their K x K transitions take the place of the decays
-  const auto cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K * d.K,
+  auto cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K * d.K,
                             kept ? FLA_SCAN_DELTA_KEPT : FLA_SCAN_DELTA);
   auto scan_cut = [&](const Tensor& rstd, const GdrKept& x) {
     check(fla_chunk_gated_delta_rule_fwd_scan_split(ptr(q), ptr(k), ptr(v), ptr(AT), fptr(gc), fptr(rstd), fptr(h0), ptr(o),
@@ -383,6 +383,10 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
     x.v_new = fresh_like(v);
     x.hT = fresh({d.chunks, d.H, d.K, d.V}, q, q.scalar_type());
     x.Aqk = fresh_like(AT);
+    if (cut) {
+      x.Mt = fresh_like(cut->transitions);
+      cut->s.transitions_t = fptr(x.Mt);
+    }
   }
   check(fla_gdr_fwd_prep(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), ptr(x.w), ptr(x.Aw), offs(a.plan), idx(a.plan),
                          d.NT, dt(q), d.B, d.T, d.H, d.K, st),
@@ -413,7 +417,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     Tensor ht;
     GdrKept x;
     Tensor o = gdr_forward(q, k, v, g, beta, h0, a, &ht, &x);
-    ctx->save_for_backward({q, k, v, beta, x.gc, x.w, x.Aw, x.v_new, x.hT, x.Aqk});
+    ctx->save_for_backward({q, k, v, beta, x.gc, x.w, x.Aw, x.v_new, x.hT, x.Aqk, x.Mt});
     ctx->set_materialize_grads(false);
     Rest r{a, std::nullopt, beta_.scalar_type(), h0.defined()};
     if (g_) r.g_type = g_->scalar_type();
@@ -428,7 +432,8 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     const GdrArgs& a = r.a;
     const Dims& d = a.d;
     const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &beta = saved[3], &gc = saved[4], &w = saved[5], &Aw = saved[6],
-                 &v_new = saved[7], &hT = saved[8], &Aqk = saved[9];
+                 &v_new = saved[7], &hT = saved[8], &Aqk = saved[9],
+                 &Mt = saved[10];
     const Tensor dout = grads[0].defined() ? as(grads[0], q.scalar_type()).contiguous() : at::zeros(v.sizes(), v.options());
     const Tensor dht = a.want_ht ? f32(grads[1]) : Tensor();
     Tensor dv2 = fresh_like(v), dh = fresh_like(hT), dw = fresh_like(k), dkp = fresh_like(k);
@@ -436,6 +441,19 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     Tensor dq = fresh_like(q), dk = fresh_like(k), dv = fresh_like(v);
     Tensor dbeta = fresh({d.B, d.T, d.H}, q, at::kFloat), dg = fresh({d.B, d.T, d.H}, q, at::kFloat);
     Tensor dh0 = r.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
+    std::optional<Cut> cut;
+    if (Mt.defined())
+      cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), true, q, d.K * d.V, 0, FLA_SCAN_DELTA_KEPT);
+    if (cut) {
+      cut->s.decays = fptr(Mt);
+      check(fla_chunk_gated_delta_rule_bwd_split(
+                ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout), fptr(dht), ptr(hT),
+                ptr(Aqk), ptr(dv2), ptr(dh), ptr(dw), ptr(dkp), fptr(dgam), ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg),
+                fptr(dh0), offs(a.plan), idx(a.plan), coff(a.plan), &cut->s, d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
+                (float)a.scale, stream_of(q)),
+            "fla_chunk_gated_delta_rule_bwd_split");
+      return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor()};
+    }
     check(fla_chunk_gated_delta_rule_bwd(ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout),
                                          fptr(dht), ptr(hT), ptr(Aqk), nullptr, ptr(dv2), ptr(dh), ptr(dw), ptr(dkp),
                                          fptr(dgam), ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg), fptr(dh0),

@@ -26,7 +26,7 @@ P, I64, I, F = c_void_p, c_int64, c_int, c_float
 class Split(ctypes.Structure):
     """``fla_split`` of include/fla_hip.h: how a scan cuts its sequences into segments."""
     _fields_ = [(n, ctypes.c_int32) for n in ("sub_chunks", "ratio", "nseg", "nsub", "slots", "reserved")] + \
-               [(n, c_void_p) for n in ("seg_table", "sub_table", "sub_base", "states", "decays")]
+               [(n, c_void_p) for n in ("seg_table", "sub_table", "sub_base", "states", "decays", "transitions_t")]
 
 
 # name -> (restype, argtypes); mirrors include/fla_hip.h declaration by declaration
@@ -80,6 +80,7 @@ SIGNATURES = {
     "fla_chunk_bwd_dh": (c_int, [P] * 9 + [I, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_states_to_fragments": (c_int, [P, P, I, I, I, I64, I64, I64, P]),
     "fla_chunk_bwd_dv_local": (c_int, [P] * 7 + [I64, I, I64, I64, I64, I64, I64, F, P]),
+    "fla_chunk_gated_delta_rule_bwd_split": (c_int, [P] * 27 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_bwd": (c_int, [P] * 27 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_bwd_dhu": (c_int, [P] * 12 + [I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_bwd_dqkwg": (c_int, [P] * 15 + [I64, I, I64, I64, I64, I64, I64, F, P]),

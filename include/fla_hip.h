@@ -63,7 +63,8 @@ int fla_prepare_chunk_indices(const int64_t* offsets_host, int64_t n_seqs, int64
  * Equal-length sequences: nseg segments and nsub sub-blocks each, no tables.  Packed batches: nseg rows of seg_table
  * (sequence, segment), nsub rows of sub_table (sequence, sub-block: those the first pass forms), sub_base [N+1] the first
  * slot of a sequence.  states [slots, H, K, V] and decays [slots, H, K] (GLA) or its transitions, [slots, H, K, K] words
- * (delta rule), are workspaces. */
+ * (delta rule), are workspaces; transitions_t [slots, H, K, K] words, or NULL: a forward that keeps its intermediates leaves
+ * the transposed transitions there for its backward. */
 typedef struct fla_split {
   int32_t sub_chunks, ratio, nseg, nsub, slots, reserved;
   const int32_t* seg_table;
@@ -71,6 +72,7 @@ typedef struct fla_split {
   const int32_t* sub_base;
   float* states;
   float* decays;
+  float* transitions_t;
 } fla_split;
 
 enum fla_scan_kind { FLA_SCAN_GLA = 0, FLA_SCAN_DELTA = 1, FLA_SCAN_DELTA_KEPT = 2 /* keeps its intermediates */ };
@@ -613,6 +615,16 @@ int fla_chunk_gated_delta_rule_bwd(
     void* dq, void* dk, void* dv, float* dbeta, float* dg, float* dh0,
     const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, int64_t NT, int qkv_dtype,
     int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
+
+/* The same on sequences cut into segments as the forward cut them (fla_scan_split with V / 64 slabs, reverse, kind
+ * FLA_SCAN_DELTA_KEPT); split->decays holds the transposed transitions the forward left.  Needs Aqk. */
+int fla_chunk_gated_delta_rule_bwd_split(
+    const void* q, const void* k, const void* v, const void* w, const void* v_new, const float* beta,
+    const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
+    void* ws_dv2, void* ws_dh_frag_t, void* ws_dw, void* ws_dk_partial, float* ws_dgam_partial,
+    void* dq, void* dk, void* dv, float* dbeta, float* dg, float* dh0,
+    const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split, int64_t NT,
+    int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
 
 /* The launches of fla_chunk_gated_delta_rule_bwd one by one, for callers that hold the reference's own
  * intermediates (the sibling operators that call these stages directly).  States cross this boundary in

@@ -96,7 +96,7 @@ def test_gdr_cut_sequences(device, B, T, H, K, V, bounds, dtype, gated):
     from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(N, T, H, V // 64, False, bounds, 1)
+    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
     print("cut delta rule", B, T, H, K, V, bounds, dtype, gated, flush=True)
     q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=2000.0, N=N)
     beta = beta * 0.02
