@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256, 2) void gla_split_pass_kernel(SplitPassParams 
           Es[r] = run;
           run = fmaf(R.gh[r], LOG2E, run);
         }
-        const float suf = row_suffix16(run), later = suf - run + carry[0];
+        const float suf = row_suffix16(run), later = dpp_f32<0x101>(suf) + carry[0];   // row_shl:1, the later row groups
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -147,7 +147,9 @@ __global__ __launch_bounds__(256, 2) void gla_split_pass_kernel(SplitPassParams 
             if constexpr (MODE == kPassGateLogits) run += log2_sigmoid_gate((float)R.g[r][jx], p.gate_inv_norm, clamp2);
             else run = fmaf((float)R.g[r][jx], LOG2E, run);
           }
-          const float suf = row_suffix16(run), later = suf - run + carry[jx];
+          // the later row groups' sum from the lane that has it: as a difference it would be lost behind a gate that
+          // resets the state (-1e30), and NaN behind -inf
+          const float suf = row_suffix16(run), later = dpp_f32<0x101>(suf) + carry[jx];
 #pragma unroll
           for (int r = 0; r < 4; ++r) E[r][jx] += later;
           carry[jx] += dpp_f32<0x150>(suf);

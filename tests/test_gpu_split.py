@@ -139,3 +139,26 @@ def test_gdr_cut_l2norm_in_kernel(device, K, V):
     ro, rht = naive_recurrent_gated_delta_rule(l2norm(q), l2norm(k), v, g, beta, initial_state=h0, output_final_state=True)
     assert_close("o", ro, o, 1e-2)
     assert_close("ht", rht, ht, 5e-3)
+
+
+@pytest.mark.parametrize("heads", [False, True])
+def test_gla_cut_state_behind_a_reset(device, heads):
+    """A gate of -1e30 drops the state.  The tokens behind it inside its chunk keep their own decays, which a difference
+    of sums that contain the reset would lose; what enters the next segment is made of them."""
+    from fla_amd import _backend as be
+    from fla_amd.ops.gla import chunk_gla
+    T = 1000
+    sp = be.Split()
+    assert be.lib().fla_scan_split(None, 1, T, 2, 1, 0, 0, ctypes.byref(sp), None, None, None)
+    seg = 64 * sp.sub_chunks * sp.ratio
+    q, k, v, g, h0 = gla_inputs(1, T, 2, 64, 64, seed=9, normalizer=16.0)
+    g[:, seg - 64 + 8] = -1e30          # the first row of a group of four, 55 tokens ahead of the next segment
+    if heads:
+        g = g[..., :1].expand(-1, -1, -1, 64).contiguous()
+    print("cut, reset", heads, sp.sub_chunks, sp.ratio, flush=True)
+    with torch.no_grad():
+        o, ht = chunk_gla(*(t.to(device) for t in (q, k, v, g)), initial_state=h0.to(device), output_final_state=True,
+                          head_first=False)
+    ro, rht = naive_recurrent_gla(q, k, v, g, initial_state=h0, output_final_state=True)
+    assert_close("o of the segments behind", ro[:, seg:], o[:, seg:], 1e-2)
+    assert_close("ht", rht, ht, 5e-3)
