@@ -10,6 +10,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -90,6 +91,7 @@ const X& held(AutogradContext* ctx) {
 // ---------------------------------------------------------------------------------------------------- packed batches
 struct SplitTables {
   bool cut = false;
+  std::optional<c10::hip::HIPStream> home;   // the stream the tables were allocated on
   fla_split ints{};
   Tensor seg, sub, base;
 };
@@ -101,9 +103,14 @@ struct Plan : torch::CustomClassHolder {
   std::mutex mu;
   std::map<std::tuple<int64_t, int, bool, int>, SplitTables> splits;
 
-  // The tables of a cut are used by later calls on any stream: the copies to the device are synchronous.
+  // The tables of a cut are used by later calls on any stream: the copies to the device are synchronous.  A stream that is
+  // being captured takes no such copy; a call whose tables are not there yet runs uncut under it.
   SplitTables split(int64_t H, int slabs, bool reverse, int kind) {
     std::lock_guard<std::mutex> lock(mu);
+    const auto stream = c10::hip::getCurrentHIPStream(offsets.device().index());
+    if (!splits.count({H, slabs, reverse, kind}) &&
+        c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+      return {};
     auto [it, fresh] = splits.try_emplace({H, slabs, reverse, kind});
     SplitTables& s = it->second;
     if (fresh && N > 0) {
@@ -122,9 +129,14 @@ struct Plan : torch::CustomClassHolder {
         sp.sub_table = (const int32_t*)s.sub.data_ptr();
         sp.sub_base = (const int32_t*)s.base.data_ptr();
         s.ints = sp;
+        s.home = stream;
         s.cut = true;
       }
     }
+    // the plan may be dropped while another stream still reads its tables
+    if (s.cut && *s.home != stream)
+      for (Tensor* t : {&s.seg, &s.sub, &s.base})   // (tensors of this build call their device CUDA)
+        t->record_stream(c10::Stream(c10::Stream::UNSAFE, offsets.device(), stream.id()));
     return s;
   }
 };

@@ -162,3 +162,34 @@ def test_gla_cut_state_behind_a_reset(device, heads):
     ro, rht = naive_recurrent_gla(q, k, v, g, initial_state=h0, output_final_state=True)
     assert_close("o of the segments behind", ro[:, seg:], o[:, seg:], 1e-2)
     assert_close("ht", rht, ht, 5e-3)
+
+
+def test_packed_batch_first_met_under_capture(device):
+    """The tables of a cut are copied to the device by the first call that needs them, which a stream being captured does
+    not take: such a call runs uncut, and one on another stream is cut with the same result."""
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.utils import VarlenPlan
+    bounds = [0, 1290, 1354, 2200]
+    q, k, v, g, _ = (x.to(device) for x in gla_inputs(1, 2200, 1, 64, 64, seed=2, normalizer=600.0))
+    offs = torch.tensor(bounds, device=device)
+    VarlenPlan(offs, 64).native
+    assert _cut(3, 2200, 1, 1, False, bounds)
+    print("capture", flush=True)
+    with torch.no_grad():
+        chunk_gla(q, k, v, g, head_first=False)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            o, _ = chunk_gla(q, k, v, g, cu_seqlens=offs, head_first=False)
+        side = torch.cuda.Stream()
+        eager, _ = chunk_gla(q, k, v, g, cu_seqlens=offs, head_first=False)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            other, _ = chunk_gla(q, k, v, g, cu_seqlens=offs, head_first=False)
+        torch.cuda.synchronize()
+        assert torch.equal(eager, other)
+        for _ in range(3):
+            o.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close("o", eager.float().cpu(), o.cpu(), 1e-2)
