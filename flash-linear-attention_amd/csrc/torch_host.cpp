@@ -54,7 +54,11 @@ Tensor f32(const Tensor& x) {
   if (!x.defined()) return x;
   return (x.scalar_type() == at::kFloat ? x : x.to(at::kFloat)).contiguous();
 }
+// Whether a call has to go through its autograd node.  An operand with a tangent does too, also where nothing requires a
+// gradient: the nodes have no forward-mode derivative and say so, a launch beside them would drop the tangent.
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->defined() && t->_fw_grad(0).defined()) return true;
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
     if (t->defined() && t->requires_grad()) return true;

@@ -193,3 +193,17 @@ def test_packed_batch_first_met_under_capture(device):
             graph.replay()
             torch.cuda.synchronize()
             assert_close("o", eager.float().cpu(), o.cpu(), 1e-2)
+
+
+def test_forward_mode_is_refused(device):
+    """No operator has a forward-mode derivative: a tangent is an error, not dropped."""
+    import torch.autograd.forward_ad as fw
+    from fla_amd.modules import l2_norm
+    from fla_amd.ops.gla import chunk_gla
+    q, k, v, g, _ = (x.to(device) for x in gla_inputs(1, 70, 1, 64, 64, seed=1))
+    with fw.dual_level():
+        x = fw.make_dual(q, torch.ones_like(q))
+        with pytest.raises(RuntimeError):
+            chunk_gla(x, k, v, g, head_first=False)
+        with pytest.raises(RuntimeError):
+            l2_norm(x)
