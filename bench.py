@@ -9,7 +9,7 @@ returned), inputs resident in HBM.  Prints ONE JSON line:
 
 * value            tokens/s of the whole forward: tokens of the K timed steps / the wall time between the two
                    synchronisations that bracket them (ms_per_step = that wall time / K; the host time of a
-                   call with the launches stubbed out is in extra.chunk_gla_fwd.host_us_per_call)
+                   call, the device working beside it, is in extra.chunk_gla_fwd.host_us_per_call)
 * roofline         the dominant kernel of that forward against the HBM roofline:
                    algorithmic bytes per launch / its median duration measured
                    here with HIP events on the launch stream; traffic = HBM bytes per launch from
@@ -189,7 +189,7 @@ def bench_gla(device, steps, warmup):
     ms = wall_us * 1e-3
     tokens_per_s = B * T / (wall_us * 1e-6)
 
-    # host side of one step: the same call with the launch replaced by a stub that returns at once
+    # host side of one step: how long the call takes to return
     host_us = host_time_us(step)
 
     # device time of the kernels of the forward, HIP events on the launch stream.  The operator is one launch
