@@ -207,3 +207,32 @@ def test_forward_mode_is_refused(device):
             chunk_gla(x, k, v, g, head_first=False)
         with pytest.raises(RuntimeError):
             l2_norm(x)
+
+
+@pytest.mark.parametrize("dtype,heads", [(torch.float16, False), (torch.float16, True), (torch.float32, False)])
+def test_gla_cut_keeps_decayed_keys(device, dtype, heads):
+    """Keys whose weight has decayed by e^-14 when their sub-block ends are all that its state is made of (the rest of the
+    keys is zero, as behind a mask).  The decays of whole chunks multiply fp32 numbers: only the rounding of the 16-bit
+    operands k e^{E} (E within a chunk) is left, 2^-11 of each at most and 2^-11 / sqrt(3) of their sum; fp32 inputs
+    round v too."""
+    from fla_amd import _backend as be
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    T, H, D = 2048, 64, 64
+    sp = be.Split()
+    assert be.lib().fla_scan_split(None, 1, T, H, 1, 0, 0, ctypes.byref(sp), None, None, None)
+    sub = 64 * sp.sub_chunks
+    assert sub >= 512 and sub < T
+    q, k, v, g, _ = gla_inputs(1, T, H, D, D, seed=4, dtype=dtype, h0=False)
+    k[:, sub - 280:] = 0
+    g[:, :sub], g[:, sub:] = -0.05, 0.0
+    print("cut, decayed keys", dtype, heads, sub, flush=True)
+    with torch.no_grad():
+        x = [t.to(device) for t in (q, k, v, g)]
+        if heads:
+            o, ht = chunk_simple_gla(*x[:3], x[3][..., 0].contiguous(), output_final_state=True, head_first=False)
+        else:
+            o, ht = chunk_gla(*x, output_final_state=True, head_first=False)
+    w = torch.exp(torch.flip(torch.cumsum(torch.flip(g.double(), [1]), 1), [1]) - g.double())
+    ref = torch.einsum("bthk,bthv->bhkv", k.double() * w, v.double())
+    assert_close("ht", ref, ht, 5e-4)
