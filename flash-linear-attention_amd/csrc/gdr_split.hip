@@ -14,9 +14,12 @@
 // in registers: 2.0 us per chunk (25 us for 7 segments of 10 chunks of 16 heads, K = V = 128).  Tiles staged by the waves
 // that multiply, one chunk ahead: 3.9 - 4.5 us.
 // gdr_split_fold_kernel: h <- M h + S; a workgroup carries 16 value columns of one head through the segments, 16 key rows
-// per wave.  M and h are multiplied as sums of two bf16 numbers (three products, 2^-16 of the result), M is stored that
-// way in operand order by the first launch and requested two segments ahead: a step is 64 KB of M into every CU (11 us for 7 steps).
-// (fp32 M in rows, 16x16x4 fp32 instructions, one segment ahead: 2.1 us per segment.)
+// per wave.  The state is fp32 in the scan and stays so between the segments: M and h are multiplied as sums of three bf16
+// numbers (exactly their 24 bits; six products, what is left out is below 2^-23 of the result), a transition that is the
+// identity hands on every bit.  M is stored in fp32, in operand order, and requested two segments ahead: a step is 64 KB of
+// M into every CU.  Two bf16 numbers apiece and three products lost the last 8 bits for 3 us less of the forward of one
+// sequence of 5003 tokens, 16 heads (79.6 against 82.5); fp32 M in rows, 16x16x4 fp32 instructions, one segment ahead: 2.1 us
+// per segment.
 #include "seq_split.h"
 
 namespace {
@@ -28,14 +31,34 @@ struct GdrPassParams {
   const float* gam;     // chunk-local prefix sums of the gate, or NULL
   const float* rk;      // L2N: 1 / |k|, [rows, H]
   float* states;        // out: S, [slots, H, K, V]
-  bf16* trans;          // out: M, [slots, H, 2 (high, low part), K/32 slices, K/16 row tiles, 64 lanes, 8]
-  bf16* trans_t;        // out, or NULL: M^T in the same order
+  float* trans;         // out: M, [slots, H, K/32 slices, K/16 row tiles, 2, 64 lanes, 4]
+  float* trans_t;       // out, or NULL: M^T in the same order
   const int64_t* offsets;
   const int64_t* chunk_offsets;
   SplitView split;
   int64_t T;
   int H, per_seq, col_wgs;
 };
+
+// Eight fp32 numbers as sums of three bf16 numbers each, exactly: 8 significant bits apiece, cut off, never rounded up (a
+// finite number stays finite).
+FLA_DEVICE void split3(f32x4 a, f32x4 b, bf16x8* out) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  u4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float x0 = i < 2 ? a[2 * i] : b[2 * i - 4], x1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+      const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+      w[part][i] = __builtin_amdgcn_perm(u1, u0, 0x07060302);   // the upper halves, x0's in the low one
+      x0 -= __uint_as_float(u0 & 0xffff0000u);
+      x1 -= __uint_as_float(u1 & 0xffff0000u);
+    }
+  }
+#pragma unroll
+  for (int part = 0; part < 3; ++part) out[part] = __builtin_bit_cast(bf16x8, w[part]);
+}
 
 template <typename T, int K, int V, bool L2N>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdr_split_pass_kernel(GdrPassParams p) {
@@ -328,61 +351,48 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 4; ++r) out[(16 * kt + 4 * g + r) * V + 16 * jb] = acc[jb][kt][r];
   } else if (is_m) {
-    // This wave's columns are one slice of 32 of the contraction index.  An accumulator pair converted to 16 bits and
-    // multiplied by the identity in accumulator-row order comes out with lanes and registers exchanged (exact for the
-    // 16-bit values): a lane then holds four columns of one row, and both column blocks of the wave together are its
-    // eight slots of the fold's operand.
+    // This wave's columns are one slice of 32 of the contraction index.  An accumulator pair multiplied by the identity in
+    // accumulator-row order, part by part, comes out with lanes and registers exchanged and every bit in place: a lane then
+    // holds four columns of one row, and both column blocks of the wave together are its eight slots of the fold's operand.
     typedef bf16x8 b8;
     b8 eye[2];
 #pragma unroll
     for (int half = 0; half < 2; ++half)
 #pragma unroll
       for (int e = 0; e < 8; ++e) eye[half][e] = (bf16)(((e >> 2) == half && 4 * g + (e & 3) == c) ? 1.f : 0.f);
-    bf16* out = p.trans + (slot * H + hh) * (int64_t)(2 * K * K) + ((col - V) / 32 * KT * 64 + lane) * 8;
+    float* out = p.trans + (slot * H + hh) * (int64_t)(K * K) + ((col - V) / 32 * KT * 128 + lane) * 4;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      b8 hi[2], lo[2];
 #pragma unroll
-      for (int jb = 0; jb < 2; ++jb)
+      for (int jb = 0; jb < 2; ++jb) {
+        b8 x[3];
+        split3(acc[jb][2 * ks], acc[jb][2 * ks + 1], x);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = acc[jb][2 * ks + (e >> 2)][e & 3];
-          hi[jb][e] = (bf16)x;
-          lo[jb][e] = (bf16)(x - (float)hi[jb][e]);
+        for (int half = 0; half < 2; ++half) {
+          f32x4 t = Elem<bf16>::mfma16(x[0], eye[half], zero4());
+          t = Elem<bf16>::mfma16(x[1], eye[half], t);
+          *(f32x4*)(out + ((2 * ks + half) * 2 + jb) * 256) = Elem<bf16>::mfma16(x[2], eye[half], t);
         }
-#pragma unroll
-      for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          b8 y;
-#pragma unroll
-          for (int jb = 0; jb < 2; ++jb) {
-            const f32x4 t = Elem<bf16>::mfma16(part ? lo[jb] : hi[jb], eye[half], zero4());
-#pragma unroll
-            for (int r = 0; r < 4; ++r) y[4 * jb + r] = (bf16)t[r];
-          }
-          *(b8*)(out + part * K * K + (2 * ks + half) * 64 * 8) = y;
-        }
+      }
       if (p.trans_t) {   // a column of M is a row of M^T: the accumulators are the operand as they are
-        bf16* ot = p.trans_t + (slot * H + hh) * (int64_t)(2 * K * K) + ((ks * KT + (col - V) / 16) * 64 + lane) * 8;
+        float* ot = p.trans_t + (slot * H + hh) * (int64_t)(K * K) + ((ks * KT + (col - V) / 16) * 128 + lane) * 4;
 #pragma unroll
-        for (int jb = 0; jb < 2; ++jb) {
-          *(b8*)(ot + jb * 64 * 8) = hi[jb];
-          *(b8*)(ot + K * K + jb * 64 * 8) = lo[jb];
-        }
+        for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) *(f32x4*)(ot + (jb * 2 + half) * 256) = acc[jb][2 * ks + half];
       }
     }
   }
 }
 
 template <int K, bool REVERSE>
-__global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* states, const bf16* trans, const float* init,
+__global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* states, const float* trans, const float* init,
                                                                        SplitView split, const int64_t* offsets, int64_t T,
                                                                        int H, int V) {
   constexpr int KS = K / 32, KT = K / 16;
   typedef bf16x4 b4;
   typedef bf16x8 b8;
-  __shared__ __attribute__((aligned(16))) bf16 sH[2][2][KT * 64 * 4];   // high and low part of the slab, [row tile][lane][4]
+  __shared__ __attribute__((aligned(16))) bf16 sH[2][3][KT * 64 * 4];   // the parts of the slab, [row tile][lane][4]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // heads fastest: the column slabs of a head, which read the same M, land on one XCD and its L2
@@ -392,54 +402,55 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
   const int nseg = (int)split_nsub(split, (sp.len + BT - 1) / BT);   // a segment is one sub-block
   const int64_t base = split.sub_base ? split.sub_base[n] : (int64_t)n * split.nsub;
   float* S = states + (base * H + hh) * (int64_t)K * V + (int64_t)(16 * wave + 4 * g) * V + cb + c;
-  const bf16* M = trans + (base * H + hh) * (int64_t)(2 * K * K) + (wave * 64 + lane) * 8;
-  const int64_t sstr = (int64_t)H * K * V, mstr = (int64_t)H * 2 * K * K;
+  const float* M = trans + (base * H + hh) * (int64_t)(K * K) + (wave * 128 + lane) * 4;
+  const int64_t sstr = (int64_t)H * K * V, mstr = (int64_t)H * K * K;
   f32x4 h;   // rows 16 wave + 4 g .. + 3 of column cb + c
 #pragma unroll
   for (int r = 0; r < 4; ++r) h[r] = init ? init[(int64_t)nh * K * V + (int64_t)(16 * wave + 4 * g + r) * V + cb + c] : 0.f;
   struct Regs {
-    b8 m[2][KS];
+    f32x4 m[KS][2];
     f32x4 s;
   } A, B;
   auto load = [&](Regs& R, int seg) __attribute__((always_inline)) {
     // `seg` counts in the order of the walk: backwards the segments come from the last to the second
     const int y = seg < nseg - 1 ? seg : nseg - 2, x = REVERSE ? nseg - 1 - y : y;
 #pragma unroll
-    for (int part = 0; part < 2; ++part)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) R.m[part][ks] = *(const b8*)(M + x * mstr + part * K * K + ks * KT * 64 * 8);
+      for (int half = 0; half < 2; ++half) R.m[ks][half] = *(const f32x4*)(M + x * mstr + ks * KT * 512 + half * 256);
 #pragma unroll
     for (int r = 0; r < 4; ++r) R.s[r] = S[x * sstr + (int64_t)r * V];
   };
   auto step = [&](Regs& R, int seg) __attribute__((always_inline)) {
-    b4 hi, lo;
+    b8 hp[3];
+    split3(h, h, hp);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      hi[r] = (bf16)h[r];
-      lo[r] = (bf16)(h[r] - (float)hi[r]);
-    }
-    *(b4*)&sH[seg & 1][0][(wave * 64 + lane) * 4] = hi;
-    *(b4*)&sH[seg & 1][1][(wave * 64 + lane) * 4] = lo;
+    for (int part = 0; part < 3; ++part)
+      *(b4*)&sH[seg & 1][part][(wave * 64 + lane) * 4] = __builtin_shufflevector(hp[part], hp[part], 0, 1, 2, 3);
     // the state entering this segment takes the place of its S, which this lane has read
-    f32x4 a0 = R.s, a1 = zero4(), a2 = zero4();
+    f32x4 a[6] = {R.s, zero4(), zero4(), zero4(), zero4(), zero4()};
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[(REVERSE ? nseg - 1 - seg : seg) * sstr + (int64_t)r * V] = h[r];
     lds_barrier();
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      b8 x[2];
+      b8 m[3], x[3];
+      split3(R.m[ks][0], R.m[ks][1], m);
 #pragma unroll
-      for (int part = 0; part < 2; ++part) {
+      for (int part = 0; part < 3; ++part) {
         const b4 t0 = *(const b4*)&sH[seg & 1][part][(2 * ks * 64 + lane) * 4];
         const b4 t1 = *(const b4*)&sH[seg & 1][part][((2 * ks + 1) * 64 + lane) * 4];
         x[part] = __builtin_shufflevector(t0, t1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
-      a0 = Elem<bf16>::mfma16(R.m[0][ks], x[0], a0);
-      a1 = Elem<bf16>::mfma16(R.m[0][ks], x[1], a1);
-      a2 = Elem<bf16>::mfma16(R.m[1][ks], x[0], a2);
+      a[0] = Elem<bf16>::mfma16(m[0], x[0], a[0]);
+      a[1] = Elem<bf16>::mfma16(m[0], x[1], a[1]);
+      a[2] = Elem<bf16>::mfma16(m[1], x[0], a[2]);
+      a[3] = Elem<bf16>::mfma16(m[0], x[2], a[3]);
+      a[4] = Elem<bf16>::mfma16(m[1], x[1], a[4]);
+      a[5] = Elem<bf16>::mfma16(m[2], x[0], a[5]);
     }
     load(R, seg + 2);
-    h = a0 + (a1 + a2);
+    h = a[0] + ((a[1] + a[2]) + (a[3] + (a[4] + a[5])));
   };
   if (nseg > 1) {
     load(A, 0);
@@ -477,10 +488,10 @@ int launch_gdr_fold(const float* init, const fla_split* split, const int64_t* of
                     int64_t N, hipStream_t st) {
   const dim3 grid((unsigned)(N * H), (unsigned)(V / 16));
   if (K == 128)
-    hipLaunchKernelGGL((gdr_split_fold_kernel<128, REVERSE>), grid, dim3(512), 0, st, split->states, (const bf16*)split->decays,
+    hipLaunchKernelGGL((gdr_split_fold_kernel<128, REVERSE>), grid, dim3(512), 0, st, split->states, split->decays,
                        init, split_view(split), offsets, T, (int)H, (int)V);
   else
-    hipLaunchKernelGGL((gdr_split_fold_kernel<64, REVERSE>), grid, dim3(256), 0, st, split->states, (const bf16*)split->decays,
+    hipLaunchKernelGGL((gdr_split_fold_kernel<64, REVERSE>), grid, dim3(256), 0, st, split->states, split->decays,
                        init, split_view(split), offsets, T, (int)H, (int)V);
   FLA_CHECK_LAUNCH();
   return FLA_OK;
@@ -495,7 +506,7 @@ int gdr_split_states(const void* k, const void* v, const void* AT, const float* 
   if (rc) return rc;
   FLA_REQUIRE(split->decays && split->ratio == 1, FLA_E_INVALID);
   FLA_REQUIRE(BT * H * K * 2 <= 0x7fffffffLL && BT * H * V * 2 <= 0x7fffffffLL, FLA_E_UNSUPPORTED);   // 32-bit offsets in a chunk
-  GdrPassParams p{k, v, AT, g_cumsum, k_rstd, split->states, (bf16*)split->decays, (bf16*)split->transitions_t, offsets,
+  GdrPassParams p{k, v, AT, g_cumsum, k_rstd, split->states, split->decays, split->transitions_t, offsets,
                   chunk_offsets, split_view(split), T, (int)H, split->nseg - (split->transitions_t ? 0 : 1),
                   (int)((V + K + 127) / 128)};
   const int64_t subs = offsets ? split->nsub : (int64_t)p.per_seq * N;

@@ -236,3 +236,33 @@ def test_gla_cut_keeps_decayed_keys(device, dtype, heads):
     w = torch.exp(torch.flip(torch.cumsum(torch.flip(g.double(), [1]), 1), [1]) - g.double())
     ref = torch.einsum("bthk,bthv->bhkv", k.double() * w, v.double())
     assert_close("ht", ref, ht, 5e-4)
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.bfloat16), (128, 128, torch.float16), (64, 128, torch.bfloat16),
+                                       (128, 64, torch.bfloat16)])
+@pytest.mark.parametrize("bounds", [None, [0, 1, 1, 2460, 2500]])
+def test_gdr_cut_state_passes_in_fp32(device, K, V, dtype, bounds):
+    """Tokens without a correction (beta = 0) and without decay leave the state, and from the right its gradient, as they
+    are, bit by bit: every segment's transition is the identity and no bit of a state may be lost between them.  An entry
+    that is not finite stays in its value column."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    T, H = 2500, 2
+    N = 1 if bounds is None else len(bounds) - 1
+    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
+    q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, T, H, K, V, seed=6, dtype=dtype, N=N))
+    kw = dict(output_final_state=True, head_first=False,
+              cu_seqlens=None if bounds is None else torch.tensor(bounds, device=device))
+    print("cut, state passes", K, V, dtype, bounds, flush=True)
+    with torch.no_grad():
+        _, ht = chunk_gated_delta_rule(q, k, v, g * 0, beta * 0, initial_state=h0, **kw)
+        assert torch.equal(ht, h0)
+        h0[..., 3, 5] = float("inf")
+        _, ht = chunk_gated_delta_rule(q, k, v, g * 0, beta * 0, initial_state=h0, **kw)
+        rest = torch.arange(V, device=device) != 5
+        assert torch.equal(ht[..., rest], h0[..., rest])
+        h0[..., 3, 5] = 0.0
+    h0.requires_grad_()
+    o, ht = chunk_gated_delta_rule(q, k, v, g * 0, beta * 0, initial_state=h0, **kw)
+    dht = torch.randn(ht.shape, device=device)
+    torch.autograd.backward((o, ht), (torch.zeros_like(o), dht))
+    assert torch.equal(ht, h0) and torch.equal(h0.grad, dht)
