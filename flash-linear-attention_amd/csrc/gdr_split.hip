@@ -15,11 +15,11 @@
 // that multiply, one chunk ahead: 3.9 - 4.5 us.
 // gdr_split_fold_kernel: h <- M h + S; a workgroup carries 16 value columns of one head through the segments, 16 key rows
 // per wave.  The state is fp32 in the scan and stays so between the segments: M and h are multiplied as sums of three bf16
-// numbers (exactly their 24 bits; six products, what is left out is below 2^-23 of the result), a transition that is the
+// numbers (exactly their 24 bits; eight products, the ninth is below 2^-30 of the result), a transition that is the
 // identity hands on every bit.  M is stored in fp32, in operand order, and requested two segments ahead: a step is 64 KB of
-// M into every CU.  Two bf16 numbers apiece and three products lost the last 8 bits for 3 us less of the forward of one
-// sequence of 5003 tokens, 16 heads (79.6 against 82.5); fp32 M in rows, 16x16x4 fp32 instructions, one segment ahead: 2.1 us
-// per segment.
+// M into every CU, 15.4 us for 7 steps.  Two bf16 numbers apiece and three products lost the last 8 bits for 11.5 us (forward
+// of one sequence of 5003 tokens, 16 heads: 80.4 against 84.0); M split a step ahead out of three register sets: 15.6 us;
+// fp32 M in rows, 16x16x4 fp32 instructions, one segment ahead: 2.1 us per segment.
 #include "seq_split.h"
 
 namespace {
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
     for (int part = 0; part < 3; ++part)
       *(b4*)&sH[seg & 1][part][(wave * 64 + lane) * 4] = __builtin_shufflevector(hp[part], hp[part], 0, 1, 2, 3);
     // the state entering this segment takes the place of its S, which this lane has read
-    f32x4 a[6] = {R.s, zero4(), zero4(), zero4(), zero4(), zero4()};
+    f32x4 a[6] = {R.s, zero4(), zero4(), zero4(), zero4(), zero4()};   // by the order of the products
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[(REVERSE ? nseg - 1 - seg : seg) * sstr + (int64_t)r * V] = h[r];
     lds_barrier();
@@ -448,6 +448,8 @@ __global__ __launch_bounds__(64 * (K / 16)) void gdr_split_fold_kernel(float* st
       a[3] = Elem<bf16>::mfma16(m[0], x[2], a[3]);
       a[4] = Elem<bf16>::mfma16(m[1], x[1], a[4]);
       a[5] = Elem<bf16>::mfma16(m[2], x[0], a[5]);
+      a[3] = Elem<bf16>::mfma16(m[1], x[2], a[3]);
+      a[5] = Elem<bf16>::mfma16(m[2], x[1], a[5]);
     }
     load(R, seg + 2);
     h = a[0] + ((a[1] + a[2]) + (a[3] + (a[4] + a[5])));
