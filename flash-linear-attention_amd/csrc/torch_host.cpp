@@ -99,7 +99,9 @@ struct SplitTables {
   fla_split ints{};
   Tensor seg, sub, base;
 };
-// The device tables of a packed batch, made once per offsets tensor by fla_amd.utils.VarlenPlan.
+// The device tables of a packed batch, made once per offsets tensor by fla_amd.utils.VarlenPlan.  `offsets` is the caller's
+// own tensor where it is int64: a node saves it, so that a backward after it has been written to is refused instead of
+// combining the other tables, made from the old boundaries, with the new ones.
 struct Plan : torch::CustomClassHolder {
   Tensor offsets, indices, chunk_offsets, seq_order;
   std::vector<int64_t> host;
@@ -272,7 +274,7 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     bool has_h0;
   };
   static variable_list forward(AutogradContext* ctx, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& g_,
-                               const Maybe& h0_, const GlaArgs& a) {
+                               const Maybe& h0_, const Maybe& offsets, const GlaArgs& a) {
     at::AutoDispatchBelowADInplaceOrView guard;
     const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous();
     const Tensor g = (a.head_gates ? f32(g_) : g_.contiguous());
@@ -280,7 +282,7 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     Tensor ht;
     GlaKept x;
     Tensor o = gla_forward(q, k, v, g, h0, a, &ht, &x);
-    ctx->save_for_backward({q, k, v, g, x.wide, x.hT, x.qg, x.decay, x.kh, x.sc});
+    ctx->save_for_backward({q, k, v, g, x.wide, x.hT, x.qg, x.decay, x.kh, x.sc, given(offsets)});
     ctx->set_materialize_grads(false);
     hold(ctx, Rest{a, g_.scalar_type(), h0.defined()});
     return a.want_ht ? variable_list{o, ht} : variable_list{o};
@@ -322,7 +324,7 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
                                    d.T, d.H, d.K, d.V, d.N, (float)a.scale, st),
             "fla_chunk_gla_bwd_kept");
     }
-    return {dq, dk, dv, as(dg, rest.g_type), dh0, Tensor()};
+    return {dq, dk, dv, as(dg, rest.g_type), dh0, Tensor(), Tensor()};
   }
 };
 
@@ -426,14 +428,14 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     bool has_h0;
   };
   static variable_list forward(AutogradContext* ctx, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Maybe& g_,
-                               const Tensor& beta_, const Maybe& h0_, const GdrArgs& a) {
+                               const Tensor& beta_, const Maybe& h0_, const Maybe& offsets, const GdrArgs& a) {
     at::AutoDispatchBelowADInplaceOrView guard;
     const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous(), g = f32(given(g_)), beta = f32(beta_);
     const Tensor h0 = h0_ ? h0_->contiguous() : Tensor();
     Tensor ht;
     GdrKept x;
     Tensor o = gdr_forward(q, k, v, g, beta, h0, a, &ht, &x);
-    ctx->save_for_backward({q, k, v, beta, x.gc, x.w, x.Aw, x.v_new, x.hT, x.Aqk, x.Mt});
+    ctx->save_for_backward({q, k, v, beta, x.gc, x.w, x.Aw, x.v_new, x.hT, x.Aqk, x.Mt, given(offsets)});
     ctx->set_materialize_grads(false);
     Rest r{a, std::nullopt, beta_.scalar_type(), h0.defined()};
     if (g_) r.g_type = g_->scalar_type();
@@ -468,7 +470,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
                 fptr(dh0), offs(a.plan), idx(a.plan), coff(a.plan), &cut->s, d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
                 (float)a.scale, stream_of(q)),
             "fla_chunk_gated_delta_rule_bwd_split");
-      return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor()};
+      return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor(), Tensor()};
     }
     check(fla_chunk_gated_delta_rule_bwd(ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout),
                                          fptr(dht), ptr(hT), ptr(Aqk), nullptr, ptr(dv2), ptr(dh), ptr(dw), ptr(dkp),
@@ -476,7 +478,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
                                          offs(a.plan), idx(a.plan), coff(a.plan), d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
                                          (float)a.scale, stream_of(q)),
           "fla_chunk_gated_delta_rule_bwd");
-    return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor()};
+    return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor(), Tensor()};
   }
 };
 
@@ -669,12 +671,13 @@ PyObject* py_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// chunk_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat, normalizer, clamp)
+// chunk_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat, normalizer, clamp, offsets)
 //   normalizer None: g holds log-gates
 PyObject* py_chunk_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 12);
-  Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]);
+  expect(n, 13);
+  Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]),
+         offsets = arg_tensor(p[12]);
   GlaArgs a{};
   a.plan = arg_plan(p[7]);
   if (!chunk_operands(q, k, v, h0, a.plan, &a.d) || !g.defined() || !g.is_cuda() || g.sizes() != q.sizes()) return none();
@@ -692,7 +695,7 @@ PyObject* py_chunk_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
     a.clamp = arg_opt_double(p[11]);
   }
   if (grad) {
-    auto out = GlaNode::apply(q, k, v, g, maybe(h0), a);
+    auto out = GlaNode::apply(q, k, v, g, maybe(h0), maybe(offsets), a);
     return pair(out[0], a.want_ht ? out[1] : Tensor());
   }
   at::AutoDispatchBelowADInplaceOrView guard;
@@ -703,11 +706,12 @@ PyObject* py_chunk_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// chunk_simple_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat)
+// chunk_simple_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat, offsets)
 PyObject* py_chunk_simple_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 10);
-  Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]);
+  expect(n, 11);
+  Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]),
+         offsets = arg_tensor(p[10]);
   GlaArgs a{};
   a.plan = arg_plan(p[7]);
   if (!chunk_operands(q, k, v, h0, a.plan, &a.d) || !g.defined() || !g.is_cuda() || g.dim() != 3 || g.size(0) != a.d.B ||
@@ -721,7 +725,7 @@ PyObject* py_chunk_simple_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   a.keep_khat = arg_bool(p[9]);
   a.head_gates = true;
   if (grad) {
-    auto out = GlaNode::apply(q, k, v, g, maybe(h0), a);
+    auto out = GlaNode::apply(q, k, v, g, maybe(h0), maybe(offsets), a);
     return pair(out[0], a.want_ht ? out[1] : Tensor());
   }
   at::AutoDispatchBelowADInplaceOrView guard;
@@ -731,12 +735,12 @@ PyObject* py_chunk_simple_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// chunk_gdr(q, k, v, g | None, beta, scale, h0, want_ht, plan, may_differentiate, l2norm_eps | None)
+// chunk_gdr(q, k, v, g | None, beta, scale, h0, want_ht, plan, may_differentiate, l2norm_eps | None, offsets)
 PyObject* py_chunk_gdr(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 11);
+  expect(n, 12);
   Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), beta = arg_tensor(p[4]),
-         h0 = arg_tensor(p[6]);
+         h0 = arg_tensor(p[6]), offsets = arg_tensor(p[11]);
   GdrArgs a{};
   a.plan = arg_plan(p[8]);
   if (!chunk_operands(q, k, v, h0, a.plan, &a.d) || !beta.defined() || !on_gpu({&g, &beta})) return none();
@@ -755,7 +759,7 @@ PyObject* py_chunk_gdr(PyObject*, PyObject* const* p, Py_ssize_t n) {
       k = L2NormNode::apply(k, *a.l2norm_eps);
       a.l2norm_eps.reset();
     }
-    auto out = GdrNode::apply(q, k, v, maybe(g), beta, maybe(h0), a);
+    auto out = GdrNode::apply(q, k, v, maybe(g), beta, maybe(h0), maybe(offsets), a);
     return pair(out[0], a.want_ht ? out[1] : Tensor());
   }
   at::AutoDispatchBelowADInplaceOrView guard;

@@ -254,7 +254,7 @@ def _launch(q, k, v, g, beta, scale, initial_state, output_final_state, offsets,
     if ONEPASS_FORWARD:
         return None
     return host().chunk_gdr(q, k, v, g, beta, scale, initial_state, output_final_state, native_plan(offsets),
-                            KEEP_STATES_FOR_BACKWARD, l2norm_eps)
+                            KEEP_STATES_FOR_BACKWARD, l2norm_eps, offsets)
 
 
 def _apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, head_first):

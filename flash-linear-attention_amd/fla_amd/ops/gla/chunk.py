@@ -655,7 +655,7 @@ def _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offse
     if h0 is not None and (KP, VP) != (K, V):
         h0 = F.pad(h0, (0, VP - V, 0, KP - K))
     res = host().chunk_gla(q, k, v, g, scale, h0, output_final_state, native_plan(offsets), True, KEEP_KHAT_AND_SCORES,
-                           None, None)
+                           None, None, offsets)
     if res is None:
         raise ValueError(f"fla_amd chunk_gla: inconsistent operands q {tuple(q.shape)}, k {tuple(k.shape)}, "
                          f"v {tuple(v.shape)}, g {tuple(g.shape)}")
@@ -737,7 +737,8 @@ def chunk_gla(
     if not head_first:
         # seq-first operands as the kernels read them: nothing left to do in Python
         res = host().chunk_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
-                               KEEP_STATES_FOR_BACKWARD, KEEP_KHAT_AND_SCORES, gate_logit_normalizer, gate_clamp_min)
+                               KEEP_STATES_FOR_BACKWARD, KEEP_KHAT_AND_SCORES, gate_logit_normalizer, gate_clamp_min,
+                               offsets)
         if res is not None:
             return res
     if gate_logit_normalizer is not None:

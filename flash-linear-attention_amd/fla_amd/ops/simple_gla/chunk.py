@@ -114,7 +114,7 @@ def chunk_simple_gla(
         check_varlen_args(q, offsets, head_first, initial_state)
     if SCAN_FORWARD and not head_first:
         res = host().chunk_simple_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
-                                      gla_chunk.KEEP_STATES_FOR_BACKWARD, gla_chunk.KEEP_KHAT_AND_SCORES)
+                                      gla_chunk.KEEP_STATES_FOR_BACKWARD, gla_chunk.KEEP_KHAT_AND_SCORES, offsets)
         if res is not None:
             return res
     if scale is None:

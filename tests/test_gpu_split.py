@@ -266,3 +266,26 @@ def test_gdr_cut_state_passes_in_fp32(device, K, V, dtype, bounds):
     dht = torch.randn(ht.shape, device=device)
     torch.autograd.backward((o, ht), (torch.zeros_like(o), dht))
     assert torch.equal(ht, h0) and torch.equal(h0.grad, dht)
+
+
+@pytest.mark.parametrize("op", ["chunk_gla", "chunk_simple_gla", "chunk_gated_delta_rule", "fp32", "K=96"])
+def test_offsets_written_before_the_backward(device, op):
+    """A cu_seqlens buffer that is filled again between a forward and its backward: refused, as for any saved tensor."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    dtype, K = torch.float32 if op == "fp32" else torch.bfloat16, 96 if op == "K=96" else 64
+    q, k, v, g, beta, _ = (x.to(device) for x in gdr_inputs(1, 300, 2, K, K, seed=8, dtype=dtype, N=2))
+    leaves = [x.requires_grad_() for x in (q, k, v)]
+    offs = torch.tensor([0, 100, 300], device=device)
+    print("offsets written", op, flush=True)
+    kw = dict(head_first=False, cu_seqlens=offs)
+    if op == "chunk_gated_delta_rule":
+        o, _ = chunk_gated_delta_rule(*leaves, g, beta, **kw)
+    elif op == "chunk_simple_gla":
+        o, _ = chunk_simple_gla(*leaves, g, **kw)
+    else:
+        o, _ = chunk_gla(*leaves, g[..., None].expand(-1, -1, -1, K).contiguous(), **kw)
+    offs.copy_(torch.tensor([0, 200, 300]))
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        o.sum().backward()
