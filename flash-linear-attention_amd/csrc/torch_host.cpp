@@ -56,9 +56,13 @@ Tensor f32(const Tensor& x) {
 }
 // Whether a call has to go through its autograd node.  An operand with a tangent does too, also where nothing requires a
 // gradient: the nodes have no forward-mode derivative and say so, a launch beside them would drop the tangent.
-bool wants_grad(std::initializer_list<const Tensor*> ts) {
+bool has_tangent(std::initializer_list<const Tensor*> ts) {
   for (const Tensor* t : ts)
     if (t->defined() && t->_fw_grad(0).defined()) return true;
+  return false;
+}
+bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  if (has_tangent(ts)) return true;
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
     if (t->defined() && t->requires_grad()) return true;
@@ -894,6 +898,7 @@ PyObject* py_conv_update(PyObject*, PyObject* const* p, Py_ssize_t n) {
   if (!x.defined() || !cache.defined() || !x.is_cuda() || !cache.is_cuda() || x.dim() != 2 || x.numel() == 0 ||
       !(is16(x) || x.scalar_type() == at::kFloat) || !conv_weights_ok(w, b, x.size(1)))
     return none();
+  if (has_tangent({&x, &cache, &w, &b})) return none();   // (the wrapper refuses it)
   const int64_t B = x.size(0), D = x.size(1), W = w.size(-1);
   if (cache.dim() != 3 || cache.size(0) != B || cache.size(1) != D || cache.size(2) != W || !cache.is_contiguous() ||
       cache.scalar_type() != x.scalar_type())

@@ -8,6 +8,7 @@ import torch.nn.functional as F
 
 from .. import _backend as be
 from .._native import host
+from ..utils import needs_node
 
 
 def _act_flag(activation: Optional[str]) -> int:
@@ -67,10 +68,14 @@ def causal_conv1d(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
 
 def causal_conv1d_update(x: torch.Tensor, cache: torch.Tensor, weight: torch.Tensor,
                          bias: Optional[torch.Tensor] = None, activation: Optional[str] = None) -> torch.Tensor:
-    """Single-token step: ``x`` [B,D]; ``cache`` [B,D,W] is shifted and updated in place."""
+    """Single-token step: ``x`` [B,D]; ``cache`` [B,D,W] is shifted and updated in place.  No derivative: gradients stop
+    here, forward-mode tangents are refused."""
     y = host().causal_conv1d_update(x, cache, weight, bias, _act_flag(activation))
     if y is not None:
         return y
+    with torch.no_grad():
+        if needs_node(x, cache, weight, bias):
+            raise NotImplementedError("fla_amd causal_conv1d_update has no forward-mode derivative")
     be.require_gpu(x, cache)
     B, D = x.shape
     W = weight.shape[-1]

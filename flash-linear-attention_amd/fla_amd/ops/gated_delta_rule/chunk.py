@@ -19,7 +19,7 @@ import torch.nn.functional as F
 from ... import _backend as be
 from ..._native import host
 from ...utils import (VarlenPlan, autocast_custom_bwd, autocast_custom_fwd, check_varlen_args, contiguous,
-                      empty_batch_result, native_plan, resolve_offsets)
+                      empty_batch_result, native_plan, needs_node, resolve_offsets)
 from ..common.chunk_delta_h import (chunk_gated_delta_rule_fwd_h, chunk_gated_delta_rule_fwd_h_both,
                                     chunk_gated_delta_rule_fwd_onepass, chunk_gated_delta_rule_fwd_scan)
 from ..common.chunk_o import chunk_fwd_o
@@ -263,7 +263,7 @@ def _apply(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, 
     and the one-launch forward go through the autograd function."""
     K, V = k.shape[-1], v.shape[-1]
     KP, VP = _round_k(K), _round64(V)
-    grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (q, k, v, g, beta, initial_state))
+    grad = needs_node(q, k, v, g, beta, initial_state)
     if KP <= _FUSED_MAX_K and not ONEPASS_FORWARD and not (grad and not KEEP_STATES_FOR_BACKWARD):
         be.require_gpu(q, k, v, beta)
         x, h0 = (q, k, v, g, beta), initial_state

@@ -7,7 +7,7 @@ import torch
 
 from ... import _backend as be
 from ..._native import host
-from ...utils import check_varlen_args, contiguous, resolve_offsets
+from ...utils import check_varlen_args, contiguous, needs_node, resolve_offsets
 
 L2NORM_EPS = 1e-6   # the eps of fla.modules.l2norm
 
@@ -121,8 +121,7 @@ def fused_recurrent_gated_delta_rule(
         res = host().recurrent_gdr(q, k, v, g, beta, scale, initial_state, output_final_state, inplace_state, l2norm_eps)
         if res is not None:
             return res
-    if not (torch.is_grad_enabled() and any(t is not None and t.requires_grad
-                                            for t in (q, k, v, g, beta, initial_state))):
+    if not needs_node(q, k, v, g, beta, initial_state):
         # decode loops: no autograd node to build, and the host time of a step is of the order of its device time
         return fused_recurrent_gated_delta_rule_fwd(q, k, v, g, beta, scale, initial_state, output_final_state,
                                                     offsets, head_first, inplace_state, l2norm_eps)

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 
 from ... import _backend as be
 from ..._native import host
-from ...utils import (VarlenPlan, check_varlen_args, contiguous, empty_batch_result, native_plan,
+from ...utils import (VarlenPlan, check_varlen_args, contiguous, empty_batch_result, native_plan, needs_node,
                       resolve_offsets)
 from ..common.chunk_h import chunk_fwd_h
 from ..utils.cumsum import chunk_local_cumsum, chunk_local_cumsum_inverse
@@ -112,7 +112,7 @@ class _ScaledFp16ChunkGla(torch.autograd.Function):
 
 
 def _chunk_gla_fp32_via_fp16(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first):
-    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (q, k, v, g, initial_state)):
+    if needs_node(q, k, v, g, initial_state):
         return _ScaledFp16ChunkGla.apply(q, k, v, g, initial_state, scale, output_final_state, offsets, head_first)
     sq, sk, sv = _pow2_scale(q), _pow2_scale(k), _pow2_scale(v)
     skv = sk * sv
@@ -631,10 +631,6 @@ class ChunkGLAFunction(torch.autograd.Function):
         return dq.to(qd), dk.to(kd), dv.to(vd), dg.to(gd), None, dh0, None, None, None
 
 
-def _needs_grad(*tensors) -> bool:
-    return torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors)
-
-
 def _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first):
     """16-bit q with K, V <= 128 in any layout: converted to what the host extension takes (seq-first, one dtype, head
     dims 64 or 128, fp32 state) by differentiable torch operations, and the results back."""
@@ -779,6 +775,6 @@ def chunk_gla(
             outs.append(o)
             states.append(ht)
         return torch.cat(outs, dim=-1), (torch.cat(states, dim=-1) if output_final_state else None)
-    if _needs_grad(q, k, v, g, initial_state) and (not KEEP_STATES_FOR_BACKWARD or float(scale) == 0.0):
+    if needs_node(q, k, v, g, initial_state) and (not KEEP_STATES_FOR_BACKWARD or float(scale) == 0.0):
         return ChunkGLAFunction.apply(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first)
     return _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offsets, head_first)

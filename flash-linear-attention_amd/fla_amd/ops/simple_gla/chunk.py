@@ -14,7 +14,7 @@ import os
 
 from ... import _backend as be
 from ..._native import host
-from ...utils import VarlenPlan, check_varlen_args, contiguous, native_plan, resolve_offsets
+from ...utils import VarlenPlan, check_varlen_args, contiguous, native_plan, needs_node, resolve_offsets
 from ..gla import chunk as gla_chunk
 from ..gla.chunk import chunk_gla, chunk_gla_bwd_device, chunk_gla_fwd_fused
 
@@ -121,11 +121,9 @@ def chunk_simple_gla(
         scale = k.shape[-1] ** -0.5
     K = k.shape[-1]
     V = v.shape[-1]
-    needs_grad = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (q, k, v, g, initial_state))
     if (g is not None and not head_first and K in (64, 128) and V in (64, 128)
             and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype):
-        if needs_grad:
+        if needs_node(q, k, v, g, initial_state):
             return ChunkSimpleGLAFunction.apply(q, k, v, g, scale, initial_state, output_final_state, offsets)
         if SCAN_FORWARD:
             return chunk_simple_gla_fwd_scan(q.contiguous(), k.contiguous(), v.contiguous(), g, scale, initial_state,

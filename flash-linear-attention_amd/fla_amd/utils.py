@@ -11,6 +11,7 @@ import weakref
 from typing import Optional, Tuple
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 
 from . import _backend as be
 
@@ -23,6 +24,15 @@ def contiguous(fn):
                   *(a.contiguous() if isinstance(a, torch.Tensor) else a for a in args),
                   **{k: (v.contiguous() if isinstance(v, torch.Tensor) else v) for k, v in kwargs.items()})
     return wrapper
+
+
+def needs_node(*tensors) -> bool:
+    """Whether a call has to go through its autograd function.  An operand with a forward-mode tangent does too, also where
+    nothing requires a gradient: the functions have no forward-mode derivative and say so, a launch beside them would drop
+    the tangent."""
+    given = [t for t in tensors if t is not None]
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in given)
+            or any(forward_ad.unpack_dual(t).tangent is not None for t in given))
 
 
 autocast_custom_fwd = functools.partial(torch.amp.custom_fwd, device_type="cuda")

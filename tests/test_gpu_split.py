@@ -195,18 +195,46 @@ def test_packed_batch_first_met_under_capture(device):
             assert_close("o", eager.float().cpu(), o.cpu(), 1e-2)
 
 
-def test_forward_mode_is_refused(device):
+@pytest.mark.parametrize("op", ["chunk_gla", "chunk_gla fp32", "chunk_gla head-first", "chunk_simple_gla",
+                                "chunk_simple_gla, 16-bit state", "chunk_gated_delta_rule", "fused_recurrent_gla",
+                                "fused_recurrent_gated_delta_rule", "fused_recurrent_gated_delta_rule, packed", "l2_norm",
+                                "causal_conv1d", "causal_conv1d_update", "rms_norm_swish_gate", "gla_gate"])
+@pytest.mark.parametrize("grad", [True, False])
+def test_forward_mode_is_refused(device, op, grad):
     """No operator has a forward-mode derivative: a tangent is an error, not dropped."""
     import torch.autograd.forward_ad as fw
-    from fla_amd.modules import l2_norm
-    from fla_amd.ops.gla import chunk_gla
-    q, k, v, g, _ = (x.to(device) for x in gla_inputs(1, 70, 1, 64, 64, seed=1))
-    with fw.dual_level():
+    from fla_amd import modules as m
+    from fla_amd.modules.convolution import causal_conv1d, causal_conv1d_update
+    from fla_amd.modules.fused_norm_gate import rms_norm_swish_gate_fn
+    from fla_amd.modules.gate_activations import gla_gate
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
+    from fla_amd.ops.gla import chunk_gla, fused_recurrent_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, 70, 1, 64, 64, seed=1))
+    gk, w, kw = g[..., None].expand(-1, -1, -1, 64).contiguous(), torch.randn(64, 4, device=device), dict(head_first=False)
+    offs = torch.tensor([0, 30, 70], device=device)
+    calls = {
+        "chunk_gla": lambda x: chunk_gla(x, k, v, gk, **kw),
+        "chunk_gla fp32": lambda x: chunk_gla(x.float(), k.float(), v.float(), gk, **kw),
+        "chunk_gla head-first": lambda x: chunk_gla(x, k, v, gk),
+        "chunk_simple_gla": lambda x: chunk_simple_gla(x, k, v, g, **kw),
+        "chunk_simple_gla, 16-bit state": lambda x: chunk_simple_gla(x, k, v, g, initial_state=h0.bfloat16(), **kw),
+        "chunk_gated_delta_rule": lambda x: chunk_gated_delta_rule(x, k, v, g, beta, **kw),
+        "fused_recurrent_gla": lambda x: fused_recurrent_gla(x, k, v, gk, **kw),
+        "fused_recurrent_gated_delta_rule": lambda x: fused_recurrent_gated_delta_rule(x, k, v, g, beta, **kw),
+        "fused_recurrent_gated_delta_rule, packed":
+            lambda x: fused_recurrent_gated_delta_rule(x, k, v, g, beta, cu_seqlens=offs, **kw),
+        "l2_norm": m.l2_norm,
+        "causal_conv1d": lambda x: causal_conv1d(x[:, :, 0], w),
+        "causal_conv1d_update": lambda x: causal_conv1d_update(x[:, 0, 0], torch.zeros_like(w)[None].to(x.dtype), w),
+        "rms_norm_swish_gate": lambda x: rms_norm_swish_gate_fn(x, v, None, None),
+        "gla_gate": lambda x: gla_gate(x, 16.0),
+    }
+    with fw.dual_level(), torch.set_grad_enabled(grad):
         x = fw.make_dual(q, torch.ones_like(q))
+        print("forward mode", op, flush=True)
         with pytest.raises(RuntimeError):
-            chunk_gla(x, k, v, g, head_first=False)
-        with pytest.raises(RuntimeError):
-            l2_norm(x)
+            calls[op](x)
 
 
 @pytest.mark.parametrize("dtype,heads", [(torch.float16, False), (torch.float16, True), (torch.float32, False)])
