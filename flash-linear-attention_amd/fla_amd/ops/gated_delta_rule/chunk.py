@@ -249,10 +249,25 @@ class ChunkGatedDeltaRuleFunction(torch.autograd.Function):
                 None, None, None)
 
 
+def _launch_onepass(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, l2norm_eps):
+    """A forward that is not differentiated, where ``ONEPASS_FORWARD`` asks for the one-launch form (which normalises q and
+    k inside the launch too); ``None`` if the operands need a conversion."""
+    ts = [t for t in (q, k, v, g, beta, initial_state) if t is not None]
+    if (q.dtype not in (torch.bfloat16, torch.float16) or k.shape[-1] > _FUSED_MAX_K
+            or (k.shape[-1], v.shape[-1]) not in _SUPPORTED_KV or needs_node(*ts)
+            or not all(t.is_cuda and t.is_contiguous() for t in ts)
+            or (initial_state is not None and initial_state.dtype != torch.float32)):
+        return None
+    _, o, _, _, ht = chunk_gated_delta_rule_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, offsets=offsets,
+                                                head_first=False, chunk_size=BT, store_A=False, l2norm_eps=l2norm_eps,
+                                                want_g_cumsum=False)
+    return o, ht
+
+
 def _launch(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, l2norm_eps=None):
     """Seq-first operands as the kernels read them through the host extension; ``None`` if they need a conversion."""
     if ONEPASS_FORWARD:
-        return None
+        return _launch_onepass(q, k, v, g, beta, scale, initial_state, output_final_state, offsets, l2norm_eps)
     return host().chunk_gdr(q, k, v, g, beta, scale, initial_state, output_final_state, native_plan(offsets),
                             KEEP_STATES_FOR_BACKWARD, l2norm_eps, offsets)
 

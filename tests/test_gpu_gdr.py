@@ -541,3 +541,22 @@ def test_chunk_gdr_onepass_forward(device, monkeypatch, dtype, K, V, T, varlen, 
     assert_close("ht", rht, ht, TOL_HT)
     assert_close("o vs two-launch", o2, o, 6e-3)
     assert_close("ht vs two-launch", ht2, ht, 6e-3)
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128)])
+def test_chunk_gdr_onepass_l2norm_in_kernel(device, monkeypatch, K, V):
+    """Raw q and k: the one-launch form normalises them itself, without launches ahead of it."""
+    import fla_amd.modules.l2norm as l2
+    import fla_amd.ops.gated_delta_rule.chunk as mod
+    from oracle.modules import l2norm
+    from oracle.recurrent import naive_recurrent_gated_delta_rule
+    q, k, v, g, beta, s0 = gdr_inputs(1, 200, 2, K, V, seed=K)
+    k = torch.randn(k.shape).to(k.dtype) * 3
+    monkeypatch.setattr(mod, "_ONEPASS_MIN_WORKGROUPS", 1)
+    monkeypatch.setattr(mod, "ONEPASS_FORWARD", True)
+    monkeypatch.setattr(l2, "l2_norm", lambda *a: pytest.fail("normalised by launches of its own"))
+    o, ht = mod.chunk_gated_delta_rule(*(x.to(device) for x in (q, k, v, g, beta)), initial_state=s0.to(device),
+                                       output_final_state=True, head_first=False, use_qk_l2norm_in_kernel=True)
+    ro, rht = naive_recurrent_gated_delta_rule(l2norm(q), l2norm(k), v, g, beta, initial_state=s0, output_final_state=True)
+    assert_close("o", ro, o, TOL_O)
+    assert_close("ht", rht, ht, TOL_HT)
