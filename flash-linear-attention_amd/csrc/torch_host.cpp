@@ -10,6 +10,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -97,11 +98,32 @@ const X& held(AutogradContext* ctx) {
 }
 
 // ---------------------------------------------------------------------------------------------------- packed batches
+// A pinned host tensor as a device tensor that any stream may read from now on.  The copy goes through a stream of its own
+// and is waited for there: the streams that compute go on (a blocking copy would wait for everything queued on its stream:
+// a whole forward, where it is a backward's tables).  The memory belongs to that stream: readers call record_stream.
+Tensor upload(const Tensor& host, at::Device device) {
+  static std::mutex mu;
+  static std::map<int, hipStream_t> streams;   // one per device, never destroyed
+  c10::DeviceGuard on_device(device);
+  std::lock_guard<std::mutex> lock(mu);
+  hipStream_t& raw = streams[device.index()];
+  if (!raw) TORCH_CHECK(hipStreamCreateWithFlags(&raw, hipStreamNonBlocking) == hipSuccess, "fla_amd: no stream for uploads");
+  const auto own = c10::hip::getStreamFromExternal(raw, device.index());
+  struct Current {
+    c10::hip::HIPStream before;
+    ~Current() { c10::hip::setCurrentHIPStream(before); }
+  } current{c10::hip::getCurrentHIPStream(device.index())};
+  c10::hip::setCurrentHIPStream(own);
+  Tensor out = at::empty(host.sizes(), host.options().device(device).pinned_memory(false));
+  out.copy_(host, /*non_blocking=*/true);
+  own.synchronize();
+  return out;
+}
+
 struct SplitTables {
   bool cut = false;
-  std::optional<c10::hip::HIPStream> home;   // the stream the tables were allocated on
   fla_split ints{};
-  Tensor seg, sub, base;
+  Tensor tables;   // seg_table, sub_table and sub_base, one behind the other
 };
 // The device tables of a packed batch, made once per offsets tensor by fla_amd.utils.VarlenPlan.  `offsets` is the caller's
 // own tensor where it is int64: a node saves it, so that a backward after it has been written to is refused instead of
@@ -113,8 +135,8 @@ struct Plan : torch::CustomClassHolder {
   std::mutex mu;
   std::map<std::tuple<int64_t, int, bool, int>, SplitTables> splits;
 
-  // The tables of a cut are used by later calls on any stream: the copies to the device are synchronous.  A stream that is
-  // being captured takes no such copy; a call whose tables are not there yet runs uncut under it.
+  // The tables of a cut are used by later calls on any stream.  A stream that is being captured takes no copy: a call whose
+  // tables are not there yet runs uncut under it.
   SplitTables split(int64_t H, int slabs, bool reverse, int kind) {
     std::lock_guard<std::mutex> lock(mu);
     const auto stream = c10::hip::getCurrentHIPStream(offsets.device().index());
@@ -129,24 +151,21 @@ struct Plan : torch::CustomClassHolder {
         return fla_scan_split(host.data(), N, 0, H, slabs, reverse, kind, &sp, a, b, c);
       };
       if (plan(nullptr, nullptr, nullptr)) {
-        auto opts = at::TensorOptions().dtype(at::kInt);
-        Tensor a = at::empty({sp.nseg, 2}, opts), b = at::empty({sp.nsub, 2}, opts), c = at::empty({N + 1}, opts);
-        plan((int32_t*)a.data_ptr(), (int32_t*)b.data_ptr(), (int32_t*)c.data_ptr());
-        s.seg = a.to(offsets.device());
-        s.sub = b.to(offsets.device());
-        s.base = c.to(offsets.device());
-        sp.seg_table = (const int32_t*)s.seg.data_ptr();
-        sp.sub_table = (const int32_t*)s.sub.data_ptr();
-        sp.sub_base = (const int32_t*)s.base.data_ptr();
+        const int64_t sub = 2 * (int64_t)sp.nseg, base = sub + 2 * (int64_t)sp.nsub;
+        const Tensor host_tables = at::empty({base + N + 1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        int32_t* h = host_tables.data_ptr<int32_t>();
+        plan(h, h + sub, h + base);
+        s.tables = upload(host_tables, offsets.device());
+        const int32_t* d = s.tables.data_ptr<int32_t>();
+        sp.seg_table = d;
+        sp.sub_table = d + sub;
+        sp.sub_base = d + base;
         s.ints = sp;
-        s.home = stream;
         s.cut = true;
       }
     }
-    // the plan may be dropped while another stream still reads its tables
-    if (s.cut && *s.home != stream)
-      for (Tensor* t : {&s.seg, &s.sub, &s.base})   // (tensors of this build call their device CUDA)
-        t->record_stream(c10::Stream(c10::Stream::UNSAFE, offsets.device(), stream.id()));
+    // the plan may be dropped while this stream still reads its tables (tensors of this build call their device CUDA)
+    if (s.cut) s.tables.record_stream(c10::Stream(c10::Stream::UNSAFE, offsets.device(), stream.id()));
     return s;
   }
 };

@@ -317,3 +317,40 @@ def test_offsets_written_before_the_backward(device, op):
     offs.copy_(torch.tensor([0, 200, 300]))
     with pytest.raises(RuntimeError, match="inplace operation"):
         o.sum().backward()
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_tables_of_a_cut_do_not_wait_for_the_device(device, delta):
+    """New boundaries behind a queue of work: neither the forward nor the backward waits until it is done."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.utils import VarlenPlan
+    T, bounds = 3200, [0, 1790, 1854, 3200]
+    assert _cut(3, T, 1, 1, False, bounds, 2 * delta) and _cut(3, T, 1, 1 + (not delta), True, bounds, 2 * delta)
+    q, k, v, g, beta, _ = (x.to(device) for x in gdr_inputs(1, T, 1, 64, 64, seed=2, normalizer=600.0))
+    gk = g[..., None].expand(-1, -1, -1, 64).contiguous()
+    q.requires_grad_()
+    do, a = torch.randn_like(v), torch.randn(8192, 8192, device=device, dtype=torch.bfloat16)
+
+    def busy():
+        for _ in range(40):
+            torch.mm(a, a)
+        done = torch.cuda.Event()
+        done.record()
+        return done
+
+    for turn in range(3):   # the first two fill the allocators' pools
+        q.grad = None
+        offs = torch.tensor(bounds, device=device)
+        VarlenPlan(offs, 64).native
+        torch.cuda.synchronize()
+        print("busy, forward", delta, flush=True)
+        done = busy()
+        kw = dict(head_first=False, cu_seqlens=offs)
+        o, _ = chunk_gated_delta_rule(q, k, v, g, beta, **kw) if delta else chunk_gla(q, k, v, gk, **kw)
+        assert turn < 2 or not done.query()
+        torch.cuda.synchronize()
+        done = busy()
+        o.backward(do)
+        assert turn < 2 or not done.query()
+        torch.cuda.synchronize()
