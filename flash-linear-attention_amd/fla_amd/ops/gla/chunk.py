@@ -279,8 +279,7 @@ def _guard_workspaces(q, chunks, H, KV, keep):
 
 
 def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets=None, exact_guard=True,
-                        return_flags=False, states_out=None, head_gates=False, first_launch_only=False,
-                        gate_logits=None):
+                        return_flags=False, states_out=None, head_gates=False, first_launch_only=False):
     """Forward through ``fla_chunk_gla_fwd_fused``: seq-first, K in {64,128}, V % 64 == 0.
     With ``exact_guard`` (needs V <= 128) chunks whose cumulative log-gate leaves the
     single-reference range are detected on the device and recomputed exactly; ``return_flags``
@@ -289,9 +288,7 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
     order, what the backward kernels read) and appends it, followed (per-key gates only) by the gated queries
     ``q e^{G}`` ``[B,T,H,K]`` and the chunk decays ``e^{G_last}`` ``[chunks,H,K]`` the backward's reverse state scan
     streams (``fla_chunk_gla_fwd_fused_kept``).  ``head_gates``: ``g`` is one fp32 log-gate
-    per (token, head), ``[B,T,H]`` (``fla_chunk_simple_gla_fwd_fused``).  ``gate_logits = (normalizer, clamp_min)``:
-    ``g`` is the gate projection's output and the kernel forms ``logsigmoid(g) / normalizer`` (clamped from below
-    unless ``clamp_min`` is None) itself (``fla_chunk_gla_fwd_fused_logits``; no kept states, per-key gates)."""
+    per (token, head), ``[B,T,H]`` (``fla_chunk_simple_gla_fwd_fused``)."""
     B, T, H, K = q.shape
     V = v.shape[-1]
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
@@ -310,14 +307,7 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
             0 if plan is None else plan.NT,
             be.dt(q), be.dt(g), B, T, H, K, V, N, float(scale), be.stream_of(q))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(h0), be.ptr(o), be.ptr(ht), be.ptr(wide), be.ptr(hwide))
-    if gate_logits is not None:
-        if head_gates or states_out is not None or first_launch_only:
-            raise ValueError("gate logits: per-key gates, forward without kept states")
-        normalizer, clamp_min = gate_logits
-        be.check(be.lib().fla_chunk_gla_fwd_fused_logits(*head, *tail[:-1], float(normalizer), int(clamp_min is not None),
-                                                         float(clamp_min or 0.0), tail[-1]),
-                 "fla_chunk_gla_fwd_fused_logits")
-    elif head_gates:
+    if head_gates:
         if g.dtype != torch.float32 or g.shape != q.shape[:3]:
             raise ValueError("head gates must be fp32 [B, T, H]")
         hT = qg = decay = kh = sc = None
