@@ -64,15 +64,11 @@ def _compile(src, force):
 
 def _build_host(force):
     """The CPython extension over libfla_hip.so (host code only; torch is asked for its include and library folders)."""
-    header = os.path.join(HERE, "..", "include", "fla_hip.h")
-    if (not force and os.path.exists(HOST_PATH)
-            and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(HOST_SRC), os.path.getmtime(header))):
-        return ""
+    import torch
     from torch.utils import cpp_extension as ext
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
     includes = [p for p in ext.include_paths() if os.path.isdir(p)] + [os.path.join(rocm, "include"), "/opt/rocm/include",
                                                                        sysconfig.get_path("include")]
-    import torch
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
     for p in includes:
@@ -82,9 +78,21 @@ def _build_host(force):
         cmd += ["-L" + p]
     cmd += ["-L" + LIB_DIR, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-lfla_hip",
             "-Wl,-rpath,$ORIGIN"]
+    # Up to date: newer than its sources and built by this very command against this torch, whose C++ interface changes
+    # from version to version without a file here becoming newer.
+    stamp = os.path.join(OBJ_DIR, "_fla_host.stamp")
+    built_for = "\n".join([torch.__version__, str(torch.version.git_version)] + cmd)
+    header = os.path.join(HERE, "..", "include", "fla_hip.h")
+    if (not force and os.path.exists(HOST_PATH) and os.path.exists(stamp)
+            and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(HOST_SRC), os.path.getmtime(header))):
+        with open(stamp) as f:
+            if f.read() == built_for:
+                return ""
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed on torch_host.cpp:\n" + r.stdout + r.stderr)
+    with open(stamp, "w") as f:
+        f.write(built_for)
     return r.stderr
 
 
