@@ -1,0 +1,101 @@
+"""CPU: where fla_scan_split cuts sequences.  Host arithmetic, whose tables the kernels index memory with."""
+import ctypes
+import random
+
+import pytest
+
+CHUNK, CUS = 64, 256
+
+
+def _plan(bounds, N, T, H, slabs, reverse, kind):
+    """The plan and, for a packed batch, its tables (from buffers with guard words behind them)."""
+    from fla_amd import _backend as be
+    fn, sp = be.lib().fla_scan_split, be.Split()
+    offs = None if bounds is None else (ctypes.c_int64 * len(bounds))(*bounds)
+    if not fn(offs, N, T, H, slabs, reverse, kind, ctypes.byref(sp), None, None, None):
+        return None
+    if bounds is None:
+        return sp, None, None, None
+    sizes = [2 * sp.nseg, 2 * sp.nsub, N + 1]
+    tables = [(ctypes.c_int32 * (n + 8))(*([-7] * (n + 8))) for n in sizes]
+    again = be.Split()
+    assert fn(offs, N, T, H, slabs, reverse, kind, ctypes.byref(again), *tables)
+    for name in ("sub_chunks", "ratio", "nseg", "nsub", "slots"):
+        assert getattr(sp, name) == getattr(again, name)
+    assert all(list(t[n:]) == [-7] * 8 for t, n in zip(tables, sizes))
+    seg, sub, base = (list(t[:n]) for t, n in zip(tables, sizes))
+    return sp, list(zip(seg[::2], seg[1::2])), list(zip(sub[::2], sub[1::2])), base
+
+
+def _check(sp, seg, sub, base, chunks, H, slabs, reverse, kind):
+    """``chunks``: chunks of every sequence; ``seg`` and the others None for sequences of equal length."""
+    assert sp.sub_chunks > 0 and sp.ratio > 0 and (kind == 0 or sp.ratio == 1)
+    subs = [max(1, -(-c // sp.sub_chunks)) for c in chunks]
+    segs = [-(-s // sp.ratio) for s in subs]
+    assert max(segs) > 1                                 # something is cut,
+    assert sum(segs) * H * slabs <= CUS                  # every workgroup of the scan has a CU of its own,
+    assert sp.slots == sum(subs)                         # and every sub-block a slot
+    # the sub-blocks the first pass forms: all whose end another segment begins at (and those whose transition a backward wants)
+    def formed(n):
+        return range(sp.ratio, subs[n]) if reverse else range(subs[n] if kind == 2 else (segs[n] - 1) * sp.ratio)
+    if seg is None:
+        assert len(set(chunks)) == 1 and sp.nseg == segs[0] and sp.nsub == subs[0]
+        return
+    assert sorted(seg) == [(n, s) for n in range(len(chunks)) for s in range(segs[n])] and sp.nseg == len(seg)
+    assert sorted(sub) == [(n, j) for n in range(len(chunks)) for j in formed(n)] and sp.nsub == len(sub)
+    assert base == [sum(subs[:n]) for n in range(len(chunks) + 1)]
+    last = [i for i, (n, s) in enumerate(seg) if s == segs[n] - 1]
+    assert last == list(range(len(seg) - len(last), len(seg)))     # the shorter last pieces start last
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_packed_batches(kind):
+    rng, cut = random.Random(kind), 0
+    for _ in range(3000):
+        N = rng.randint(1, 40)
+        longest = int(2 ** rng.uniform(4, 18))
+        bounds = [0]
+        for _ in range(N):
+            bounds.append(bounds[-1] + (0 if rng.random() < 0.1 else rng.randint(1, longest)))
+        H, slabs, reverse = rng.choice((1, 2, 3, 4, 8, 16, 32)), rng.choice((1, 2, 4)), rng.randint(0, 1)
+        got = _plan(bounds, N, bounds[-1], H, slabs, reverse, kind)
+        if got:
+            cut += 1
+            _check(*got, [-(-(b - a) // CHUNK) for a, b in zip(bounds, bounds[1:])], H, slabs, reverse, kind)
+    assert cut > 300
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_sequences_of_equal_length(kind):
+    cut = 0
+    for N in (1, 2, 3, 5, 8, 16, 33, 128):
+        for T in (1, 64, 704, 833, 1600, 4096, 5003, 8192, 100001, 262144):
+            for H in (1, 2, 3, 4, 16, 64, 128):
+                for slabs in (1, 2, 4):
+                    for reverse in (0, 1):
+                        got = _plan(None, N, T, H, slabs, reverse, kind)
+                        if got:
+                            cut += 1
+                            _check(*got, [-(-T // CHUNK)] * N, H, slabs, reverse, kind)
+    assert cut > 100
+
+
+def test_forward_and_backward_of_the_delta_rule_are_cut_alike():
+    """The backward folds with the transitions the forward left, slot by slot."""
+    rng = random.Random(5)
+    for _ in range(300):
+        bounds = [0]
+        for _ in range(rng.randint(1, 12)):
+            bounds.append(bounds[-1] + rng.randint(0, 20000))
+        N, H, slabs = len(bounds) - 1, rng.choice((1, 2, 4, 8)), rng.choice((1, 2))
+        f, r = (_plan(bounds, N, bounds[-1], H, slabs, reverse, 2) for reverse in (0, 1))
+        assert (f is None) == (r is None)
+        if f:
+            assert (f[0].sub_chunks, f[0].slots, f[3]) == (r[0].sub_chunks, r[0].slots, r[3]) and f[1] == r[1]
+
+
+def test_nothing_to_cut():
+    assert _plan([0, 0, 0], 2, 0, 1, 1, 0, 0) is None
+    assert _plan(None, 1, 0, 1, 1, 0, 0) is None
+    assert _plan(None, 0, 64, 1, 1, 0, 0) is None
+    assert _plan(None, 1, 64 * 200, 512, 2, 0, 0) is None
