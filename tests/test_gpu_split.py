@@ -354,3 +354,160 @@ def test_tables_of_a_cut_do_not_wait_for_the_device(device, delta):
         o.backward(do)
         assert turn < 2 or not done.query()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", CASES)
+def test_gla_cut_16bit_gates(device, B, T, H, K, V, bounds, dtype):
+    """Gates in the dtype of q, k and v: log-gates forward and backward, and pre-activations."""
+    from fla_amd.ops.gla import chunk_gla
+    N = B if bounds is None else len(bounds) - 1
+    offs = None if bounds is None else torch.tensor(bounds, device=device)
+    assert _cut(N, T, H, V // 64, False, bounds) and _cut(N, T, H, V // 32, True, bounds)
+    print("cut, 16-bit gates", B, T, H, K, V, bounds, dtype, flush=True)
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
+    g, do = g.to(dtype), torch.randn(B, T, H, V).to(dtype)
+    kw = dict(output_final_state=True, cu_seqlens=offs, head_first=False)
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, h0)]
+    o, ht = chunk_gla(*leaves[:4], initial_state=leaves[4], **kw)
+    torch.autograd.backward((o, ht), (do.to(device), torch.zeros_like(ht)))
+    refs = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*refs[:4], initial_state=refs[4], output_final_state=True, offsets=bounds)
+    ro.backward(do.float())
+    assert_close("o", ro, o, 1e-2)
+    assert_close("ht", rht, ht, 5e-3)
+    for name, r, d in zip(("dq", "dk", "dv", "dg", "dh0"), refs, leaves):
+        assert_close(name, r.grad, d.grad, 2e-2)
+    x = torch.randn(g.shape).to(dtype)
+    with torch.no_grad():
+        o, ht = chunk_gla(*leaves[:3], x.to(device), gate_logit_normalizer=600.0, **kw)
+        ro, rht = naive_recurrent_gla(*refs[:3], F.logsigmoid(x.float()) / 600.0, output_final_state=True, offsets=bounds)
+    assert_close("o from logits", ro, o, 1e-2)
+    assert_close("ht from logits", rht, ht, 5e-3)
+
+
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", GDR_CASES)
+@pytest.mark.parametrize("normalizer,states", [(1.0, True), (200.0, False), (200.0, True)])
+def test_gdr_cut_ordinary_corrections(device, B, T, H, K, V, bounds, dtype, normalizer, states):
+    """beta = sigmoid with ordinary and with weak gates, with and without states given from outside: the transition of a
+    segment is far from the identity, and the folds start from zero."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    N = B if bounds is None else len(bounds) - 1
+    offs = None if bounds is None else torch.tensor(bounds, device=device)
+    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
+    print("cut, ordinary beta", B, T, H, K, V, bounds, dtype, normalizer, states, flush=True)
+    q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=normalizer, N=N, h0=states)
+    kw = dict(output_final_state=states, cu_seqlens=offs, head_first=False)
+    leaves = [None if x is None else x.to(device).requires_grad_() for x in (q, k, v, g, beta, h0)]
+    with torch.no_grad():
+        o1, ht1 = chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], **kw)
+    o, ht = chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], **kw)
+    do, dht = torch.randn(B, T, H, V).to(dtype), torch.randn(N, H, K, V) * 0.1
+    torch.autograd.backward((o, ht) if states else (o,), (do.to(device), dht.to(device)) if states else (do.to(device),))
+    refs = [None if x is None else x.float().requires_grad_() for x in (q, k, v, g, beta, h0)]
+    ro, rht = naive_recurrent_gated_delta_rule(*refs[:5], initial_state=refs[5], output_final_state=True, offsets=bounds)
+    torch.autograd.backward((ro, rht) if states else (ro,), (do.float(), dht) if states else (do.float(),))
+    for a, b in ((o1, ht1), (o, ht)):
+        assert_close("o", ro, a, 1e-2)
+        if states:
+            assert_close("ht", rht, b, 5e-3)
+    for name, r, d in zip(("dq", "dk", "dv", "dg", "dbeta", "dh0"), refs, leaves):
+        if r is not None:
+            assert_close(name, r.grad, d.grad, 2e-2)
+
+
+def _split(like, N, T, H, slabs, kind, state, transition):
+    """A cut of sequences of equal length with its workspaces."""
+    from fla_amd import _backend as be
+    sp = be.Split()
+    assert be.lib().fla_scan_split(None, N, T, H, slabs, 0, kind, ctypes.byref(sp), None, None, None)
+    bufs = [torch.empty(sp.slots * H * n, device=like.device) for n in (state, transition)]
+    sp.states, sp.decays = (b.data_ptr() for b in bufs)
+    return sp, bufs
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.float16), (128, 128, torch.bfloat16), (64, 128, torch.bfloat16),
+                                       (128, 64, torch.bfloat16)])
+@pytest.mark.parametrize("op", ["gla", "gated_delta_rule"])
+def test_cut_entry_against_the_uncut_one(device, K, V, dtype, op):
+    """The same inputs through both entry points of the library, and the operator, which takes the cut one.  In the first
+    segment they run the same instructions (equal bits).  Behind it the states that enter differ by the order of their fp32
+    sums and by the rounding of their operands, 2^-9 (bf16) or 2^-12 of each at most; four times that bounds o and ht, which
+    round by as much themselves."""
+    from fla_amd import _backend as be
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from fla_amd.ops.gla import chunk_gla
+    B, T, H, delta = 2, 2020, 2, op != "gla"
+    q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(B, T, H, K, V, seed=3, dtype=dtype, normalizer=200.0))
+    if not delta:
+        g = gla_inputs(B, T, H, K, V, seed=3, normalizer=200.0)[3].to(device)
+    lib, p, scale, st = be.lib(), be.ptr, K ** -0.5, be.stream_of(q)
+    sp, bufs = _split(q, B, T, H, V // 64, int(delta), K * V, K * K if delta else K)
+    assert sp.nseg > 1
+    print("cut against uncut", op, K, V, dtype, sp.nseg, sp.sub_chunks, sp.ratio, flush=True)
+    o, ht = [torch.empty_like(v) for _ in range(2)], [torch.empty_like(h0) for _ in range(2)]
+    dims, chunks = (B, T, H, K, V, B), -(-T // 64) * B
+    if delta:
+        AT, gc = q.new_empty(chunks, H, 10, 16, 16), torch.empty_like(g)
+        be.check(lib.fla_gdr_fwd_prep(p(k), p(beta), p(g), 0, p(gc), p(AT), None, None, None, None, 0, be.dt(q), *dims[:4], st), "prep")
+        be.check(lib.fla_chunk_gated_delta_rule_fwd_scan(p(q), p(k), p(v), p(AT), p(gc), p(h0), p(o[0]), p(ht[0]), *[None] * 6,
+                                                         be.dt(q), *dims, scale, st), "scan")
+        be.check(lib.fla_chunk_gated_delta_rule_fwd_scan_split(p(q), p(k), p(v), p(AT), p(gc), None, p(h0), p(o[1]), p(ht[1]),
+                                                               *[None] * 5, ctypes.byref(sp), be.dt(q), *dims, scale, 0.0, st),
+                 "scan_split")
+        call = lambda: chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True, head_first=False)
+    else:
+        ws = [torch.empty(chunks, H, dtype=torch.int32, device=device), q.new_empty(chunks, H, K * V)]
+        be.check(lib.fla_chunk_gla_fwd_fused(*map(p, (q, k, v, g, h0, o[0], ht[0], *ws)), *[None] * 4, 0, be.dt(q), be.dt(g), *dims,
+                                             scale, st), "fused")
+        be.check(lib.fla_chunk_gla_fwd_fused_split(*map(p, (q, k, v, g, h0, o[1], ht[1], *ws)), *[None] * 8, ctypes.byref(sp), 0,
+                                                   be.dt(q), be.dt(g), *dims, scale, 0, 1.0, 0, 0.0, st), "fused_split")
+        call = lambda: chunk_gla(q, k, v, g, initial_state=h0, output_final_state=True, head_first=False)
+    tol = 4 * 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    assert_close("o", o[0].cpu(), o[1].cpu(), tol)
+    assert_close("ht", ht[0].cpu(), ht[1].cpu(), tol)
+    first = 64 * sp.sub_chunks * sp.ratio
+    assert torch.equal(o[0][:, :first], o[1][:, :first])
+    assert not torch.equal(ht[0], ht[1])   # (so that the comparison below tells the two apart)
+    with torch.no_grad():
+        oo, hh = call()
+    assert torch.equal(oo, o[1]) and torch.equal(hh, ht[1])
+
+
+@pytest.mark.parametrize("bounds", [None, [0, 1790, 1854, 3200]])
+def test_gdr_cut_forward_with_its_backward_under_capture(device, bounds):
+    """The forward runs eagerly and leaves its transitions.  A backward that is captured finds no tables of its own for a
+    packed batch and runs uncut; for one sequence it needs none."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    T, N = 3200, 1 if bounds is None else 3
+    assert _cut(N, T, 1, 1, False, bounds, 2) and _cut(N, T, 1, 1, True, bounds, 2)
+    leaves = [x.to(device).requires_grad_() for x in gdr_inputs(1, T, 1, 64, 64, seed=2, normalizer=600.0, h0=False)[:5]]
+    do = torch.randn(1, T, 1, 64, device=device).to(leaves[0].dtype)
+    offs = None if bounds is None else torch.tensor(bounds, device=device)
+    other = None if bounds is None else offs.clone()   # tables of its own
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+
+    def forward(offs):
+        return chunk_gated_delta_rule(*leaves, cu_seqlens=offs, head_first=False)[0]
+
+    def backward(o):
+        return torch.autograd.grad(o, leaves, do, retain_graph=True)
+
+    with torch.cuda.stream(side):
+        backward(forward(other))
+        o = forward(offs)
+    torch.cuda.synchronize()
+    print("capture a backward", bounds, flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        grads = backward(o)
+    with torch.cuda.stream(side):
+        eager = backward(o)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for x in grads:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, r, d in zip(("dq", "dk", "dv", "dg", "dbeta"), eager, grads):
+            assert_close(name, r.float().cpu(), d.float().cpu(), 2e-2)
