@@ -23,7 +23,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define FLA_DEVICE __device__ __forceinline__
 
-// Four consecutive floats at any float address in one load (weights are slices of parameters, aligned to 4 bytes only)
+// Four consecutive floats at any float address in one load (weights are slices of parameters, states of larger buffers:
+// aligned to 4 bytes only)
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 #define FLA_CHECK_LAUNCH()                         \

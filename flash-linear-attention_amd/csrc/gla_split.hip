@@ -267,7 +267,8 @@ __global__ __launch_bounds__(256) void gla_split_fold_kernel(float* __restrict__
   f32x4* S = (f32x4*)states + (base * H + hh) * (int64_t)KV4 + e4;
   const float* D = decays + (base * H + hh) * (int64_t)K + kk;
   const int64_t sstr = (int64_t)H * KV4, dstr = (int64_t)H * K;
-  f32x4 h = init ? ((const f32x4*)init)[(int64_t)nh * KV4 + e4] : f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 h = {0.f, 0.f, 0.f, 0.f};
+  if (init) h = ((const f32x4_any*)init)[(int64_t)nh * KV4 + e4];   // the caller's: aligned to 4 bytes only
   constexpr int U = 8;
   const int todo = REVERSE ? nsub - split.ratio : (nseg - 1) * split.ratio;   // sub-blocks the first pass formed
   for (int d = 0; d < todo; d += U) {

@@ -511,3 +511,36 @@ def test_gdr_cut_forward_with_its_backward_under_capture(device, bounds):
         torch.cuda.synchronize()
         for name, r, d in zip(("dq", "dk", "dv", "dg", "dbeta"), eager, grads):
             assert_close(name, r.float().cpu(), d.float().cpu(), 2e-2)
+
+
+@pytest.mark.parametrize("op", ["chunk_gla", "chunk_simple_gla", "chunk_gated_delta_rule"])
+def test_cut_states_at_any_float_address(device, op):
+    """An initial state and a gradient of the final one that begin four bytes behind a 16-byte boundary: the same bits."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    T, K = 2020, 64
+    delta = op == "chunk_gated_delta_rule"
+    assert _cut(1, T, 2, 1, False, None, 2 * delta) and _cut(1, T, 2, 1 if delta else 2, True, None, 2 * delta)
+    q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, T, 2, K, K, seed=4, normalizer=200.0))
+    do, dht = torch.randn(v.shape, device=device).to(v.dtype), torch.randn(h0.shape, device=device)
+
+    def moved(x):
+        y = torch.empty(x.numel() + 1, device=device)[1:].view(x.shape)
+        assert y.data_ptr() % 16 == 4
+        return y.copy_(x)
+
+    def call(h0, dht):
+        print("states at", h0.data_ptr() % 16, op, flush=True)
+        leaves = [q.detach().requires_grad_(), h0.requires_grad_()]
+        kw = dict(initial_state=h0, output_final_state=True, head_first=False)
+        if delta:
+            o, ht = chunk_gated_delta_rule(leaves[0], k, v, g, beta, **kw)
+        elif op == "chunk_simple_gla":
+            o, ht = chunk_simple_gla(leaves[0], k, v, g, **kw)
+        else:
+            o, ht = chunk_gla(leaves[0], k, v, g[..., None].expand(-1, -1, -1, K).contiguous(), **kw)
+        return [o, ht, *torch.autograd.grad((o, ht), leaves, (do, dht))]
+
+    for a, b in zip(call(h0.clone(), dht), call(moved(h0), moved(dht))):
+        assert torch.equal(a, b)
