@@ -41,8 +41,9 @@ def norm_gate_fwd(x, o, weight, bias, eps, is_rms_norm, residual=None, residual_
     rstd = torch.empty(M, dtype=torch.float32, device=x.device)
     if M == 0:
         return y, mean, rstd, residual_out if keep else x
+    w32, b32 = _f32(weight), _f32(bias)
     be.check(be.lib().fla_norm_swish_gate_residual_fwd(
-        be.ptr(x), be.ptr(o), be.ptr(_f32(weight)), be.ptr(_f32(bias)), be.ptr(residual),
+        be.ptr(x), be.ptr(o), be.ptr(w32), be.ptr(b32), be.ptr(residual),
         be.dt(residual) if residual is not None else be.dt(x), be.ptr(y), be.ptr(residual_out),
         be.dt(residual_out) if keep else be.dt(x), be.ptr(mean), be.ptr(rstd), M, N, float(eps), int(is_rms_norm),
         be.dt(x), be.stream_of(x)), "fla_norm_swish_gate_residual_fwd")
@@ -68,8 +69,9 @@ def norm_gate_bwd(dy, x, o, weight, bias, eps, mean, rstd, is_rms_norm, dresidua
     nwg = be.lib().fla_norm_swish_gate_workgroups(M, N)
     dwp = torch.empty(nwg, N, dtype=torch.float32, device=x.device) if weight is not None else None
     dbp = torch.empty(nwg, N, dtype=torch.float32, device=x.device) if bias is not None else None
+    w32, b32 = _f32(weight), _f32(bias)
     be.check(be.lib().fla_norm_swish_gate_residual_bwd(
-        be.ptr(dy), be.ptr(x), be.dt(x), be.ptr(o), be.ptr(_f32(weight)), be.ptr(_f32(bias)), be.ptr(mean),
+        be.ptr(dy), be.ptr(x), be.dt(x), be.ptr(o), be.ptr(w32), be.ptr(b32), be.ptr(mean),
         be.ptr(rstd), be.ptr(dresidual), be.ptr(dx), be.ptr(do), be.ptr(dresidual_in), be.ptr(dwp), be.ptr(dbp), M, N,
         float(eps), int(is_rms_norm), be.dt(dx), be.stream_of(x)), "fla_norm_swish_gate_residual_bwd")
     dw = None if dwp is None else dwp.sum(0).to(weight.dtype)

@@ -144,6 +144,30 @@ def test_norm_swish_gate_residual_prenorm(device, dtype, is_rms, res_kind, preno
         assert_close("dresidual", rr.grad, rd.grad, bt)
 
 
+@pytest.mark.parametrize("residual", [False, True])
+@pytest.mark.parametrize("is_rms", [True, False])
+def test_norm_swish_gate_16bit_weight_and_bias(device, is_rms, residual):
+    """Weight and bias of a module in bf16, both converted for the launch.  The fp32 sums are exact to 1e-5; a
+    gradient in bf16 (8 significant bits) is off by its rounding, at most 2^-8 of each element."""
+    from fla_amd.modules import layer_norm_swish_gate_fn, rms_norm_swish_gate_fn
+    from oracle.modules import norm_swish_gate
+    gen = torch.Generator().manual_seed(12)
+    N = 128
+    x, o, r, dy = (torch.randn(40, N, generator=gen) for _ in range(4))
+    w, b = (torch.randn(N, generator=gen).bfloat16() for _ in range(2))
+    print("norm gate, 16-bit weight and bias", is_rms, residual, flush=True)
+    leaves = [t.to(device).requires_grad_() for t in (x, o, w, b)]
+    fn = rms_norm_swish_gate_fn if is_rms else layer_norm_swish_gate_fn
+    y = fn(*leaves, residual=r.to(device) if residual else None, eps=1e-5)
+    y.backward(dy.to(device))
+    refs = [t.float().requires_grad_() for t in (x, o, w, b)]
+    yr = norm_swish_gate(*refs, eps=1e-5, is_rms_norm=is_rms, residual=r if residual else None)
+    yr.backward(dy)
+    assert_close("y", yr, y, 1e-5)
+    for name, ref, d in zip(("dx", "do", "dw", "db"), refs, leaves):
+        assert_close(name, ref.grad, d.grad, 1e-5 if name in ("dx", "do") else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W", [2, 3, 4])
 @pytest.mark.parametrize("T,D,bias,act", [(1, 64, False, "silu"), (5, 64, True, "silu"), (64, 200, False, None),
