@@ -53,23 +53,28 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 
 // Where a sequence is cut.  A scan's time is its longest workgroup's chunks times the chunk period once every workgroup
 // has a CU of its own, so the segments are as short as 256 CUs allow (GLA forward of 16 heads x 8192 tokens, K = V = 128:
-// 4, 8, 16 and 32 segments 112, 80, 86 and 111 us, uncut 293).  The first pass gets about as many workgroups as there are
-// CUs: 1, 2 and 4 sub-blocks per segment of that forward 94, 80 and 84 us, of one of 64 pairs in two segments 169, 136 and
-// 125 us (uncut 155).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands,
+// 4, 8, 16 and 32 segments 112, 81, 88 and 104 us, uncut 291).  The first pass gets about as many workgroups as there are
+// CUs: 1, 2 and 4 sub-blocks per segment of that forward 97, 80 and 83 us, of one of 64 pairs in two segments 177, 141 and
+// 126 us (uncut 156).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands,
 // which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us).
 //
-// The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 1.2 us per
-// segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16 chunks 76, 63
-// and 74 us, uncut 175; training step of 64 chunks, 8 heads, in 4 and 8 172 and 158 us, uncut 251), twenty chunks to save
-// (16 chunks: 32 us uncut, 38 cut; training step of 24 chunks 94 / 87) and at least three of them (forward of K = V = 128, 16
-// heads, uncut against cut in us: one sequence of 5003 tokens in 8 119 / 74, of 16384 in 8 359 / 163, two of 4096 in 4
-// 105 / 94, four in 2 127 / 158).  A forward that keeps its intermediates and its backward gain from five on (training
-// step: three sequences of 4096, 8 heads, in 5 377 / 352, two of 16 heads in 4 462 / 468).
+// The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 2.2 us per
+// segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16 chunks 92, 71
+// and 77 us, uncut 174; training step of 64 chunks, 8 heads, in 4 and 8 187 and 165 us, uncut 251), and at least three of
+// them (forward of K = V = 128, 16 heads, uncut against cut in us: one sequence of 5003 tokens in 8 119 / 78, of 16384 in 8
+// 359 / 168, two of 4096 in 4 105 / 96, four in 2 125 / 160).  A forward that keeps its intermediates and its backward gain
+// from five on (training step: three sequences of 4096, 8 heads, in 5 379 / 356, two of 16 heads in 4 462 / 472).  Twenty
+// chunks to save pay for both launches up to 16 (sequence, head, slab) triples (24 chunks, uncut / cut: 8 heads 46.3 / 45.7,
+// training step 123 / 116).  With more of them the segments are fewer and longer, and so is the first pass, and the fold
+// reads more: forward of 16 heads, 24, 28 and 32 chunks 48.4 / 51.8, 54.1 / 55.3 and 59.9 / 58.9, of 32 heads, 32, 40, 48
+// and 64 chunks 62.6 / 68.3, 75.1 / 77.2, 86.7 / 85.2 and 109.5 / 100.9; training step of 16 heads, 24, 32 and 40 chunks
+// 136 / 148, 168 / 172 and 203 / 193 (K = V = 128; launches replayed from a graph).
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
   const bool delta = kind != FLA_SCAN_GLA;
-  const int64_t kMinSaved = delta ? 20 : 8, kMinSegments = kind == FLA_SCAN_DELTA_KEPT ? 5 : delta ? 3 : 2;
+  const bool delta_kept = kind == FLA_SCAN_DELTA_KEPT;
+  const int64_t kMinSegments = delta_kept ? 5 : delta ? 3 : 2;
   int64_t min_seg = 4;
   if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_DELTA_KEPT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
@@ -82,7 +87,7 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   if (delta)
     while (100 * min_seg * min_seg < 49 * longest) ++min_seg;
   const int64_t room = kCUs / (H * slabs);   // segments the chip holds at once
-  if (room < 2 || N > room || longest > 0x7fffffff / kChunk) return 0;
+  if (longest == 0 || room < 2 || N > room || longest > 0x7fffffff / kChunk) return 0;
   // the shortest segment with which all of them fit
   auto segments = [&](int64_t len) {
     int64_t s = 0;
@@ -95,7 +100,10 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   int64_t seg = fla_cdiv(total, room);
   seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
-  if (longest - seg < kMinSaved || longest < (kMinSegments - 1) * seg + 1) return 0;
+  const int64_t triples = fla_cdiv(total, longest) * H * slabs;   // sequences of other lengths: as many of the longest
+  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : 14 + triples * 11 / 32;
+  const int64_t min_saved = !delta ? 8 : line > 20 ? line : 20;
+  if (longest - seg < min_saved || longest < (kMinSegments - 1) * seg + 1) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;
   ratio = ratio > seg / 2 ? seg / 2 : ratio;

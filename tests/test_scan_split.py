@@ -99,3 +99,18 @@ def test_nothing_to_cut():
     assert _plan(None, 1, 0, 1, 1, 0, 0) is None
     assert _plan(None, 0, 64, 1, 1, 0, 0) is None
     assert _plan(None, 1, 64 * 200, 512, 2, 0, 0) is None
+
+
+@pytest.mark.parametrize("kind,heads,chunks,cut", [
+    # kind 1, the delta rule's forward, 2, one that keeps its intermediates; K = V = 128, so two slabs a head
+    (1, 8, 24, True), (1, 16, 24, False), (1, 16, 28, False), (1, 16, 32, True), (1, 32, 28, False), (1, 32, 40, False),
+    (1, 32, 48, True), (2, 8, 24, True), (2, 16, 24, False), (2, 16, 32, False), (2, 16, 40, True)])
+def test_delta_rule_is_cut_where_it_pays(kind, heads, chunks, cut):
+    """The cuts that were measured to lose (forward of 32 heads, 28 chunks: 57 us uncut, 65 cut) are not made, also not in
+    a packed batch whose other sequences are short."""
+    for reverse in (0, 1):
+        for bounds in (None, [0, chunks * CHUNK], [0, chunks * CHUNK, chunks * CHUNK + 3]):
+            N = 1 if bounds is None else len(bounds) - 1
+            if N > 1 and cut:   # (what the short sequence takes lengthens the segments)
+                continue
+            assert (_plan(bounds, N, chunks * CHUNK, heads, 2, reverse, kind) is not None) == cut
