@@ -69,14 +69,20 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // reads more: forward of 16 heads, 24, 28 and 32 chunks 48.4 / 51.8, 54.1 / 55.3 and 59.9 / 58.9, of 32 heads, 32, 40, 48
 // and 64 chunks 62.6 / 68.3, 75.1 / 77.2, 86.7 / 85.2 and 109.5 / 100.9; training step of 16 heads, 24, 32 and 40 chunks
 // 136 / 148, 168 / 172 and 203 / 193 (K = V = 128; launches replayed from a graph).
+//
+// The plain scan of chunk_simple_gla's forward takes half as long per chunk as the GLA kernel and fills the chip with half
+// the pairs (slabs of 32 columns), so its line lies higher and rises too, and it wants three segments: K = V = 128, uncut
+// against cut in us, 16 heads, 12, 24 and 32 chunks 22.9 / 27.7, 35.4 / 34.5 and 43.9 / 36.6, two sequences of them, 16, 32
+// and 64 chunks 28.2 / 34.8, 44.8 / 45.0 and 77.5 / 64.8, four, in two segments, 24, 64 and 128 chunks 39.6 / 55.7, 84.7 /
+// 95.5 and 174.8 / 170.3; 4 heads, 12 and 16 chunks 22.1 / 23.6 and 26.0 / 24.3.
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
-  const bool delta = kind != FLA_SCAN_GLA;
-  const bool delta_kept = kind == FLA_SCAN_DELTA_KEPT;
-  const int64_t kMinSegments = delta_kept ? 5 : delta ? 3 : 2;
+  const bool delta_kept = kind == FLA_SCAN_DELTA_KEPT, delta = kind == FLA_SCAN_DELTA || delta_kept,
+             simple = kind == FLA_SCAN_SIMPLE;
+  const int64_t kMinSegments = delta_kept ? 5 : delta || simple ? 3 : 2;
   int64_t min_seg = 4;
-  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_DELTA_KEPT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
+  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_SIMPLE || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
   int64_t longest = 0, total = 0;
   for (int64_t n = 0; n < N; ++n) {
@@ -101,8 +107,8 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
   const int64_t triples = fla_cdiv(total, longest) * H * slabs;   // sequences of other lengths: as many of the longest
-  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : 14 + triples * 11 / 32;
-  const int64_t min_saved = !delta ? 8 : line > 20 ? line : 20;
+  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : delta ? 14 + triples * 11 / 32 : simple ? 8 + triples * 9 / 32 : 8;
+  const int64_t min_saved = delta && line < 20 ? 20 : line;
   if (longest - seg < min_saved || longest < (kMinSegments - 1) * seg + 1) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;

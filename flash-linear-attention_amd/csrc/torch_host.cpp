@@ -357,7 +357,8 @@ Tensor simple_gla_scan(const Tensor& q, const Tensor& k, const Tensor& v, const 
   const Dims& d = a.d;
   Tensor o = fresh_like(v);
   if (a.want_ht) *ht = fresh({d.N, d.H, d.K, d.V}, q, at::kFloat);
-  if (auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K)) {
+  if (auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K,
+                        FLA_SCAN_SIMPLE)) {
     check(fla_chunk_gated_delta_rule_fwd_scan_split(ptr(q), ptr(k), ptr(v), nullptr, fptr(g), nullptr, fptr(h0), ptr(o),
                                                     fptr(*ht), nullptr, nullptr, nullptr, offs(a.plan), coff(a.plan), &c->s,
                                                     dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale, 0.f, stream_of(q)),

@@ -75,7 +75,12 @@ typedef struct fla_split {
   float* transitions_t;
 } fla_split;
 
-enum fla_scan_kind { FLA_SCAN_GLA = 0, FLA_SCAN_DELTA = 1, FLA_SCAN_DELTA_KEPT = 2 /* keeps its intermediates */ };
+enum fla_scan_kind {
+  FLA_SCAN_GLA = 0,
+  FLA_SCAN_DELTA = 1,
+  FLA_SCAN_DELTA_KEPT = 2, /* keeps its intermediates */
+  FLA_SCAN_SIMPLE = 3      /* the plain scan: AT == NULL in fla_chunk_gated_delta_rule_fwd_scan_split */
+};
 
 /* The plan for N sequences of T tokens (or, with offsets_host [N+1], of a packed batch) and H heads in `slabs` workgroups
  * per (sequence, head); reverse: for a scan from right to left; kind: the recurrence (the delta rule: segments of one

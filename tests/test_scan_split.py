@@ -29,7 +29,7 @@ def _plan(bounds, N, T, H, slabs, reverse, kind):
 
 def _check(sp, seg, sub, base, chunks, H, slabs, reverse, kind):
     """``chunks``: chunks of every sequence; ``seg`` and the others None for sequences of equal length."""
-    assert sp.sub_chunks > 0 and sp.ratio > 0 and (kind == 0 or sp.ratio == 1)
+    assert sp.sub_chunks > 0 and sp.ratio > 0 and (kind in (0, 3) or sp.ratio == 1)
     subs = [max(1, -(-c // sp.sub_chunks)) for c in chunks]
     segs = [-(-s // sp.ratio) for s in subs]
     assert max(segs) > 1                                 # something is cut,
@@ -48,7 +48,7 @@ def _check(sp, seg, sub, base, chunks, H, slabs, reverse, kind):
     assert last == list(range(len(seg) - len(last), len(seg)))     # the shorter last pieces start last
 
 
-@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
 def test_packed_batches(kind):
     rng, cut = random.Random(kind), 0
     for _ in range(3000):
@@ -65,7 +65,7 @@ def test_packed_batches(kind):
     assert cut > 300
 
 
-@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
 def test_sequences_of_equal_length(kind):
     cut = 0
     for N in (1, 2, 3, 5, 8, 16, 33, 128):
@@ -102,12 +102,15 @@ def test_nothing_to_cut():
 
 
 @pytest.mark.parametrize("kind,heads,chunks,cut", [
-    # kind 1, the delta rule's forward, 2, one that keeps its intermediates; K = V = 128, so two slabs a head
+    # kind 1, the delta rule's forward, 2, one that keeps its intermediates, 3, the plain scan of chunk_simple_gla; K = V =
+    # 128, so two slabs a head
     (1, 8, 24, True), (1, 16, 24, False), (1, 16, 28, False), (1, 16, 32, True), (1, 32, 28, False), (1, 32, 40, False),
-    (1, 32, 48, True), (2, 8, 24, True), (2, 16, 24, False), (2, 16, 32, False), (2, 16, 40, True)])
-def test_delta_rule_is_cut_where_it_pays(kind, heads, chunks, cut):
-    """The cuts that were measured to lose (forward of 32 heads, 28 chunks: 57 us uncut, 65 cut) are not made, also not in
-    a packed batch whose other sequences are short."""
+    (1, 32, 48, True), (2, 8, 24, True), (2, 16, 24, False), (2, 16, 32, False), (2, 16, 40, True),
+    (3, 4, 12, False), (3, 4, 16, True), (3, 16, 16, False), (3, 16, 24, True), (3, 32, 24, False), (3, 32, 40, True),
+    (3, 48, 64, False), (3, 64, 64, False)])
+def test_cut_where_it_pays(kind, heads, chunks, cut):
+    """The cuts that were measured to lose (delta-rule forward of 32 heads, 28 chunks: 57 us uncut, 65 cut; plain scan of 64
+    heads, 24 chunks: 40 uncut, 56 cut) are not made, also not in a packed batch whose other sequences are short."""
     for reverse in (0, 1):
         for bounds in (None, [0, chunks * CHUNK], [0, chunks * CHUNK, chunks * CHUNK + 3]):
             N = 1 if bounds is None else len(bounds) - 1
