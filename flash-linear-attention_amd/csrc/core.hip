@@ -56,7 +56,9 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // 4, 8, 16 and 32 segments 112, 81, 88 and 104 us, uncut 291).  The first pass gets about as many workgroups as there are
 // CUs: 1, 2 and 4 sub-blocks per segment of that forward 97, 80 and 83 us, of one of 64 pairs in two segments 177, 141 and
 // 126 us (uncut 156).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands,
-// which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us).
+// which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us) up to 64 (sequence, head, slab) triples.  128, in
+// two segments, need twelve (64 heads or four sequences of 16, uncut / cut: forward of 16, 20 and 24 chunks 50.4 / 53.5, 59.3
+// / 61.6 and 68.4 / 65.8 us, training step 145 / 162, 198 / 202 and 237 / 237).
 //
 // The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 2.2 us per
 // segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16 chunks 92, 71
@@ -64,7 +66,7 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // them (forward of K = V = 128, 16 heads, uncut against cut in us: one sequence of 5003 tokens in 8 119 / 78, of 16384 in 8
 // 359 / 168, two of 4096 in 4 105 / 96, four in 2 125 / 160).  A forward that keeps its intermediates and its backward gain
 // from five on (training step: three sequences of 4096, 8 heads, in 5 379 / 356, two of 16 heads in 4 462 / 472).  Twenty
-// chunks to save pay for both launches up to 16 (sequence, head, slab) triples (24 chunks, uncut / cut: 8 heads 46.3 / 45.7,
+// chunks to save pay for both launches up to 16 triples (24 chunks, uncut / cut: 8 heads 46.3 / 45.7,
 // training step 123 / 116).  With more of them the segments are fewer and longer, and so is the first pass, and the fold
 // reads more: forward of 16 heads, 24, 28 and 32 chunks 48.4 / 51.8, 54.1 / 55.3 and 59.9 / 58.9, of 32 heads, 32, 40, 48
 // and 64 chunks 62.6 / 68.3, 75.1 / 77.2, 86.7 / 85.2 and 109.5 / 100.9; training step of 16 heads, 24, 32 and 40 chunks
@@ -107,8 +109,8 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
   const int64_t triples = fla_cdiv(total, longest) * H * slabs;   // sequences of other lengths: as many of the longest
-  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : delta ? 14 + triples * 11 / 32 : simple ? 8 + triples * 9 / 32 : 8;
-  const int64_t min_saved = delta && line < 20 ? 20 : line;
+  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : delta ? 14 + triples * 11 / 32 : simple ? 8 + triples * 9 / 32 : 4 + triples / 16;
+  const int64_t least = delta ? 20 : 8, min_saved = line < least ? least : line;
   if (longest - seg < min_saved || longest < (kMinSegments - 1) * seg + 1) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;

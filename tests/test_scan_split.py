@@ -102,8 +102,9 @@ def test_nothing_to_cut():
 
 
 @pytest.mark.parametrize("kind,heads,chunks,cut", [
-    # kind 1, the delta rule's forward, 2, one that keeps its intermediates, 3, the plain scan of chunk_simple_gla; K = V =
+    # kind 0, GLA, 1, the delta rule's forward, 2, one that keeps its intermediates, 3, the plain scan of chunk_simple_gla; K = V =
     # 128, so two slabs a head
+    (0, 16, 12, True), (0, 32, 12, True), (0, 64, 16, False), (0, 64, 20, False), (0, 64, 24, True),
     (1, 8, 24, True), (1, 16, 24, False), (1, 16, 28, False), (1, 16, 32, True), (1, 32, 28, False), (1, 32, 40, False),
     (1, 32, 48, True), (2, 8, 24, True), (2, 16, 24, False), (2, 16, 32, False), (2, 16, 40, True),
     (3, 4, 12, False), (3, 4, 16, True), (3, 16, 16, False), (3, 16, 24, True), (3, 32, 24, False), (3, 32, 40, True),
