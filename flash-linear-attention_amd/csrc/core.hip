@@ -55,34 +55,29 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // has a CU of its own, so the segments are as short as 256 CUs allow (GLA forward of 16 heads x 8192 tokens, K = V = 128:
 // 4, 8, 16 and 32 segments 112, 81, 88 and 104 us, uncut 291).  The first pass gets about as many workgroups as there are
 // CUs: 1, 2 and 4 sub-blocks per segment of that forward 97, 80 and 83 us, of one of 64 pairs in two segments 177, 141 and
-// 126 us (uncut 156).  Cutting costs the two launches ahead of the scan and another read of two thirds of the operands,
-// which eight chunk periods pay for (16 chunks in 4 segments: 42 -> 33 us) up to 64 (sequence, head, slab) triples.  128, in
-// two segments, need twelve (64 heads or four sequences of 16, uncut / cut: forward of 16, 20 and 24 chunks 50.4 / 53.5, 59.3
-// / 61.6 and 68.4 / 65.8 us, training step 145 / 162, 198 / 202 and 237 / 237).
+// 126 us (uncut 156).  The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its
+// fold 2.2 us per segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16
+// chunks 92, 71 and 77 us, uncut 174; training step of 64 chunks, 8 heads, in 4 and 8 187 and 165 us, uncut 251).
 //
-// The delta rule's first pass costs as much as its scan (it walks K + V columns instead of V) and its fold 2.2 us per
-// segment: segments of at least 0.7 sqrt(chunks) (forward of 128 chunks, 4 heads, in segments of 4, 8 and 16 chunks 92, 71
-// and 77 us, uncut 174; training step of 64 chunks, 8 heads, in 4 and 8 187 and 165 us, uncut 251), and at least three of
-// them (forward of K = V = 128, 16 heads, uncut against cut in us: one sequence of 5003 tokens in 8 119 / 78, of 16384 in 8
-// 359 / 168, two of 4096 in 4 105 / 96, four in 2 125 / 160).  A forward that keeps its intermediates and its backward gain
-// from five on (training step: three sequences of 4096, 8 heads, in 5 379 / 356, two of 16 heads in 4 462 / 472).  Twenty
-// chunks to save pay for both launches up to 16 triples (24 chunks, uncut / cut: 8 heads 46.3 / 45.7,
-// training step 123 / 116).  With more of them the segments are fewer and longer, and so is the first pass, and the fold
-// reads more: forward of 16 heads, 24, 28 and 32 chunks 48.4 / 51.8, 54.1 / 55.3 and 59.9 / 58.9, of 32 heads, 32, 40, 48
-// and 64 chunks 62.6 / 68.3, 75.1 / 77.2, 86.7 / 85.2 and 109.5 / 100.9; training step of 16 heads, 24, 32 and 40 chunks
-// 136 / 148, 168 / 172 and 203 / 193 (K = V = 128; launches replayed from a graph).
-//
-// The plain scan of chunk_simple_gla's forward takes half as long per chunk as the GLA kernel and fills the chip with half
-// the pairs (slabs of 32 columns), so its line lies higher and rises too, and it wants three segments: K = V = 128, uncut
-// against cut in us, 16 heads, 12, 24 and 32 chunks 22.9 / 27.7, 35.4 / 34.5 and 43.9 / 36.6, two sequences of them, 16, 32
-// and 64 chunks 28.2 / 34.8, 44.8 / 45.0 and 77.5 / 64.8, four, in two segments, 24, 64 and 128 chunks 39.6 / 55.7, 84.7 /
-// 95.5 and 174.8 / 170.3; 4 heads, 12 and 16 chunks 22.1 / 23.6 and 26.0 / 24.3.
+// Whether cutting pays is the longest sequence's chunk periods against those of a segment in the scan and in the first pass
+// and the launches ahead of the scan, fitted to the times below (K = V = 128, uncut / cut in us, launches replayed from a
+// graph; packed batches back to back).  The busier the CUs (triples of sequence, head and slab), the less a cut gains.
+//   GLA: one sequence of 16 heads, 12 and 16 chunks 37.7 / 36.1 and 46.0 / 37.2; four, 16, 20 and 24 chunks 50.4 / 53.5,
+//     59.3 / 61.6 and 68.4 / 65.8, their training steps 145 / 162, 198 / 202 and 237 / 237.
+//   Delta rule: 4 and 8 heads, 24 chunks 45.9 / 44.0 and 46.3 / 45.7; 16 heads, 24, 28, 32 and 40 chunks 48.4 / 51.8, 54.1 /
+//     55.3, 59.9 / 58.9 and 70.6 / 63.0; 32 heads, 28, 40, 48 and 64 chunks 57.1 / 65.3, 75.1 / 77.2, 86.8 / 85.4 and 109.5 /
+//     100.9; packed, 16 heads, 54, 94 and 77 chunks 152 / 160, 80 and 171 chunks 253 / 174.
+//   Delta rule, a forward that keeps its intermediates and its backward: from five segments on (training step of two
+//     sequences of 64 chunks, 16 heads, in 4 462 / 472, three of 8 heads in 5 379 / 356); 8 heads, 24 chunks 123 / 116; 16
+//     heads, 24, 32 and 40 chunks 136 / 148, 168 / 172 and 203 / 193.
+//   The plain scan of chunk_simple_gla's forward takes half as long per chunk as the GLA kernel and fills the chip with half
+//     the pairs (slabs of 32 columns): 4 heads, 12 and 16 chunks 22.1 / 23.6 and 26.0 / 24.3; 16 heads, 12, 24 and 32 chunks
+//     22.9 / 27.7, 35.4 / 34.5 and 43.9 / 36.6, two sequences of them, 16, 32 and 64 chunks 28.2 / 34.8, 44.8 / 45.0 and 77.5 /
+//     64.8, four, 24 and 64 chunks 39.6 / 55.7 and 84.7 / 95.5; packed, 54, 94 and 77 chunks 103 / 94.
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
-  const bool delta_kept = kind == FLA_SCAN_DELTA_KEPT, delta = kind == FLA_SCAN_DELTA || delta_kept,
-             simple = kind == FLA_SCAN_SIMPLE;
-  const int64_t kMinSegments = delta_kept ? 5 : delta || simple ? 3 : 2;
+  const bool delta = kind == FLA_SCAN_DELTA || kind == FLA_SCAN_DELTA_KEPT;
   int64_t min_seg = 4;
   if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_SIMPLE || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
@@ -109,9 +104,15 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
   const int64_t triples = fla_cdiv(total, longest) * H * slabs;   // sequences of other lengths: as many of the longest
-  const int64_t line = delta_kept ? 8 + triples * 3 / 4 : delta ? 14 + triples * 11 / 32 : simple ? 8 + triples * 9 / 32 : 4 + triples / 16;
-  const int64_t least = delta ? 20 : 8, min_saved = line < least ? least : line;
-  if (longest - seg < min_saved || longest < (kMinSegments - 1) * seg + 1) return 0;
+  const int64_t L = longest, steps = fla_cdiv(L, seg) - 1;
+  bool pays;
+  switch (kind) {   // the scan of whole sequences against that of the segments and what stands ahead of it: see above
+    case FLA_SCAN_DELTA: pays = 4 * L >= 11 * seg + 7 * steps + (triples < 32 ? 7 + triples * 5 / 8 : 22 + triples * 5 / 32); break;
+    case FLA_SCAN_DELTA_KEPT: pays = steps >= 4 && L - seg >= 20 && L - seg >= 8 + triples * 3 / 4; break;
+    case FLA_SCAN_SIMPLE: pays = 5 * L >= 11 * seg + 28 + (triples < 64 ? triples : 64) * 3 / 4; break;
+    default: pays = 5 * L >= 7 * seg + 31;
+  }
+  if (steps == 0 || !pays) return 0;
   const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;
   ratio = ratio > seg / 2 ? seg / 2 : ratio;

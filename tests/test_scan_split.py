@@ -118,3 +118,17 @@ def test_cut_where_it_pays(kind, heads, chunks, cut):
             if N > 1 and cut:   # (what the short sequence takes lengthens the segments)
                 continue
             assert (_plan(bounds, N, chunks * CHUNK, heads, 2, reverse, kind) is not None) == cut
+
+
+@pytest.mark.parametrize("kind,heads,chunks,cut", [
+    (1, 16, [54, 94, 77], False), (1, 16, [46, 42, 40, 40], False), (1, 16, [60, 20, 20, 20], False), (1, 16, [80, 171], True),
+    (1, 16, [64, 67, 21, 163], True), (1, 8, [54, 94, 77], True), (3, 16, [46, 42, 40, 40], False), (3, 16, [54, 94, 77], True),
+    (0, 16, [46, 42, 40, 40], True), (2, 8, [30, 10, 10], False), (2, 8, [20, 63, 49, 26], True)])
+def test_packed_batches_are_cut_where_it_pays(kind, heads, chunks, cut):
+    """The measured packed batches: segments are as long as room for all of them makes them (delta rule, 16 heads, 54, 94 and
+    77 chunks in segments of 32: 152 us uncut, 160 cut)."""
+    bounds = [0]
+    for c in chunks:
+        bounds.append(bounds[-1] + c * CHUNK - 5)
+    for reverse in (0, 1):
+        assert (_plan(bounds, len(chunks), bounds[-1], heads, 2, reverse, kind) is not None) == cut
