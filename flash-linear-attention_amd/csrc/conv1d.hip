@@ -3,8 +3,8 @@
 // Replaces the external causal_conv1d package the reference's ShortConvolution needs
 // (fla/modules/convolution.py:79-211; forward :171-186, single-token step :188-211).
 //
-// HBM-streaming kernels: a lane owns 8 (backward: 4; half of that where little work has to fill the chip) adjacent
-// channels (one 16-byte access per row for 16-bit storage) and walks a tile of consecutive time steps with the last W inputs (and, in
+// HBM-streaming kernels: a lane owns 8 (fp32 and backward: 4; half of that where little work has to fill the chip) adjacent
+// channels (one 16-byte access per row) and walks a tile of consecutive time steps with the last W inputs (and, in
 // backward, the last W pre-activation gradients) in registers, so every input row is read
 // once per tile plus a (W-1)-row halo that the neighbouring tile has just pulled into L2.
 // The weight/bias gradients are accumulated in registers over all tiles a lane visits, summed
@@ -293,14 +293,16 @@ int launch_conv(const ConvParams& p, bool bwd, hipStream_t st) {
     else hipLaunchKernelGGL((conv_bwd_kernel<T, W, 4>), grid, block, 0, st, p);
   } else {
     // tiles of 4 steps x 4 channels while those of 8 x 8 leave fewer than one wave per SIMD (B=1, T=300, 512 channels:
-    // 5.5 -> 3.7 us; at two waves, B=2, T=2048, 2048 channels, 11.6 -> 13 us)
+    // 5.5 -> 3.7 us; at two waves, B=2, T=2048, 2048 channels, 11.6 -> 13 us).  In fp32 four channels are 16 bytes: tiles of
+    // 8 x 4 (B=2, T=2048, 2048 channels: 12.8 us, 8 x 8 20.3, 16 x 8 16.5; B=8, T=4096 96, 119, 112)
+    constexpr int CV = sizeof(T) == 4 ? 4 : 8;
     const bool brief = p.B * fla_cdiv(p.T, kTileFwd) * cblocks(8) < 1024;
-    const int64_t cb = cblocks(brief ? 4 : 8);
+    const int64_t cb = cblocks(brief ? 4 : CV);
     int64_t gy = fla_cdiv(p.B * fla_cdiv(p.T, brief ? kTileFwdShort : kTileFwd), 4);
     if (gy * cb > 4096) gy = fla_cdiv(4096, cb);   // a few tiles per lane: weights are loaded once
     const dim3 grid((unsigned)cb, (unsigned)(gy < 1 ? 1 : gy > 65535 ? 65535 : gy));
     if (brief) hipLaunchKernelGGL((conv_fwd_kernel<T, W, kTileFwdShort, 4>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((conv_fwd_kernel<T, W, kTileFwd, 8>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((conv_fwd_kernel<T, W, kTileFwd, CV>), grid, block, 0, st, p);
   }
   FLA_CHECK_LAUNCH();
   return FLA_OK;

@@ -168,6 +168,29 @@ def test_norm_swish_gate_16bit_weight_and_bias(device, is_rms, residual):
         assert_close(name, ref.grad, d.grad, 1e-5 if name in ("dx", "do") else 2.0 ** -8)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,T,D,W", [(2, 2055, 1048, 4), (3, 1800, 1048, 3), (2, 2055, 1048, 2), (1, 8195, 2048, 4)])
+def test_causal_conv1d_on_wide_tiles(device, dtype, B, T, D, W):
+    """Sizes that fill the chip: the forward on its wide tiles, the last case's backward too, ragged in time and channels."""
+    from fla_amd.modules.convolution import causal_conv1d as conv
+    from oracle.modules import causal_conv1d
+    gen = torch.Generator().manual_seed(T)
+    x, dy = (torch.randn(B, T, D, generator=gen).to(dtype) for _ in range(2))
+    w, b = torch.rand(D, W, generator=gen) - 0.5, torch.randn(D, generator=gen)
+    print("short conv on wide tiles", dtype, B, T, D, W, flush=True)
+    leaves = [t.to(device).requires_grad_() for t in (x, w, b)]
+    y = conv(*leaves, "silu")
+    y.backward(dy.to(device))
+    refs = [t.float().requires_grad_() for t in (x, w, b)]
+    yr = causal_conv1d(*refs, "silu")
+    yr.backward(dy.float())
+    ft, bt = _tols(dtype)
+    sums = 2e-3 if dtype != torch.float32 else 2e-5   # fp32 sums over B T terms
+    assert_close("y", yr, y, ft)
+    for name, r, d, tol in zip(("dx", "dw", "db"), refs, leaves, (bt, sums, sums)):
+        assert_close(name, r.grad, d.grad, tol)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W", [2, 3, 4])
 @pytest.mark.parametrize("T,D,bias,act", [(1, 64, False, "silu"), (5, 64, True, "silu"), (64, 200, False, None),
