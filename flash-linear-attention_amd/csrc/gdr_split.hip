@@ -11,7 +11,7 @@
 // 16-column blocks, so that an operand read from LDS serves two matrix instructions (16 columns per wave: twice the LDS
 // reads), beside four waves that stage the tiles.  Neither q nor an output is touched: a chunk costs 21 KB of k and Tu, and
 // 16 KB of v for the columns of S, and its load latency is longer than its arithmetic: the staging waves hold three chunks
-// in registers: 2.0 us per chunk (25 us for 7 segments of 10 chunks of 16 heads, K = V = 128).  Tiles staged by the waves
+// in registers: 2.0 us per chunk (23 us for 7 segments of 10 chunks of 16 heads, K = V = 128).  Tiles staged by the waves
 // that multiply, one chunk ahead: 3.9 - 4.5 us.
 // gdr_split_fold_kernel: h <- M h + S; a workgroup carries 16 value columns of one head through the segments, 16 key rows
 // per wave.  The state is fp32 in the scan and stays so between the segments: M and h are multiplied as sums of three bf16

@@ -12,8 +12,8 @@
 //
 // One workgroup of four waves per (sub-block, head) holds the whole K x V tile (a wave a quarter of it), reads every
 // operand once and runs two to a CU: 64 KB (GLA forward, fp32 gates) of loads per chunk against 64 matrix instructions, so
-// it is bound by the loads: 27 us for 16 heads x 7168 tokens, K = V = 128 (117 MB in, 15 MB out: 4.8 TB/s, a large copy
-// moves 5.2).  The fold behind it takes 6 us, the scan over 8 segments 54 us instead of 293 us over the whole sequences.
+// it is bound by the loads: 28 us for 16 heads x 7168 tokens, K = V = 128 (117 MB in, 15 MB out: 4.7 TB/s, a large copy
+// moves 5.1).  The fold behind it takes 6 us, the scan over 8 segments 50 us instead of 291 us over the whole sequences.
 #include "gla_fused_staging.h"
 #include "seq_split.h"
 
