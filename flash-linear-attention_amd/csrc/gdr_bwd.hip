@@ -11,6 +11,8 @@
 //                              store dH_c;  dv2 = dv_loc + (k e^{gamma_last-gamma}) dH_c;
 //                              dH <- e^{gamma_last} dH + (s q e^gamma)^T do - (w e^gamma)^T dv2
 //                                                                                (chunk_delta_h.py:136-237)
+//   gdr_bwd_chunk_kernel     (gdr_bwd_chunk.hip) the two below as one launch, for up to 128 key channels; they remain for
+//                            256 and as the reference's separate stages
 //   gdr_bwd_dqkwg_kernel     per (chunk, head, 64-wide half of K):
 //                              ds = s tril((do v_new^T) * Gamma)
 //                              dq = s e^gamma (do h_c^T) + ds k
@@ -30,6 +32,7 @@
 //                            (wy_fast.py:440-562, written for the single inverse Aw).
 #include <type_traits>
 
+#include "gdr_bwd_chunk.h"
 #include "seq_split.h"
 
 namespace {
@@ -1543,6 +1546,9 @@ int launch_gdr_bwd(const void* q, const void* k, const void* v, const void* w, c
                split_view(split), nullptr, 0};
   if (split && (rc = dhu_split<T>(p2, split, K, st))) return rc;
   if ((rc = launch_dhu<T>(p2, K, st))) return rc;
+  if (K <= 128)
+    return gdr_bwd_chunk(q, k, v, vnew, beta, gam, Aw, dout, dv2, hT, dhtf, dq, dk, dv, dbeta, dgam2, offsets, indices,
+                         grid.x, ntfix, std::is_same<T, bf16>::value ? FLA_BF16 : FLA_F16, T_, H, K, V, scale, st);
   DqkwgParams p3{q, k, vnew, w, dout, dv2, gam, hT, dhtf, dq, dkp, dw, dgam_part, offsets, indices, T_,
                  B * T_, (int)H, (int)K, ntfix, scale};
   if ((rc = launch_dqkwg<T>(p3, V, grid, st))) return rc;
@@ -1580,8 +1586,9 @@ static int gdr_bwd_impl(
     int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream,
     const fla_split* split) {
   FLA_REQUIRE(q && k && v && w && v_new && beta && Aw && dout && hT && (ws_dv_local || Aqk) && ws_dv2 && ws_dh_frag_t &&
-                  ws_dw && ws_dk_partial && ws_dgam_partial && dq && dk && dv && dbeta && dgam2,
+                  dq && dk && dv && dbeta && dgam2,
               FLA_E_INVALID);
+  FLA_REQUIRE(K <= 128 || (ws_dw && ws_dk_partial && ws_dgam_partial), FLA_E_INVALID);
   FLA_REQUIRE(B >= 0 && T >= 0 && H > 0 && K > 0 && V > 0 && N >= 0 && NT >= 0, FLA_E_INVALID);
   FLA_REQUIRE((K == 64 || K == 128 || K == 256) && (V == 64 || V == 128), FLA_E_UNSUPPORTED);
   if (Aqk) FLA_REQUIRE(K <= 128 && (uintptr_t)Aqk % 16 == 0, FLA_E_UNSUPPORTED);

@@ -478,8 +478,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
                  &Mt = saved[10];
     const Tensor dout = grads[0].defined() ? as(grads[0], q.scalar_type()).contiguous() : at::zeros(v.sizes(), v.options());
     const Tensor dht = a.want_ht ? f32(grads[1]) : Tensor();
-    Tensor dv2 = fresh_like(v), dh = fresh_like(hT), dw = fresh_like(k), dkp = fresh_like(k);
-    Tensor dgam = fresh({d.K / 64, d.B * d.T, d.H}, q, at::kFloat);
+    Tensor dv2 = fresh_like(v), dh = fresh_like(hT);
     Tensor dq = fresh_like(q), dk = fresh_like(k), dv = fresh_like(v);
     Tensor dbeta = fresh({d.B, d.T, d.H}, q, at::kFloat), dg = fresh({d.B, d.T, d.H}, q, at::kFloat);
     Tensor dh0 = r.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
@@ -490,15 +489,15 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
       cut->s.decays = fptr(Mt);
       check(fla_chunk_gated_delta_rule_bwd_split(
                 ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout), fptr(dht), ptr(hT),
-                ptr(Aqk), ptr(dv2), ptr(dh), ptr(dw), ptr(dkp), fptr(dgam), ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg),
+                ptr(Aqk), ptr(dv2), ptr(dh), nullptr, nullptr, nullptr, ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg),
                 fptr(dh0), offs(a.plan), idx(a.plan), coff(a.plan), &cut->s, d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
                 (float)a.scale, stream_of(q)),
             "fla_chunk_gated_delta_rule_bwd_split");
       return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor(), Tensor()};
     }
     check(fla_chunk_gated_delta_rule_bwd(ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout),
-                                         fptr(dht), ptr(hT), ptr(Aqk), nullptr, ptr(dv2), ptr(dh), ptr(dw), ptr(dkp),
-                                         fptr(dgam), ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg), fptr(dh0),
+                                         fptr(dht), ptr(hT), ptr(Aqk), nullptr, ptr(dv2), ptr(dh), nullptr, nullptr,
+                                         nullptr, ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg), fptr(dh0),
                                          offs(a.plan), idx(a.plan), coff(a.plan), d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
                                          (float)a.scale, stream_of(q)),
           "fla_chunk_gated_delta_rule_bwd");

@@ -154,11 +154,13 @@ def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do
             chunk_offsets=co)
     ws_dvl, ws_dv2 = (torch.empty_like(v) if Aqk is None else None), torch.empty_like(v)
     ws_dh = torch.empty_like(hT)
-    ws_dw, ws_dkp = torch.empty_like(k), torch.empty_like(k)
-    ws_dgam = q.new_empty(K // 64, B * T, H, dtype=torch.float32)
+    ws_dw = ws_dkp = ws_dgam = None
+    if K > _FUSED_MAX_K:   # up to 128 key channels these stay on the chip
+        ws_dw, ws_dkp = torch.empty_like(k), torch.empty_like(k)
+        ws_dgam = q.new_empty(K // 64, B * T, H, dtype=torch.float32)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dbeta = q.new_empty(B, T, H, dtype=torch.float32)
-    dg = q.new_empty(B, T, H, dtype=torch.float32)   # the last launch sums the partials and takes the reverse cumsum
+    dg = q.new_empty(B, T, H, dtype=torch.float32)   # the last launch takes the reverse cumsum
     dh0 = q.new_empty(N, H, K, V, dtype=torch.float32) if initial_state is not None else None
     if dht is not None:
         dht = (dht if dht.dtype == torch.float32 else dht.float()).contiguous()

@@ -597,19 +597,19 @@ int fla_chunk_bwd_dv_local(const void* q, const void* k, const float* g_cumsum, 
  * chunk_gated_delta_rule_bwd (fla/ops/gated_delta_rule/chunk.py:76-177):
  * chunk_bwd_dv_local (common/chunk_o.py:551), chunk_gated_delta_rule_bwd_dhu
  * (common/chunk_delta_h.py:323), chunk_bwd_dqkwg (common/chunk_o.py:602) and
- * bwd_prepare_wy_repr (gated_delta_rule/wy_fast.py:565).  Four launches, or three with Aqk.
+ * bwd_prepare_wy_repr (gated_delta_rule/wy_fast.py:565).  K up to 128: dv_local (unless Aqk is given), the reverse
+ * scan and one launch for everything behind it; K = 256: the last one as two.
  * Inputs recomputed by the caller with the forward entry points: w, v_new, Aw
  * (fla_gdr_fwd_wy, fla_chunk_gated_delta_rule_fwd_h) and hT (the per-chunk
  * states in FLA_H_FRAGMENT_T order).  g_cumsum fp32 [B,T,H] or NULL.
  * Aqk: the packed score tiles [chunks,H,10,16,16] that fla_chunk_gated_delta_rule_fwd_scan leaves on request, or
  * NULL.  With them (K <= 128) the reverse state scan forms dv_local = Aqk^T do itself: the chunk_bwd_dv_local
  * launch is skipped and ws_dv_local may be NULL.
- * Workspaces: ws_dv_local, ws_dv2 like v; ws_dh_frag_t like hT; ws_dw,
- * ws_dk_partial like k; ws_dgam_partial fp32 [K/64, B*T, H].
+ * Workspaces: ws_dv_local, ws_dv2 like v; ws_dh_frag_t like hT; with K = 256 (unused, may be NULL, up to 128)
+ * ws_dw, ws_dk_partial like k and ws_dgam_partial fp32 [K/64, B*T, H].
  * Outputs: dq, dk [B,T,H,K], dv [B,T,H,V] (q/k/v dtype); dbeta and dg fp32
  * [B,T,H]; dh0 fp32 [N,H,K,V] or NULL.  dg is the gradient w.r.t. the raw gate: the last launch
- * adds the slices of ws_dgam_partial to its own gate terms and takes the reverse chunk-local
- * cumulative sum (the reference's chunk_local_cumsum(dg, reverse=True), chunk.py:170-171);
+ * adds up all gate terms and takes the reverse chunk-local cumulative sum (the reference's chunk_local_cumsum(dg, reverse=True), chunk.py:170-171);
  * without a gate (g_cumsum NULL) it holds nothing meaningful.
  * K in {64,128,256}, V in {64,128}.
  * ---------------------------------------------------------------------- */

@@ -312,6 +312,31 @@ def test_chunk_gdr_backward(device, T, K, V):
         assert_close(name, r, x, tol)
 
 
+@pytest.mark.parametrize("B,T,H", [(1, 1, 1), (2, 63, 3), (1, 65, 2), (2, 1285, 16)])
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (64, 128), (128, 64)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_chunk_gdr_backward_chunk_launch(device, B, T, H, K, V, gated):
+    """The launch behind the reverse scan: single rows, chunks one row short and one row over, and more (chunk, head) items
+    (672) than workgroups run at once (512), so that tiles are reused from item to item.  fp16: its tolerances are a
+    quarter of the bf16 ones, 8x the resolution less the fp32 reference's own order of summation."""
+    q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=70 + T, h0_std=1.0, dtype=torch.float16)
+    if not gated:
+        g = torch.zeros_like(g)
+    gen = torch.Generator().manual_seed(9)
+    do = torch.randn(B, T, H, V, generator=gen).half()
+    dht = torch.randn(B, H, K, V, generator=gen) * 0.1
+    print(f"chunk_gdr backward, one launch per chunk B={B} T={T} H={H} K={K} V={V} gated={gated}", flush=True)
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    leaves = [None if x is None else x.to(device).requires_grad_() for x in (q, k, v, g if gated else None, beta, h0)]
+    o, ht = chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], output_final_state=True, head_first=False)
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    torch.cuda.synchronize()
+    ref = _grads_ref(q, k, v, g, beta, h0, do, dht)
+    for name, r, x, tol in zip(NAMES, ref, leaves, TOLS):
+        if x is not None:
+            assert_close(name, r, x.grad, tol / 4)
+
+
 def test_chunk_gdr_backward_varlen_and_headfirst(device):
     gen = torch.Generator().manual_seed(8)
     T, N, H, D = 500, 4, 2, 128
