@@ -7,7 +7,7 @@
 // gradients stay on the chip, and w is not needed: its gate term is the row sum of w . dw = Aw ((dw k^T) diag beta), whose
 // second factor the WY gradient forms anyway.  191 us there, 4.75 TB/s (a large copy: 5.0), where the two launches it
 // replaces took 200 + 146 us for 1.3 GB; 2 x 2048 tokens 50 us instead of 50 + 39.
-#include "chunk_common.h"
+#include "chunk_rows.h"
 #include "gdr_bwd_chunk.h"
 
 namespace {
@@ -35,61 +35,6 @@ struct ChunkBwdParams {
   int H, NTfix;
   float scale;
 };
-
-// A [64][D] tile moved in 16-byte pieces, whole rows per group of D / 8 lanes.  Rows past the end of a short chunk
-// re-read its last row (no load sits under a branch) and are cleared on the way to LDS.
-template <typename T, int D>
-struct RowTile {
-  typedef typename Elem<T>::v8 v8;
-  static constexpr int C8 = D / 8, N = BT * C8 / 256;
-  static FLA_DEVICE void load(const void* src, int64_t r0h, int L, int H, int tid, v8* reg) {
-    const char* base = (const char*)src + r0h * D * (int64_t)sizeof(T);
-    const uint32_t pitch = (uint32_t)H * D * (uint32_t)sizeof(T), col = (uint32_t)(tid % C8) * 16u;
-    const uint32_t lim = (uint32_t)(L - 1) * pitch + col;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const uint32_t o = (uint32_t)((tid + 256 * i) / C8) * pitch + col;
-      reg[i] = *(const v8*)(base + (o < lim ? o : lim));
-    }
-  }
-  static FLA_DEVICE void put(T* dst, int ld, int L, int tid, const v8* reg) {
-    const v8 z = {(T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f};
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int e = tid + 256 * i, row = e / C8, c8 = (e % C8) * 8;
-      *(v8*)&dst[row * ld + c8] = row < L ? reg[i] : z;
-    }
-  }
-  static FLA_DEVICE void get(const T* tile, int ld, int tid, v8* reg) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int e = tid + 256 * i;
-      reg[i] = *(const v8*)&tile[e / C8 * ld + (e % C8) * 8];
-    }
-  }
-  static FLA_DEVICE void store(void* dst, int64_t r0h, int L, int H, int tid, const v8* reg) {
-    char* base = (char*)dst + r0h * D * (int64_t)sizeof(T);
-    const uint32_t pitch = (uint32_t)H * D * (uint32_t)sizeof(T), col = (uint32_t)(tid % C8) * 16u;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const int row = (tid + 256 * i) / C8;
-      // nobody reads the gradients soon: they need not push the operands of other workgroups out of the L2 (204 -> 198 us)
-      if (row < L) __builtin_nontemporal_store(reg[i], (v8*)(base + ((uint32_t)row * pitch + col)));
-    }
-  }
-};
-
-// The lane id through an opaque copy: addresses formed from it are formed where they are used.  Left to itself the compiler
-// forms the LDS and row addresses of all phases once per item and keeps them, a hundred registers it then spills - and every
-// reload of a spilled register waits for all loads and stores in flight (245 us instead of 204).
-FLA_DEVICE int fresh_tid(int tid) {
-  asm volatile("" : "+v"(tid));
-  return tid;
-}
-#define FLA_PHASE(t0)                                    \
-  const int tid = fresh_tid(t0), lane = tid & 63;        \
-  const int l32 = lane & 31, hi4 = 4 * (lane >> 5);      \
-  (void)l32, (void)hi4
 
 // Four waves.  In products with K (V) result columns a wave owns 32 of them and, with 128 columns, all 64 rows, with 64
 // columns one half of the rows: what a wave later needs of such a result (gate terms, in-place replacement of q by dq, k

@@ -227,13 +227,13 @@ struct GlaArgs {
   Dims d;
   PlanPtr plan;
   double scale;
-  bool want_ht, head_gates, keep_khat;
+  bool want_ht, head_gates;
   int gate_form = 0;
   double normalizer = 1.0;
   std::optional<double> clamp;
 };
 struct GlaKept {
-  Tensor wide, hT, qg, decay, kh, sc;
+  Tensor wide, hT, qg, decay;
 };
 
 Tensor gla_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& h0, const GlaArgs& a,
@@ -249,23 +249,19 @@ Tensor gla_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
     x.hT = fresh({d.chunks, d.H, d.K, d.V}, q, q.scalar_type());
     x.qg = fresh_like(q);
     x.decay = fresh({d.chunks, d.H, d.K}, q, at::kFloat);
-    if (a.keep_khat) {
-      x.kh = fresh({d.chunks, d.H, d.K, BT}, q, q.scalar_type());
-      x.sc = fresh({d.chunks, d.H, BT, BT}, q, q.scalar_type());
-    }
   }
   const fla_stream_t st = stream_of(q);
   const int form = a.head_gates ? 1 : a.gate_form;
   if (auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K)) {
     check(fla_chunk_gla_fwd_fused_split(ptr(q), ptr(k), ptr(v), ptr(g), fptr(h0), ptr(o), fptr(*ht), (int*)ptr(wide),
-                                        ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), ptr(x.kh), ptr(x.sc), offs(a.plan),
+                                        ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), nullptr, nullptr, offs(a.plan),
                                         idx(a.plan), coff(a.plan), &c->s, d.NT, dt(q), dt(g), d.B, d.T, d.H, d.K, d.V, d.N,
                                         (float)a.scale, form, (float)a.normalizer, a.clamp.has_value(),
                                         (float)a.clamp.value_or(0.0), st),
           "fla_chunk_gla_fwd_fused_split");
   } else if (form == 1) {
     check(fla_chunk_simple_gla_fwd_fused(ptr(q), ptr(k), ptr(v), fptr(g), fptr(h0), ptr(o), fptr(*ht), (int*)ptr(wide),
-                                         ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), ptr(x.kh), ptr(x.sc), offs(a.plan),
+                                         ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), nullptr, nullptr, offs(a.plan),
                                          idx(a.plan), coff(a.plan), order(a.plan), d.NT, dt(q), d.B, d.T, d.H, d.K, d.V,
                                          d.N, (float)a.scale, st),
           "fla_chunk_simple_gla_fwd_fused");
@@ -277,7 +273,7 @@ Tensor gla_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
           "fla_chunk_gla_fwd_fused_logits");
   } else if (kept) {
     check(fla_chunk_gla_fwd_fused_kept(ptr(q), ptr(k), ptr(v), ptr(g), fptr(h0), ptr(o), fptr(*ht), (int*)ptr(wide),
-                                       ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), ptr(x.kh), ptr(x.sc), offs(a.plan),
+                                       ptr(hwide), ptr(x.hT), ptr(x.qg), fptr(x.decay), nullptr, nullptr, offs(a.plan),
                                        idx(a.plan), coff(a.plan), order(a.plan), d.NT, dt(q), dt(g), d.B, d.T, d.H, d.K,
                                        d.V, d.N, (float)a.scale, st),
           "fla_chunk_gla_fwd_fused_kept");
@@ -305,7 +301,7 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     Tensor ht;
     GlaKept x;
     Tensor o = gla_forward(q, k, v, g, h0, a, &ht, &x);
-    ctx->save_for_backward({q, k, v, g, x.wide, x.hT, x.qg, x.decay, x.kh, x.sc, given(offsets)});
+    ctx->save_for_backward({q, k, v, g, x.wide, x.hT, x.qg, x.decay, given(offsets)});
     ctx->set_materialize_grads(false);
     hold(ctx, Rest{a, g_.scalar_type(), h0.defined()});
     return a.want_ht ? variable_list{o, ht} : variable_list{o};
@@ -318,31 +314,30 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     const GlaArgs& a = rest.a;
     const Dims& d = a.d;
     const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &g = saved[3], &wide = saved[4], &hT = saved[5], &qg = saved[6],
-                 &decay = saved[7], &kh = saved[8], &sc = saved[9];
+                 &decay = saved[7];
     const Tensor dout = grads[0].defined() ? as(grads[0], q.scalar_type()).contiguous() : at::zeros(v.sizes(), v.options());
     const Tensor dht = a.want_ht ? f32(grads[1]) : Tensor();
     Tensor dhtf = fresh_like(hT), dq = fresh_like(q), dk = fresh_like(k), dv = fresh_like(v);
-    // per-head gates: the kernels add their slices' sums to it
-    Tensor dg = a.head_gates ? at::zeros({d.B, d.T, d.H}, g.options()) : fresh(q.sizes(), q, at::kFloat);
+    Tensor dg = a.head_gates ? fresh({d.B, d.T, d.H}, q, at::kFloat) : fresh(q.sizes(), q, at::kFloat);
     Tensor dh0 = rest.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
     const fla_stream_t st = stream_of(q);
-    std::optional<Cut> c;
-    if (kh.defined()) c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 32), true, q, d.K * d.V, d.K);
+    // (the reverse scan's workgroups hold 64 x 64 tiles of a state)
+    auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.K / 64 * (d.V / 64)), true, q, d.K * d.V, d.K);
     if (c) {
       check(fla_chunk_gla_bwd_split(ptr(q), ptr(k), ptr(v), ptr(g), ptr(dout), fptr(dht), ptr(hT), ptr(qg), fptr(decay),
-                                    ptr(kh), ptr(sc), ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
+                                    nullptr, nullptr, ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
                                     (const int*)ptr(wide), offs(a.plan), idx(a.plan), coff(a.plan), &c->s, d.NT, dt(q), dt(g),
                                     d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale, a.head_gates, st),
             "fla_chunk_gla_bwd_split");
     } else if (a.head_gates) {
       check(fla_chunk_simple_gla_bwd(ptr(q), ptr(k), ptr(v), fptr(g), ptr(dout), fptr(dht), ptr(hT), ptr(qg), fptr(decay),
-                                     ptr(kh), ptr(sc), ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
+                                     nullptr, nullptr, ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
                                      (const int*)ptr(wide), offs(a.plan), idx(a.plan), coff(a.plan), d.NT, dt(q), d.B, d.T,
                                      d.H, d.K, d.V, d.N, (float)a.scale, st),
             "fla_chunk_simple_gla_bwd");
     } else {
       check(fla_chunk_gla_bwd_kept(ptr(q), ptr(k), ptr(v), ptr(g), ptr(dout), fptr(dht), ptr(hT), ptr(qg), fptr(decay),
-                                   ptr(kh), ptr(sc), ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
+                                   nullptr, nullptr, ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),
                                    (const int*)ptr(wide), offs(a.plan), idx(a.plan), coff(a.plan), d.NT, dt(q), dt(g), d.B,
                                    d.T, d.H, d.K, d.V, d.N, (float)a.scale, st),
             "fla_chunk_gla_bwd_kept");
@@ -694,28 +689,27 @@ PyObject* py_plan(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// chunk_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat, normalizer, clamp, offsets)
+// chunk_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, normalizer, clamp, offsets)
 //   normalizer None: g holds log-gates
 PyObject* py_chunk_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 13);
+  expect(n, 12);
   Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]),
-         offsets = arg_tensor(p[12]);
+         offsets = arg_tensor(p[11]);
   GlaArgs a{};
   a.plan = arg_plan(p[7]);
   if (!chunk_operands(q, k, v, h0, a.plan, &a.d) || !g.defined() || !g.is_cuda() || g.sizes() != q.sizes()) return none();
   if (g.scalar_type() != at::kFloat && g.scalar_type() != q.scalar_type()) return none();
   const bool grad = wants_grad({&q, &k, &v, &g, &h0});
-  const auto normalizer = arg_opt_double(p[10]);
+  const auto normalizer = arg_opt_double(p[9]);
   if (grad && (normalizer || !arg_bool(p[8]))) return none();
   a.scale = p[4] == Py_None ? 1.0 / std::sqrt((double)a.d.K) : arg_double(p[4]);
   if (grad && a.scale == 0.0) return none();
   a.want_ht = arg_bool(p[6]);
-  a.keep_khat = arg_bool(p[9]);
   if (normalizer) {
     a.gate_form = 2;
     a.normalizer = *normalizer;
-    a.clamp = arg_opt_double(p[11]);
+    a.clamp = arg_opt_double(p[10]);
   }
   if (grad) {
     auto out = GlaNode::apply(q, k, v, g, maybe(h0), maybe(offsets), a);
@@ -729,12 +723,12 @@ PyObject* py_chunk_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// chunk_simple_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, keep_khat, offsets)
+// chunk_simple_gla(q, k, v, g, scale, h0, want_ht, plan, may_differentiate, offsets)
 PyObject* py_chunk_simple_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  expect(n, 11);
+  expect(n, 10);
   Tensor q = arg_tensor(p[0]), k = arg_tensor(p[1]), v = arg_tensor(p[2]), g = arg_tensor(p[3]), h0 = arg_tensor(p[5]),
-         offsets = arg_tensor(p[10]);
+         offsets = arg_tensor(p[9]);
   GlaArgs a{};
   a.plan = arg_plan(p[7]);
   if (!chunk_operands(q, k, v, h0, a.plan, &a.d) || !g.defined() || !g.is_cuda() || g.dim() != 3 || g.size(0) != a.d.B ||
@@ -745,7 +739,6 @@ PyObject* py_chunk_simple_gla(PyObject*, PyObject* const* p, Py_ssize_t n) {
   a.scale = p[4] == Py_None ? 1.0 / std::sqrt((double)a.d.K) : arg_double(p[4]);
   if (grad && a.scale == 0.0) return none();
   a.want_ht = arg_bool(p[6]);
-  a.keep_khat = arg_bool(p[9]);
   a.head_gates = true;
   if (grad) {
     auto out = GlaNode::apply(q, k, v, g, maybe(h0), maybe(offsets), a);

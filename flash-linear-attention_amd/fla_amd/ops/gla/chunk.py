@@ -30,9 +30,6 @@ _SUPPORTED_KV = {(64, 64), (128, 128), (64, 128), (128, 64)}
 # pass, which the reference starts by recomputing those states (fla/ops/gla/chunk.py:1239-1253).
 # FLA_AMD_RECOMPUTE_STATES=1 (or setting this flag to False) restores the reference's behaviour.
 KEEP_STATES_FOR_BACKWARD = os.environ.get("FLA_AMD_RECOMPUTE_STATES", "0") in ("", "0")
-# With the states, a differentiated forward (per-key gates, V <= 128) also keeps k^ = k e^{G_last - G} and the score tile
-# of every chunk (1.5 more tensors of k's size), from which the backward's reverse state scan forms dv on its way.
-KEEP_KHAT_AND_SCORES = os.environ.get("FLA_AMD_GLA_FUSED_DV", "1") not in ("", "0")
 # fp32 q/k/v run through the fp16 chunk kernels, as the reference runs them through its chunk kernels with fp32 operands
 # on the matrix pipe at reduced precision (tests/ops/test_gla.py:149-201): q, k and v are divided by a power of two >= their
 # largest magnitude (exact; found on the device, no synchronisation) and rounded to fp16, gates and states stay fp32, and
@@ -279,7 +276,8 @@ def _guard_workspaces(q, chunks, H, KV, keep):
 
 
 def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets=None, exact_guard=True,
-                        return_flags=False, states_out=None, head_gates=False, first_launch_only=False):
+                        return_flags=False, states_out=None, head_gates=False, first_launch_only=False,
+                        khat_and_scores=True):
     """Forward through ``fla_chunk_gla_fwd_fused``: seq-first, K in {64,128}, V % 64 == 0.
     With ``exact_guard`` (needs V <= 128) chunks whose cumulative log-gate leaves the
     single-reference range are detected on the device and recomputed exactly; ``return_flags``
@@ -287,7 +285,8 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
     ``states_out`` the launch also writes the state entering every chunk (transposed fragment
     order, what the backward kernels read) and appends it, followed (per-key gates only) by the gated queries
     ``q e^{G}`` ``[B,T,H,K]`` and the chunk decays ``e^{G_last}`` ``[chunks,H,K]`` the backward's reverse state scan
-    streams (``fla_chunk_gla_fwd_fused_kept``).  ``head_gates``: ``g`` is one fp32 log-gate
+    streams (``fla_chunk_gla_fwd_fused_kept``), and, unless ``khat_and_scores`` is off,
+    ``k e^{G_last - G}`` ``[chunks,H,K,64]`` and the score tiles ``[chunks,H,64,64]``.  ``head_gates``: ``g`` is one fp32 log-gate
     per (token, head), ``[B,T,H]`` (``fla_chunk_simple_gla_fwd_fused``)."""
     B, T, H, K = q.shape
     V = v.shape[-1]
@@ -319,7 +318,7 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
                 qg = torch.empty_like(q)
                 decay = q.new_empty(B, nt, H, K, dtype=torch.float32)
                 states_out.extend((qg, decay))
-                if KEEP_KHAT_AND_SCORES and V <= 128:
+                if khat_and_scores and V <= 128:
                     kh = q.new_empty(B, nt, H, K, BT)
                     sc = q.new_empty(B, nt, H, BT, BT)
                     states_out.extend((kh, sc))
@@ -332,7 +331,7 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
             qg = torch.empty_like(q)
             decay = q.new_empty(B, nt, H, K, dtype=torch.float32)
             kh = sc = None
-            if KEEP_KHAT_AND_SCORES and V <= 128:
+            if khat_and_scores and V <= 128:
                 kh = q.new_empty(B, nt, H, K, BT)
                 sc = q.new_empty(B, nt, H, BT, BT)
             be.check(be.lib().fla_chunk_gla_fwd_fused_kept(*head, be.ptr(hT), be.ptr(qg), be.ptr(decay), be.ptr(kh),
@@ -442,7 +441,7 @@ def chunk_gla_fwd(q, k, v, g, g_cumsum, scale, initial_state, output_final_state
 
 
 def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wide=None, hT=None, qg=None,
-                         decay=None, head_gates=False, kh=None, scores=None):
+                         decay=None, head_gates=False):
     """Backward on prepared tensors (seq-first, 16-bit, 64-aligned head dims).
     Returns ``(dq, dk, dv, dg, dh0)``; without ``hT`` (the states a forward pass kept) it
     recomputes the per-chunk states as the reference does (``fla/ops/gla/chunk.py:1239-1253``).  ``qg``, ``decay``:
@@ -470,10 +469,7 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
                             fragment_layout=True, transposed_fragments=True, chunk_offsets=co)
     dhtf = torch.empty_like(hT)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    if kept and head_gates:
-        dg = q.new_zeros(B, T, H, dtype=torch.float32)   # the kernels add their slices' sums to it
-    else:
-        dg = q.new_empty(B, T, H, K, dtype=torch.float32)
+    dg = q.new_empty(q.shape[:3] if kept and head_gates else q.shape, dtype=torch.float32)
     dh0 = q.new_empty(N, H, K, V, dtype=torch.float32) if initial_state is not None else None
     if dht is not None:
         dht = (dht if dht.dtype == torch.float32 else dht.float()).contiguous()
@@ -482,11 +478,11 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
     outs = (be.ptr(dhtf), be.ptr(dq), be.ptr(dk), be.ptr(dv), be.ptr(dg))
     head = (be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(g), be.ptr(do), be.ptr(dht), be.ptr(hT))
     if kept and head_gates:
-        be.check(be.lib().fla_chunk_simple_gla_bwd(*head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs,
+        be.check(be.lib().fla_chunk_simple_gla_bwd(*head, be.ptr(qg), be.ptr(decay), None, None, *outs,
                                                    *tail[:7], *tail[8:]),
                  "fla_chunk_simple_gla_bwd")
     elif kept:
-        be.check(be.lib().fla_chunk_gla_bwd_kept(*head, be.ptr(qg), be.ptr(decay), be.ptr(kh), be.ptr(scores), *outs,
+        be.check(be.lib().fla_chunk_gla_bwd_kept(*head, be.ptr(qg), be.ptr(decay), None, None, *outs,
                                                  *tail), "fla_chunk_gla_bwd_kept")
     else:
         be.check(be.lib().fla_chunk_gla_bwd(*head, *outs, *tail), "fla_chunk_gla_bwd")
@@ -540,13 +536,11 @@ def chunk_gla_bwd(q, k, v, g, g_cumsum, scale, initial_state, h, A, do, dht,
     else:
         states = []
         _, _, wide = chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, False, offsets, return_flags=True,
-                                         states_out=states)
+                                         states_out=states, khat_and_scores=False)
         dq, dk, dv, dg, dh0 = chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wide,
                                                    hT=states[0],
                                                    qg=states[1] if len(states) > 1 else None,
-                                                   decay=states[2] if len(states) > 2 else None,
-                                                   kh=states[3] if len(states) > 4 else None,
-                                                   scores=states[4] if len(states) > 4 else None)
+                                                   decay=states[2] if len(states) > 2 else None)
     if head_first:
         dq, dk, dv, dg = (x.transpose(1, 2) for x in (dq, dk, dv, dg))
     return dq, dk, dv, dg, dh0
@@ -640,7 +634,7 @@ def _chunk_gla_16bit(q, k, v, g, scale, initial_state, output_final_state, offse
     q, k, g, v = _pad_dim(q, KP), _pad_dim(k, KP), _pad_dim(g, KP), _pad_dim(v, VP)
     if h0 is not None and (KP, VP) != (K, V):
         h0 = F.pad(h0, (0, VP - V, 0, KP - K))
-    res = host().chunk_gla(q, k, v, g, scale, h0, output_final_state, native_plan(offsets), True, KEEP_KHAT_AND_SCORES,
+    res = host().chunk_gla(q, k, v, g, scale, h0, output_final_state, native_plan(offsets), True,
                            None, None, offsets)
     if res is None:
         raise ValueError(f"fla_amd chunk_gla: inconsistent operands q {tuple(q.shape)}, k {tuple(k.shape)}, "
@@ -723,7 +717,7 @@ def chunk_gla(
     if not head_first:
         # seq-first operands as the kernels read them: nothing left to do in Python
         res = host().chunk_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
-                               KEEP_STATES_FOR_BACKWARD, KEEP_KHAT_AND_SCORES, gate_logit_normalizer, gate_clamp_min,
+                               KEEP_STATES_FOR_BACKWARD, gate_logit_normalizer, gate_clamp_min,
                                offsets)
         if res is not None:
             return res

@@ -64,7 +64,8 @@ class ChunkSimpleGLAFunction(torch.autograd.Function):
         h0 = initial_state
         flags_states = [] if gla_chunk.KEEP_STATES_FOR_BACKWARD and any(ctx.needs_input_grad) else None
         o, ht, wide = chunk_gla_fwd_fused(q, k, v, gf, scale, h0, output_final_state, offsets=offsets,
-                                          return_flags=True, states_out=flags_states, head_gates=True)
+                                          return_flags=True, states_out=flags_states, head_gates=True,
+                                          khat_and_scores=False)
         ctx.save_for_backward(q, k, v, gf, h0, offsets, wide, *(flags_states or ()))
         ctx.scale, ctx.g_dtype = scale, g.dtype
         ctx.h0_dtype = None if initial_state is None else initial_state.dtype
@@ -76,11 +77,9 @@ class ChunkSimpleGLAFunction(torch.autograd.Function):
         q, k, v, gf, h0, offsets, wide, *kept = ctx.saved_tensors
         hT = kept[0] if kept else None
         qg, decay = (kept[1], kept[2]) if len(kept) > 2 else (None, None)
-        kh, scores = (kept[3], kept[4]) if len(kept) > 4 else (None, None)
         h0f = None if h0 is None else h0.float().contiguous()
         dq, dk, dv, dg, dh0 = chunk_gla_bwd_device(q, k, v, gf, ctx.scale, h0f, do.to(q.dtype).contiguous(), dht,
-                                                   offsets, wide, hT=hT, qg=qg, decay=decay, head_gates=True, kh=kh,
-                                                   scores=scores)
+                                                   offsets, wide, hT=hT, qg=qg, decay=decay, head_gates=True)
         if dh0 is not None:
             dh0 = dh0.to(ctx.h0_dtype)
         return dq, dk, dv, dg.to(ctx.g_dtype), None, dh0, None, None
@@ -114,7 +113,7 @@ def chunk_simple_gla(
         check_varlen_args(q, offsets, head_first, initial_state)
     if SCAN_FORWARD and not head_first:
         res = host().chunk_simple_gla(q, k, v, g, scale, initial_state, output_final_state, native_plan(offsets),
-                                      gla_chunk.KEEP_STATES_FOR_BACKWARD, gla_chunk.KEEP_KHAT_AND_SCORES, offsets)
+                                      gla_chunk.KEEP_STATES_FOR_BACKWARD, offsets)
         if res is not None:
             return res
     if scale is None:

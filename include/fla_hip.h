@@ -292,8 +292,8 @@ int fla_chunk_gla_fwd_fused_states(const void* q, const void* k, const void* v, 
  * queries q_gated = q e^{G} ([B,T,H,K] in the q/k/v dtype, G the chunk-local prefix sum of the log-gates; rows
  * past the end of a short chunk are not written) and chunk_decay = e^{G_last} (fp32 [chunks, H, K]).  Hand both
  * to fla_chunk_gla_bwd_kept.  khat_t and scores (both or neither, q/k/v dtype): k^ = k e^{G_last - G} per chunk,
- * key-major [chunks, H, K, 64], and the chunk's causal score tile tril(q~ k~^T) (unscaled), [chunks, H, 64, 64]; with
- * them fla_chunk_gla_bwd_kept forms dv inside its reverse state scan. */
+ * key-major [chunks, H, K, 64], and the chunk's causal score tile tril(q~ k~^T) (unscaled), [chunks, H, 64, 64]
+ * (no launch of this library reads them). */
 int fla_chunk_gla_fwd_fused_kept(const void* q, const void* k, const void* v, const void* gates,
                                  const float* h0, void* o, float* ht, int* ws_wide, void* ws_hwide,
                                  void* h_frag_t, void* q_gated, float* chunk_decay, void* khat_t, void* scores,
@@ -473,7 +473,7 @@ int fla_chunk_gated_delta_rule_fwd_onepass(const void* q, const void* k, const v
  * Chunked GLA backward (chunk size 64), replaces chunk_gla_bwd
  * (fla/ops/gla/chunk.py:1217-1320: chunk_bwd_dh common/chunk_h.py:338-402,
  * chunk_gla_bwd_dv :1018, _dA :982, _dqk_intra :1057, _dqkg :1102).
- * Three launches on `stream`: reverse state scan, dv, dq/dk/dg.
+ * Two launches on `stream`: reverse state scan, dq/dk/dv/dg.
  *   gates   raw log-gates [B,T,H,K] (fp32 or the q/k/v dtype)
  *   dout    gradient of o, [B,T,H,V] in the q/k/v dtype; dht fp32 [N,H,K,V] or NULL
  *   hT      forward states in FLA_H_FRAGMENT_T order (kept by fla_chunk_gla_fwd_fused_states
@@ -485,7 +485,7 @@ int fla_chunk_gated_delta_rule_fwd_onepass(const void* q, const void* k, const v
  *   wide    int32 [chunks, H] flags written by fla_chunk_gla_fwd_fused (ws_wide), or
  *           NULL.  The kernels score a chunk with one reference point (exact while
  *           the chunk-cumulative log-gate stays within +-80); for flagged chunks the
- *           intra-chunk terms are instead added by a fourth launch with pairwise
+ *           intra-chunk terms are instead added by a third launch with pairwise
  *           exponents <= 0 (the reference's sub-block arithmetic,
  *           fla/ops/gla/chunk.py:409-567).
  * ---------------------------------------------------------------------- */
@@ -500,8 +500,7 @@ int fla_chunk_gla_bwd(const void* q, const void* k, const void* v, const void* g
 /* The same with q_gated and chunk_decay from fla_chunk_gla_fwd_fused_kept: the reverse state scan
  * (chunk_bwd_dh, fla/ops/common/chunk_h.py:338-402) streams them and do instead of re-forming prefix sums and
  * exponentials from q and the gates; results equal fla_chunk_gla_bwd's to rounding.  scale must not be 0.
- * khat_t and scores (both or NULL) as the forward left them: the scan then also forms dv = s P^T do + k^ dH
- * (chunk_gla_bwd_dv, fla/ops/gla/chunk.py:1037-1061) and the launch of its own for dv is skipped: two launches. */
+ * khat_t and scores (both or NULL) as the forward can leave them: accepted, not read. */
 int fla_chunk_gla_bwd_kept(const void* q, const void* k, const void* v, const void* gates, const void* dout,
                            const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,
                            const void* khat_t, const void* scores, void* dh_frag_t, void* dq, void* dk, void* dv, float* dg, float* dh0, const int* wide,
@@ -510,10 +509,9 @@ int fla_chunk_gla_bwd_kept(const void* q, const void* k, const void* v, const vo
                            int64_t N, float scale, fla_stream_t stream);
 
 /* The backward of chunk_simple_gla (fla/ops/simple_gla/chunk.py:134-210: chunk_bwd_dh, chunk_bwd_dqkwg,
- * chunk_bwd_dv with one gate per (token, head)) on the same three launches: g fp32 [B,T,H] is read as it is (a lane
- * broadcasts its row's gate over its key channels) and dg, fp32 [B,T,H], which the caller zeroes, receives the
- * gate gradient summed over the key channels (each 64-channel slice of a head adds its share; the additions of
- * one entry happen in a fixed order).  hT, q_gated and chunk_decay as fla_chunk_simple_gla_fwd_fused left them;
+ * chunk_bwd_dv with one gate per (token, head)) on the same launches: g fp32 [B,T,H] is read as it is (a lane
+ * broadcasts its row's gate over its key channels) and dg, fp32 [B,T,H], receives the gate gradient summed over the
+ * key channels in a fixed order.  hT, q_gated and chunk_decay as fla_chunk_simple_gla_fwd_fused left them;
  * everything else as for fla_chunk_gla_bwd_kept. */
 int fla_chunk_simple_gla_bwd(const void* q, const void* k, const void* v, const float* g, const void* dout,
                              const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,
@@ -522,8 +520,8 @@ int fla_chunk_simple_gla_bwd(const void* q, const void* k, const void* v, const 
                              int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N,
                              float scale, fla_stream_t stream);
 
-/* fla_chunk_gla_bwd_kept (head_gates: fla_chunk_simple_gla_bwd) with khat_t and scores on sequences cut into segments
- * (fla_scan_split with V / 32 slabs, reverse): the state gradient leaving every segment is formed first and the reverse
+/* fla_chunk_gla_bwd_kept (head_gates: fla_chunk_simple_gla_bwd) on sequences cut into segments
+ * (fla_scan_split with (K / 64) (V / 64) slabs, reverse): the state gradient leaving every segment is formed first and the reverse
  * state scan runs over the segments. */
 int fla_chunk_gla_bwd_split(const void* q, const void* k, const void* v, const void* gates, const void* dout,
                             const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,

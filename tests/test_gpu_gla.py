@@ -262,6 +262,36 @@ def test_chunk_gla_backward_extreme_gates(device, normalizer):
         assert_close(name, r, x, tol)
 
 
+@pytest.mark.parametrize("B,T,H,K,V", [(1, 1, 1, 128, 128), (1, 1, 1, 64, 64), (2, 63, 3, 128, 64), (1, 65, 2, 64, 128),
+                                       (1, 65, 2, 128, 128), (1, 127, 2, 64, 64), (1, 2309, 16, 64, 64)])
+@pytest.mark.parametrize("gates", ["float32", "float16", "head"])
+def test_chunk_gla_backward_chunk_launch(device, B, T, H, K, V, gates):
+    """The launch that forms all gradients of a (chunk, head): single rows, chunks one row short and one row over, every pair
+    of head dims, more items (592) than workgroups run at once (512), per-key gates of both types and one gate per head.
+    fp16: its tolerances are a quarter of the bf16 ones, 8x the resolution less the fp32 reference's own order of
+    summation."""
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    from oracle.recurrent import naive_recurrent_gla
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=90 + T, normalizer=16.0, h0_std=1.0, dtype=torch.float16)
+    g = g[..., 0].contiguous() if gates == "head" else g.to(getattr(torch, gates))
+    gen = torch.Generator().manual_seed(11)
+    do = torch.randn(B, T, H, V, generator=gen).half()
+    dht = torch.randn(B, H, K, V, generator=gen) * 0.1
+    print(f"chunk_gla backward, one launch per chunk B={B} T={T} H={H} K={K} V={V} gates={gates}", flush=True)
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, h0)]
+    op = chunk_simple_gla if gates == "head" else chunk_gla
+    o, ht = op(*leaves[:4], initial_state=leaves[4], output_final_state=True, head_first=False)
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    torch.cuda.synchronize()
+    ref = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*ref[:3], **{"g" if gates == "head" else "gk": ref[3]}, initial_state=ref[4],
+                                  output_final_state=True)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for name, r, x, tol in zip(("dq", "dk", "dv", "dg", "dh0"), ref, leaves, (8e-3, 8e-3, 8e-3, 1e-2, 5e-3)):
+        assert_close(name, r.grad, x.grad, tol / 4)
+
+
 def test_chunk_gla_backward_extreme_gates_mixed_varlen(device):
     """Only some chunks and channels are flagged; packed batch, K != V."""
     gen = torch.Generator().manual_seed(82)
