@@ -281,9 +281,9 @@ __global__ __launch_bounds__(512) void gdr_bwd_dhu_kernel(DhuParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = p.H, V = p.V;
   const int nvt = V / BV;
-  int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int vt = (int)(id % nvt);
-  const int item = (int)(id / nvt);
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int vt = (int)(id % (uint32_t)nvt);
+  const int item = (int)(id / (uint32_t)nvt);
   const int hh = item % H;
   const int vbase = vt * BV;
   const ScanSpan span = PASS ? pass_span(p.split, item / H, p.per_seq, p.offsets, p.chunk_offsets, p.T)

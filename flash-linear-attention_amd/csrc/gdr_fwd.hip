@@ -699,9 +699,9 @@ __global__ __launch_bounds__(256) void gdr_fwd_h_kernel(DHParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = p.H, V = p.V;
   const int nvt = V / BV;
-  int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int vt = (int)(id % nvt);
-  const int nh = (int)(id / nvt);
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int vt = (int)(id % (uint32_t)nvt);
+  const int nh = (int)(id / (uint32_t)nvt);
   const int n = nh / H, hh = nh % H;
   const int vbase = vt * BV;
   SeqSpan sp = seq_span(p.offsets, n, p.T);

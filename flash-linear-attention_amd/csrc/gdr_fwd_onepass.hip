@@ -98,8 +98,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int nvb = V / BV;
   const ScanItem wi = scan_item(nvb);
   const int vb = wi.slab;
-  const int hh = (int)(wi.item % H);
-  const int n = p.seq_order ? (int)p.seq_order[wi.item / H] : (int)(wi.item / H);
+  const int hh = (int)(wi.item % (uint32_t)H);
+  const int n = p.seq_order ? (int)p.seq_order[wi.item / (uint32_t)H] : (int)(wi.item / (uint32_t)H);
   const int nh = n * H + hh;
   const int vbase = vb * BV;
   SeqSpan sp = seq_span(p.offsets, n, p.T);

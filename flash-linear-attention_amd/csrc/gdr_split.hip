@@ -79,10 +79,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = p.H;
-  const int cw = (int)(blockIdx.x % p.col_wgs);     // which 128 of the V + K columns
-  const int64_t item = blockIdx.x / p.col_wgs;
-  const int hh = (int)(item % H);
-  const int64_t i = item / H;
+  const int cw = (int)(blockIdx.x % (uint32_t)p.col_wgs);     // which 128 of the V + K columns
+  const uint32_t item = blockIdx.x / (uint32_t)p.col_wgs;
+  const int hh = (int)(item % (uint32_t)H);
+  const int64_t i = item / (uint32_t)H;
   int n, j;
   if (p.split.sub_table) {
     n = p.split.sub_table[2 * i];

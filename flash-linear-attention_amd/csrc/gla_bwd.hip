@@ -60,9 +60,9 @@ __global__ __launch_bounds__(256) void gla_bwd_dh_qg_kernel(BDhParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = p.H, K = p.K, V = p.V;
   const int nkt = K / 64, nvt = V / 64, ntile = nkt * nvt;
-  int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(id % ntile);
-  const int item = (int)(id / ntile), hh = item % H;
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = (int)(id % (uint32_t)ntile);
+  const int item = (int)(id / (uint32_t)ntile), hh = item % H;
   const int kbase = (tile % nkt) * 64, vbase = (tile / nkt) * 64;
   const ScanSpan span = scan_span<true>(p.split, item / H, nullptr, p.offsets, p.chunk_offsets, p.T);
   const int nh = span.n * H + hh;
@@ -197,9 +197,9 @@ __global__ __launch_bounds__(256) void gla_bwd_dh_kernel(BDhParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = p.H, K = p.K, V = p.V;
   const int nkt = K / 64, nvt = V / 64, ntile = nkt * nvt;
-  int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(id % ntile);
-  const int nh = (int)(id / ntile);
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = (int)(id % (uint32_t)ntile);
+  const int nh = (int)(id / (uint32_t)ntile);
   const int n = nh / H, hh = nh % H;
   const int kbase = (tile % nkt) * 64, vbase = (tile / nkt) * 64;
   SeqSpan sp = seq_span(p.offsets, n, p.T);

@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     TK::put(sD, LDK, L, tid, R.q);
   };
 
-  uint32_t it = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);   // adjacent heads of a chunk at the same time on one XCD
+  uint32_t it = xcd_remap(blockIdx.x, gridDim.x);   // adjacent heads of a chunk at the same time on one XCD
   if (it >= nitems) return;
   Item im = locate(it);
   Raw R;

@@ -70,7 +70,7 @@ struct Load<f16> {
 
 // Workgroups of one launch are dealt round-robin to the 8 XCDs by linear id.
 // Renumber so that consecutive logical ids share an XCD (and its L2).
-FLA_DEVICE int64_t xcd_remap(int64_t id, int64_t total) {
+FLA_DEVICE uint32_t xcd_remap(uint32_t id, uint32_t total) {
   if (total % 8 != 0) return id;
   return (id % 8) * (total / 8) + id / 8;
 }
@@ -108,9 +108,9 @@ __global__ __launch_bounds__(256) void gla_fwd_h_kernel(HParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = p.H, K = p.K, V = p.V;
   const int nkt = K / 64, nvt = V / 64, ntile = nkt * nvt;
-  int64_t id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(id % ntile);
-  const int nh = (int)(id / ntile);
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = (int)(id % (uint32_t)ntile);
+  const int nh = (int)(id / (uint32_t)ntile);
   const int n = nh / H, hh = nh % H;
   const int kbase = (tile % nkt) * 64, vbase = (tile / nkt) * 64;
   SeqSpan sp = seq_span(p.offsets, n, p.T);

@@ -268,9 +268,9 @@ __global__ __launch_bounds__(256 + 64 * NSTG) void gla_fwd_fused_kernel(FusedPar
   const int nvb = V / BV;
   const ScanItem wi = scan_item(nvb);
   const int vb = wi.slab;
-  const int hh = (int)(wi.item % H);
+  const int hh = (int)(wi.item % (uint32_t)H);
   const int vbase = vb * BV;
-  const ScanSpan span = scan_span<false>(p.split, wi.item / H, p.seq_order, p.offsets, p.chunk_offsets, p.T);
+  const ScanSpan span = scan_span<false>(p.split, wi.item / (uint32_t)H, p.seq_order, p.offsets, p.chunk_offsets, p.T);
   const int nh = span.n * H + hh;
   const SeqSpan sp = span.sp;
   const int64_t nchunks = span.nchunks, chunk0 = span.chunk0;

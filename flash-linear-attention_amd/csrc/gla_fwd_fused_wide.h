@@ -56,9 +56,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // wave-uniform by construction: keeps the role split and the barriers on scalar branches
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = p.H;
-  const int64_t item = blockIdx.x;
-  const int hh = (int)(item % H);
-  const int n = p.seq_order ? (int)p.seq_order[item / H] : (int)(item / H);
+  const int hh = (int)(blockIdx.x % (uint32_t)H);
+  const int n = p.seq_order ? (int)p.seq_order[blockIdx.x / (uint32_t)H] : (int)(blockIdx.x / (uint32_t)H);
   const int nh = n * H + hh;
   SeqSpan sp = seq_span(p.offsets, n, p.T);
   const int64_t nchunks = (sp.len + BT - 1) / BT;

@@ -54,9 +54,8 @@ __global__ __launch_bounds__(256, 2) void gla_split_pass_kernel(SplitPassParams 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = p.H;
-  const int64_t item = blockIdx.x;
-  const int hh = (int)(item % H);
-  const int64_t i = item / H;
+  const int hh = (int)(blockIdx.x % (uint32_t)H);
+  const int64_t i = blockIdx.x / (uint32_t)H;
   int n, j;
   if (p.split.sub_table) {
     n = p.split.sub_table[2 * i];

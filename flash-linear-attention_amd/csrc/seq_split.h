@@ -50,7 +50,7 @@ inline int check_split(const fla_split* s, const int64_t* offsets) {
 
 // Sub-blocks of a sequence of `chunks` chunks (an empty sequence keeps one slot: its state passes through it).
 FLA_DEVICE int64_t split_nsub(const SplitView& v, int64_t chunks) {
-  const int64_t n = (chunks + v.sub_chunks - 1) / v.sub_chunks;
+  const int64_t n = ((uint32_t)chunks + (uint32_t)v.sub_chunks - 1) / (uint32_t)v.sub_chunks;   // (below 2^31)
   return n > 0 ? n : 1;
 }
 
