@@ -74,12 +74,19 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 //     the pairs (slabs of 32 columns): 4 heads, 12 and 16 chunks 22.1 / 23.6 and 26.0 / 24.3; 16 heads, 12, 24 and 32 chunks
 //     22.9 / 27.7, 35.4 / 34.5 and 43.9 / 36.6, two sequences of them, 16, 32 and 64 chunks 28.2 / 34.8, 44.8 / 45.0 and 77.5 /
 //     64.8, four, 24 and 64 chunks 39.6 / 55.7 and 84.7 / 95.5; packed, 54, 94 and 77 chunks 103 / 94.
+//   The reverse scan of GLA's backward forms the state gradient alone, in half the time per chunk, and leaves every pass of the
+//     backward behind it alone, so only what it saves itself counts (whole training steps; per-key gates, K = V = 128): 4
+//     heads, 16, 24 and 32 chunks 63.5 / 67.3, 72.1 / 72.3 and 77.3 / 73.8; 8 heads, 24, 32 and 64 chunks 75.3 / 77.1, 84.0 /
+//     83.1 and 118 / 106; 16 heads, 32, 48 and 64 chunks 99.2 / 101.6, 137.0 / 135.5 and 155.7 / 148.7; 24 heads, 64 and 96
+//     chunks 225 / 229 and 340 / 336; two sequences of 16 heads, 32, 64 and 96 chunks 138 / 152, 286 / 291 and 400.0 / 398.5.
+//     Per-head gates, K = V = 64: 8, 16, 32, 64, 96 and 128 heads, 24 chunks 52.9 / 51.5, 59.5 / 58.9, 65.9 / 66.9, 85.4 / 89.9,
+//     107.8 / 115.1 and 120.8 / 131.5, 48 chunks 72.1 / 61.2, 79.5 / 68.9, 97.7 / 89.8, 137.4 / 138.9, 196.5 / 202.1 and 262 / 267.
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
   const bool delta = kind == FLA_SCAN_DELTA || kind == FLA_SCAN_DELTA_KEPT;
   int64_t min_seg = 4;
-  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_SIMPLE || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
+  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_GLA_GRADIENT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
   int64_t longest = 0, total = 0;
   for (int64_t n = 0; n < N; ++n) {
@@ -110,6 +117,7 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
     case FLA_SCAN_DELTA: pays = 4 * L >= 11 * seg + 7 * steps + (triples < 32 ? 7 + triples * 5 / 8 : 22 + triples * 5 / 32); break;
     case FLA_SCAN_DELTA_KEPT: pays = steps >= 4 && L - seg >= 20 && L - seg >= 8 + triples * 3 / 4; break;
     case FLA_SCAN_SIMPLE: pays = 5 * L >= 11 * seg + 28 + (triples < 64 ? triples : 64) * 3 / 4; break;
+    case FLA_SCAN_GLA_GRADIENT: pays = 11 * (L - seg) >= 165 + 3 * triples; break;
     default: pays = 5 * L >= 7 * seg + 31;
   }
   if (steps == 0 || !pays) return 0;

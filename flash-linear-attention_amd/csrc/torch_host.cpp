@@ -322,7 +322,8 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     Tensor dh0 = rest.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
     const fla_stream_t st = stream_of(q);
     // (the reverse scan's workgroups hold 64 x 64 tiles of a state)
-    auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.K / 64 * (d.V / 64)), true, q, d.K * d.V, d.K);
+    auto c = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.K / 64 * (d.V / 64)), true, q, d.K * d.V, d.K,
+                      FLA_SCAN_GLA_GRADIENT);
     if (c) {
       check(fla_chunk_gla_bwd_split(ptr(q), ptr(k), ptr(v), ptr(g), ptr(dout), fptr(dht), ptr(hT), ptr(qg), fptr(decay),
                                     nullptr, nullptr, ptr(dhtf), ptr(dq), ptr(dk), ptr(dv), fptr(dg), fptr(dh0),

@@ -79,7 +79,8 @@ enum fla_scan_kind {
   FLA_SCAN_GLA = 0,
   FLA_SCAN_DELTA = 1,
   FLA_SCAN_DELTA_KEPT = 2, /* keeps its intermediates */
-  FLA_SCAN_SIMPLE = 3      /* the plain scan: AT == NULL in fla_chunk_gated_delta_rule_fwd_scan_split */
+  FLA_SCAN_SIMPLE = 3,     /* the plain scan: AT == NULL in fla_chunk_gated_delta_rule_fwd_scan_split */
+  FLA_SCAN_GLA_GRADIENT = 4 /* the state gradient alone: fla_chunk_gla_bwd_split */
 };
 
 /* The plan for N sequences of T tokens (or, with offsets_host [N+1], of a packed batch) and H heads in `slabs` workgroups
@@ -521,7 +522,7 @@ int fla_chunk_simple_gla_bwd(const void* q, const void* k, const void* v, const 
                              float scale, fla_stream_t stream);
 
 /* fla_chunk_gla_bwd_kept (head_gates: fla_chunk_simple_gla_bwd) on sequences cut into segments
- * (fla_scan_split with (K / 64) (V / 64) slabs, reverse): the state gradient leaving every segment is formed first and the reverse
+ * (fla_scan_split with (K / 64) (V / 64) slabs, reverse, kind FLA_SCAN_GLA_GRADIENT): the state gradient leaving every segment is formed first and the reverse
  * state scan runs over the segments. */
 int fla_chunk_gla_bwd_split(const void* q, const void* k, const void* v, const void* gates, const void* dout,
                             const float* dht, const void* hT, const void* q_gated, const float* chunk_decay,

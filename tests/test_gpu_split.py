@@ -142,6 +142,36 @@ def test_gdr_cut_l2norm_in_kernel(device, K, V):
 
 
 @pytest.mark.parametrize("heads", [False, True])
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", [
+    (1, 1985, 1, 64, 64, None, torch.bfloat16),                     # 32 chunks, the last of one token
+    (2, 2303, 2, 128, 128, None, torch.float16),                    # 36 chunks, the last of 63 tokens
+    (1, 2500, 2, 128, 64, [0, 0, 2111, 2112, 2500], torch.bfloat16)])   # an empty sequence, one of a token, uneven ones
+def test_gla_cut_state_gradients(device, B, T, H, K, V, bounds, dtype, heads):
+    """A reverse scan over cut sequences against the fp32 recurrence (the cases above are cut in the forward only).  The
+    tolerances are those of the cases above."""
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    N = B if bounds is None else len(bounds) - 1
+    assert _cut(N, T, H, K // 64 * (V // 64), True, bounds, 4)
+    print("cut state gradients", B, T, H, K, V, bounds, dtype, heads, flush=True)
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
+    if heads:
+        g = g[..., 0].contiguous()
+    do, dht = torch.randn(B, T, H, V).to(dtype), torch.randn(N, H, K, V) * 0.1
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, h0)]
+    o, ht = (chunk_simple_gla if heads else chunk_gla)(
+        *leaves[:4], initial_state=leaves[4], output_final_state=True, head_first=False,
+        cu_seqlens=None if bounds is None else torch.tensor(bounds, device=device))
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    refs = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*refs[:3], **{"g" if heads else "gk": refs[3]}, initial_state=refs[4],
+                                  output_final_state=True, offsets=bounds)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for name, a, r in zip(("dq", "dk", "dv", "dg", "dh0"), leaves, refs):
+        assert_close(name, r.grad, a.grad, 2e-2)
+
+
+@pytest.mark.parametrize("heads", [False, True])
 def test_gla_cut_state_behind_a_reset(device, heads):
     """A gate of -1e30 drops the state.  The tokens behind it inside its chunk keep their own decays, which a difference
     of sums that contain the reset would lose; what enters the next segment is made of them."""

@@ -120,6 +120,19 @@ def test_cut_where_it_pays(kind, heads, chunks, cut):
             assert (_plan(bounds, N, chunks * CHUNK, heads, 2, reverse, kind) is not None) == cut
 
 
+@pytest.mark.parametrize("heads,slabs,chunks,cut", [
+    (4, 4, 16, False), (4, 4, 32, True), (8, 4, 24, False), (8, 4, 48, True), (16, 4, 32, False), (16, 4, 48, True),
+    (24, 4, 64, False), (24, 4, 96, True), (32, 4, 64, False), (8, 1, 16, False), (8, 1, 24, True), (32, 1, 24, False),
+    (32, 1, 32, True), (64, 1, 32, False), (96, 1, 48, False), (128, 1, 48, False)])
+def test_state_gradients_are_cut_where_it_pays(heads, slabs, chunks, cut):
+    """The reverse scan of GLA's backward (kind 4), on both sides of the measured lines."""
+    for bounds in (None, [0, chunks * CHUNK]):
+        got = _plan(bounds, 1, chunks * CHUNK, heads, slabs, 1, 4)
+        assert (got is not None) == cut
+        if cut:
+            _check(*got, [chunks], heads, slabs, 1, 0)
+
+
 @pytest.mark.parametrize("kind,heads,chunks,cut", [
     (1, 16, [54, 94, 77], False), (1, 16, [46, 42, 40, 40], False), (1, 16, [60, 20, 20, 20], False), (1, 16, [80, 171], True),
     (1, 16, [64, 67, 21, 163], True), (1, 8, [54, 94, 77], True), (3, 16, [46, 42, 40, 40], False), (3, 16, [54, 94, 77], True),
