@@ -34,7 +34,7 @@ FLAGS = [
 # Only where it measured faster (gdr_bwd_dhu 216 -> 204 us, gla_bwd_dh 166 -> 162 us); the forward state
 # scans lose with it.
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-VGPR_FORM_SOURCES = {"gdr_bwd.hip", "gdr_bwd_chunk.hip", "gla_bwd.hip", "gla_bwd_chunk.hip"}
+VGPR_FORM_SOURCES = {"gdr_bwd.hip", "gdr_bwd_chunk.hip", "gdr_bwd_scan.hip", "gla_bwd.hip", "gla_bwd_chunk.hip"}
 
 
 def sources():

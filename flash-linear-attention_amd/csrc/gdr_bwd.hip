@@ -11,6 +11,8 @@
 //                              store dH_c;  dv2 = dv_loc + (k e^{gamma_last-gamma}) dH_c;
 //                              dH <- e^{gamma_last} dH + (s q e^gamma)^T do - (w e^gamma)^T dv2
 //                                                                                (chunk_delta_h.py:136-237)
+//   gdr_bwd_scan_kernel      (gdr_bwd_scan.hip) the same scan from the forward's tiles, without dv_loc and w: the operators'
+//                            own path for up to 128 key channels; the two above serve callers that hold w
 //   gdr_bwd_chunk_kernel     (gdr_bwd_chunk.hip) the two below as one launch, for up to 128 key channels; they remain for
 //                            256 and as the reference's separate stages
 //   gdr_bwd_dqkwg_kernel     per (chunk, head, 64-wide half of K):
@@ -33,6 +35,7 @@
 #include <type_traits>
 
 #include "gdr_bwd_chunk.h"
+#include "gdr_bwd_scan.h"
 #include "seq_split.h"
 
 namespace {
@@ -1634,6 +1637,41 @@ extern "C" int fla_chunk_gated_delta_rule_bwd_split(
   return gdr_bwd_impl(q, k, v, w, v_new, beta, g_cumsum, Aw, dout, dht, hT, Aqk, nullptr, ws_dv2, ws_dh_frag_t, ws_dw,
                       ws_dk_partial, ws_dgam_partial, dq, dk, dv, dbeta, dgam2, dh0, offsets, indices, chunk_offsets, NT, qkv_dtype,
                       B, T, H, K, V, N, scale, stream, split);
+}
+
+extern "C" int fla_chunk_gated_delta_rule_bwd_tiles(
+    const void* q, const void* k, const void* v, const void* AT, const void* v_new, const float* beta,
+    const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
+    void* ws_dv2, void* ws_dh_frag_t, void* dq, void* dk, void* dv, float* dbeta, float* dg, float* dh0,
+    const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split, int64_t NT,
+    int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream) {
+  FLA_REQUIRE(q && k && v && AT && v_new && beta && Aw && dout && hT && Aqk && ws_dv2 && ws_dh_frag_t && dq && dk && dv &&
+                  dbeta && dg,
+              FLA_E_INVALID);
+  FLA_REQUIRE(B >= 0 && T >= 0 && H > 0 && K > 0 && V > 0 && N >= 0 && NT >= 0, FLA_E_INVALID);
+  FLA_REQUIRE((K == 64 || K == 128) && (V == 64 || V == 128), FLA_E_UNSUPPORTED);
+  FLA_REQUIRE(qkv_dtype == FLA_BF16 || qkv_dtype == FLA_F16, FLA_E_UNSUPPORTED);
+  FLA_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)AT | (uintptr_t)v_new | (uintptr_t)Aw |
+               (uintptr_t)dout | (uintptr_t)hT | (uintptr_t)Aqk | (uintptr_t)ws_dv2 | (uintptr_t)ws_dh_frag_t |
+               (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) % 16 == 0, FLA_E_ALIGNMENT);
+  if (offsets) FLA_REQUIRE(indices && chunk_offsets && B == 1, FLA_E_INVALID);
+  else FLA_REQUIRE(N == B, FLA_E_INVALID);
+  if (split) {
+    const int rc = check_split(split, offsets);
+    if (rc) return rc;
+    FLA_REQUIRE(split->decays && split->ratio == 1, FLA_E_INVALID);
+  }
+  hipStream_t st = (hipStream_t)stream;
+  dim3 grid;
+  int ntfix;
+  int rc = chunk_grid(offsets, indices, B, T, H, NT, &grid, &ntfix);
+  if (rc) return rc;
+  if (grid.x == 0) return copy_or_zero(dht, dh0, N * H * K * V, st);   // no chunk at all: d h0 = d ht
+  if ((rc = gdr_bwd_scan(q, k, AT, Aqk, g_cumsum, dout, dht, ws_dv2, ws_dh_frag_t, dh0, offsets, chunk_offsets, split,
+                         qkv_dtype, T, H, K, V, N, scale, st)))
+    return rc;
+  return gdr_bwd_chunk(q, k, v, v_new, beta, g_cumsum, Aw, dout, ws_dv2, hT, ws_dh_frag_t, dq, dk, dv, dbeta, dg, offsets,
+                       indices, grid.x, ntfix, qkv_dtype, T, H, K, V, scale, st);
 }
 
 extern "C" int fla_chunk_gated_delta_rule_bwd_dhu(const void* q, const void* k, const void* w, const float* g_cumsum,

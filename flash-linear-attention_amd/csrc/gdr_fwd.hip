@@ -361,8 +361,8 @@ struct PrepParams {
   const int64_t* indices;
   int64_t T;
   int H, NTfix;
-  void* w;             // KEEP: w = Aw (beta k) [rows, H, K] and Aw [rows, H, 64], what the backward reads
-  void* Aw;
+  void* w;             // KEEP: w = Aw (beta k) [rows, H, K]
+  void* Aw;            // KEPT: Aw [rows, H, 64]
   float l2_eps;        // L2N: k is un-normalised; the launch works with k / sqrt(sum k^2 + l2_eps) ...
   float* rk_out;       //      ... and leaves the factors 1 / sqrt(sum k^2 + l2_eps), fp32 [rows, H], for the scan
 };
@@ -376,15 +376,17 @@ FLA_DEVICE int tri_block(int tt, int jb) { return tt * (tt + 1) / 2 + jb; }
 // accumulators: the loads land while the inversion runs (measured: worth about 4 %; the launch is a chain
 // of short dependent phases - removing the inversion, the stores or the loads each saves 15-20 % - rather
 // than bound by one resource).
-// KEEP: the forward of a pass that will be differentiated also leaves w = Aw (beta k) and Aw in memory (the WY
-// launch of the reference's decomposition, without a second inversion and a second pass over k).
+// KEPT 1: the forward of a pass that will be differentiated also leaves Aw in memory, the one thing the backward from the
+// tiles cannot do without (13 us for 4096 tokens of 16 heads, K = 128, against 19 with w).  KEPT 2: w = Aw (beta k) too (the WY
+// launch of the reference's decomposition, without a second inversion and a second pass over k), for callers that hand w on.
 // L2N: k arrives un-normalised (what l2_norm(k) in front of the operator would normalise,
 // fla/layers/gated_deltanet.py:235).  The rows are not rewritten: k^ = r k with r = 1 / sqrt(sum k^2 + eps) per row, so
 // k^ k^T = diag(r) (k k^T) diag(r) and the factors go onto the rows and columns of the product; r comes from the
 // pieces the lanes hold anyway (a row of K elements sits in K / 8 adjacent lanes) and is left in memory for the scan.
-template <typename T, int K, bool KEEP, bool L2N = false>
-__global__ __launch_bounds__(256, KEEP ? kPrepResidentKeep : kPrepResident) void gdr_fwd_prep_kernel(PrepParams p, int64_t total) {
-  static_assert(!(KEEP && L2N), "a forward that keeps w and Aw takes normalised keys");
+template <typename T, int K, int KEPT, bool L2N = false>
+__global__ __launch_bounds__(256, KEPT == 2 ? kPrepResidentKeep : kPrepResident) void gdr_fwd_prep_kernel(PrepParams p, int64_t total) {
+  constexpr bool KEEP = KEPT == 2;
+  static_assert(!(KEPT && L2N), "a forward that keeps w and Aw takes normalised keys");
   typedef typename Elem<T>::v8 v8;
   typedef typename Elem<T>::v4 v4;
   constexpr int LDK = K + 8;
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(256, KEEP ? kPrepResidentKeep : kPrepResident) void
             tu[e] = (T)(x[e] * __expf(tt != jb || c4 + e <= r ? d : 0.f) * bj[e]);
           }
           *(v4*)(at + idx * 256 + 4 * lane) = tu;
-          if constexpr (KEEP) {
+          if constexpr (KEPT) {
             // Aw row piece to memory; Aw diag(beta) as a row-major 16-bit tile in region A (M is dead)
             v4 aw, ab;
 #pragma unroll
@@ -594,12 +596,12 @@ __global__ __launch_bounds__(256, KEEP ? kPrepResidentKeep : kPrepResident) void
               aw[e] = (T)x[e];
               ab[e] = (T)(x[e] * bj[e]);
             }
-            *(v4*)&sAb[i * LDT + j0] = ab;
+            if constexpr (KEEP) *(v4*)&sAb[i * LDT + j0] = ab;
             if (i < L) *(v4*)((T*)p.Aw + ((row0 + i) * H + hh) * (int64_t)BT + j0) = aw;
           }
         }
       }
-      if constexpr (KEEP) {
+      if constexpr (KEPT) {
         // the blocks above the diagonal of Aw and of Aw diag(beta) are zero
         const v4 z4 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
 #pragma unroll
@@ -609,7 +611,7 @@ __global__ __launch_bounds__(256, KEEP ? kPrepResidentKeep : kPrepResident) void
             const int tt = u >= 5 ? 2 : u >= 3 ? 1 : 0;
             const int jb = u - (tt == 0 ? 0 : tt == 1 ? 3 : 5) + tt + 1;
             const int i = 16 * tt + r, j0 = 16 * jb + c4;
-            *(v4*)&sAb[i * LDT + j0] = z4;
+            if constexpr (KEEP) *(v4*)&sAb[i * LDT + j0] = z4;
             if (i < L) *(v4*)((T*)p.Aw + ((row0 + i) * H + hh) * (int64_t)BT + j0) = z4;
           }
         }
@@ -1214,16 +1216,20 @@ int launch_prep(const PrepParams& p, int K, dim3 chunk_grid_, hipStream_t st) {
   dim3 grid((unsigned)(total < resident ? total : resident));
   if (p.l2_eps >= 0.f) {
     if (p.w) return FLA_E_UNSUPPORTED;
-    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, false, true>), grid, dim3(256), 0, st, p, total);
-    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, false, true>), grid, dim3(256), 0, st, p, total);
+    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, 0, true>), grid, dim3(256), 0, st, p, total);
+    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, 0, true>), grid, dim3(256), 0, st, p, total);
     else return FLA_E_UNSUPPORTED;
   } else if (p.w) {
-    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, true>), grid, dim3(256), 0, st, p, total);
-    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, true>), grid, dim3(256), 0, st, p, total);
+    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, 2>), grid, dim3(256), 0, st, p, total);
+    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, 2>), grid, dim3(256), 0, st, p, total);
+    else return FLA_E_UNSUPPORTED;
+  } else if (p.Aw) {
+    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, 1>), grid, dim3(256), 0, st, p, total);
+    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, 1>), grid, dim3(256), 0, st, p, total);
     else return FLA_E_UNSUPPORTED;
   } else {
-    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, false>), grid, dim3(256), 0, st, p, total);
-    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, false>), grid, dim3(256), 0, st, p, total);
+    if (K == 64) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 64, 0>), grid, dim3(256), 0, st, p, total);
+    else if (K == 128) hipLaunchKernelGGL((gdr_fwd_prep_kernel<T, 128, 0>), grid, dim3(256), 0, st, p, total);
     else return FLA_E_UNSUPPORTED;
   }
   FLA_CHECK_LAUNCH();
@@ -1238,7 +1244,6 @@ static int gdr_fwd_prep_impl(const void* k, const float* beta, const float* g, i
                              int64_t K, float l2_eps, fla_stream_t stream, float* rk_out = nullptr) {
   FLA_REQUIRE(k && beta && AT, FLA_E_INVALID);
   FLA_REQUIRE((l2_eps >= 0.f) == (rk_out != nullptr), FLA_E_INVALID);
-  FLA_REQUIRE((w == nullptr) == (Aw == nullptr), FLA_E_INVALID);
   FLA_REQUIRE(B >= 0 && T >= 0 && H > 0 && K > 0 && NT >= 0, FLA_E_INVALID);
   FLA_REQUIRE(((uintptr_t)k | (uintptr_t)AT | (uintptr_t)w | (uintptr_t)Aw) % 16 == 0, FLA_E_ALIGNMENT);
   dim3 grid;
@@ -1256,7 +1261,17 @@ extern "C" int fla_gdr_fwd_prep(const void* k, const float* beta, const float* g
                                 float* g_cumsum_out, void* AT, void* w, void* Aw, const int64_t* offsets,
                                 const int64_t* indices, int64_t NT, int qkv_dtype, int64_t B, int64_t T, int64_t H,
                                 int64_t K, fla_stream_t stream) {
+  FLA_REQUIRE((w == nullptr) == (Aw == nullptr), FLA_E_INVALID);
   return gdr_fwd_prep_impl(k, beta, g, g_is_cumsum, g_cumsum_out, AT, w, Aw, offsets, indices, NT, qkv_dtype, B, T,
+                           H, K, -1.f, stream);
+}
+
+extern "C" int fla_gdr_fwd_prep_kept(const void* k, const float* beta, const float* g, int g_is_cumsum,
+                                     float* g_cumsum_out, void* AT, void* Aw, const int64_t* offsets,
+                                     const int64_t* indices, int64_t NT, int qkv_dtype, int64_t B, int64_t T, int64_t H,
+                                     int64_t K, fla_stream_t stream) {
+  FLA_REQUIRE(Aw, FLA_E_INVALID);
+  return gdr_fwd_prep_impl(k, beta, g, g_is_cumsum, g_cumsum_out, AT, nullptr, Aw, offsets, indices, NT, qkv_dtype, B, T,
                            H, K, -1.f, stream);
 }
 

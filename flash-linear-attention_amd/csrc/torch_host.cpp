@@ -377,7 +377,7 @@ struct GdrArgs {
   std::optional<double> l2norm_eps;
 };
 struct GdrKept {
-  Tensor gc, w, Aw, v_new, hT, Aqk, Mt;   // Mt: the segments' transposed transitions where the forward was cut
+  Tensor gc, AT, Aw, v_new, hT, Aqk, Mt;   // Mt: the segments' transposed transitions where the forward was cut
 };
 
 Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& h0,
@@ -416,7 +416,7 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   GdrKept none, &x = kept ? *kept : none;
   if (kept) {
     x.gc = gc;
-    x.w = fresh_like(k);
+    x.AT = AT;
     x.Aw = fresh({d.B, d.T, d.H, BT}, q, q.scalar_type());
     x.v_new = fresh_like(v);
     x.hT = fresh({d.chunks, d.H, d.K, d.V}, q, q.scalar_type());
@@ -426,9 +426,14 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
       cut->s.transitions_t = fptr(x.Mt);
     }
   }
-  check(fla_gdr_fwd_prep(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), ptr(x.w), ptr(x.Aw), offs(a.plan), idx(a.plan),
-                         d.NT, dt(q), d.B, d.T, d.H, d.K, st),
-        "fla_gdr_fwd_prep");
+  if (kept)
+    check(fla_gdr_fwd_prep_kept(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), ptr(x.Aw), offs(a.plan), idx(a.plan),
+                                d.NT, dt(q), d.B, d.T, d.H, d.K, st),
+          "fla_gdr_fwd_prep_kept");
+  else
+    check(fla_gdr_fwd_prep(ptr(k), fptr(beta), fptr(g), 0, fptr(gc), ptr(AT), nullptr, nullptr, offs(a.plan), idx(a.plan),
+                           d.NT, dt(q), d.B, d.T, d.H, d.K, st),
+          "fla_gdr_fwd_prep");
   if (cut) {
     scan_cut({}, x);
     return o;
@@ -455,7 +460,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     Tensor ht;
     GdrKept x;
     Tensor o = gdr_forward(q, k, v, g, beta, h0, a, &ht, &x);
-    ctx->save_for_backward({q, k, v, beta, x.gc, x.w, x.Aw, x.v_new, x.hT, x.Aqk, x.Mt, given(offsets)});
+    ctx->save_for_backward({q, k, v, beta, x.gc, x.AT, x.Aw, x.v_new, x.hT, x.Aqk, x.Mt, given(offsets)});
     ctx->set_materialize_grads(false);
     Rest r{a, std::nullopt, beta_.scalar_type(), h0.defined()};
     if (g_) r.g_type = g_->scalar_type();
@@ -469,7 +474,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     const Rest& r = held<Rest>(ctx);
     const GdrArgs& a = r.a;
     const Dims& d = a.d;
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &beta = saved[3], &gc = saved[4], &w = saved[5], &Aw = saved[6],
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &beta = saved[3], &gc = saved[4], &AT = saved[5], &Aw = saved[6],
                  &v_new = saved[7], &hT = saved[8], &Aqk = saved[9],
                  &Mt = saved[10];
     const Tensor dout = grads[0].defined() ? as(grads[0], q.scalar_type()).contiguous() : at::zeros(v.sizes(), v.options());
@@ -481,22 +486,13 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     std::optional<Cut> cut;
     if (Mt.defined())
       cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), true, q, d.K * d.V, 0, FLA_SCAN_DELTA_KEPT);
-    if (cut) {
-      cut->s.decays = fptr(Mt);
-      check(fla_chunk_gated_delta_rule_bwd_split(
-                ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout), fptr(dht), ptr(hT),
-                ptr(Aqk), ptr(dv2), ptr(dh), nullptr, nullptr, nullptr, ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg),
-                fptr(dh0), offs(a.plan), idx(a.plan), coff(a.plan), &cut->s, d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
-                (float)a.scale, stream_of(q)),
-            "fla_chunk_gated_delta_rule_bwd_split");
-      return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor(), Tensor()};
-    }
-    check(fla_chunk_gated_delta_rule_bwd(ptr(q), ptr(k), ptr(v), ptr(w), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout),
-                                         fptr(dht), ptr(hT), ptr(Aqk), nullptr, ptr(dv2), ptr(dh), nullptr, nullptr,
-                                         nullptr, ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg), fptr(dh0),
-                                         offs(a.plan), idx(a.plan), coff(a.plan), d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N,
-                                         (float)a.scale, stream_of(q)),
-          "fla_chunk_gated_delta_rule_bwd");
+    if (cut) cut->s.decays = fptr(Mt);
+    check(fla_chunk_gated_delta_rule_bwd_tiles(
+              ptr(q), ptr(k), ptr(v), ptr(AT), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout), fptr(dht), ptr(hT),
+              ptr(Aqk), ptr(dv2), ptr(dh), ptr(dq), ptr(dk), ptr(dv), fptr(dbeta), fptr(dg), fptr(dh0), offs(a.plan),
+              idx(a.plan), coff(a.plan), cut ? &cut->s : nullptr, d.NT, dt(q), d.B, d.T, d.H, d.K, d.V, d.N, (float)a.scale,
+              stream_of(q)),
+          "fla_chunk_gated_delta_rule_bwd_tiles");
     return {dq, dk, dv, r.g_type ? as(dg, *r.g_type) : Tensor(), as(dbeta, r.beta_type), dh0, Tensor(), Tensor()};
   }
 };

@@ -66,6 +66,7 @@ SIGNATURES = {
     "fla_gdr_fwd_prep": (c_int, [P, P, P, I, P, P, P, P, P, P, I64, I, I64, I64, I64, I64, P]),
     "fla_chunk_gated_delta_rule_fwd_scan": (c_int, [P] * 14 + [I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_simple_gla_fwd_scan": (c_int, [P] * 10 + [I, I64, I64, I64, I64, I64, I64, F, P]),
+    "fla_gdr_fwd_prep_kept": (c_int, [P, P, P, I, P, P, P, P, P, I64, I, I64, I64, I64, I64, P]),
     "fla_gdr_fwd_prep_l2norm": (c_int, [P, P, P, I, P, P, P, P, P, I64, I, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_fwd_scan_l2norm": (c_int, [P] * 12 + [I, I64, I64, I64, I64, I64, I64, F, F, P]),
     "fla_chunk_gated_delta_rule_fwd_onepass": (c_int, [P] * 11 + [I, I64, I64, I64, I64, I64, I64, F, I, F, P]),
@@ -80,6 +81,7 @@ SIGNATURES = {
     "fla_chunk_bwd_dh": (c_int, [P] * 9 + [I, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_states_to_fragments": (c_int, [P, P, I, I, I, I64, I64, I64, P]),
     "fla_chunk_bwd_dv_local": (c_int, [P] * 7 + [I64, I, I64, I64, I64, I64, I64, F, P]),
+    "fla_chunk_gated_delta_rule_bwd_tiles": (c_int, [P] * 24 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_bwd_split": (c_int, [P] * 27 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_bwd": (c_int, [P] * 27 + [I64, I, I64, I64, I64, I64, I64, I64, F, P]),
     "fla_chunk_gated_delta_rule_bwd_dhu": (c_int, [P] * 12 + [I, I64, I64, I64, I64, I64, I64, F, P]),

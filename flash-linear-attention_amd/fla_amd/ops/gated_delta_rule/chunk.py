@@ -103,20 +103,21 @@ def chunk_gated_delta_rule_fwd(q, k, v, g, beta, scale, initial_state, output_fi
 
 def chunk_gated_delta_rule_fwd_keep(q, k, v, g, beta, scale, initial_state, output_final_state, offsets=None):
     """Forward of a pass that will be differentiated.  Returns ``(g_cumsum, o, final_state, kept)``
-    with ``kept = (w, Aw, v_new, hT[, Aqk])`` for :func:`chunk_gated_delta_rule_bwd`.  Key dims up to 128: the
-    two-launch forward, whose first launch also writes ``w`` and ``Aw`` and whose scan also writes ``v_new`` and
-    the state entering every chunk.  K = 256: the reference's decomposition (WY launch, state scan, output stage)."""
+    with ``kept`` for :func:`chunk_gated_delta_rule_bwd`.  Key dims up to 128: ``(AT, Aw, v_new, hT, Aqk)`` of the
+    two-launch forward, whose first launch also writes ``Aw`` and whose scan also writes ``v_new``, the score tiles and
+    the state entering every chunk.  K = 256: ``(w, Aw, v_new, hT)`` of the reference's decomposition (WY launch, state scan,
+    output stage)."""
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
     offs = None if plan is None else plan.offsets
     idx = None if plan is None else plan.indices
     co = None if plan is None else plan.chunk_offsets
     beta = beta.float().contiguous()
     if q.shape[-1] <= _FUSED_MAX_K:
-        AT, g, w, Aw = fwd_prepare_scan_operands(k, beta, g, offsets=offs, indices=idx, keep_w=True)
+        AT, g, Aw = fwd_prepare_scan_operands(k, beta, g, offsets=offs, indices=idx, keep_Aw=True)
         o, final_state, v_new, hT, Aqk = chunk_gated_delta_rule_fwd_scan(
             q, k, v, AT, g, scale, initial_state, output_final_state, offsets=offs, chunk_offsets=co,
             seq_order=None if plan is None else plan.seq_order, keep=True)
-        return g, o, final_state, (w, Aw, v_new, hT, Aqk)
+        return g, o, final_state, (AT, Aw, v_new, hT, Aqk)
     g = None if g is None else chunk_local_cumsum(g, BT, offsets=offs, indices=idx, head_first=False)
     w, u, Aw, _ = fwd_prepare_wy_repr(k, v, beta, g, offsets=offs, indices=idx, head_first=False, chunk_size=BT,
                                       store_A=True, store_Au=False)
@@ -144,7 +145,7 @@ def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do
     Aqk = None
     if kept is not None:
         w, Aw, v_new, hT = kept[:4]
-        Aqk = kept[4] if len(kept) > 4 else None   # the score tiles of the two-launch forward (K <= 128)
+        Aqk = kept[4] if len(kept) > 4 else None   # the two-launch forward (K <= 128): tiles, AT in place of w
     else:
         w, u, Aw, _ = fwd_prepare_wy_repr(k, v, beta, g_cumsum, offsets=offs, indices=idx, head_first=False,
                                           chunk_size=BT, store_A=True, store_Au=False)
@@ -164,6 +165,13 @@ def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do
     dh0 = q.new_empty(N, H, K, V, dtype=torch.float32) if initial_state is not None else None
     if dht is not None:
         dht = (dht if dht.dtype == torch.float32 else dht.float()).contiguous()
+    if Aqk is not None:
+        be.check(be.lib().fla_chunk_gated_delta_rule_bwd_tiles(
+            be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(w), be.ptr(v_new), be.ptr(beta), be.ptr(g_cumsum), be.ptr(Aw),
+            be.ptr(do), be.ptr(dht), be.ptr(hT), be.ptr(Aqk), be.ptr(ws_dv2), be.ptr(ws_dh), be.ptr(dq), be.ptr(dk),
+            be.ptr(dv), be.ptr(dbeta), be.ptr(dg), be.ptr(dh0), be.ptr(offs), be.ptr(idx), be.ptr(co), None, NT,
+            be.dt(q), B, T, H, K, V, N, float(scale), be.stream_of(q)), "fla_chunk_gated_delta_rule_bwd_tiles")
+        return dq, dk, dv, dbeta, (dg if g_cumsum is not None else None), dh0
     be.check(be.lib().fla_chunk_gated_delta_rule_bwd(
         be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(w), be.ptr(v_new), be.ptr(beta), be.ptr(g_cumsum), be.ptr(Aw),
         be.ptr(do), be.ptr(dht), be.ptr(hT), be.ptr(Aqk), be.ptr(ws_dvl), be.ptr(ws_dv2), be.ptr(ws_dh), be.ptr(ws_dw),

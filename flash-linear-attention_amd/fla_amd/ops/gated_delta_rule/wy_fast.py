@@ -67,6 +67,7 @@ def fwd_prepare_scan_operands(
     g_is_cumsum: bool = False,
     keep_w: bool = False,
     l2norm_eps: Optional[float] = None,
+    keep_Aw: bool = False,
 ):
     """Chunk-parallel half of the one-pass forward (``fla_gdr_fwd_prep``): the work of ``chunk_local_cumsum``
     and ``fwd_prepare_wy_repr`` (``fla/ops/gated_delta_rule/wy_fast.py:320-376``), leaving per (chunk, head) the
@@ -75,8 +76,9 @@ def fwd_prepare_scan_operands(
     ``[B, T, H]`` (or its chunk-local cumsum with ``g_is_cumsum``; ``None`` for the un-gated rule).
     Seq-first, K in {64, 128}.  Returns ``(AT, g_cumsum)``; with ``keep_w`` the launch also writes
     ``w = Aw (beta k)`` and ``Aw`` (what ``fwd_prepare_wy_repr`` leaves for the backward) and the return value
-    is ``(AT, g_cumsum, w, Aw)``.  ``l2norm_eps``: ``k`` is un-normalised and the launch works with its
-    l2-normalised rows (``fla_gdr_fwd_prep_l2norm``; not with ``keep_w``); the return value is then
+    is ``(AT, g_cumsum, w, Aw)``; with ``keep_Aw`` it writes ``Aw`` beside the tiles and returns ``(AT, g_cumsum, Aw)``
+    (``fla_gdr_fwd_prep_kept``: what a backward from the tiles reads).  ``l2norm_eps``: ``k`` is un-normalised and the launch works with its
+    l2-normalised rows (``fla_gdr_fwd_prep_l2norm``; not with ``keep_w`` or ``keep_Aw``); the return value is then
     ``(AT, g_cumsum, k_rstd)`` with the per-row factors ``1 / sqrt(sum k^2 + eps)`` (fp32 ``[B,T,H]``) the scan reads."""
     be.require_gpu(k, beta)
     B, T, H, K = k.shape
@@ -92,9 +94,9 @@ def fwd_prepare_scan_operands(
         gc = g if g_is_cumsum else torch.empty_like(g)
     AT = k.new_empty(chunks, H, TRI_BLOCKS, 16, 16)
     w = torch.empty_like(k) if keep_w else None
-    Aw = k.new_empty(B, T, H, BT) if keep_w else None
+    Aw = k.new_empty(B, T, H, BT) if keep_w or keep_Aw else None
     if l2norm_eps is not None:
-        if keep_w:
+        if keep_w or keep_Aw:
             raise ValueError("l2norm_eps: forward without kept intermediates only")
         k_rstd = k.new_empty(B, T, H, dtype=torch.float32)
         be.check(be.lib().fla_gdr_fwd_prep_l2norm(
@@ -102,6 +104,12 @@ def fwd_prepare_scan_operands(
             be.ptr(k_rstd), be.ptr(offsets), be.ptr(indices), NT, be.dt(k), B, T, H, K, float(l2norm_eps),
             be.stream_of(k)), "fla_gdr_fwd_prep_l2norm")
         return AT, gc, k_rstd
+    if keep_Aw and not keep_w:
+        be.check(be.lib().fla_gdr_fwd_prep_kept(
+            be.ptr(k), be.ptr(beta), be.ptr(g), int(g_is_cumsum), be.ptr(None if g_is_cumsum else gc), be.ptr(AT),
+            be.ptr(Aw), be.ptr(offsets), be.ptr(indices), NT, be.dt(k), B, T, H, K, be.stream_of(k)),
+            "fla_gdr_fwd_prep_kept")
+        return AT, gc, Aw
     be.check(be.lib().fla_gdr_fwd_prep(
         be.ptr(k), be.ptr(beta), be.ptr(g), int(g_is_cumsum), be.ptr(None if g_is_cumsum else gc),
         be.ptr(AT), be.ptr(w), be.ptr(Aw), be.ptr(offsets), be.ptr(indices), NT, be.dt(k), B, T, H, K,

@@ -410,7 +410,8 @@ int fla_chunk_fwd_o(const void* q, const void* k, const void* v, const float* g_
  * written to g_cumsum_out, fp32 [B,T,H], if that is given), or already the prefix sum (== 1), or NULL (no gate).
  * w [B,T,H,K] and Aw [B,T,H,64] in the q/k/v dtype, both given or both NULL: w = Aw (beta k) and Aw = (I + M)^-1 as
  * fwd_prepare_wy_repr leaves them (fla/ops/gated_delta_rule/wy_fast.py:320-376), for a forward that will be
- * differentiated (fla_chunk_gated_delta_rule_bwd reads them).
+ * differentiated (fla_chunk_gated_delta_rule_bwd reads them).  fla_gdr_fwd_prep_kept writes AT and Aw alone, what
+ * fla_chunk_gated_delta_rule_bwd_tiles reads.
  * K in {64, 128}.
  * fla_chunk_gated_delta_rule_fwd_scan is the serial part (state scan + output, replaces
  * chunk_gated_delta_rule_fwd_h + chunk_fwd_o, fla/ops/gated_delta_rule/chunk.py:47-72): with h the state entering
@@ -427,6 +428,9 @@ int fla_gdr_fwd_prep(const void* k, const float* beta, const float* g, int g_is_
                      float* g_cumsum_out, void* AT, void* w, void* Aw, const int64_t* offsets,
                      const int64_t* indices,
                      int64_t NT, int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, fla_stream_t stream);
+int fla_gdr_fwd_prep_kept(const void* k, const float* beta, const float* g, int g_is_cumsum, float* g_cumsum_out,
+                          void* AT, void* Aw, const int64_t* offsets, const int64_t* indices, int64_t NT,
+                          int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, fla_stream_t stream);
 
 int fla_chunk_gated_delta_rule_fwd_scan(const void* q, const void* k, const void* v, const void* AT,
                                         const float* g_cumsum, const float* h0, void* o, float* ht,
@@ -627,6 +631,16 @@ int fla_chunk_gated_delta_rule_bwd_split(
     const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
     void* ws_dv2, void* ws_dh_frag_t, void* ws_dw, void* ws_dk_partial, float* ws_dgam_partial,
     void* dq, void* dk, void* dv, float* dbeta, float* dg, float* dh0,
+    const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split, int64_t NT,
+    int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
+
+/* The same from the tiles the two-launch forward leaves: AT (Tu, fla_gdr_fwd_prep_kept) in place of w, and Aqk.  The
+ * reverse scan takes the gradient through the corrected values as k^T (Tu^T dv2), so w is neither kept nor read.  split:
+ * as for the entry above, or NULL.  K in {64,128}, V in {64,128}. */
+int fla_chunk_gated_delta_rule_bwd_tiles(
+    const void* q, const void* k, const void* v, const void* AT, const void* v_new, const float* beta,
+    const float* g_cumsum, const void* Aw, const void* dout, const float* dht, const void* hT, const void* Aqk,
+    void* ws_dv2, void* ws_dh_frag_t, void* dq, void* dk, void* dv, float* dbeta, float* dg, float* dh0,
     const int64_t* offsets, const int64_t* indices, const int64_t* chunk_offsets, const fla_split* split, int64_t NT,
     int qkv_dtype, int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t N, float scale, fla_stream_t stream);
 

@@ -77,6 +77,11 @@ def test_argument_validation_without_device():
     scan = lambda vn, hT, aqk: lib.fla_chunk_gated_delta_rule_fwd_scan(p, p, p, p, None, None, p, None, vn, hT, aqk, None, None,
                                                                        None, 0, 1, 64, 1, 64, 64, 1, 1.0, None)
     assert scan(p, None, None) == -1 and scan(None, None, p) == -1
+    # its backward from the forward's tiles: both tiles, Aw, K in {64, 128}
+    assert lib.fla_gdr_fwd_prep_kept(p, p, None, 0, None, p, None, None, None, 0, 0, 1, 64, 1, 64, None) == -1
+    tiles = lambda AT, Aqk, K: lib.fla_chunk_gated_delta_rule_bwd_tiles(p, p, p, AT, p, p, None, p, p, None, p, Aqk, *(p,) * 7, None,
+                                                                        *z, 0, 0, 1, 64, 1, K, 64, 1, 1.0, None)
+    assert tiles(None, p, 64) == -1 and tiles(p, None, 64) == -1 and tiles(p, p, 256) == -2
 
 
 @pytest.mark.parametrize("bt", [16, 64])

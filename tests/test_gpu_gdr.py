@@ -337,6 +337,47 @@ def test_chunk_gdr_backward_chunk_launch(device, B, T, H, K, V, gated):
             assert_close(name, r, x.grad, tol / 4)
 
 
+@pytest.mark.parametrize("T,K,V", [(1, 64, 64), (64, 128, 64), (65, 128, 128), (129, 64, 128), (193, 128, 128), (256, 64, 64),
+                                   (260, 128, 64), (385, 128, 128)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_chunk_gdr_reverse_scan_from_tiles(device, T, K, V, gated):
+    """The reverse scan from the forward's tiles: one to seven chunks (the first, the last and the second one processed are
+    peeled off the loop), ends one row past a chunk and on its edge.  The same gradients come from the entry that takes w
+    in place of Tu.  fp16, a quarter of the bf16 tolerances as above; the two forms round w here and dr there, once each to
+    16 bits, so they differ by no more than twice what either may differ from the reference."""
+    from fla_amd import _backend as be
+    from fla_amd.ops.gated_delta_rule.chunk import chunk_gated_delta_rule_bwd, chunk_gated_delta_rule_fwd_scan
+    from fla_amd.ops.gated_delta_rule.wy_fast import fwd_prepare_scan_operands
+    B, H = 2, 3
+    q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=90 + T, h0_std=1.0, dtype=torch.float16)
+    gen = torch.Generator().manual_seed(10)
+    do = torch.randn(B, T, H, V, generator=gen).half()
+    dht = torch.randn(B, H, K, V, generator=gen) * 0.1
+    print(f"chunk_gdr reverse scan from tiles T={T} K={K} V={V} gated={gated}", flush=True)
+    qd, kd, vd, gd, bd, hd, dod, dhd = (x.to(device) for x in (q, k, v, g, beta, h0, do, dht))
+    scale = K ** -0.5
+    AT, gc, w, Aw = fwd_prepare_scan_operands(kd, bd, gd if gated else None, keep_w=True)
+    AT2, gc2, Aw2 = fwd_prepare_scan_operands(kd, bd, gd if gated else None, keep_Aw=True)
+    assert torch.equal(AT, AT2) and torch.equal(Aw, Aw2) and (not gated or torch.equal(gc, gc2))
+    _, _, v_new, hT, Aqk = chunk_gated_delta_rule_fwd_scan(qd, kd, vd, AT, gc, scale, hd, True, keep=True)
+    got = chunk_gated_delta_rule_bwd(qd, kd, vd, gc, bd, scale, hd, dod, dhd, kept=(AT, Aw, v_new, hT, Aqk))
+    ref = _grads_ref(q, k, v, g if gated else torch.zeros_like(g), beta, h0, do, dht)
+    dq, dk, dv, db, dg, dh0 = got
+    dv2, dh = torch.empty_like(vd), torch.empty_like(hT)
+    alt = [torch.empty_like(x) for x in (dq, dk, dv, db, db, dh0)]
+    be.check(be.lib().fla_chunk_gated_delta_rule_bwd(
+        *(be.ptr(x) for x in (qd, kd, vd, w, v_new, bd, gc, Aw, dod, dhd, hT, Aqk, None, dv2, dh, None, None, None)),
+        *(be.ptr(x) for x in alt), None, None, None, 0, be.dt(qd), B, T, H, K, V, B, float(scale), be.stream_of(qd)), "bwd")
+    torch.cuda.synchronize()
+    order = dict(zip(NAMES, (dq, dk, dv, dg, db, dh0)))
+    other = dict(zip(NAMES, (alt[0], alt[1], alt[2], alt[4], alt[3], alt[5])))
+    for name, r, tol in zip(NAMES, ref, TOLS):
+        if name == NAMES[3] and not gated:
+            continue
+        assert_close(name, r, order[name], tol / 4)
+        assert_close(name + " (from w)", other[name].float().cpu(), order[name], tol / 2)
+
+
 def test_chunk_gdr_backward_varlen_and_headfirst(device):
     gen = torch.Generator().manual_seed(8)
     T, N, H, D = 500, 4, 2, 128
