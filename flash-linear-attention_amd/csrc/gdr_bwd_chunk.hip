@@ -94,7 +94,8 @@ __global__ __launch_bounds__(256, 2) void gdr_bwd_chunk_kernel(ChunkBwdParams p,
     TV::load(p.vnew, r0h, im.cl.L, H, tid, R.vn);
     TK::load(p.k, r0h, im.cl.L, H, tid, R.k);
     TK::load(p.q, r0h, im.cl.L, H, tid, R.q);
-    const int row = (tid & (BT - 1)) < im.cl.L ? (tid & (BT - 1)) : im.cl.L - 1;
+    // a column of 64 gates is 64 requests to the L2: the waves that do not use it read one word
+    const int row = tid >= BT ? 0 : tid < im.cl.L ? tid : im.cl.L - 1;
     R.beta = p.beta[r0h + (int64_t)row * H];
     R.gam = *(p.gam ? p.gam + r0h + (int64_t)row * H : &kZeroWord);   // (without gates one zero word: no branch)
   };

@@ -242,13 +242,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < NPW; ++i) offq[i] = 2 * ((uint32_t)q_row(st + 256 * i) * HK + q_col(st + 256 * i));
 #pragma unroll
     for (int i = 0; i < RV; ++i) offv[i] = 2 * ((uint32_t)(urg * RV + i) * HV + uc4);
-    const uint32_t offg = 4 * (uint32_t)lane * H;
+    // Only the first staging wave uses the gate rows and the last 64 pieces of Tu; the others' loads (no branch) are all of one
+    // word: a column of 64 gates, H apart, is 64 requests to the L2, as many as half of a q tile (4 x 4096 tokens, 16 heads:
+    // 166.5 -> 162 us).
+    const uint32_t offg = wave == 4 ? 4 * (uint32_t)lane * H : 0u;
     const int64_t row00 = sp.bos * H + hh;
     const char* lq = (const char*)p.q + row00 * K * 2;
     const char* lk = (const char*)p.k + row00 * K * 2;
     const char* lv = (const char*)p.v + (row00 * V + vbase) * 2;
     const char* la = (const char*)p.AT + (chunk0 * H + hh) * (int64_t)ATS * 2;
-    const uint32_t offa0 = 16 * (uint32_t)st, offa1 = 16 * (uint32_t)(256 + lane);
+    const uint32_t offa0 = 16 * (uint32_t)st, offa1 = 16 * (uint32_t)(256 + (wave == 4 ? lane : 0));
     // The gate load is unconditional (a load under a branch would make the wave drain its whole load
     // queue at the join); without gates it reads a dummy address and the bits are masked to zero.
     const uint32_t gmask = p.gam ? 0xffffffffu : 0u;
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const uint32_t limv = (last ? limv_last : limv_full) + colv;
       if constexpr (DELTA) {
         R.a0 = *(const v8*)(la + offa0);   // a full tile whatever the chunk length
-        R.a1 = *(const v8*)(la + offa1);   // its last 64 pieces: every wave loads them, the first one writes them
+        R.a1 = *(const v8*)(la + offa1);   // its last 64 pieces: the first wave writes them
       }
 #pragma unroll
       for (int i = 0; i < RV; ++i) R.v[i] = *(const v4*)(lv + (offv[i] < limv ? offv[i] : limv));

@@ -117,6 +117,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int x = 0; x < NPV; ++x) offv[x] = (uint32_t)((st + 256 * x) / CV) * pitchv + colv;
     const int Llast = rows - (nc - 1) * BT;   // < BT at the end of a sequence only
+    const uint32_t tail = wave == 4 ? (uint32_t)lane : 0u, grow = wave == 7 ? (uint32_t)lane : 0u;
     // One barrier per chunk: it publishes the next chunk's tiles and says that the matrix waves are done with the other
     // buffer.  Every memory operation is unconditional (rows and chunks past the end are read from the last one), so
     // that the compiler's wait counts leave the other register sets in flight.
@@ -139,8 +140,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         const char* tb = (const char*)p.AT + ((chunk0 + cc) * H + hh) * (int64_t)kTriElems * 2;
         R.tu0 = *(const v8*)(tb + st * 16);
-        R.tu1 = *(const v8*)(tb + (256 + lane) * 16);   // the last 64 pieces: every wave loads them, one writes them
-        const uint32_t gr = ((uint32_t)lane < last ? (uint32_t)lane : last) * (uint32_t)H;
+        // the last 64 pieces of Tu and the gates: one wave's each; the others load one word, without a branch (a column of
+        // 64 gates is 64 requests to the L2)
+        R.tu1 = *(const v8*)(tb + (256 + tail) * 16);
+        const uint32_t gr = (grow < last ? grow : last) * (uint32_t)H;
         R.gam = *(p.gam ? p.gam + r0 + gr : &kZeroWord);
         if constexpr (L2N) R.rk = p.rk[r0 + gr];
         ++lc;

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     const int64_t r0h = im.cl.row0 * H + im.hh;
     const int L = im.cl.L;
     if constexpr (PH) {
-      const int row = (tid & (BT - 1)) < L ? (tid & (BT - 1)) : L - 1;
+      const int row = tid >= BT ? 0 : tid < L ? tid : L - 1;   // (one wave's; the others read one word, not 64 lines)
       R.gh = ((const float*)p.g)[r0h + (int64_t)row * H];
     } else {
       constexpr int CG = K / GP;
