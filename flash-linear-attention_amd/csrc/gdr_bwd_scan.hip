@@ -70,7 +70,7 @@ struct BwdScanParams {
 // PASS: the first pass over sequences cut into segments (seq_split.h): every segment but a sequence's first, from a zero
 // gradient, without outputs but the gradient it ends with.
 template <typename T, int K, bool PASS>
-__global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
+__global__ __launch_bounds__(512, K == 64 ? 4 : 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
   typedef typename Elem<T>::v8 v8;
   typedef typename Elem<T>::v4 v4;
   typedef short s4 __attribute__((ext_vector_type(4)));
@@ -305,6 +305,9 @@ __global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
     // wave w: rows 32 w .. of dH; rows 16 w .. of dv2 and dr (16 x 16 tiles: a lane holds four time rows of one column)
     const bool own = KT32 >= 4 || wave < KT32;
     const int tr = wave * 16 + 4 * (lane >> 4), l16 = lane & 15;
+    // operands of q^T and k^T read a phase ahead of their products: not with 64 key channels, where two workgroups share a CU
+    // (128 registers) and hide each other's latency (one sequence of 16384 tokens, 8 heads: step 211 -> 195 us)
+    constexpr bool EARLY = K == 128;
     f32x16 acc = zero16();
     if (dht && own) {
 #pragma unroll
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
         for (int i = 0; i < K / 32; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) b[j][i] = *(const v8*)&sDHt[j * 16 * K + roff[i]];
-        if (own) load_qd(0);
+        if (EARLY && own) load_qd(0);
         __builtin_amdgcn_sched_barrier(0);   // all reads in flight before the first product waits
         f32x4 d[2] = {zero4(), zero4()};
 #pragma unroll
@@ -402,6 +405,14 @@ __global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
       lds_barrier();  // B2(c)
       const T* kc = sK[c & 1];
       v8 fk[BT / 16];
+      auto load_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < BT / 16; ++s) {
+          s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)&kc[klo + 16 * s * K]);
+          s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)&kc[khi + 16 * s * K]);
+          fk[s] = __builtin_shufflevector(__builtin_bit_cast(v4, lo), __builtin_bit_cast(v4, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      };
       {
         v8 ua[2], db[2][2];
 #pragma unroll
@@ -414,11 +425,11 @@ __global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
             db[s][j] = __builtin_shufflevector(*(const v4*)d2, *(const v4*)(d2 + 16), 0, 1, 2, 3, 4, 5, 6, 7);
           }
         }
-        if (own) load_qd(2);
+        if (EARLY && own) load_qd(2);
         const f32x4 eg = *(const f32x4*)&sG[c & 1][0][tr];
         const float dec = sG[c & 1][0][L - 1];
         __builtin_amdgcn_sched_barrier(0);
-        if (own) {   // in the shade of those reads
+        if (EARLY && own) {   // in the shade of those reads
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[r] *= dec;
 #pragma unroll
@@ -437,17 +448,21 @@ __global__ __launch_bounds__(512, 2) void gdr_bwd_scan_kernel(BwdScanParams p) {
           for (int r = 0; r < 4; ++r) o[r] = (T)(-eg[r] * dr[j][r]);
           *(v4*)&sDrT[(16 * j + l16) * LDT + tr] = o;
         }
-        if (own) {
+        if (EARLY && own) load_k();
+        if (!EARLY && own) {
 #pragma unroll
-          for (int s = 0; s < BT / 16; ++s) {
-            s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)&kc[klo + 16 * s * K]);
-            s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)&kc[khi + 16 * s * K]);
-            fk[s] = __builtin_shufflevector(__builtin_bit_cast(v4, lo), __builtin_bit_cast(v4, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+          for (int r = 0; r < 16; ++r) acc[r] *= dec;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            load_qd(2 * h);
+#pragma unroll
+            for (int s = 2 * h; s < 2 * h + 2; ++s) acc = Elem<T>::mfma32(fq[s], fd[s], acc);
           }
         }
       }
       lds_barrier();  // B3(c)
       if (own) {
+        if (!EARLY) load_k();
         v8 f2[BT / 16];
 #pragma unroll
         for (int s = 0; s < BT / 16; ++s) f2[s] = lds_frag32<T>(sDrT, LDT, 0, 16 * s, lane);
