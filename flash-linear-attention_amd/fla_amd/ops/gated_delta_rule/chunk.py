@@ -5,8 +5,8 @@ Forward on the device (chunk size 64), two launches: ``fla_gdr_fwd_prep`` (chunk
 the gate, KK^T, block inverse; leaves one packed triangular 64x64 tile per chunk and head) ->
 ``fla_chunk_gated_delta_rule_fwd_scan`` (gated causal q k^T scores, state scan and output in one pass over q, k,
 v; w, u, v_new and the per-chunk states are never formed).
-A forward pass that will be differentiated runs the same two launches with more outputs and keeps w, Aw, v_new
-and the per-chunk states for the backward; with ``KEEP_STATES_FOR_BACKWARD = False`` the backward recomputes
+A forward pass that will be differentiated runs the same two launches with more outputs and keeps Aw, v_new, the two
+launches' tiles and the per-chunk states for the backward; with ``KEEP_STATES_FOR_BACKWARD = False`` the backward recomputes
 them with ``fla_chunk_gated_delta_rule_fwd_h`` like the reference.
 """
 import os
@@ -31,8 +31,8 @@ _SUPPORTED_KV = {(64, 64), (128, 128), (64, 128), (128, 64), (256, 64), (256, 12
 L2NORM_EPS = 1e-6   # the eps of fla.modules.l2norm
 _FUSED_MAX_K = 128  # the one-pass forward kernel holds at most 128 key channels of the state
 
-# A forward pass that will be differentiated keeps w, Aw, v_new and the per-chunk states for its
-# backward pass (about 2.3 bytes per q/k/v byte) instead of recomputing them there as the reference
+# A forward pass that will be differentiated keeps Aw, v_new, its packed tiles (K = 256: w) and the per-chunk states for
+# its backward pass (about 1.4 bytes per q/k/v byte) instead of recomputing them there as the reference
 # does (fla/ops/gated_delta_rule/chunk.py:95-116): with 288 GB of HBM the second WY launch and the
 # second state scan cost more than the memory.  FLA_AMD_RECOMPUTE_STATES=1 (or setting this flag to
 # False) restores the reference's behaviour.
@@ -130,7 +130,8 @@ def chunk_gated_delta_rule_fwd_keep(q, k, v, g, beta, scale, initial_state, outp
 
 def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do, dht, offsets=None, kept=None):
     """Backward on prepared tensors (seq-first, 16-bit, 64-aligned head dims; ``g_cumsum``
-    the fp32 chunk-local cumsum saved by the forward).  Without ``kept`` it recomputes w, u, Aw, the
+    the fp32 chunk-local cumsum saved by the forward).  ``kept``: ``(AT, Aw, v_new, hT, Aqk)``, or
+    ``(w, Aw, v_new, hT[, Aqk])``.  Without it it recomputes w, u, Aw, the
     per-chunk states and v_new like the reference (``fla/ops/gated_delta_rule/chunk.py:95-116``).
     Returns ``(dq, dk, dv, dbeta, dg, dh0)``."""
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
@@ -145,7 +146,7 @@ def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do
     Aqk = None
     if kept is not None:
         w, Aw, v_new, hT = kept[:4]
-        Aqk = kept[4] if len(kept) > 4 else None   # the two-launch forward (K <= 128): tiles, AT in place of w
+        Aqk = kept[4] if len(kept) > 4 else None   # the two-launch forward (K <= 128): its tiles, w or AT beside them
     else:
         w, u, Aw, _ = fwd_prepare_wy_repr(k, v, beta, g_cumsum, offsets=offs, indices=idx, head_first=False,
                                           chunk_size=BT, store_A=True, store_Au=False)
@@ -165,7 +166,7 @@ def chunk_gated_delta_rule_bwd(q, k, v, g_cumsum, beta, scale, initial_state, do
     dh0 = q.new_empty(N, H, K, V, dtype=torch.float32) if initial_state is not None else None
     if dht is not None:
         dht = (dht if dht.dtype == torch.float32 else dht.float()).contiguous()
-    if Aqk is not None:
+    if Aqk is not None and w.dim() == 5:   # AT [chunks, H, 10, 16, 16]; w has q's four dims
         be.check(be.lib().fla_chunk_gated_delta_rule_bwd_tiles(
             be.ptr(q), be.ptr(k), be.ptr(v), be.ptr(w), be.ptr(v_new), be.ptr(beta), be.ptr(g_cumsum), be.ptr(Aw),
             be.ptr(do), be.ptr(dht), be.ptr(hT), be.ptr(Aqk), be.ptr(ws_dv2), be.ptr(ws_dh), be.ptr(dq), be.ptr(dk),
