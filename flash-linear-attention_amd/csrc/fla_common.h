@@ -106,6 +106,13 @@ FLA_DEVICE T from_f32(float x) { return (T)x; }
 // (fla/ops/utils/exp.py:9-10).
 FLA_DEVICE float safe_exp(float x) { return x <= 0.f ? __expf(x) : 0.f; }
 
+// `sum` and one more log-gate, in units of log 2.  Gates of their type's lowest value (masks) and -inf hold it at -2^120, whose
+// decay is 0 just the same: the sums over a chunk stay finite, and with them the differences of two sums.  NaN stays NaN.
+constexpr float kLog2GateMin = -0x1p120f;
+FLA_DEVICE float add_log2_gate(float sum, float g) {
+  return __builtin_elementwise_maximum(fmaf(g, 1.4426950408889634f, sum), kLog2GateMin);
+}
+
 // DPP row operations (a DPP row is 16 consecutive lanes); lanes without a source read 0.
 template <int CTRL>
 FLA_DEVICE float dpp_f32(float x) {

@@ -292,6 +292,42 @@ def test_chunk_gla_backward_chunk_launch(device, B, T, H, K, V, gates):
         assert_close(name, r.grad, x.grad, tol / 4)
 
 
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (64, 128), (128, 64)])
+@pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
+def test_chunk_gla_lowest_gates(device, monkeypatch, gates, K, V, keep):
+    """A log-gate of its type's lowest value (at most one a chunk and channel, as a mask leaves it) resets the state as one
+    of -1e30 does: times log2 e it must not become -inf, whose differences are NaN.  Both swallow every other gate of the
+    sums over their chunk and have a decay of 0, so outputs and gradients are the same bits, from the states the forward
+    kept and from recomputed ones."""
+    from fla_amd.ops.gla import chunk as mod
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    monkeypatch.setattr(mod, "KEEP_STATES_FOR_BACKWARD", keep)
+    B, T, H = 2, 200, 3
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=83, normalizer=16.0, h0_std=1.0)
+    gen = torch.Generator().manual_seed(12)
+    do = torch.randn(B, T, H, V, generator=gen).bfloat16()
+    dht = torch.randn(B, H, K, V, generator=gen) * 0.1
+    g = g[..., 0].contiguous() if gates == "head" else g.to(getattr(torch, gates))
+    reset = torch.zeros(g.shape, dtype=torch.bool)
+    for t0 in range(0, T, 64):
+        at = t0 + torch.randint(min(64, T - t0), (B, 1) + tuple(g.shape[2:]), generator=gen)
+        reset.scatter_(1, at, torch.rand(at.shape, generator=gen) < 0.5)
+    print(f"chunk_gla lowest gates {gates} K={K} V={V} keep={keep}", flush=True)
+
+    def step(low):
+        leaves = [x.to(device).requires_grad_() for x in (q, k, v, g.masked_fill(reset, low), h0)]
+        o, ht = (chunk_simple_gla if gates == "head" else chunk_gla)(*leaves[:4], initial_state=leaves[4],
+                                                                     output_final_state=True, head_first=False)
+        torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+        return [o, ht] + [x.grad for x in leaves]
+
+    for name, want, got in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), step(-1e30), step(torch.finfo(g.dtype).min)):
+        assert torch.isfinite(want).all(), name
+        assert torch.equal(want, got), name
+
+
 def test_chunk_gla_backward_extreme_gates_mixed_varlen(device):
     """Only some chunks and channels are flagged; packed batch, K != V."""
     gen = torch.Generator().manual_seed(82)
