@@ -344,6 +344,13 @@ __global__ __launch_bounds__(512, K == 64 ? 4 : 2) void gdr_bwd_scan_kernel(BwdS
       hi = t1 >= wave ? hi : z;
       return __builtin_shufflevector(__builtin_bit_cast(v4, lo), __builtin_bit_cast(v4, hi), 0, 1, 2, 3, 4, 5, 6, 7);
     };
+    // The first 32 rows lie above the diagonal for waves 2 and 3: their product is left out and not formed with zeros, which
+    // would make every later row NaN where an earlier one of do holds an infinity or NaN.
+    auto tri_product = [&](const v8* a, v8 b0, v8 b1) __attribute__((always_inline)) {
+      f32x4 x = zero4();
+      if (wave < 2) x = Elem<T>::mfma16(a[0], b0, x);   // wave-uniform
+      return Elem<T>::mfma16(a[1], b1, x);
+    };
     // what dv2 of chunk c takes that does not depend on dH: this wave's rows of k, dl = Aqk^T do, the gate factors
     v8 ka[K / 32];
     f32x4 dl[2], ed;
@@ -360,10 +367,7 @@ __global__ __launch_bounds__(512, K == 64 ? 4 : 2) void gdr_bwd_scan_kernel(BwdS
       for (int i = 0; i < K / 32; ++i) ka[i] = *(const v8*)&kc[wave * 16 * K + roff[i]];
       ed = *(const f32x4*)&sG[c & 1][1][tr];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        dl[j] = Elem<T>::mfma16(pa[0], db[0][j], zero4());
-        dl[j] = Elem<T>::mfma16(pa[1], db[1][j], dl[j]);
-      }
+      for (int j = 0; j < 2; ++j) dl[j] = tri_product(pa, db[0][j], db[1][j]);
     };
     if (nchunks > 0) {
       publish();
@@ -437,10 +441,7 @@ __global__ __launch_bounds__(512, K == 64 ? 4 : 2) void gdr_bwd_scan_kernel(BwdS
         }
         f32x4 dr[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          dr[j] = Elem<T>::mfma16(ua[0], db[0][j], zero4());
-          dr[j] = Elem<T>::mfma16(ua[1], db[1][j], dr[j]);
-        }
+        for (int j = 0; j < 2; ++j) dr[j] = tri_product(ua, db[0][j], db[1][j]);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           v4 o;

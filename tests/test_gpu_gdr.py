@@ -373,6 +373,33 @@ def test_chunk_gdr_reverse_scan_from_tiles(device, T, K, V, gated):
         assert_close(name + " (from w)", other[name].float().cpu(), order[name], tol / 2)
 
 
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (64, 128), (128, 64)])
+@pytest.mark.parametrize("row", [5, 31])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_chunk_gdr_backward_nan_stays_behind(device, K, V, row, bad):
+    """dv and dg of a token come from do of that token and later ones.  What is not finite in do in the first half of a chunk
+    leaves the rows of its second half and of the chunks behind it as they are, bit for bit (the kernels' products skip
+    blocks of 32 rows above the diagonal)."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    B, T, H = 1, 200, 2
+    q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=97, h0_std=1.0)
+    gen = torch.Generator().manual_seed(13)
+    do = torch.randn(B, T, H, V, generator=gen).to(q.dtype)
+    print(f"chunk_gdr backward with {bad} in row {row} of a chunk, K={K} V={V}", flush=True)
+
+    def grads(do):
+        leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, beta, h0)]
+        o, _ = chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], output_final_state=True, head_first=False)
+        o.backward(do.to(device))
+        return leaves[2].grad, leaves[3].grad
+
+    poisoned = do.clone()
+    poisoned[0, 64 + row, 1, 7] = bad
+    for name, want, got in zip(("dv", "dg"), grads(do), grads(poisoned)):
+        assert torch.isfinite(want).all() and not torch.isfinite(got).all(), name
+        assert torch.equal(want[:, 96:], got[:, 96:]), name
+
+
 def test_chunk_gdr_backward_varlen_and_headfirst(device):
     gen = torch.Generator().manual_seed(8)
     T, N, H, D = 500, 4, 2, 128
