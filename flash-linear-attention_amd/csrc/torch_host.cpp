@@ -135,6 +135,8 @@ struct Plan : torch::CustomClassHolder {
   std::mutex mu;
   std::map<std::tuple<int64_t, int, bool, int>, SplitTables> splits;
 
+  bool covers(int64_t begin, int64_t end) const { return !host.empty() && host.front() == begin && host.back() == end; }
+
   // The tables of a cut are used by later calls on any stream.  A stream that is being captured takes no copy: a call whose
   // tables are not there yet runs uncut under it.
   SplitTables split(int64_t H, int slabs, bool reverse, int kind) {
@@ -318,7 +320,10 @@ struct GlaNode : torch::autograd::Function<GlaNode> {
     const Tensor dout = grads[0].defined() ? as(grads[0], q.scalar_type()).contiguous() : at::zeros(v.sizes(), v.options());
     const Tensor dht = a.want_ht ? f32(grads[1]) : Tensor();
     Tensor dhtf = fresh_like(hT), dq = fresh_like(q), dk = fresh_like(k), dv = fresh_like(v);
-    Tensor dg = a.head_gates ? fresh({d.B, d.T, d.H}, q, at::kFloat) : fresh(q.sizes(), q, at::kFloat);
+    // per-head gates: rows of a packed batch that belong to no sequence have a gradient of zero
+    Tensor dg = !a.head_gates                       ? fresh(q.sizes(), q, at::kFloat)
+                : !a.plan || a.plan->covers(0, d.T) ? fresh({d.B, d.T, d.H}, q, at::kFloat)
+                                                    : at::zeros({d.B, d.T, d.H}, g.options());
     Tensor dh0 = rest.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
     const fla_stream_t st = stream_of(q);
     // (the reverse scan's workgroups hold 64 x 64 tiles of a state)

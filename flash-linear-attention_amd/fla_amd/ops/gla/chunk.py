@@ -470,6 +470,8 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
     dhtf = torch.empty_like(hT)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dg = q.new_empty(q.shape[:3] if kept and head_gates else q.shape, dtype=torch.float32)
+    if kept and head_gates and plan is not None and not plan.covers(0, T):
+        dg.zero_()   # rows of a packed batch that belong to no sequence have a gradient of zero
     dh0 = q.new_empty(N, H, K, V, dtype=torch.float32) if initial_state is not None else None
     if dht is not None:
         dht = (dht if dht.dtype == torch.float32 else dht.float()).contiguous()

@@ -131,6 +131,8 @@ class VarlenPlan:
         order = sorted(range(self.N), key=lambda i: -lens[i])
         self.seq_order = torch.tensor(order, dtype=torch.int64).to(dev, non_blocking=True)
 
+    def covers(self, begin: int, end: int) -> bool:
+        return self._host[0] == begin and self._host[-1] == end
 
     @property
     def native(self):

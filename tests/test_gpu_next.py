@@ -314,6 +314,35 @@ def test_chunk_simple_gla_per_head_gate_kernel_fp16_and_gradients(device):
     assert_close("dh0", rh0.grad, h0l.grad, TOL_G)
 
 
+@pytest.mark.parametrize("native", [True, False])   # the compiled node / the Python one
+@pytest.mark.parametrize("bounds", [[0, 70, 200], [30, 70, 300], [30, 70, 200]])
+def test_chunk_simple_gla_rows_outside_the_sequences(device, native, bounds, monkeypatch):
+    """Rows of a packed batch that belong to no sequence (padding ahead of the first one or behind the last): their gates get
+    a gradient of zero, whatever the memory held before; the other rows' gradients are those of the batch without them."""
+    import fla_amd.ops.simple_gla.chunk as sg_mod
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    monkeypatch.setattr(sg_mod, "SCAN_FORWARD", native)
+    T, H, D, b, e = 300, 3, 64, bounds[0], bounds[-1]
+    gen = torch.Generator().manual_seed(92)
+    q, k, v, do = (torch.randn(1, T, H, D, generator=gen).bfloat16() for _ in range(4))
+    g = F.logsigmoid(torch.randn(1, T, H, generator=gen)) / 16
+    dev = _dev(device)
+    print(f"chunk_simple_gla rows outside the sequences {bounds} native={native}", flush=True)
+
+    def grad(x, do, bounds):
+        leaves = [dev(t.contiguous()).requires_grad_() for t in x]
+        junk = [torch.full((1, T, H), float("nan"), device=device) for _ in range(64)]   # what freed memory may hold
+        o, _ = chunk_simple_gla(*leaves, cu_seqlens=dev(torch.tensor(bounds)), head_first=False)
+        del junk
+        o.backward(dev(do.contiguous()))
+        return leaves[3].grad
+
+    dg = grad((q, k, v, g), do, bounds)
+    want = grad([x[:, b:e] for x in (q, k, v, g)], do[:, b:e], [x - b for x in bounds])
+    assert torch.equal(dg[:, b:e], want)
+    assert torch.equal(dg[:, :b], torch.zeros_like(dg[:, :b])) and torch.equal(dg[:, e:], torch.zeros_like(dg[:, e:]))
+
+
 @pytest.mark.parametrize("varlen", [False, True])
 def test_chunk_simple_gla_strong_gates_backward_reproducible(device, varlen, monkeypatch):
     """Gates strong enough that chunks leave the single-reference range (their intra-chunk terms come from the
