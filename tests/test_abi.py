@@ -2,6 +2,7 @@
 the ctypes signature table covers them all, and the host-side integer
 bookkeeping is bit-exact against the oracle.  No device compute."""
 import ctypes
+import hashlib
 import os
 import re
 
@@ -27,6 +28,30 @@ def test_library_exports_every_declared_symbol():
         assert hasattr(handle, n), f"{n} declared in fla_hip.h but not exported"
     assert sorted(be.SIGNATURES) == names, "ctypes signature table out of sync with fla_hip.h"
     assert be.lib().fla_abi_version() == be.ABI_VERSION
+
+
+# What a binding relies on, by version: a digest of the C declarations and of the argument counts of the host extension.
+INTERFACES = {15: "b7a4f7cfed6a371e", 16: "087cb7b8a1fcb11d"}
+
+
+def _interface():
+    text = open(os.path.join(ROOT, "include", "fla_hip.h")).read()
+    text = re.sub(r"/\*.*?\*/|^#define FLA_ABI_VERSION.*?$", "", text, flags=re.S | re.M)
+    host = open(os.path.join(ROOT, "flash-linear-attention_amd", "csrc", "torch_host.cpp")).read()
+    counts = re.findall(r"^PyObject\* (py_\w+)\(.*?expect\(n, (\d+)\)", host, flags=re.S | re.M)
+    assert len(counts) >= 10
+    return hashlib.sha256(repr((text.split(), counts)).encode()).hexdigest()[:16]
+
+
+def test_version_moves_with_the_interface():
+    """A library or extension built before a declaration changed must be refused when it is loaded, not fail at a call: another
+    interface takes another FLA_ABI_VERSION (in the header and in _backend.py) and a line in the table above."""
+    from fla_amd import _backend as be
+    header = open(os.path.join(ROOT, "include", "fla_hip.h")).read()
+    version = int(re.search(r"#define FLA_ABI_VERSION (\d+)", header).group(1))
+    assert version == be.ABI_VERSION
+    assert INTERFACES.get(version) == _interface()
+    assert len(set(INTERFACES.values())) == len(INTERFACES)
 
 
 def test_error_strings():
