@@ -30,6 +30,9 @@ _SUPPORTED_KV = {(64, 64), (128, 128), (64, 128), (128, 64)}
 # pass, which the reference starts by recomputing those states (fla/ops/gla/chunk.py:1239-1253).
 # FLA_AMD_RECOMPUTE_STATES=1 (or setting this flag to False) restores the reference's behaviour.
 KEEP_STATES_FOR_BACKWARD = os.environ.get("FLA_AMD_RECOMPUTE_STATES", "0") in ("", "0")
+# What chunk_gla_fwd_fused leaves beside the states unless its caller says: k^ = k e^{G_last - G} and the score tile of every
+# chunk too (V <= 128).  The operators do not ask for them and the backward does not read them.
+KEEP_KHAT_AND_SCORES = os.environ.get("FLA_AMD_GLA_FUSED_DV", "1") not in ("", "0")
 # fp32 q/k/v run through the fp16 chunk kernels, as the reference runs them through its chunk kernels with fp32 operands
 # on the matrix pipe at reduced precision (tests/ops/test_gla.py:149-201): q, k and v are divided by a power of two >= their
 # largest magnitude (exact; found on the device, no synchronisation) and rounded to fp16, gates and states stay fp32, and
@@ -277,7 +280,7 @@ def _guard_workspaces(q, chunks, H, KV, keep):
 
 def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets=None, exact_guard=True,
                         return_flags=False, states_out=None, head_gates=False, first_launch_only=False,
-                        khat_and_scores=True):
+                        khat_and_scores=None):
     """Forward through ``fla_chunk_gla_fwd_fused``: seq-first, K in {64,128}, V % 64 == 0.
     With ``exact_guard`` (needs V <= 128) chunks whose cumulative log-gate leaves the
     single-reference range are detected on the device and recomputed exactly; ``return_flags``
@@ -285,9 +288,11 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
     ``states_out`` the launch also writes the state entering every chunk (transposed fragment
     order, what the backward kernels read) and appends it, followed (per-key gates only) by the gated queries
     ``q e^{G}`` ``[B,T,H,K]`` and the chunk decays ``e^{G_last}`` ``[chunks,H,K]`` the backward's reverse state scan
-    streams (``fla_chunk_gla_fwd_fused_kept``), and, unless ``khat_and_scores`` is off,
+    streams (``fla_chunk_gla_fwd_fused_kept``), and, with ``khat_and_scores`` (default ``KEEP_KHAT_AND_SCORES``),
     ``k e^{G_last - G}`` ``[chunks,H,K,64]`` and the score tiles ``[chunks,H,64,64]``.  ``head_gates``: ``g`` is one fp32 log-gate
     per (token, head), ``[B,T,H]`` (``fla_chunk_simple_gla_fwd_fused``)."""
+    if khat_and_scores is None:
+        khat_and_scores = KEEP_KHAT_AND_SCORES
     B, T, H, K = q.shape
     V = v.shape[-1]
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
@@ -441,7 +446,7 @@ def chunk_gla_fwd(q, k, v, g, g_cumsum, scale, initial_state, output_final_state
 
 
 def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wide=None, hT=None, qg=None,
-                         decay=None, head_gates=False):
+                         decay=None, head_gates=False, kh=None, scores=None):
     """Backward on prepared tensors (seq-first, 16-bit, 64-aligned head dims).
     Returns ``(dq, dk, dv, dg, dh0)``; without ``hT`` (the states a forward pass kept) it
     recomputes the per-chunk states as the reference does (``fla/ops/gla/chunk.py:1239-1253``).  ``qg``, ``decay``:
@@ -450,7 +455,8 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
     from the exact kernel.  Without it the result is exact only while the chunk-cumulative
     log-gate stays within +-80.  ``head_gates``: ``g`` is one fp32 log-gate per (token, head), ``[B, T, H]``, and
     ``dg`` comes back in that shape (``fla_chunk_simple_gla_bwd`` when the forward kept its gated queries; otherwise
-    the gates are broadcast over the key channels and the per-key gradient is summed afterwards)."""
+    the gates are broadcast over the key channels and the per-key gradient is summed afterwards).  ``kh``, ``scores``: what
+    else a forward may have left; accepted, not read."""
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
     offs = None if plan is None else plan.offsets
     idx = None if plan is None else plan.indices

@@ -604,6 +604,36 @@ def test_chunk_gla_kept_gated_queries_and_decays(device, B, H, varlen):
     torch.testing.assert_close(got_decay, want_decay, rtol=2e-5, atol=1e-30)
 
 
+@pytest.mark.parametrize("head_gates", [False, True])
+def test_chunk_gla_backward_takes_all_kept_tensors(device, monkeypatch, head_gates):
+    """A caller may hand the backward everything the forward left, k^ and the score tiles among it: the gradients are those
+    without them.  KEEP_KHAT_AND_SCORES decides whether a forward that is not told leaves them."""
+    from fla_amd.ops.gla import chunk as mod
+    B, T, H, D = 1, 150, 2, 64
+    q, k, v, g, h0 = (x.to(device) for x in gla_inputs(B, T, H, D, D, seed=84))
+    g = g[..., 0].contiguous() if head_gates else g
+    do, dht = torch.randn_like(v), torch.randn_like(h0)
+    print(f"chunk_gla backward on all kept tensors head_gates={head_gates}", flush=True)
+    names = ("hT", "qg", "decay", "kh", "scores")
+
+    def forward(**kw):
+        kept = []
+        _, _, wide = mod.chunk_gla_fwd_fused(q, k, v, g, D ** -0.5, h0, True, return_flags=True, states_out=kept,
+                                             head_gates=head_gates, **kw)
+        return wide, kept
+
+    def backward(wide, kept):
+        return mod.chunk_gla_bwd_device(q, k, v, g, D ** -0.5, h0, do, dht, None, wide, head_gates=head_gates,
+                                        **dict(zip(names, kept)))
+
+    wide, kept = forward()
+    assert len(kept) == 5 and len(forward(khat_and_scores=False)[1]) == 3
+    for a, b in zip(backward(wide, kept), backward(wide, kept[:3])):
+        assert torch.equal(a, b)
+    monkeypatch.setattr(mod, "KEEP_KHAT_AND_SCORES", False)
+    assert len(forward()[1]) == 3 and len(forward(khat_and_scores=True)[1]) == 5
+
+
 @pytest.mark.parametrize("logit_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("K,V,T,normalizer,clamp_min,varlen", [
     (128, 128, 300, 16.0, None, False),
