@@ -106,12 +106,12 @@ FLA_DEVICE T from_f32(float x) { return (T)x; }
 // (fla/ops/utils/exp.py:9-10).
 FLA_DEVICE float safe_exp(float x) { return x <= 0.f ? __expf(x) : 0.f; }
 
-// `sum` and one more log-gate, in units of log 2.  Gates of their type's lowest value (masks) and -inf hold it at -2^120, whose
-// decay is 0 just the same: the sums over a chunk stay finite, and with them the differences of two sums.  NaN stays NaN.
-constexpr float kLog2GateMin = -0x1p120f;
-FLA_DEVICE float add_log2_gate(float sum, float g) {
-  return __builtin_elementwise_maximum(fmaf(g, 1.4426950408889634f, sum), kLog2GateMin);
-}
+// A log-gate on its way into a sum over a chunk.  What resets the state (a mask: -1e30, the type's lowest value, -inf) counts as
+// -256, whose decay is 0 in fp32 just the same.  Sums of 64 then stay finite, and so does the difference of two sums; the gates
+// behind a reset are not lost in them, and several resets add up in any order.  Each gate is held and not the sum, so that two
+// masked tokens in a row still differ by one of them.  NaN stays NaN.
+constexpr float kGateMin = -256.f;
+FLA_DEVICE float finite_gate(float g) { return __builtin_elementwise_maximum(g, kGateMin); }
 
 // DPP row operations (a DPP row is 16 consecutive lanes); lanes without a source read 0.
 template <int CTRL>

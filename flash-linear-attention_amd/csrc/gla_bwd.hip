@@ -277,8 +277,8 @@ __global__ __launch_bounds__(256) void gla_bwd_dh_kernel(BDhParams p) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         bool valid = (rg * 8 + i) < L;
-        r0 += valid ? (float)R.g[i][0] : 0.f;
-        r1 += valid ? (float)R.g[i][1] : 0.f;
+        r0 += valid ? finite_gate((float)R.g[i][0]) : 0.f;
+        r1 += valid ? finite_gate((float)R.g[i][1]) : 0.f;
         G[i][0] = r0;
         G[i][1] = r1;
       }
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void gla_bwd_intra_exact_kernel(BExactParams p
       kv = *(const v4*)((const T*)p.k + off);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sG[row * LDG + c4 + j] = gv[j];
+    for (int j = 0; j < 4; ++j) sG[row * LDG + c4 + j] = finite_gate(gv[j]);
     *(v4*)&sQ[row * LDQ + c4] = qv;
     *(v4*)&sK[row * LDQ + c4] = kv;
   }

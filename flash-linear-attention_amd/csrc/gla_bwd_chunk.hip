@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
   constexpr int GP = 16 / sizeof(GE), NG = PH ? 1 : BT * K / GP / 256;   // gates: elements per 16-byte piece, pieces per lane
   typedef GE gvec __attribute__((ext_vector_type(GP)));
   constexpr int LDK = K + 8, LDV = V + 8, LDG = K + 4;
-  // the gates and their sums are carried times log2 e (add_log2_gate)
-  constexpr float kInvLimit = InvDecayLimit<T>::value * 1.4426950408889634f;
+  // the gates and their sums are carried times log2 e
+  constexpr float kLog2e = 1.4426950408889634f, kInvLimit = InvDecayLimit<T>::value * kLog2e;
   constexpr int VT32 = V / 32, KT32 = K / 32;
   constexpr int RK = K / 64, RV = V / 64;   // row tiles of a wave in products with K (V) result columns
   constexpr int AB_DOV = 2 * BT * LDV * 2, AB_G = PH ? 0 : BT * LDG * 4, AB_DH = K * LDV * 2;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     const int L = im.cl.L;
     if constexpr (PH) {
       if (wave == 0) {
-        float x = half_prefix(lane < L ? add_log2_gate(0.f, R.gh) : 0.f);
+        float x = half_prefix(lane < L ? finite_gate(R.gh) * kLog2e : 0.f);
         x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x143, 0xC, 0xF, true));   // row_bcast:31
         sGam[lane] = x;
       }
@@ -148,11 +148,12 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
 #pragma unroll
       for (int i = 0; i < NG; ++i) {
         const int e = tid + 256 * i, row = e / CG, c = (e % CG) * GP;
+        const float unit = row < L ? kLog2e : 0.f;
 #pragma unroll
         for (int j = 0; j < GP; j += 4) {
           f32x4 x;
 #pragma unroll
-          for (int b = 0; b < 4; ++b) x[b] = row < L ? add_log2_gate(0.f, (float)R.g[i][j + b]) : 0.f;
+          for (int b = 0; b < 4; ++b) x[b] = finite_gate((float)R.g[i][j + b]) * unit;
           *(f32x4*)&sG[row * LDG + c + j] = x;
         }
       }

@@ -209,14 +209,14 @@ FLA_DEVICE void gla_stage_waves(const FusedParams& p, const StageLds<T>& L, cons
     begin_loads();
     float G[RPT][CPL], glast[CPL];
     float gabs = 0.f;
-    [[maybe_unused]] const float clamp2 = fmaxf(p.gate_clamp_min * LOG2E, kLog2GateMin);
+    [[maybe_unused]] const float clamp2 = fmaxf(p.gate_clamp_min * LOG2E, kGateMin);
     if constexpr (SG) {
       // one gate per row: a single prefix sum, shared by all key channels of the lane (the
       // exponentials below then collapse to one pair per row)
       float run = 0.f, Gs[RPT];
 #pragma unroll
       for (int i = 0; i < RPT; ++i) {
-        run = add_log2_gate(run, (float)R.g[i][0]);
+        run = fmaf(finite_gate((float)R.g[i][0]), LOG2E, run);
         Gs[i] = run;
       }
       const float pre = row_prefix16(run);
@@ -240,7 +240,7 @@ FLA_DEVICE void gla_stage_waves(const FusedParams& p, const StageLds<T>& L, cons
 #pragma unroll
       for (int i = 0; i < RPT; ++i) {
         if constexpr (LOGITS) run += log2_sigmoid_gate((float)R.g[i][j], p.gate_inv_norm, clamp2);
-        else run = add_log2_gate(run, (float)R.g[i][j]);   // prefix sums in the log2 domain
+        else run = fmaf(finite_gate((float)R.g[i][j]), LOG2E, run);   // prefix sums in the log2 domain
         G[i][j] = run;
       }
       const float pre = row_prefix16(run);

@@ -202,8 +202,8 @@ __global__ __launch_bounds__(256) void gla_fwd_h_kernel(HParams p) {
       float r0 = 0.f, r1 = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        r0 += (float)R0.g[i][0];
-        r1 += (float)R0.g[i][1];
+        r0 += finite_gate((float)R0.g[i][0]);
+        r1 += finite_gate((float)R0.g[i][1]);
         G[i][0] = r0;
         G[i][1] = r1;
       }

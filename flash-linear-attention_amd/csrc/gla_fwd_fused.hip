@@ -125,7 +125,7 @@ FLA_DEVICE void gla_exact_chunk(const ExactParams& p, const ExactLds<T>& S, cons
     for (int i = 0; i < RPT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        run[j] += gq[i][j];
+        run[j] += finite_gate(gq[i][j]);
         G[i][j] = run[j];
       }
     *(f32x4*)&S.part[rg * K + c4] = f32x4{run[0], run[1], run[2], run[3]};

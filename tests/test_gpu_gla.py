@@ -297,9 +297,9 @@ def test_chunk_gla_backward_chunk_launch(device, B, T, H, K, V, gates):
 @pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
 def test_chunk_gla_lowest_gates(device, monkeypatch, gates, K, V, keep):
     """A log-gate of its type's lowest value (at most one a chunk and channel, as a mask leaves it) resets the state as one
-    of -1e30 does: times log2 e it must not become -inf, whose differences are NaN.  Both swallow every other gate of the
-    sums over their chunk and have a decay of 0, so outputs and gradients are the same bits, from the states the forward
-    kept and from recomputed ones."""
+    of -1e30 does: times log2 e it must not become -inf, whose differences are NaN.  Both have a decay of 0 and count as the
+    same gate in the sums over their chunk, so outputs and gradients are the same bits, from the states the forward kept
+    and from recomputed ones."""
     from fla_amd.ops.gla import chunk as mod
     from fla_amd.ops.gla import chunk_gla
     from fla_amd.ops.simple_gla import chunk_simple_gla
@@ -326,6 +326,50 @@ def test_chunk_gla_lowest_gates(device, monkeypatch, gates, K, V, keep):
     for name, want, got in zip(("o", "ht", "dq", "dk", "dv", "dg", "dh0"), step(-1e30), step(torch.finfo(g.dtype).min)):
         assert torch.isfinite(want).all(), name
         assert torch.equal(want, got), name
+
+
+@pytest.mark.parametrize("form", ["kept", "recomputed", "cut"])
+@pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
+def test_chunk_gla_runs_of_lowest_gates(device, monkeypatch, gates, form):
+    """Masked tokens next to each other: the state is reset at every one of them, not at the first alone, and the tokens
+    between and behind them keep their own decays, which a sum holding gates of -1e30 would lose.  Against the fp32
+    recurrence at the tolerances of ordinary gates; whatever low value the mask has, the same bits.  From kept and
+    recomputed states, and where the sequence is cut."""
+    from fla_amd.ops.gla import chunk as mod
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    from oracle.recurrent import naive_recurrent_gla
+    monkeypatch.setattr(mod, "KEEP_STATES_FOR_BACKWARD", form != "recomputed")
+    B, T, H, K, V = 1, 4096 if form == "cut" else 200, 2, 64, 64
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=84, normalizer=16.0, h0_std=1.0)
+    gen = torch.Generator().manual_seed(14)
+    do = torch.randn(B, T, H, V, generator=gen).bfloat16()
+    dht = torch.randn(B, H, K, V, generator=gen) * 0.1
+    g = g[..., 0].contiguous() if gates == "head" else g.to(getattr(torch, gates))
+    reset = torch.zeros(g.shape, dtype=torch.bool)
+    for t0, n in ((3, 2), (20, 5), (62, 4), (130, 1), (136, 1), (192, 8)):   # within four rows, across them, across chunks
+        reset[:, t0:t0 + n] = torch.rand((B, 1) + tuple(g.shape[2:]), generator=gen) < 0.7
+    names = ("o", "ht", "dq", "dk", "dv", "dg", "dh0")
+    print(f"chunk_gla runs of lowest gates {gates} {form}", flush=True)
+
+    def step(low):
+        leaves = [x.to(device).requires_grad_() for x in (q, k, v, g.masked_fill(reset, low), h0)]
+        o, ht = (chunk_simple_gla if gates == "head" else chunk_gla)(*leaves[:4], initial_state=leaves[4],
+                                                                     output_final_state=True, head_first=False)
+        torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+        return [o, ht] + [x.grad for x in leaves]
+
+    refs = [x.float().clone().requires_grad_() for x in (q, k, v, g.masked_fill(reset, -1e30), h0)]
+    ro, rht = naive_recurrent_gla(*refs[:3], **{"g" if gates == "head" else "gk": refs[3]}, initial_state=refs[4],
+                                  output_final_state=True)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    wanted = [ro, rht] + [x.grad for x in refs]
+    first = step(-1e30)
+    for name, want, got, tol in zip(names, wanted, first, (TOL_O, TOL_HT) + (2e-2,) * 5):
+        assert_close(name, want.detach(), got.detach().cpu(), tol)
+    for low in (torch.finfo(g.dtype).min, float("-inf")):
+        for name, want, got in zip(names, first, step(low)):
+            assert torch.equal(want, got), (name, low)
 
 
 def test_chunk_gla_backward_extreme_gates_mixed_varlen(device):
