@@ -267,8 +267,8 @@ def test_chunk_gla_backward_extreme_gates(device, normalizer):
 @pytest.mark.parametrize("gates", ["float32", "float16", "head"])
 def test_chunk_gla_backward_chunk_launch(device, B, T, H, K, V, gates):
     """The launch that forms all gradients of a (chunk, head): single rows, chunks one row short and one row over, every pair
-    of head dims, more items (592) than workgroups run at once (512), per-key gates of both types and one gate per head.
-    fp16: its tolerances are a quarter of the bf16 ones, 8x the resolution less the fp32 reference's own order of
+    of head dims, 592 items of a workgroup each (768 of 64 x 64 run at once; below more than run at once), per-key gates of
+    both types and one gate per head.  fp16: its tolerances are a quarter of the bf16 ones, 8x the resolution less the fp32 reference's own order of
     summation."""
     from fla_amd.ops.gla import chunk_gla
     from fla_amd.ops.simple_gla import chunk_simple_gla
@@ -290,6 +290,36 @@ def test_chunk_gla_backward_chunk_launch(device, B, T, H, K, V, gates):
     torch.autograd.backward((ro, rht), (do.float(), dht))
     for name, r, x, tol in zip(("dq", "dk", "dv", "dg", "dh0"), ref, leaves, (8e-3, 8e-3, 8e-3, 1e-2, 5e-3)):
         assert_close(name, r.grad, x.grad, tol / 4)
+
+
+@pytest.mark.parametrize("B,K,V", [(52, 64, 64), (36, 128, 64), (36, 64, 128), (36, 128, 128)])
+@pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
+def test_chunk_gla_backward_chunk_launch_many_items(device, B, K, V, gates):
+    """More (chunk, head) items than workgroups run at once (three per CU with 64 x 64 heads, i.e. 768, two with the others,
+    512): a workgroup takes two and three, requests the next one's rows while it forms the last one's gradients and stages
+    them over its tiles.  The same sequences a few at a time, an item per workgroup, give the same bits."""
+    from fla_amd.ops.gla import chunk as mod
+    T, H, head = 127, 16, gates == "head"
+    q, k, v, g, h0 = (x.to(device) for x in gla_inputs(B, T, H, K, V, seed=95, normalizer=16.0, h0_std=1.0))
+    g = g[..., 0].contiguous() if head else g.to(getattr(torch, gates))
+    do, dht = torch.randn_like(v), torch.randn_like(h0)
+    print(f"chunk_gla backward, {2 * B * H} items K={K} V={V} gates={gates}", flush=True)
+    kept = []
+    _, _, wide = mod.chunk_gla_fwd_fused(q, k, v, g, K ** -0.5, h0, True, return_flags=True, states_out=kept, head_gates=head,
+                                         khat_and_scores=False)
+    hT, qg, decay = kept
+    wide = wide.view(B, 2, H)
+
+    def backward(s):
+        c = lambda x: x[s].contiguous()
+        n = c(q).shape[0]
+        return mod.chunk_gla_bwd_device(c(q), c(k), c(v), c(g), K ** -0.5, c(h0), c(do), c(dht), None,
+                                        c(wide).view(2 * n, H), hT=c(hT), qg=c(qg), decay=c(decay), head_gates=head)
+
+    whole = backward(slice(0, B))
+    for b in range(0, B, 4):
+        for name, a, x in zip(("dq", "dk", "dv", "dg", "dh0"), whole, backward(slice(b, b + 4))):
+            assert torch.equal(a[b:b + 4], x), (name, b)
 
 
 @pytest.mark.parametrize("keep", [True, False])

@@ -39,7 +39,7 @@ def test_gla_cut_sequences(device, B, T, H, K, V, bounds, dtype, heads):
     from fla_amd.ops.simple_gla import chunk_simple_gla
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(N, T, H, V // 64, False, bounds) and _cut(N, T, H, V // 32, True, bounds)
+    assert _cut(N, T, H, V // 64, False, bounds)   # (the reverse scan runs uncut: test_gla_cut_state_gradients)
     print("cut", B, T, H, K, V, bounds, dtype, heads, flush=True)
     q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
     if heads:
@@ -141,11 +141,16 @@ def test_gdr_cut_l2norm_in_kernel(device, K, V):
     assert_close("ht", rht, ht, 5e-3)
 
 
-@pytest.mark.parametrize("heads", [False, True])
-@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", [
+GRADIENT_CASES = [
     (1, 1985, 1, 64, 64, None, torch.bfloat16),                     # 32 chunks, the last of one token
     (2, 2303, 2, 128, 128, None, torch.float16),                    # 36 chunks, the last of 63 tokens
-    (1, 2500, 2, 128, 64, [0, 0, 2111, 2112, 2500], torch.bfloat16)])   # an empty sequence, one of a token, uneven ones
+    (1, 2500, 2, 128, 64, [0, 0, 2111, 2112, 2500], torch.bfloat16),    # an empty sequence, one of a token, uneven ones
+    (1, 2300, 2, 64, 128, [0, 2100, 2300], torch.float16),
+]
+
+
+@pytest.mark.parametrize("heads", [False, True])
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", GRADIENT_CASES)
 def test_gla_cut_state_gradients(device, B, T, H, K, V, bounds, dtype, heads):
     """A reverse scan over cut sequences against the fp32 recurrence (the cases above are cut in the forward only).  The
     tolerances are those of the cases above."""
@@ -169,6 +174,82 @@ def test_gla_cut_state_gradients(device, B, T, H, K, V, bounds, dtype, heads):
     torch.autograd.backward((ro, rht), (do.float(), dht))
     for name, a, r in zip(("dq", "dk", "dv", "dg", "dh0"), leaves, refs):
         assert_close(name, r.grad, a.grad, 2e-2)
+
+
+@pytest.mark.parametrize("B,T,H,K,V,bounds,dtype", GRADIENT_CASES)
+def test_gla_cut_state_gradients_16bit_gates(device, B, T, H, K, V, bounds, dtype):
+    """The same with gates in the dtype of q, k and v."""
+    from fla_amd.ops.gla import chunk_gla
+    N = B if bounds is None else len(bounds) - 1
+    assert _cut(N, T, H, K // 64 * (V // 64), True, bounds, 4)
+    print("cut state gradients, 16-bit gates", B, T, H, K, V, bounds, dtype, flush=True)
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T + 1, dtype=dtype, normalizer=600.0, N=N)
+    g, do, dht = g.to(dtype), torch.randn(B, T, H, V).to(dtype), torch.randn(N, H, K, V) * 0.1
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, h0)]
+    o, ht = chunk_gla(*leaves[:4], initial_state=leaves[4], output_final_state=True, head_first=False,
+                      cu_seqlens=None if bounds is None else torch.tensor(bounds, device=device))
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    refs = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*refs[:4], initial_state=refs[4], output_final_state=True, offsets=bounds)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for name, a, r in zip(("dq", "dk", "dv", "dg", "dh0"), leaves, refs):
+        assert_close(name, r.grad, a.grad, 2e-2)
+
+
+@pytest.mark.parametrize("K,V,dtype", [(64, 64, torch.float16), (128, 128, torch.bfloat16), (64, 128, torch.bfloat16),
+                                       (128, 64, torch.float16)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_gdr_cut_backward_that_reads_w(device, K, V, dtype, gated):
+    """The cut form of the entry that takes w (the operator's own backward reads the tiles) against its uncut form on the
+    same kept tensors.  Where nothing enters from the right, the last segment, they run the same instructions (equal bits).
+    Ahead of it the gradients that enter differ by the order of their fp32 sums and the rounding of the operands; either
+    form may be off the recurrence by 2e-2 (bf16) or an eighth of it, twice that bounds their difference."""
+    from fla_amd import _backend as be
+    from fla_amd.ops.gated_delta_rule.wy_fast import fwd_prepare_scan_operands
+    B, T, H = 2, 2020, 2
+    q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(B, T, H, K, V, seed=5, dtype=dtype, normalizer=200.0))
+    do, dht = torch.randn_like(v), torch.randn_like(h0)
+    lib, p, scale, st, dims = be.lib(), be.ptr, K ** -0.5, be.stream_of(q), (B, T, H, K, V, B)
+    AT, gc, w, Aw = fwd_prepare_scan_operands(k, beta, g if gated else None, keep_w=True)
+    chunks = AT.shape[0]
+    new = lambda *shape: q.new_empty(*shape)
+    o, ht, v_new, hT, Aqk = torch.empty_like(v), torch.empty_like(h0), torch.empty_like(v), new(chunks, H, K * V), torch.empty_like(AT)
+    sp, bufs = _split(q, B, T, H, V // 64, 2, K * V, K * K)
+    back = be.Split()
+    assert lib.fla_scan_split(None, B, T, H, V // 64, 1, 2, ctypes.byref(back), None, None, None)
+    assert (back.nseg, back.sub_chunks, back.ratio, back.slots) == (sp.nseg, sp.sub_chunks, 1, sp.slots) and sp.nseg > 1
+    Mt = torch.empty_like(bufs[1])
+    sp.transitions_t = Mt.data_ptr()
+    print("cut backward from w", K, V, dtype, gated, sp.nseg, sp.sub_chunks, flush=True)
+    be.check(lib.fla_chunk_gated_delta_rule_fwd_scan_split(
+        *map(p, (q, k, v, AT, gc)), None, *map(p, (h0, o, ht, v_new, hT, Aqk)), None, None, ctypes.byref(sp), be.dt(q), *dims, scale,
+        0.0, st), "scan_split")
+    states = torch.empty_like(bufs[0])
+    back.states, back.decays = states.data_ptr(), Mt.data_ptr()
+    results = []
+    for split in (None, back):
+        out = [torch.empty_like(x) for x in (q, k, v, beta, beta, h0)]
+        dv2, dh = torch.empty_like(v), torch.empty_like(hT)
+        head = (*map(p, (q, k, v, w, v_new, beta, gc, Aw, do, dht, hT, Aqk)),)
+        tail = (p(dv2), p(dh), None, None, None, *map(p, out), None, None, None)
+        if split is None:
+            be.check(lib.fla_chunk_gated_delta_rule_bwd(*head, None, *tail, 0, be.dt(q), *dims, scale, st), "bwd")
+        else:
+            be.check(lib.fla_chunk_gated_delta_rule_bwd_split(*head, *tail, ctypes.byref(split), 0, be.dt(q), *dims, scale, st),
+                     "bwd_split")
+        results.append(dict(zip(("dq", "dk", "dv", "dbeta", "dg", "dh0"), out)))
+    torch.cuda.synchronize()
+    last = 64 * sp.sub_chunks * (sp.nseg - 1)
+    assert last < T
+    tol = 4e-2 / (1 if dtype == torch.bfloat16 else 8)
+    for name, a in results[0].items():
+        b = results[1][name]
+        if name == "dg" and not gated:
+            continue
+        if name != "dh0":
+            assert torch.equal(a[:, last:], b[:, last:]), name
+        assert_close(name, a.float().cpu(), b.cpu(), tol)
+    assert not torch.equal(results[0]["dh0"], results[1]["dh0"])   # (so that the comparison tells the two apart)
 
 
 @pytest.mark.parametrize("heads", [False, True])
@@ -356,7 +437,7 @@ def test_tables_of_a_cut_do_not_wait_for_the_device(device, delta):
     from fla_amd.ops.gla import chunk_gla
     from fla_amd.utils import VarlenPlan
     T, bounds = 3200, [0, 1790, 1854, 3200]
-    assert _cut(3, T, 1, 1, False, bounds, 2 * delta) and _cut(3, T, 1, 1 + (not delta), True, bounds, 2 * delta)
+    assert _cut(3, T, 1, 1, False, bounds, 2 * delta) and _cut(3, T, 1, 1, True, bounds, 2 if delta else 4)
     q, k, v, g, beta, _ = (x.to(device) for x in gdr_inputs(1, T, 1, 64, 64, seed=2, normalizer=600.0))
     gk = g[..., None].expand(-1, -1, -1, 64).contiguous()
     q.requires_grad_()
@@ -392,7 +473,7 @@ def test_gla_cut_16bit_gates(device, B, T, H, K, V, bounds, dtype):
     from fla_amd.ops.gla import chunk_gla
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(N, T, H, V // 64, False, bounds) and _cut(N, T, H, V // 32, True, bounds)
+    assert _cut(N, T, H, V // 64, False, bounds)   # (the reverse scan runs uncut: test_gla_cut_state_gradients)
     print("cut, 16-bit gates", B, T, H, K, V, bounds, dtype, flush=True)
     q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=600.0, N=N)
     g, do = g.to(dtype), torch.randn(B, T, H, V).to(dtype)
@@ -551,7 +632,7 @@ def test_cut_states_at_any_float_address(device, op):
     from fla_amd.ops.simple_gla import chunk_simple_gla
     T, K = 2020, 64
     delta = op == "chunk_gated_delta_rule"
-    assert _cut(1, T, 2, 1, False, None, 2 * delta) and _cut(1, T, 2, 1 if delta else 2, True, None, 2 * delta)
+    assert _cut(1, T, 2, 1, False, None, 2 * delta) and _cut(1, T, 2, 1, True, None, 2 if delta else 4)
     q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, T, 2, K, K, seed=4, normalizer=200.0))
     do, dht = torch.randn(v.shape, device=device).to(v.dtype), torch.randn(h0.shape, device=device)
 
