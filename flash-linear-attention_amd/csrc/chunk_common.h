@@ -42,9 +42,8 @@ struct Load<f16> {
 
 // Workgroups of one launch are dealt round-robin to the 8 XCDs by linear id.
 // Renumber so that consecutive logical ids share an XCD (and its L2).  (Workgroup numbers are 32-bit, here and below: a 64-bit
-// division by a number the compiler does not know is 150 dependent instructions, a quarter of a microsecond, and the scans
-// took up to five of them ahead of their first load: reverse delta-rule scan of 32 chunks 58.6 -> 57.0 us, GLA forward of 31
-// chunks 27.1 -> 26.4.)
+// division by a number the compiler does not know is 150 dependent instructions, and the scans took up to five of them
+// ahead of their first load: reverse delta-rule scan of 32 chunks 58.6 -> 57.0 us, GLA forward of 31 chunks 27.1 -> 26.4.)
 FLA_DEVICE uint32_t xcd_remap(uint32_t id, uint32_t total) {
   if (total % 8 != 0) return id;
   return (id % 8) * (total / 8) + id / 8;

@@ -42,8 +42,10 @@ struct RowTile {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int row = (tid + 256 * i) / C8;
-      // nobody reads the gradients soon: they need not push the operands of other workgroups out of the L2
-      // (gdr_bwd_chunk_kernel: 204 -> 198 us)
+      // This launch does not read the gradients again: they need not push the operands of other workgroups out of the L2.
+      // Whole steps with plain stores / with these: gla_bwd_chunk, 4 x 4096 tokens, 16 heads of 128, 474 / 465 us, 2 x 2000
+      // tokens, 32 heads of 64, 117 / 102; gdr_bwd_chunk, the first shape, 527 / 525; a mixing layer of 2 x 2048 tokens, whose
+      // norms and convolutions read them in the next launches, 319.9 / 320.7 (the runs of one side differ by 0.6).
       if (row < L) __builtin_nontemporal_store(reg[i], (v8*)(base + ((uint32_t)row * pitch + col)));
     }
   }
