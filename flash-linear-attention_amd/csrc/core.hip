@@ -62,6 +62,9 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // Whether cutting pays is the longest sequence's chunk periods against those of a segment in the scan and in the first pass
 // and the launches ahead of the scan, fitted to the times below (K = V = 128, uncut / cut in us, launches replayed from a
 // graph; packed batches back to back).  The busier the CUs (triples of sequence, head and slab), the less a cut gains.
+// (The training steps of GLA were read with a forward that also wrote k^ and the score tiles and with per-key gates, those of the
+// delta rule with a forward that wrote w and a reverse scan of 162 us where today's takes 141: today's scans gain a little
+// less from a cut than these figures say.)
 //   GLA: one sequence of 16 heads, 12 and 16 chunks 37.7 / 36.1 and 46.0 / 37.2; four, 16, 20 and 24 chunks 50.4 / 53.5,
 //     59.3 / 61.6 and 68.4 / 65.8, their training steps 145 / 162, 198 / 202 and 237 / 237.
 //   Delta rule: 4 and 8 heads, 24 chunks 45.9 / 44.0 and 46.3 / 45.7; 16 heads, 24, 28, 32 and 40 chunks 48.4 / 51.8, 54.1 /

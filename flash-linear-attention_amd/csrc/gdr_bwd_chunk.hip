@@ -5,8 +5,9 @@
 // What bounds it: bytes.  q, k, v, v_new, do, dv2, Aw and the two states enter once, dq, dk and dv leave once (0.91 GB for
 // 4 x 4096 tokens, 16 heads, K = V = 128); dw, the part of dk that does not go through the inverse and the partial gate
 // gradients stay on the chip, and w is not needed: its gate term is the row sum of w . dw = Aw ((dw k^T) diag beta), whose
-// second factor the WY gradient forms anyway.  191 us there, 4.75 TB/s (a large copy: 5.0), where the two launches it
-// replaces took 200 + 146 us for 1.3 GB; 2 x 2048 tokens 50 us instead of 50 + 39.
+// second factor the WY gradient forms anyway.  191 us there, 4.75 TB/s (a large copy: 5.0; 195 behind the reverse scan, 202
+// inside a training step), where the two launches it replaces took 200 + 146 us for 1.3 GB; 2 x 2048 tokens 50 us instead of
+// 50 + 39.
 #include "chunk_rows.h"
 #include "gdr_bwd_chunk.h"
 

@@ -8,7 +8,8 @@
 // (the pairs of the first sum are formed with the rounded operands of the products, so that they cancel exactly unless they
 // straddle t; see gla_bwd.hip).
 //
-// What bounds it: bytes, 1.0 GB for 4 x 4096 tokens, 16 heads, K = V = 128, in 202 us: 5.0 TB/s, the rate of a large copy.
+// What bounds it: bytes, 1.0 GB for 4 x 4096 tokens, 16 heads, K = V = 128, in 202 us: 5.0 TB/s, the rate of a large copy
+// (208 behind the gradient scan, 216 inside a training step).
 // Before, dv was formed inside the reverse state scan from three tiles the forward kept for it (P, k^ and the gated
 // queries: 128 us, and 20 us more in the forward) and the rest in a launch per 64 key channels (206 us); the scan alone is
 // 70 us.  Sums over time cost VALU cycles here, not LDS or barriers: 3600 vector instructions per wave and item are 214 us,
