@@ -355,17 +355,15 @@ def chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, of
 
 
 def _gla_forward(q, k, v, g, scale, initial_state, output_final_state, offsets, want_A=False, fused=True,
-                 flags_out=None, states_out=None):
+                 flags_out=None):
     """Seq-first forward on 64-aligned head dims.  Returns (o, ht, A); with a list ``flags_out`` the
-    gate-range flags of the fused kernel are appended to it, with a list ``states_out`` the per-chunk
-    states it kept for the backward pass."""
+    gate-range flags of the fused kernel are appended to it."""
     if fused and not want_A and q.shape[-1] in (64, 128):
         if flags_out is None:
-            o, ht = chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets,
-                                        states_out=states_out)
+            o, ht = chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets)
             return o, ht, None
         o, ht, wide = chunk_gla_fwd_fused(q, k, v, g, scale, initial_state, output_final_state, offsets,
-                                          return_flags=True, states_out=states_out)
+                                          return_flags=True)
         flags_out.append(wide)
         return o, ht, None
     plan = VarlenPlan(offsets, BT) if offsets is not None else None
