@@ -191,6 +191,34 @@ def test_causal_conv1d_on_wide_tiles(device, dtype, B, T, D, W):
         assert_close(name, r.grad, d.grad, tol)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,T,D,bias,act", [(130, 15, 1032, True, "silu"), (130, 16, 1032, False, "silu"),
+                                            (130, 17, 1032, False, None), (130, 34, 1032, True, None),
+                                            (2, 2, 8, True, "silu"), (1, 16401, 2056, False, "silu")])
+def test_causal_conv1d_at_tile_edges(device, dtype, B, T, D, bias, act):
+    """Tiles of 16 and of 8 time steps that end with their sequence, one step before and behind its end; rows of channels
+    that end inside a workgroup; the last case takes the forward's 8 x 4 tiles in 16 bits."""
+    from fla_amd.modules.convolution import causal_conv1d as conv
+    from oracle.modules import causal_conv1d
+    gen = torch.Generator().manual_seed(T)
+    W = 4
+    x, dy = (torch.randn(B, T, D, generator=gen).to(dtype) for _ in range(2))
+    w, b = torch.rand(D, W, generator=gen) - 0.5, torch.randn(D, generator=gen) if bias else None
+    print("short conv at tile edges", dtype, B, T, D, bias, act, flush=True)
+    leaves = [None if t is None else t.to(device).requires_grad_() for t in (x, w, b)]
+    y = conv(*leaves, act)
+    y.backward(dy.to(device))
+    refs = [None if t is None else t.float().requires_grad_() for t in (x, w, b)]
+    yr = causal_conv1d(*refs, act)
+    yr.backward(dy.float())
+    ft, bt = _tols(dtype)
+    sums = 2e-3 if dtype != torch.float32 else 2e-5   # fp32 sums over B T terms
+    assert_close("y", yr, y, ft)
+    for name, r, d, tol in zip(("dx", "dw", "db"), refs, leaves, (bt, sums, sums)):
+        if r is not None:
+            assert_close(name, r.grad, d.grad, tol)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W", [2, 3, 4])
 @pytest.mark.parametrize("T,D,bias,act", [(1, 64, False, "silu"), (5, 64, True, "silu"), (64, 200, False, None),
