@@ -2,9 +2,9 @@
 // K K^T blocks and their triangular solve, the state scan and the output in a single pass over q, k, v.
 // Nothing but o and the final state is written; no per-chunk tile crosses HBM.
 //
-// The workgroup is the one of gdr_fwd_scan_kernel (gdr_fwd_fused.hip): 8 waves per (sequence, head, 64 value
-// columns), waves 4-7 staging q, k, v and the per-row scalars of the coming chunks, waves 0-3 each carrying 16
-// value columns of the fp32 state in accumulators, one LDS-only barrier per chunk.  What differs is where the
+// A workgroup of 8 waves per (sequence, head, 64 value columns): waves 4-7 staging q, k, v and the per-row scalars of the
+// coming chunks, waves 0-3 each carrying 16 value columns of the fp32 state in accumulators and all products of these
+// columns, one LDS-only barrier per chunk.  What differs from the two-launch forward (gdr_fwd_fused.hip) is where the
 // WY operator of a chunk comes from.  With M = strict_lower(diag(beta) K K^T * Gamma), Gamma_ij = e^{gamma_i -
 // gamma_j} (fla/ops/gated_delta_rule/wy_fast.py:150-208), the scan needs
 //     v_new = (I + M)^-1 diag(beta) (v - e^{gamma} * (k h))          (= u - e^{gamma} (w h), chunk_delta_h.py:101-110)

@@ -517,6 +517,44 @@ def test_chunk_gdr_slab_width_independence(device):
     assert_close("ht[3,11]", rht, ht4[b:b + 1, h:h + 1], TOL_HT)
 
 
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("lens", [(1,), (64,), (65, 0, 63), (128,), (129, 192), (256, 1, 200)])
+def test_chunk_gdr_scan_lengths_in_both_slab_widths(device, K, lens):
+    """The scan's pipeline at its ends: one to four chunks, whole and short last ones, an empty sequence, in 32-column slabs (two
+    heads) and in 64-column ones (72 heads: 288 slabs of 32), plain, with q and k normalised, with everything kept (gradients)
+    and without the delta rule (chunk_simple_gla).  Both widths form the same sums: bit for bit; the narrow one against the
+    recurrence with the tolerances of the other tests."""
+    from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    from oracle.recurrent import naive_recurrent_gated_delta_rule, naive_recurrent_gla
+    H, V, N, T = 72, 128, len(lens), sum(lens)
+    q, k, v, g, beta, h0 = gdr_inputs(1, T, H, K, V, seed=83, N=N)
+    ends = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist())
+    print(f"gdr scan lengths K={K} {lens}", flush=True)
+    gen = torch.Generator().manual_seed(84)
+    do, dht = torch.randn(1, T, H, V, generator=gen).bfloat16(), torch.randn(N, H, K, V, generator=gen) * 0.1
+    run = {}
+    for heads in (H, 2):
+        x = [t[:, :, :heads].contiguous().to(device) for t in (q, k, v, g, beta)]
+        kw = dict(initial_state=h0[:, :heads].contiguous().to(device), output_final_state=True, cu_seqlens=ends.to(device),
+                  head_first=False)
+        out = list(chunk_gated_delta_rule(*x, **kw)) + list(chunk_gated_delta_rule(*x, use_qk_l2norm_in_kernel=True, **kw))
+        out += list(chunk_simple_gla(*x[:4], **kw))
+        x = [t.requires_grad_() for t in x]
+        o, ht = chunk_gated_delta_rule(*x, **kw)
+        torch.autograd.backward((o, ht), (do[:, :, :heads].to(device), dht[:, :heads].to(device)))
+        run[heads] = out + [o.detach(), ht.detach()] + [t.grad for t in x]
+        torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(run[H], run[2])):
+        assert torch.equal(a[:, :2] if a.dim() == 4 and a.shape[0] == N and a.shape[1] == H else a[:, :, :2], b), i
+    sl = [t[:, :, :2] for t in (q, k, v, g, beta)]
+    kw = dict(initial_state=h0[:, :2], output_final_state=True, offsets=ends.tolist())
+    for name, ref, got in (("delta", naive_recurrent_gated_delta_rule(*sl, **kw), run[2][:2]),
+                           ("simple", naive_recurrent_gla(*sl[:3], sl[3][..., None].expand(1, T, 2, K), **kw), run[2][4:6])):
+        assert_close(name + " o", ref[0], got[0], TOL_O)
+        assert_close(name + " ht", ref[1], got[1], TOL_HT)
+
+
 def test_chunk_gdr_slab_width_independence_backward(device):
     """The same for a forward that keeps its intermediates and the backward that reads them: gradients of the
     batch stacked twice (64-column slabs) equal those of the batch alone (32-column slabs) bit for bit, except the
