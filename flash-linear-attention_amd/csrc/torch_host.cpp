@@ -905,15 +905,18 @@ PyObject* py_conv(PyObject*, PyObject* const* p, Py_ssize_t n) {
 }
 
 // causal_conv1d_update(x [B,D], cache [B,D,W], weight, bias | None, silu): the cache is updated in place
+// short_conv_step: the same for x [B,1,D], as the module gets it (a squeeze and an unsqueeze around a launch of 2.5 us cost the
+// host 2 us)
+template <bool STEP>
 PyObject* py_conv_update(PyObject*, PyObject* const* p, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   expect(n, 5);
   const Tensor x = arg_tensor(p[0]), cache = arg_tensor(p[1]), w = arg_tensor(p[2]), b = arg_tensor(p[3]);
-  if (!x.defined() || !cache.defined() || !x.is_cuda() || !cache.is_cuda() || x.dim() != 2 || x.numel() == 0 ||
-      !(is16(x) || x.scalar_type() == at::kFloat) || !conv_weights_ok(w, b, x.size(1)))
+  if (!x.defined() || !cache.defined() || !x.is_cuda() || !cache.is_cuda() || x.dim() != (STEP ? 3 : 2) || x.numel() == 0 ||
+      (STEP && x.size(1) != 1) || !(is16(x) || x.scalar_type() == at::kFloat) || !conv_weights_ok(w, b, x.size(-1)))
     return none();
   if (has_tangent({&x, &cache, &w, &b})) return none();   // (the wrapper refuses it)
-  const int64_t B = x.size(0), D = x.size(1), W = w.size(-1);
+  const int64_t B = x.size(0), D = x.size(-1), W = w.size(-1);
   if (cache.dim() != 3 || cache.size(0) != B || cache.size(1) != D || cache.size(2) != W || !cache.is_contiguous() ||
       cache.scalar_type() != x.scalar_type())
     return none();
@@ -955,7 +958,8 @@ PyMethodDef kMethods[] = {
     ENTRY("recurrent_gdr", py_recurrent_gdr),
     ENTRY("l2_norm", py_l2_norm),
     ENTRY("causal_conv1d", py_conv),
-    ENTRY("causal_conv1d_update", py_conv_update),
+    ENTRY("causal_conv1d_update", py_conv_update<false>),
+    ENTRY("short_conv_step", py_conv_update<true>),
     ENTRY("norm_swish_gate", py_norm_gate),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fla_host", nullptr, -1, kMethods};

@@ -111,12 +111,12 @@ class ShortConvolution(nn.Conv1d):
     def forward(self, x: torch.Tensor, mask: Optional[torch.Tensor] = None, cache: Optional[torch.Tensor] = None,
                 output_final_state: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
         """``x`` [B,T,D]; ``cache`` [B,D,W] is updated in place; returns ``(y [B,T,D], cache)``."""
-        batch_size, _, hidden_size = x.shape
+        batch_size, length, hidden_size = x.shape
         if mask is not None:
             x = x.mul_(mask.unsqueeze(-1))
         if output_final_state and cache is None:
             cache = x.new_zeros(batch_size, hidden_size, self.kernel_size[0])
-        if cache is not None and x.shape[1] == 1:
+        if cache is not None and length == 1:
             return self.step(x, cache)
         if cache is not None:
             cache.copy_(F.pad(x.transpose(1, 2), (self.kernel_size[0] - x.shape[1], 0)))
@@ -125,6 +125,9 @@ class ShortConvolution(nn.Conv1d):
 
     def step(self, x: torch.Tensor, cache: torch.Tensor):
         assert x.shape[1] == 1, "Only support decoding with 1 token at a time for now"
+        y = host().short_conv_step(x, cache, self.weight, self.bias, _act_flag(self.activation))
+        if y is not None:
+            return y, cache
         y = causal_conv1d_update(x.squeeze(1), cache, self.weight, self.bias, self.activation)
         return y.unsqueeze(1), cache
 

@@ -278,6 +278,28 @@ def test_short_convolution_step(device, dtype, W):
     assert torch.equal(cache, x[:, -W:].transpose(1, 2))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_short_convolution_step_is_the_update(device, dtype):
+    """The module's step takes [B,1,D] as it comes, slices of a longer tensor and inputs with gradients among them, and is
+    causal_conv1d_update of its rows bit for bit; forward-mode tangents are refused as there."""
+    import torch.autograd.forward_ad as fwd
+    from fla_amd.modules import ShortConvolution
+    from fla_amd.modules.convolution import causal_conv1d_update
+    gen = torch.Generator().manual_seed(10)
+    B, D, W = 3, 40, 4
+    x = torch.randn(B, 5, D, generator=gen).to(dtype).to(device).requires_grad_()
+    conv = ShortConvolution(D, W, bias=True).to(device).to(dtype)
+    c0 = torch.randn(B, D, W, generator=gen).to(dtype).to(device)
+    got, want = c0.clone(), c0.clone()
+    for t in range(5):
+        y, cache = conv(x[:, t:t + 1], cache=got)
+        ref = causal_conv1d_update(x[:, t], want, conv.weight, conv.bias, "silu")
+        assert cache is got and y.shape == (B, 1, D) and not y.requires_grad
+        assert torch.equal(y[:, 0], ref) and torch.equal(got, want)
+    with fwd.dual_level(), pytest.raises(NotImplementedError):
+        conv(fwd.make_dual(x[:, :1].detach(), torch.ones_like(x[:, :1])), cache=got)
+
+
 @pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32),
                                              (torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize("normalizer,clamp_min", [(16.0, None), (1.0, None), (0.05, None), (16.0, -0.05)])
