@@ -108,17 +108,75 @@ FLA_DEVICE void wy_stage_t(T* dstT, const typename Elem<T>::v4* reg, const float
   }
 }
 
-// One step of the forward substitution of wy_invert: x[c] += nm[J] * (x[c] of lane J of this DPP row), c <= J.
+// One step of the forward substitution of wy_invert: x[c] += nm[J] * (x[c] of lane J of this DPP row), c <= J, each update one
+// instruction (the compiler makes a move and a multiply-add of it, and waits between them: 240 instructions and 110 waits
+// instead of 120 in all).  A register written by the vector ALU is read through DPP two instructions later at the earliest:
+// step J - 1 wrote x[c] J instructions ago, and the wait in front covers the first steps.
 template <int J>
 FLA_DEVICE void wy_subst_step(float (&x)[16], const float (&nm)[16]) {
-#pragma unroll
-  for (int c = 0; c <= J; ++c) x[c] = fmaf(nm[J], dpp_f32<0x150 + J>(x[c]), x[c]);   // row_newbcast:J
+#define FLA_STEP(c) "v_fmac_f32_dpp %" #c ", %" #c ", %[m] row_newbcast:%[j] row_mask:0xf bank_mask:0xf\n\t"
+  if constexpr (J == 0)
+    asm("s_nop 1\n\t" FLA_STEP(0) : "+v"(x[0]) : [m] "v"(nm[0]), [j] "i"(0));
+  if constexpr (J == 1)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) : "+v"(x[0]), "+v"(x[1]) : [m] "v"(nm[1]), [j] "i"(1));
+  if constexpr (J == 2)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]) : [m] "v"(nm[2]), [j] "i"(2));
+  if constexpr (J == 3)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : [m] "v"(nm[3]), [j] "i"(3));
+  if constexpr (J == 4)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]) : [m] "v"(nm[4]), [j] "i"(4));
+  if constexpr (J == 5)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]) : [m] "v"(nm[5]), [j] "i"(5));
+  if constexpr (J == 6)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]) : [m] "v"(nm[6]), [j] "i"(6));
+  if constexpr (J == 7)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]) : [m] "v"(nm[7]), [j] "i"(7));
+  if constexpr (J == 8)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]) : [m] "v"(nm[8]), [j] "i"(8));
+  if constexpr (J == 9)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]) : [m] "v"(nm[9]), [j] "i"(9));
+  if constexpr (J == 10)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]) : [m] "v"(nm[10]), [j] "i"(10));
+  if constexpr (J == 11)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]) : [m] "v"(nm[11]), [j] "i"(11));
+  if constexpr (J == 12)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]) : [m] "v"(nm[12]), [j] "i"(12));
+  if constexpr (J == 13)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) FLA_STEP(13) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]) : [m] "v"(nm[13]), [j] "i"(13));
+  if constexpr (J == 14)
+    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) FLA_STEP(13) FLA_STEP(14) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]) : [m] "v"(nm[14]), [j] "i"(14));
+#undef FLA_STEP
   if constexpr (J < 14) wy_subst_step<J + 1>(x, nm);
 }
 
-// X = (I + M)^-1 for a strictly lower triangular fp32 M [64][LDM] in LDS, into sX [64][LDM]
-// (lower triangle valid; the upper right quadrant is used as scratch and holds garbage afterwards).
-// 16x16 diagonal blocks by forward substitution, then block merges X_ba = -X_bb (M_ba X_aa) on the
+// The 16x16 diagonal blocks of X = (I + M)^-1 for a strictly lower triangular fp32 M [64][LDM] in LDS, by forward
+// substitution, all four at once on one wave: DPP row b is block b, a lane holds row i of its block of M (zero on and above
+// the diagonal) and of X.  Step j subtracts M[i][j] X[j][:] from every row; X[j][:] reaches the 16 lanes of the block through
+// row_newbcast:j, so the 120 dependent updates are register-to-register (the order of the products in every entry's sum is j
+// ascending, as a row-by-row substitution forms them).
+FLA_DEVICE void wy_diagonal(const float* sM, float* sX, int lane) {
+  const int b = lane >> 4, i = lane & 15;
+  const float* Mr = sM + (16 * b + i) * LDM + 16 * b;
+  float nm[16], x[16];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 m = *(const f32x4*)&Mr[4 * q];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) nm[4 * q + e] = -m[e];
+  }
+#pragma unroll
+  for (int c = 0; c < 16; ++c) x[c] = (c == i) ? 1.f : 0.f;
+  wy_subst_step<0>(x, nm);
+  float* Xr = sX + (16 * b + i) * LDM + 16 * b;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 o = {x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+    *(f32x4*)&Xr[4 * q] = o;
+  }
+}
+
+// X = (I + M)^-1 into sX [64][LDM] (lower triangle valid; the upper right quadrant is used as scratch and holds garbage
+// afterwards): the diagonal blocks, then block merges X_ba = -X_bb (M_ba X_aa) on the
 // fp32 matrix instruction.  Called by all 256 threads after a barrier behind the writes of M; ends
 // with a barrier, after which X is complete.  The barriers order LDS traffic only.
 FLA_DEVICE void wy_invert(const float* sM, float* sX, int tid) {
@@ -129,31 +187,7 @@ FLA_DEVICE void wy_invert(const float* sM, float* sX, int tid) {
     int blk = e >> 8, i = (e >> 4) & 15, j = e & 15;
     sX[(32 * blk + i) * LDM + 32 * blk + 16 + j] = 0.f;
   }
-  // 16x16 diagonal blocks by forward substitution, all four at once on the first wave: DPP row b is block b,
-  // a lane holds row i of its block of M (zero on and above the diagonal) and of X.  Step j subtracts
-  // M[i][j] X[j][:] from every row; X[j][:] reaches the 16 lanes of the block through row_newbcast:j, so the
-  // 120 dependent updates are register-to-register (the order of the products in every entry's sum is j
-  // ascending, as a row-by-row substitution forms them).
-  if (tid < 64) {
-    const int b = tid >> 4, i = tid & 15;
-    const float* Mr = sM + (16 * b + i) * LDM + 16 * b;
-    float nm[16], x[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f32x4 m = *(const f32x4*)&Mr[4 * q];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) nm[4 * q + e] = -m[e];
-    }
-#pragma unroll
-    for (int c = 0; c < 16; ++c) x[c] = (c == i) ? 1.f : 0.f;
-    wy_subst_step<0>(x, nm);
-    float* Xr = sX + (16 * b + i) * LDM + 16 * b;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f32x4 o = {x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
-      *(f32x4*)&Xr[4 * q] = o;
-    }
-  }
+  if (tid < 64) wy_diagonal(sM, sX, lane);
   lds_barrier();
   // ---- 32x32 diagonal blocks: X_ba = -X_bb (M_ba X_aa) for the block pairs (1,0) and (3,2)
   {
@@ -367,8 +401,10 @@ struct PrepParams {
   float* rk_out;       //      ... and leaves the factors 1 / sqrt(sum k^2 + l2_eps), fp32 [rows, H], for the scan
 };
 
-// resident workgroups per CU (register budget): four, or three for the variant that also writes w and Aw
-constexpr int kPrepResident = 4, kPrepResidentKeep = 3;
+// Resident workgroups per CU: as many as the registers hold without spills, for an item is a chain of short phases and only
+// other items fill its gaps (K = 128, 32768 tokens: four 45.8 us, five 43.7; K = 64, 8 x 4096 tokens, 32 heads: four 72.8, five
+// 69.2, six 67.0; five where Aw is kept and K = 128 spill, 31.5 -> 33.7).
+constexpr int prep_resident(int K, int kept) { return kept == 2 ? 3 : K == 64 ? (kept ? 5 : 6) : kept ? 4 : 5; }
 FLA_DEVICE int tri_block(int tt, int jb) { return tt * (tt + 1) / 2 + jb; }
 
 // A workgroup walks several (chunk, head) items (grid-stride) and loads the k rows, beta and the gate
@@ -384,7 +420,7 @@ FLA_DEVICE int tri_block(int tt, int jb) { return tt * (tt + 1) / 2 + jb; }
 // k^ k^T = diag(r) (k k^T) diag(r) and the factors go onto the rows and columns of the product; r comes from the
 // pieces the lanes hold anyway (a row of K elements sits in K / 8 adjacent lanes) and is left in memory for the scan.
 template <typename T, int K, int KEPT, bool L2N = false>
-__global__ __launch_bounds__(256, KEPT == 2 ? kPrepResidentKeep : kPrepResident) void gdr_fwd_prep_kernel(PrepParams p, int64_t total) {
+__global__ __launch_bounds__(256, prep_resident(K, KEPT)) void gdr_fwd_prep_kernel(PrepParams p, int64_t total) {
   constexpr bool KEEP = KEPT == 2;
   static_assert(!(KEPT && L2N), "a forward that keeps w and Aw takes normalised keys");
   typedef typename Elem<T>::v8 v8;
@@ -392,18 +428,17 @@ __global__ __launch_bounds__(256, KEPT == 2 ? kPrepResidentKeep : kPrepResident)
   constexpr int LDK = K + 8;
   constexpr int CG = K / 4, RG = 256 / CG, RPT = BT / RG;
   constexpr int R_BYTES = BT * LDK * 2 > BT * LDM * 4 ? BT * LDK * 2 : BT * LDM * 4;
-  __shared__ __attribute__((aligned(16))) char sRA[R_BYTES];   // k row-major -> M (fp32) -> packed Tu tile
-  __shared__ __attribute__((aligned(16))) char sRB[R_BYTES];   // X (fp32) -> KEEP: k row-major again
+  __shared__ __attribute__((aligned(16))) char sRA[R_BYTES];   // k row-major -> M (fp32) -> X -> KEEP: Aw diag(beta)
+  __shared__ __attribute__((aligned(16))) char sRB[KEEP ? R_BYTES : 16];   // KEEP: k row-major again
   __shared__ __attribute__((aligned(16))) float sBeta[BT];
   __shared__ __attribute__((aligned(16))) float sGam[BT];
   __shared__ __attribute__((aligned(16))) float sRk[L2N ? BT : 4];   // L2N: 1 / |k_t| (zero past the end of the chunk)
   T* sK = (T*)sRA;
   float* sM = (float*)sRA;
   T* sK2 = (T*)sRB;
-  T* sTu = (T*)sRA;
-  T* sAb = (T*)sRA + kTriElems;   // KEEP: Aw diag(beta), row-major [64][LDT], behind the packed tile
-  static_assert((kTriElems + BT * LDT) * 2 <= R_BYTES, "region A holds the packed tile and Aw diag(beta)");
-  float* sX = (float*)sRB;
+  T* sAb = (T*)sRA;   // KEEP: Aw diag(beta), row-major [64][LDT]
+  static_assert(BT * LDT * 2 <= R_BYTES, "region A holds Aw diag(beta)");
+  float* sX = sM;   // block by block, each when nobody reads that block of M any more
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int H = p.H;
@@ -546,7 +581,7 @@ __global__ __launch_bounds__(256, KEPT == 2 ? kPrepResidentKeep : kPrepResident)
         for (int e = 0; e < 4; ++e) sM[(ib + e) * LDM + j] = (j < ib + e) ? b[e] * s[4 * r4 + e] : 0.f;
       }
     }
-    lds_barrier();  // M complete; region B becomes X
+    lds_barrier();  // M complete
     // the next item's rows start their way to the registers now: the matrix products above no longer
     // hold their accumulators, and the inversion below needs few registers and no memory
     v8 kkeep[KEEP ? NPL : 1];
@@ -559,67 +594,111 @@ __global__ __launch_bounds__(256, KEPT == 2 ? kPrepResidentKeep : kPrepResident)
       fetch(cur);
     }
 
-    wy_invert(sM, sX, tid);
-
-    // ---- Tu = (X * Gamma) diag(beta): the ten 16x16 blocks of the lower triangle are dealt to the waves; a lane
-    // holds four adjacent columns of one row, and a block leaves for memory as 512 contiguous bytes straight
-    // from the registers (the packed tile is never staged)
-    {
-      const int wv = __builtin_amdgcn_readfirstlane(wave);
-      const int r = lane >> 2, c4 = 4 * (lane & 3);
-      T* at = (T*)p.AT + (cglob * H + hh) * (int64_t)kTriElems;
+    // ---- X = (I + M)^-1 and Tu = (X * Gamma) diag(beta), 16x16 block by block.  The last wave inverts the diagonal blocks D and
+    // finishes them; wave a forms block column a below the diagonal, from the top,
+    //   X_ba = -D_b S_ba,   S_ba = sum_{a <= c < b} M_bc X_ca
+    // on the fp32 matrix instruction, without the other waves: an accumulator (lane (g, c): rows 4 g .. + 3 of column c) is the
+    // right operand of the next product as it is, its register s going with column 4 g + s of the left one.  A finished block
+    // crosses the wave's own part of LDS, after which a lane has four adjacent columns of row lane / 4: 16 lanes store 128 bytes
+    // on end.  (Merges of 32x32 and 64x64 blocks through LDS, a barrier between any two, and the tile formed after them took
+    // 4100 cycles of an item's 10,000.  With that, X in the place of M and the registers and LDS for more workgroups, 32768 packed
+    // tokens of 16 heads of 128 52 -> 43.7 us, 8 x 4096 tokens of 32 heads of 64 83.6 -> 67, and where Aw is kept, 4 x 4096 tokens
+    // of 16 heads, 32.2 -> 31.5.)
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    int fl = lane;   // (an opaque copy: addresses formed from it are formed here, not kept in registers over the walk)
+    asm volatile("" : "+v"(fl));
+    const int c = fl & 15, g = fl >> 4, orow = fl >> 2, oc4 = 4 * (fl & 3);
+    T* at = (T*)p.AT + (cglob * H + hh) * (int64_t)kTriElems;
+    [[maybe_unused]] char* awb = KEPT ? (char*)p.Aw + (row0 * H + hh) * (int64_t)BT * 2 : nullptr;
+    [[maybe_unused]] const uint32_t awl = ((uint32_t)orow * (uint32_t)H * BT + (uint32_t)oc4) * 2u, awr = (uint32_t)H * BT * 32u;
+    v4 ab[KEEP ? 4 : 1];   // KEEP: this wave's blocks of Aw diag(beta)
+    auto finish = [&](int b, int a, int n) __attribute__((always_inline)) {
+      const f32x4 x = *(const f32x4*)&sX[(16 * b + orow) * LDM + 16 * a + oc4];
+      const f32x4 gj = *(const f32x4*)&sGam[16 * a + oc4], bj = *(const f32x4*)&sBeta[16 * a + oc4];
+      const float gi = sGam[16 * b + orow];
+      v4 tu;
+      // (on the diagonal X is zero above it; the exponent there is set to zero so that the product stays zero)
 #pragma unroll
-      for (int pass = 0; pass < 3; ++pass) {
-        const int idx = wv + 4 * pass;          // tri_block(tt, jb)
-        if (idx < 10) {
-          const int tt = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-          const int jb = idx - tt * (tt + 1) / 2;
-          const int i = 16 * tt + r, j0 = 16 * jb + c4;
-          const f32x4 xv = *(const f32x4*)&sX[i * LDM + j0];
-          const f32x4 gj = *(const f32x4*)&sGam[j0];
-          const f32x4 bj = *(const f32x4*)&sBeta[j0];
-          const float gi = sGam[i];
-          // X is zero above the diagonal of a diagonal block; the exponent there is set to zero so that the product stays zero
-          const f32x4 x = xv;
-          v4 tu;
+      for (int r = 0; r < 4; ++r) tu[r] = (T)(x[r] * __expf(a != b || oc4 + r <= orow ? gi - gj[r] : 0.f) * bj[r]);
+      *(v4*)(at + tri_block(b, a) * 256 + 4 * fl) = tu;
+      if constexpr (KEPT) {
+        v4 aw;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float d = gi - gj[e];
-            tu[e] = (T)(x[e] * __expf(tt != jb || c4 + e <= r ? d : 0.f) * bj[e]);
-          }
-          *(v4*)(at + idx * 256 + 4 * lane) = tu;
-          if constexpr (KEPT) {
-            // Aw row piece to memory; Aw diag(beta) as a row-major 16-bit tile in region A (M is dead)
-            v4 aw, ab;
+        for (int r = 0; r < 4; ++r) aw[r] = (T)x[r];
+        if (16 * b + orow < L) *(v4*)(awb + (awl + (uint32_t)b * awr + 32u * a)) = aw;
+        if constexpr (KEEP) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              aw[e] = (T)x[e];
-              ab[e] = (T)(x[e] * bj[e]);
-            }
-            if constexpr (KEEP) *(v4*)&sAb[i * LDT + j0] = ab;
-            if (i < L) *(v4*)((T*)p.Aw + ((row0 + i) * H + hh) * (int64_t)BT + j0) = aw;
-          }
+          for (int r = 0; r < 4; ++r) ab[n][r] = (T)(x[r] * bj[r]);
         }
       }
-      if constexpr (KEPT) {
-        // the blocks above the diagonal of Aw and of Aw diag(beta) are zero
-        const v4 z4 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
+    };
+    auto rows_of = [&](const float* m, int b, int a) __attribute__((always_inline)) {   // row c of block (b, a), columns 4 g ..
+      return *(const f32x4*)&m[(16 * b + c) * LDM + 16 * a + 4 * g];
+    };
+    auto mm = [](f32x4 l, f32x4 r, f32x4 acc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-          const int u = wv + 4 * pass;          // the six blocks (tt, jb), jb > tt
-          if (u < 6) {
-            const int tt = u >= 5 ? 2 : u >= 3 ? 1 : 0;
-            const int jb = u - (tt == 0 ? 0 : tt == 1 ? 3 : 5) + tt + 1;
-            const int i = 16 * tt + r, j0 = 16 * jb + c4;
-            if constexpr (KEEP) *(v4*)&sAb[i * LDT + j0] = z4;
-            if (i < L) *(v4*)((T*)p.Aw + ((row0 + i) * H + hh) * (int64_t)BT + j0) = z4;
-          }
-        }
+      for (int s4 = 0; s4 < 4; ++s4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(l[s4], r[s4], acc, 0, 0, 0);
+      return acc;
+    };
+    auto column = [&](auto which) __attribute__((always_inline)) {
+      constexpr int A = decltype(which)::value;
+      f32x4 m[4][4];
+#pragma unroll
+      for (int b = A + 1; b < 4; ++b)
+#pragma unroll
+        for (int cc = A; cc < b; ++cc) m[b][cc] = rows_of(sM, b, cc);
+      lds_barrier();   // the diagonal blocks of X are in their places, M below them is in registers
+      f32x4 x[4], d[4];   // the blocks of this column so far, rows 4 g .. of column c
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[A][r] = sX[(16 * A + 4 * g + r) * LDM + 16 * A + c];
+#pragma unroll
+      for (int b = A + 1; b < 4; ++b) d[b] = rows_of(sX, b, b);
+#pragma unroll
+      for (int b = A + 1; b < 4; ++b) {
+        f32x4 sum = zero4();
+#pragma unroll
+        for (int cc = A; cc < b; ++cc) sum = mm(m[b][cc], x[cc], sum);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] = -sum[r];
+        x[b] = mm(d[b], sum, zero4());
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sX[(16 * b + 4 * g + r) * LDM + 16 * A + c] = x[b][r];
+        finish(b, A, b - A - 1);
+      }
+    };
+    if (wv == 0) column(std::integral_constant<int, 0>{});
+    else if (wv == 1) column(std::integral_constant<int, 1>{});
+    else if (wv == 2) column(std::integral_constant<int, 2>{});
+    else {
+      wy_diagonal(sM, sX, fl);
+      lds_barrier();
+#pragma unroll
+      for (int b = 0; b < 4; ++b) finish(b, b, b);
+    }
+    const v4 z4 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
+    if constexpr (KEPT) {
+      if (wv == 2) {   // the blocks above the diagonal of Aw are zero
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+          for (int a = b + 1; a < 4; ++a)
+            if (16 * b + orow < L) *(v4*)(awb + (awl + (uint32_t)b * awr + 32u * a)) = z4;
       }
     }
     if constexpr (KEEP) {
-      lds_barrier();   // X fully consumed
-      // its storage takes k row-major again (rows past the end of the chunk zero)
+      lds_barrier();   // M and X fully consumed: Aw diag(beta) row-major takes the place of M ...
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const int b = wv == 3 ? n : wv + 1 + n, a = wv == 3 ? n : wv;
+        if (b < 4) *(v4*)&sAb[(16 * b + orow) * LDT + 16 * a + oc4] = ab[n];
+      }
+      if (wv == 2) {
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+          for (int a = b + 1; a < 4; ++a) *(v4*)&sAb[(16 * b + orow) * LDT + 16 * a + oc4] = z4;
+      }
+      // ... and k row-major again the other region (rows past the end of the chunk zero)
 #pragma unroll
       for (int i = 0; i < NPL; ++i) {
         const int row = r0 + RPP * i;
@@ -1212,7 +1291,7 @@ template <typename T>
 int launch_prep(const PrepParams& p, int K, dim3 chunk_grid_, hipStream_t st) {
   // (chunk, head) items, head-fastest; as many workgroups as are resident at once, each walking its share of the items
   const int64_t total = (int64_t)chunk_grid_.x * chunk_grid_.y;
-  const int64_t resident = (p.w ? kPrepResidentKeep : kPrepResident) * kNumCUs;
+  const int64_t resident = prep_resident(K, p.w ? 2 : p.Aw ? 1 : 0) * kNumCUs;
   dim3 grid((unsigned)(total < resident ? total : resident));
   if (p.l2_eps >= 0.f) {
     if (p.w) return FLA_E_UNSUPPORTED;
