@@ -11,7 +11,7 @@
 //                        states-keeping forward left: no prefix sums, no exponentials, 16-byte row pieces.
 //   gla_bwd_chunk_kernel (gla_bwd_chunk.hip) per (chunk, head):  dq, dk, dv and dg from q, k, v, the gates, do, h_c and dH_c.
 //                        As in the forward, one reference point per chunk replaces the 16x16 sub-block scheme.
-//   gla_bwd_intra_exact_kernel  the score terms of chunks whose gates leave the range of one reference point
+//                        The score terms of chunks whose gates leave its range are added behind the last item.
 #include <type_traits>
 
 #include "chunk_common.h"
@@ -363,202 +363,6 @@ __global__ __launch_bounds__(256) void gla_bwd_dh_kernel(BDhParams p) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Intra-chunk part of the backward for chunks whose cumulative log-gate leaves the range in
-// which one reference point per chunk is exact.  gla_bwd_chunk_kernel
-// leaves the score terms of such chunks out; this kernel adds them with pairwise exponents
-// G_i - G_j <= 0, the arithmetic of the reference's diagonal sub-blocks
-// (fla/ops/gla/chunk.py:409-567):
-//   A_ij  = s sum_k q_ik k_jk e^{G_ik-G_jk},  dA_ij = do_i . v_j            (j <= i)
-//   dv_j += sum_{i>=j} A_ij do_i
-//   dq_ik += s sum_{j<=i} dA_ij k_jk e^{G_ik-G_jk},  dk_jk += s sum_{i>=j} dA_ij q_ik e^{G_ik-G_jk}
-//   dg_ik += sum_{t>=i} (q_tk dq'_tk - k_tk dk'_tk)          (dq', dk': the terms added here)
-// Plain fp32 arithmetic on the vector ALU: it only runs for flagged chunks.
-struct BExactParams {
-  const void* q;
-  const void* k;
-  const void* v;
-  const void* g;
-  const void* dout;
-  const int* wide;
-  void* dq;
-  void* dk;
-  void* dv;
-  float* dg;
-  float* dg_head;
-  const int64_t* offsets;
-  const int64_t* indices;
-  int64_t T;
-  int H, NTfix;
-  float scale;
-  int64_t total;   // (chunk, head) pairs
-};
-
-template <typename T, typename GT, int K, int V>
-__global__ __launch_bounds__(256) void gla_bwd_intra_exact_kernel(BExactParams p) {
-  typedef typename Elem<T>::v4 v4;
-  constexpr int LDG = K + 1, LDQ = K + 8, LDVV = V + 8, LDA = BT + 1;
-  constexpr int VD_BYTES = 2 * BT * LDVV * 2;
-  constexpr int X_BYTES = BT * LDG * 4;
-  const int H = p.H;
-  // A few hundred workgroups walk the (chunk, head) flags (almost always none is set).  The lanes first read
-  // all flags of the workgroup side by side (one memory latency instead of one per flag) and leave if none is set.
-  {
-    int any = 0;
-    for (int64_t lin = blockIdx.x + (int64_t)threadIdx.x * gridDim.x; lin < p.total; lin += (int64_t)256 * gridDim.x)
-      any |= p.wide[lin];
-    if (!__syncthreads_or(any)) return;
-  }
-  for (int64_t lin = blockIdx.x; lin < p.total; lin += gridDim.x) {
-  if (p.wide[lin] == 0) continue;  // workgroup-uniform
-  __syncthreads();                 // the tiles of the previous flagged chunk are free
-  int hh;
-  ChunkLoc cl = locate_chunk_at(lin, p.offsets, p.indices, p.T, p.NTfix, H, &hh);
-  __shared__ float sG[BT * LDG];
-  __shared__ __attribute__((aligned(16))) T sQ[BT * LDQ];
-  __shared__ __attribute__((aligned(16))) T sK[BT * LDQ];
-  __shared__ __attribute__((aligned(16))) char sVD[VD_BYTES > X_BYTES ? VD_BYTES : X_BYTES];  // v | do, later x
-  __shared__ float sA[BT * LDA];
-  __shared__ float sdA[BT * LDA];
-  T* sV = (T*)sVD;
-  T* sDo = sV + BT * LDVV;
-  float* sX = (float*)sVD;
-  const int tid = threadIdx.x;
-  const int L = cl.L;
-  const int64_t row0 = cl.row0;
-  const int64_t strideK = (int64_t)H * K, strideV = (int64_t)H * V;
-  const int64_t baseK = (row0 * H + hh) * (int64_t)K, baseV = (row0 * H + hh) * (int64_t)V;
-
-  for (int e = tid; e < BT * (K / 4); e += 256) {
-    int row = e / (K / 4), c4 = (e % (K / 4)) * 4;
-    float gv[4] = {0.f, 0.f, 0.f, 0.f};
-    v4 qv = {(T)0.f, (T)0.f, (T)0.f, (T)0.f}, kv = qv;
-    if (row < L) {
-      int64_t off = baseK + row * strideK + c4;
-      if constexpr (GateOf<GT>::per_head) {
-        gv[0] = gv[1] = gv[2] = gv[3] = ((const float*)p.g)[(row0 + row) * H + hh];
-      } else {
-        Load<GT>::x4((const GT*)p.g + off, gv);
-      }
-      qv = *(const v4*)((const T*)p.q + off);
-      kv = *(const v4*)((const T*)p.k + off);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sG[row * LDG + c4 + j] = finite_gate(gv[j]);
-    *(v4*)&sQ[row * LDQ + c4] = qv;
-    *(v4*)&sK[row * LDQ + c4] = kv;
-  }
-  for (int e = tid; e < BT * (V / 4); e += 256) {
-    int row = e / (V / 4), c4 = (e % (V / 4)) * 4;
-    v4 vv = {(T)0.f, (T)0.f, (T)0.f, (T)0.f}, dv = vv;
-    if (row < L) {
-      int64_t off = baseV + row * strideV + c4;
-      vv = *(const v4*)((const T*)p.v + off);
-      dv = *(const v4*)((const T*)p.dout + off);
-    }
-    *(v4*)&sV[row * LDVV + c4] = vv;
-    *(v4*)&sDo[row * LDVV + c4] = dv;
-  }
-  __syncthreads();
-  // prefix sums of the gates along time, one channel per thread
-  for (int c = tid; c < K; c += 256) {
-    float run = 0.f;
-    for (int t = 0; t < BT; ++t) {
-      run += sG[t * LDG + c];
-      sG[t * LDG + c] = run;
-    }
-  }
-  __syncthreads();
-  // A and dA, one (i, j) pair at a time
-  for (int e = tid; e < BT * BT; e += 256) {
-    int i = e >> 6, j = e & 63;
-    float a = 0.f, da = 0.f;
-    if (j <= i && i < L) {
-      for (int c = 0; c < K; ++c)
-        a += (float)sQ[i * LDQ + c] * (float)sK[j * LDQ + c] * __expf(sG[i * LDG + c] - sG[j * LDG + c]);
-      for (int c = 0; c < V; ++c) da += (float)sDo[i * LDVV + c] * (float)sV[j * LDVV + c];
-    }
-    sA[i * LDA + j] = a * p.scale;
-    sdA[i * LDA + j] = da * p.scale;
-  }
-  __syncthreads();
-  // dv_j += sum_{i>=j} A_ij do_i
-  for (int e = tid; e < BT * (V / 4); e += 256) {
-    int j = e / (V / 4), c4 = (e % (V / 4)) * 4;
-    if (j >= L) continue;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int i = j; i < L; ++i) {
-      float a = sA[i * LDA + j];
-      v4 d = *(const v4*)&sDo[i * LDVV + c4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) acc[x] += a * (float)d[x];
-    }
-    T* dst = (T*)p.dv + baseV + j * strideV + c4;
-    v4 old = *(const v4*)dst, nw;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) nw[x] = (T)((float)old[x] + acc[x]);
-    *(v4*)dst = nw;
-  }
-  __syncthreads();  // v and do are consumed: their storage becomes x = q dq' - k dk'
-  for (int e = tid; e < BT * (K / 4); e += 256) {
-    int r = e / (K / 4), c4 = (e % (K / 4)) * 4;
-    float xq[4] = {0.f, 0.f, 0.f, 0.f}, xk[4] = {0.f, 0.f, 0.f, 0.f};
-    if (r < L) {
-      float dq[4] = {0.f, 0.f, 0.f, 0.f}, dk[4] = {0.f, 0.f, 0.f, 0.f};
-      float gr[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) gr[x] = sG[r * LDG + c4 + x];
-      for (int j = 0; j <= r; ++j) {       // row r as the query row i
-        float da = sdA[r * LDA + j];
-        v4 kj = *(const v4*)&sK[j * LDQ + c4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) dq[x] += da * (float)kj[x] * __expf(gr[x] - sG[j * LDG + c4 + x]);
-      }
-      for (int i = r; i < L; ++i) {        // row r as the key row j
-        float da = sdA[i * LDA + r];
-        v4 qi = *(const v4*)&sQ[i * LDQ + c4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) dk[x] += da * (float)qi[x] * __expf(sG[i * LDG + c4 + x] - gr[x]);
-      }
-      v4 qr = *(const v4*)&sQ[r * LDQ + c4], kr = *(const v4*)&sK[r * LDQ + c4];
-      T* dqp = (T*)p.dq + baseK + r * strideK + c4;
-      T* dkp = (T*)p.dk + baseK + r * strideK + c4;
-      v4 oq = *(const v4*)dqp, ok = *(const v4*)dkp, nq, nk;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        nq[x] = (T)((float)oq[x] + dq[x]);
-        nk[x] = (T)((float)ok[x] + dk[x]);
-        xq[x] = (float)qr[x] * dq[x];
-        xk[x] = (float)kr[x] * dk[x];
-      }
-      *(v4*)dqp = nq;
-      *(v4*)dkp = nk;
-    }
-#pragma unroll
-    for (int x = 0; x < 4; ++x) sX[r * LDG + c4 + x] = xq[x] - xk[x];
-  }
-  __syncthreads();
-  // dg_ik += sum_{t>=i} x_tk, one channel per thread
-  for (int c = tid; c < K; c += 256) {
-    float run = 0.f;
-    for (int t = L - 1; t >= 0; --t) {
-      run += sX[t * LDG + c];
-      if (p.dg_head) sX[t * LDG + c] = run;
-      else p.dg[baseK + t * strideK + c] += run;
-    }
-  }
-  if (p.dg_head) {
-    // one gate per (token, head): a row's channels are summed in a fixed order, one addition per row
-    __syncthreads();
-    for (int t = tid; t < L; t += 256) {
-      float sum = 0.f;
-      for (int c = 0; c < K; ++c) sum += sX[t * LDG + c];
-      atomicAdd(p.dg_head + (cl.row0 + t) * H + hh, sum);
-    }
-  }
-  }
-}
-
 template <typename T, typename GT>
 int launch_bwd(const void* q, const void* k, const void* v, const void* g, const void* dout, const float* dht,
                const void* hT, const void* qg, const float* decay, void* dhtf, void* dq, void* dk, void* dv, float* dg,
@@ -594,18 +398,7 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* g, const
   }
   rc = gla_bwd_chunk(q, k, v, g, dout, hT, dhtf, wide, dq, dk, dv, GateOf<GT>::per_head ? dg_head : dg, offsets, indices,
                      grid.x, ntfix, kDtype, kGates, GateOf<GT>::per_head, T_, H, K, V, scale, st);
-  if (rc) return rc;
-  if (wide) {
-    BExactParams p{q, k, v, g, dout, wide, dq, dk, dv, dg, dg_head, offsets, indices, T_, (int)H, ntfix, scale,
-                   (int64_t)grid.x * grid.y};
-    const dim3 gx((unsigned)(p.total < 512 ? p.total : 512));
-#define FLA_CASE(KK, VV)                                                                                      \
-  if (K == KK && V == VV) hipLaunchKernelGGL((gla_bwd_intra_exact_kernel<T, GT, KK, VV>), gx, dim3(256), 0, st, p);
-    FLA_CASE(64, 64) else FLA_CASE(128, 128) else FLA_CASE(64, 128) else FLA_CASE(128, 64) else return FLA_E_UNSUPPORTED;
-#undef FLA_CASE
-    FLA_CHECK_LAUNCH();
-  }
-  return FLA_OK;
+  return rc;
 }
 
 }  // namespace

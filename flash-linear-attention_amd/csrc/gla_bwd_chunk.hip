@@ -29,7 +29,7 @@ struct GlaChunkParams {
   const void* dout;
   const void* hT;      // forward states, FLA_H_FRAGMENT_T
   const void* dhtf;    // dH, FLA_H_FRAGMENT_T
-  const int* wide;     // [chunks, H] or NULL: chunks whose score terms (P, dA) are left to the exact kernel
+  const int* wide;     // [chunks, H] or NULL: chunks whose score terms (P, dA) are left to exact_scores()
   void* dq;
   void* dk;
   void* dv;
@@ -52,6 +52,197 @@ FLA_DEVICE X opaque(X x) {
 
 // One fp32 log-gate per (token, head) instead of per-key log-gates of type GT
 struct PerHead {};
+
+// Element (i, j), j <= i, of a 64 x 64 lower triangle of floats
+FLA_DEVICE int tri_at(int i, int j) { return i * (i + 1) / 2 + j; }
+constexpr int kTriFloats = BT * (BT + 1) / 2;
+
+// The score terms of a chunk whose gates leave the range of one reference point, added to what gla_bwd_chunk_kernel left for
+// it: pairwise exponents G_i - G_j <= 0, the arithmetic of the reference's diagonal sub-blocks (fla/ops/gla/chunk.py:409-567):
+//   A_ij  = s sum_k q_ik k_jk e^{G_ik-G_jk},  dA_ij = do_i . v_j            (j <= i)
+//   dv_j += sum_{i>=j} A_ij do_i
+//   dq_ik += s sum_{j<=i} dA_ij k_jk e^{G_ik-G_jk},  dk_jk += s sum_{i>=j} dA_ij q_ik e^{G_ik-G_jk}
+//   dg_ik += sum_{t>=i} (q_tk dq'_tk - k_tk dk'_tk)          (dq', dk': the terms added here)
+// Plain fp32 arithmetic on the vector ALU, by the workgroup that formed the chunk, behind its last item and in the LDS of the
+// items.  A launch of its own took 4 us to find that nothing is flagged: without it a training step of 2 x 2000 tokens, 32
+// heads of 64, takes 97.7 us instead of 100.8, 4 x 4096 tokens, 16 heads of 128, 468 instead of 471, and 2 x 256 tokens, 4
+// heads of 64, host and all, 74.7 instead of 79.  ab, c, d, tri: room for 64 rows of gates and sums over channels (or v and
+// do), for q, for k (or A), for dA.
+template <typename T, typename GT, int K, int V>
+FLA_DEVICE void exact_scores(const GlaChunkParams& p, const ChunkLoc& cl, int hh, char* ab, T* c, T* d, float* tri, float* sGam) {
+  typedef typename Elem<T>::v4 v4;
+  constexpr bool PH = std::is_same<GT, PerHead>::value;
+  typedef typename std::conditional<PH, float, GT>::type GE;
+  constexpr int LDG = K + 1, LDQ = K + 8, LDW = V + 8, NR = BT * (K / 4) / 256;
+  float* sG = (float*)ab;
+  T *sQ = c, *sK = d, *sV = (T*)ab, *sDo = sV + BT * LDW;
+  float *sA = (float*)d, *sdA = tri;
+  // (fresh_tid and loops left rolled: this code must not raise the registers of the kernel it stands in)
+  const int tid0 = threadIdx.x, tid = fresh_tid(tid0), H = p.H, L = cl.L;
+  const int64_t strideK = (int64_t)H * K, strideV = (int64_t)H * V;
+  const int64_t baseK = (cl.row0 * H + hh) * (int64_t)K, baseV = (cl.row0 * H + hh) * (int64_t)V;
+  const v4 z4 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
+  // gates summed along time, q, k; rows past the end of the chunk zero
+  auto load_qkg = [&]() {
+#pragma unroll 1
+    for (int e = tid; e < BT * (K / 4); e += 256) {
+      const int row = e / (K / 4), c4 = (e % (K / 4)) * 4;
+      const int64_t off = baseK + row * strideK + c4;
+      if constexpr (!PH) {
+        float gv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (row < L) Load<GE>::x4((const GE*)p.g + off, gv);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sG[row * LDG + c4 + j] = finite_gate(gv[j]);
+      }
+      *(v4*)&sQ[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.q + off) : z4;
+      *(v4*)&sK[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.k + off) : z4;
+    }
+    if (PH && tid < BT) sGam[tid] = tid < L ? finite_gate(((const float*)p.g)[(cl.row0 + tid) * H + hh]) : 0.f;
+    __syncthreads();
+    float* col = PH ? sGam : sG + tid;
+    constexpr int step = PH ? 1 : LDG;
+    if (tid < (PH ? 1 : K)) {
+      float run = 0.f;
+#pragma unroll 1
+      for (int t = 0; t < BT; ++t) {
+        run += col[t * step];
+        col[t * step] = run;
+      }
+    }
+    __syncthreads();
+  };
+  auto gsum = [&](int row, int ch) { return PH ? sGam[row] : sG[row * LDG + ch]; };
+
+  load_qkg();
+  float a[16];   // A, pairs (i, j) = (4 n + wave, lane)
+  const int j = tid & 63, i0 = tid >> 6;
+#pragma unroll
+  for (int n = 0; n < 16; ++n) {
+    const int t = fresh_tid(tid0), jj = t & 63, i = 4 * n + (t >> 6);
+    float sum = 0.f;
+    if (jj <= i && i < L) {
+#pragma unroll 1
+      for (int ch = 0; ch < K; ++ch)
+        sum += (float)sQ[i * LDQ + ch] * (float)sK[jj * LDQ + ch] * __expf(gsum(i, ch) - gsum(jj, ch));
+    }
+    a[n] = sum;
+  }
+  __syncthreads();   // q, k and the gates make room
+#pragma unroll 1
+  for (int e = tid; e < BT * (V / 4); e += 256) {
+    const int row = e / (V / 4), c4 = (e % (V / 4)) * 4;
+    const int64_t off = baseV + row * strideV + c4;
+    *(v4*)&sV[row * LDW + c4] = row < L ? *(const v4*)((const T*)p.v + off) : z4;
+    *(v4*)&sDo[row * LDW + c4] = row < L ? *(const v4*)((const T*)p.dout + off) : z4;
+  }
+#pragma unroll
+  for (int n = 0; n < 16; ++n)
+    if (j <= 4 * n + i0) sA[tri_at(4 * n + i0, j)] = a[n] * p.scale;
+  __syncthreads();
+#pragma unroll 1
+  for (int n = 0; n < 16; ++n) {
+    const int i = 4 * n + i0;
+    if (j > i) continue;
+    float da = 0.f;
+    if (i < L)
+#pragma unroll 1
+      for (int ch = 0; ch < V; ++ch) da += (float)sDo[i * LDW + ch] * (float)sV[j * LDW + ch];
+    sdA[tri_at(i, j)] = da * p.scale;
+  }
+  // dv_j += sum_{i>=j} A_ij do_i
+#pragma unroll 1
+  for (int e = tid; e < BT * (V / 4); e += 256) {
+    const int r = e / (V / 4), c4 = (e % (V / 4)) * 4;
+    if (r >= L) continue;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int i = r; i < L; ++i) {
+      const float x = sA[tri_at(i, r)];
+      const v4 y = *(const v4*)&sDo[i * LDW + c4];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) acc[z] += x * (float)y[z];
+    }
+    T* dst = (T*)p.dv + baseV + r * strideV + c4;
+    const v4 old = *(const v4*)dst;
+    v4 nw;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) nw[z] = (T)((float)old[z] + acc[z]);
+    *(v4*)dst = nw;
+  }
+  __syncthreads();   // v, do and A are consumed
+  load_qkg();
+  float x[NR][4];    // q dq' - k dk', rows and channels as below
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    const int e = fresh_tid(tid0) + 256 * n, r = e / (K / 4), c4 = (e % (K / 4)) * 4;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) x[n][z] = 0.f;
+    if (r >= L) continue;
+    float dq[4] = {0.f, 0.f, 0.f, 0.f}, dk[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int jj = 0; jj <= r; ++jj) {       // row r as the query row i
+      const float da = sdA[tri_at(r, jj)];
+      const v4 kj = *(const v4*)&sK[jj * LDQ + c4];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) dq[z] += da * (float)kj[z] * __expf(gsum(r, c4 + z) - gsum(jj, c4 + z));
+    }
+#pragma unroll 1
+    for (int i = r; i < L; ++i) {           // row r as the key row j
+      const float da = sdA[tri_at(i, r)];
+      const v4 qi = *(const v4*)&sQ[i * LDQ + c4];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) dk[z] += da * (float)qi[z] * __expf(gsum(i, c4 + z) - gsum(r, c4 + z));
+    }
+    const v4 qr = *(const v4*)&sQ[r * LDQ + c4], kr = *(const v4*)&sK[r * LDQ + c4];
+    T *dqp = (T*)p.dq + baseK + r * strideK + c4, *dkp = (T*)p.dk + baseK + r * strideK + c4;
+    const v4 oq = *(const v4*)dqp, ok = *(const v4*)dkp;
+    v4 nq, nk;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+      nq[z] = (T)((float)oq[z] + dq[z]);
+      nk[z] = (T)((float)ok[z] + dk[z]);
+      x[n][z] = (float)qr[z] * dq[z] - (float)kr[z] * dk[z];
+    }
+    *(v4*)dqp = nq;
+    *(v4*)dkp = nk;
+  }
+  __syncthreads();   // the gates make room for x
+  if constexpr (PH) {
+    // one gate per (token, head): the channels of a row are added up in the K / 4 lanes that hold it
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      float sum = (x[n][0] + x[n][1]) + (x[n][2] + x[n][3]);
+#pragma unroll
+      for (int m = K / 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
+      const int e = tid + 256 * n;
+      if (e % (K / 4) == 0) sGam[e / (K / 4)] = sum;
+    }
+    __syncthreads();
+    if (tid < L) {
+      float run = 0.f;
+#pragma unroll 1
+      for (int t = L - 1; t >= tid; --t) run += sGam[t];
+      p.dg[(cl.row0 + tid) * H + hh] += run;
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      const int e = tid + 256 * n, r = e / (K / 4), c4 = (e % (K / 4)) * 4;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) sG[r * LDG + c4 + z] = x[n][z];
+    }
+    __syncthreads();
+    if (tid < K) {
+      float run = 0.f;
+#pragma unroll 1
+      for (int t = L - 1; t >= 0; --t) {
+        run += sG[t * LDG + tid];
+        p.dg[baseK + t * strideK + tid] += run;
+      }
+    }
+  }
+  __syncthreads();
+}
 
 // Four waves.  In products with K (V) result columns a wave owns 32 of them and, with 128 columns, all 64 rows, with 64
 // columns one half of the rows; such products are formed transposed, so that a lane owns one time row and, per register
@@ -163,7 +354,13 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     TK::put(sD, LDK, L, tid, R.q);
   };
 
-  uint32_t it = xcd_remap(blockIdx.x, gridDim.x);   // adjacent heads of a chunk at the same time on one XCD
+  // room for exact_scores()
+  static_assert(2 * BT * LDV * 2 <= AB && (PH || BT * (K + 1) * 4 <= AB) && BT * (K + 8) <= BT * (LDK > LDV ? LDK : LDV) &&
+                    kTriFloats * 4 <= BT * LDK * 2 && kTriFloats * 4 <= BT * LDT * 2,
+                "tiles of the pairwise score terms");
+  bool any_flagged = false;
+  const uint32_t it0 = xcd_remap(blockIdx.x, gridDim.x);
+  uint32_t it = it0;   // adjacent heads of a chunk at the same time on one XCD
   if (it >= nitems) return;
   Item im = locate(it);
   Raw R;
@@ -174,6 +371,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     const int L = cl.L;
     const int64_t r0h = cl.row0 * H + im.hh;
     const bool flagged = p.wide && p.wide[cl.cglob * H + im.hh];
+    any_flagged |= flagged;
     // what the item needs next: do and v, and the state tiles of this wave's key columns
     v8 rd[TV::N], rv[TV::N], hf[VT32][2], dhf[VT32][2];
     {
@@ -513,6 +711,13 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
     if (!more) break;
     it = nit;
     im = nim;
+  }
+  if (!any_flagged) return;   // workgroup-uniform
+  for (it = it0; it < nitems; it += gridDim.x) {
+    im = locate(it);
+    if (!p.wide[im.cl.cglob * H + im.hh]) continue;
+    __syncthreads();   // (what this workgroup stored is what it reads back)
+    exact_scores<T, GT, K, V>(p, im.cl, im.hh, sAB, sC, sD, (float*)sS, sGam);
   }
 }
 

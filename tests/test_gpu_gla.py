@@ -322,6 +322,51 @@ def test_chunk_gla_backward_chunk_launch_many_items(device, B, K, V, gates):
             assert torch.equal(a[b:b + 4], x), (name, b)
 
 
+@pytest.mark.parametrize("B,K,V", [(26, 64, 64), (20, 128, 64), (20, 64, 128), (20, 128, 128)])
+@pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
+def test_chunk_gla_backward_flagged_items_of_many(device, B, K, V, gates):
+    """The pairwise score terms of flagged chunks, added behind the last item of a workgroup in the tiles of the items: every
+    pair of head dims and every gate type, workgroups with two items of which none, the first, the second or both are flagged
+    (512 and 768 run at once), short second chunks.  A sequence at a time gives the same bits; two heads against the
+    recurrence with the tolerances of the other tests of strong gates."""
+    from fla_amd.ops.gla import chunk as mod
+    T, H, head = 127, 16, gates == "head"
+    q, k, v, g, h0 = gla_inputs(B, T, H, K, V, seed=96, normalizer=16.0, h0_std=1.0)
+    g = g[..., 0].contiguous() if head else g
+    gen = torch.Generator().manual_seed(97)
+    strong = torch.rand(B, H, generator=gen) < 0.4
+    strong[0, 0], strong[0, 1] = True, False
+    g[strong[:, None].expand(B, T, H)] *= 40          # about -130 a chunk
+    g = g if head else g.to(getattr(torch, gates))
+    do, dht = torch.randn(B, T, H, V, generator=gen).bfloat16(), torch.randn(h0.shape, generator=gen)
+    dev = [x.to(device) for x in (q, k, v, g, h0, do, dht)]
+    print(f"chunk_gla backward, flagged ones of {2 * B * H} items K={K} V={V} gates={gates}", flush=True)
+    kept = []
+    _, _, wide = mod.chunk_gla_fwd_fused(*dev[:4], K ** -0.5, dev[4], True, return_flags=True, states_out=kept, head_gates=head,
+                                         khat_and_scores=False)
+    hT, qg, decay = kept
+    wide = wide.view(B, 2, H)
+    assert torch.equal(wide[:, 0].bool().cpu(), strong)
+
+    def backward(s):
+        c = lambda x: x[s].contiguous()
+        return mod.chunk_gla_bwd_device(*(c(x) for x in dev[:4]), K ** -0.5, *(c(x) for x in dev[4:]), None,
+                                        c(wide).view(-1, H), hT=c(hT), qg=c(qg), decay=c(decay), head_gates=head)
+
+    whole = backward(slice(0, B))
+    names = ("dq", "dk", "dv", "dg", "dh0")
+    for b in range(B):
+        for name, a, x in zip(names, whole, backward(slice(b, b + 1))):
+            assert torch.equal(a[b:b + 1], x), (name, b)
+    sl = [x[:1, :, :2] for x in (q, k, v, g)] + [h0[:1, :2], do[:1, :, :2], dht[:1, :2]]
+    ref = [x.float().requires_grad_() for x in sl[:5]]
+    from oracle.recurrent import naive_recurrent_gla
+    ro, rht = naive_recurrent_gla(*ref[:3], **{"g" if head else "gk": ref[3]}, initial_state=ref[4], output_final_state=True)
+    torch.autograd.backward((ro, rht), (sl[5].float(), sl[6]))
+    for name, r, x, tol in zip(names, ref, whole, (1e-2, 1e-2, 1e-2, 2e-2, 5e-3)):
+        assert_close(name, r.grad, x[:1, :2] if name == "dh0" else x[:1, :, :2], tol)
+
+
 @pytest.mark.parametrize("keep", [True, False])
 @pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (64, 128), (128, 64)])
 @pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
