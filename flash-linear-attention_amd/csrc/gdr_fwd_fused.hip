@@ -293,13 +293,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     asm volatile("" ::: "memory");   // the sets are issued one after the other
     load(R1);
     asm volatile("" ::: "memory");
-    load(R2);
-    write(R0);
-    load(R0);
-    lds_barrier();
-    // Iteration c (the chain works on chunk c) writes set c + 1 and loads set c + 4 into the registers just emptied.
-    write(R1);
-    load(R1);
+    // Iteration c (the chain works on chunk c) writes set c + 1 and loads set c + 4 into the registers just emptied.  Where
+    // there is one chunk nothing behind set 1 is wanted (16 sequences of 64 tokens, 32 heads of 128: 39.5 -> 36.6 us).
+    if (nchunks > 1) {
+      load(R2);
+      write(R0);
+      load(R0);
+      lds_barrier();
+      write(R1);
+      load(R1);
+    } else {
+      write(R0);
+      lds_barrier();
+      write(R1);
+    }
     lds_barrier();
     auto iter = [&](Regs& R) __attribute__((always_inline)) {
       write(R);
