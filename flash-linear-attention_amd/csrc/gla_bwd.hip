@@ -127,9 +127,19 @@ __global__ __launch_bounds__(256) void gla_bwd_dh_qg_kernel(BDhParams p) {
         lo[r] = (T)(acc2[r] * scale);
         hi[r] = (T)(acc2[r + 8] * scale);
       }
-      T* o2 = (T*)p.dhtf + blk + (((int64_t)vt32 * (K / 32) + kt32) * 64 + lane) * 16;
-      *(v8*)o2 = lo;
-      *(v8*)(o2 + 8) = hi;
+      // halves of 32 bytes exchanged between the halves of the wave: a store covers 1 KB on end instead of every other 16 bytes
+      // of 2 KB (4 x 4096 tokens, 16 heads of 128: 66.1 -> 58.6 us)
+      typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+      u4 x = __builtin_bit_cast(u4, lo), y = __builtin_bit_cast(u4, hi);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const auto sw = __builtin_amdgcn_permlane32_swap(x[r], y[r], false, false);
+        x[r] = sw[0];
+        y[r] = sw[1];
+      }
+      T* o2 = (T*)p.dhtf + blk + (((int64_t)vt32 * (K / 32) + kt32) * 64 + (lane & 31)) * 16 + 8 * (lane >> 5);
+      *(u4*)o2 = x;
+      *(u4*)(o2 + 32 * 16) = y;
     }
     const v8 z8 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f};
 #pragma unroll
