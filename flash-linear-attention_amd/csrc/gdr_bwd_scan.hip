@@ -210,17 +210,21 @@ __global__ __launch_bounds__(512, K == 64 ? 4 : 2) void gdr_bwd_scan_kernel(BwdS
       *(v8*)&sU[st * 8] = u0;
       *(uint32_t*)&sU[2048 + st * 2] = u1;
     };
-    // dH of chunk c in fragment order: transposing loads turn the 16-bit tile round (a 16-lane group takes a block of 4
-    // value columns x 16 key channels); the K / 32 tiles have two 16-byte pieces per lane of a wave
+    // dH of chunk c in fragment order: transposing loads turn the 16-bit tile round.  The K / 32 tiles have 32 bytes per lane of
+    // a wave; four adjacent lanes of a 16-lane group take the 4 key channels of an 8-byte piece, the group both halves of 8
+    // such 32 bytes, 256 bytes on end (16 bytes of every lane's 32 per store: 127.6 us for 4 x 4096 tokens, 16 heads of 128; so:
+    // 123.1)
     const T *hlo[KT32 / 2], *hhi[KT32 / 2];
     char* hdst[KT32 / 2];
 #pragma unroll
     for (int i = 0; i < KT32 / 2; ++i) {
-      const int pc = (wave - 4) * (KT32 / 2) + i, kt = pc >> 1, half = pc & 1;
-      const int hrow = 16 * half + 4 * (lane >> 5) + ((lane & 15) >> 2), hcol = kt * 32 + (lane & 16) + 4 * (lane & 3);
+      const int pc = (wave - 4) * (KT32 / 2) + i, kt = pc >> 1, x = pc & 1;
+      const int g = lane >> 4, j = lane & 15;
+      const int hrow = 16 * (j & 1) + 4 * x + (j >> 2), hcol = kt * 32 + 8 * g + 2 * (j & 2);
       hlo[i] = &sDHt[swz<K>(hrow, hcol)];
       hhi[i] = &sDHt[swz<K>(hrow + 8, hcol)];
-      hdst[i] = (char*)((T*)p.dhtf + ((chunk0 + c0) * H + hh) * (int64_t)K * V + (((int64_t)vt * KT32 + kt) * 64 + lane) * 16 + 8 * half);
+      hdst[i] = (char*)((T*)p.dhtf + ((chunk0 + c0) * H + hh) * (int64_t)K * V +
+                        (((int64_t)vt * KT32 + kt) * 64 + 32 * x + 8 * g + 4 * (j >> 3) + (j & 3)) * 16 + 8 * ((j >> 2) & 1));
     }
     const int64_t hstep = (int64_t)H * K * V * (int64_t)sizeof(T);
     auto store_dh = [&]() __attribute__((always_inline)) {
