@@ -64,181 +64,270 @@ constexpr int kTriFloats = BT * (BT + 1) / 2;
 //   dq_ik += s sum_{j<=i} dA_ij k_jk e^{G_ik-G_jk},  dk_jk += s sum_{i>=j} dA_ij q_ik e^{G_ik-G_jk}
 //   dg_ik += sum_{t>=i} (q_tk dq'_tk - k_tk dk'_tk)          (dq', dk': the terms added here)
 // Plain fp32 arithmetic on the vector ALU, by the workgroup that formed the chunk, behind its last item and in the LDS of the
-// items.  A launch of its own took 4 us to find that nothing is flagged: without it a training step of 2 x 2000 tokens, 32
-// heads of 64, takes 97.7 us instead of 100.8, 4 x 4096 tokens, 16 heads of 128, 468 instead of 471, and 2 x 256 tokens, 4
-// heads of 64, host and all, 74.7 instead of 79.  ab, c, d, tri: room for 64 rows of gates and sums over channels (or v and
-// do), for q, for k (or A), for dA.
+// items.  ab, c, d, tri: room for 64 rows of gates and sums over channels (or v and do), for q (or do), for k (or A), for dA.
+//
+// What bounds it: with per-key gates 3 x 2080 K exponentials an item and what stands around them, as long as the operands come
+// wide enough and far enough ahead.  Pairs: a thread takes rows a + 16 m and columns b + 16 n, the ten blocks m >= n, so that
+// four channels of eight rows feed forty products and all threads have the same work.  dq and dk: a thread takes four channels
+// of a row, four steps of the sum per trip, the ends of the triangle by selection.
+// Backward with every chunk flagged, us, as a launch of its own with 136 KB of LDS / here, one channel a trip and a single sum /
+// so: fp16, 2 x 2000 tokens, 32 heads of 64, per-key gates 819 / 687 / 412, per head 672 / 535 / 232; bf16, 4 x 4096 tokens, 16
+// heads of 128, per-key 3176 / 3260 / 1568, per head 2728 / 2577 / 928, a chunk in twenty flagged 987 / 1316 / 666; 2 x 256 tokens,
+// 4 heads of 64, one item a workgroup, 120 / 194 / 76.  Where nothing is flagged the launch took 4 us to find that out.
 template <typename T, typename GT, int K, int V>
 FLA_DEVICE void exact_scores(const GlaChunkParams& p, const ChunkLoc& cl, int hh, char* ab, T* c, T* d, float* tri, float* sGam) {
   typedef typename Elem<T>::v4 v4;
   constexpr bool PH = std::is_same<GT, PerHead>::value;
   typedef typename std::conditional<PH, float, GT>::type GE;
-  constexpr int LDG = K + 1, LDQ = K + 8, LDW = V + 8, NR = BT * (K / 4) / 256;
-  float* sG = (float*)ab;
-  T *sQ = c, *sK = d, *sV = (T*)ab, *sDo = sV + BT * LDW;
+  constexpr int LDG = K + 4, LDQ = K + 8, LDW = V + 8;
+  constexpr int RP = 1024 / K, NR = BT / RP;   // rows of K / 4 threads each that stand side by side, and how often
+  float *sG = (float*)ab, *sX = sG;
+  T *sQ = c, *sK = d, *sV = (T*)ab, *sDo = sV + BT * LDW, *sDo2 = c;
   float *sA = (float*)d, *sdA = tri;
-  // (fresh_tid and loops left rolled: this code must not raise the registers of the kernel it stands in)
+  // (fresh_tid: nothing formed here may live in registers over the items)
   const int tid0 = threadIdx.x, tid = fresh_tid(tid0), H = p.H, L = cl.L;
   const int64_t strideK = (int64_t)H * K, strideV = (int64_t)H * V;
   const int64_t baseK = (cl.row0 * H + hh) * (int64_t)K, baseV = (cl.row0 * H + hh) * (int64_t)V;
   const v4 z4 = {(T)0.f, (T)0.f, (T)0.f, (T)0.f};
-  // gates summed along time, q, k; rows past the end of the chunk zero
-  auto load_qkg = [&]() {
-#pragma unroll 1
-    for (int e = tid; e < BT * (K / 4); e += 256) {
-      const int row = e / (K / 4), c4 = (e % (K / 4)) * 4;
-      const int64_t off = baseK + row * strideK + c4;
-      if constexpr (!PH) {
-        float gv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (row < L) Load<GE>::x4((const GE*)p.g + off, gv);
+  auto f4 = [](v4 x) __attribute__((always_inline)) { return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; };
+  const int pa = tid >> 4, pb = tid & 15;
+  // f(block number, m, n) over the ten blocks of pairs (pa + 16 m, pb + 16 n)
+  auto blocks = [](auto f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sG[row * LDG + c4 + j] = finite_gate(gv[j]);
-      }
-      *(v4*)&sQ[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.q + off) : z4;
-      *(v4*)&sK[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.k + off) : z4;
-    }
-    if (PH && tid < BT) sGam[tid] = tid < L ? finite_gate(((const float*)p.g)[(cl.row0 + tid) * H + hh]) : 0.f;
-    __syncthreads();
-    float* col = PH ? sGam : sG + tid;
-    constexpr int step = PH ? 1 : LDG;
-    if (tid < (PH ? 1 : K)) {
-      float run = 0.f;
-#pragma unroll 1
-      for (int t = 0; t < BT; ++t) {
-        run += col[t * step];
-        col[t * step] = run;
-      }
-    }
-    __syncthreads();
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int n = 0; n <= m; ++n) f(m * (m + 1) / 2 + n, m, n);
   };
-  auto gsum = [&](int row, int ch) { return PH ? sGam[row] : sG[row * LDG + ch]; };
 
-  load_qkg();
-  float a[16];   // A, pairs (i, j) = (4 n + wave, lane)
-  const int j = tid & 63, i0 = tid >> 6;
-#pragma unroll
-  for (int n = 0; n < 16; ++n) {
-    const int t = fresh_tid(tid0), jj = t & 63, i = 4 * n + (t >> 6);
-    float sum = 0.f;
-    if (jj <= i && i < L) {
-#pragma unroll 1
-      for (int ch = 0; ch < K; ++ch)
-        sum += (float)sQ[i * LDQ + ch] * (float)sK[jj * LDQ + ch] * __expf(gsum(i, ch) - gsum(jj, ch));
-    }
-    a[n] = sum;
-  }
-  __syncthreads();   // q, k and the gates make room
-#pragma unroll 1
+#pragma unroll 4
   for (int e = tid; e < BT * (V / 4); e += 256) {
     const int row = e / (V / 4), c4 = (e % (V / 4)) * 4;
     const int64_t off = baseV + row * strideV + c4;
     *(v4*)&sV[row * LDW + c4] = row < L ? *(const v4*)((const T*)p.v + off) : z4;
     *(v4*)&sDo[row * LDW + c4] = row < L ? *(const v4*)((const T*)p.dout + off) : z4;
   }
-#pragma unroll
-  for (int n = 0; n < 16; ++n)
-    if (j <= 4 * n + i0) sA[tri_at(4 * n + i0, j)] = a[n] * p.scale;
+#pragma unroll 4
+  for (int e = tid; e < BT * (K / 4); e += 256) {
+    const int row = e / (K / 4), c4 = (e % (K / 4)) * 4;
+    const int64_t off = baseK + row * strideK + c4;
+    *(v4*)&sQ[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.q + off) : z4;
+    *(v4*)&sK[row * LDQ + c4] = row < L ? *(const v4*)((const T*)p.k + off) : z4;
+  }
+  if (PH && tid < BT) sGam[tid] = tid < L ? finite_gate(((const float*)p.g)[(cl.row0 + tid) * H + hh]) : 0.f;
   __syncthreads();
-#pragma unroll 1
-  for (int n = 0; n < 16; ++n) {
-    const int i = 4 * n + i0;
-    if (j > i) continue;
-    float da = 0.f;
-    if (i < L)
-#pragma unroll 1
-      for (int ch = 0; ch < V; ++ch) da += (float)sDo[i * LDW + ch] * (float)sV[j * LDW + ch];
-    sdA[tri_at(i, j)] = da * p.scale;
+  if (PH && tid == 0) {
+    float run = 0.f;
+#pragma unroll 16
+    for (int t = 0; t < BT; ++t) {
+      run += sGam[t];
+      sGam[t] = run;
+    }
   }
-  // dv_j += sum_{i>=j} A_ij do_i
-#pragma unroll 1
-  for (int e = tid; e < BT * (V / 4); e += 256) {
-    const int r = e / (V / 4), c4 = (e % (V / 4)) * 4;
-    if (r >= L) continue;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int i = r; i < L; ++i) {
-      const float x = sA[tri_at(i, r)];
-      const v4 y = *(const v4*)&sDo[i * LDW + c4];
+  float da[10];
+  blocks([&](int x, int, int) { da[x] = 0.f; });
+#pragma unroll 2
+  for (int ch = 0; ch < V; ch += 4) {
+    f32x4 di[4], vj[4];
 #pragma unroll
-      for (int z = 0; z < 4; ++z) acc[z] += x * (float)y[z];
+    for (int m = 0; m < 4; ++m) {
+      di[m] = f4(*(const v4*)&sDo[(pa + 16 * m) * LDW + ch]);
+      vj[m] = f4(*(const v4*)&sV[(pb + 16 * m) * LDW + ch]);
     }
-    T* dst = (T*)p.dv + baseV + r * strideV + c4;
-    const v4 old = *(const v4*)dst;
-    v4 nw;
+    blocks([&](int x, int m, int n) {
 #pragma unroll
-    for (int z = 0; z < 4; ++z) nw[z] = (T)((float)old[z] + acc[z]);
-    *(v4*)dst = nw;
+      for (int z = 0; z < 4; ++z) da[x] = fmaf(di[m][z], vj[n][z], da[x]);
+    });
   }
-  __syncthreads();   // v, do and A are consumed
-  load_qkg();
-  float x[NR][4];    // q dq' - k dk', rows and channels as below
-#pragma unroll
-  for (int n = 0; n < NR; ++n) {
-    const int e = fresh_tid(tid0) + 256 * n, r = e / (K / 4), c4 = (e % (K / 4)) * 4;
-#pragma unroll
-    for (int z = 0; z < 4; ++z) x[n][z] = 0.f;
-    if (r >= L) continue;
-    float dq[4] = {0.f, 0.f, 0.f, 0.f}, dk[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int jj = 0; jj <= r; ++jj) {       // row r as the query row i
-      const float da = sdA[tri_at(r, jj)];
-      const v4 kj = *(const v4*)&sK[jj * LDQ + c4];
-#pragma unroll
-      for (int z = 0; z < 4; ++z) dq[z] += da * (float)kj[z] * __expf(gsum(r, c4 + z) - gsum(jj, c4 + z));
-    }
-#pragma unroll 1
-    for (int i = r; i < L; ++i) {           // row r as the key row j
-      const float da = sdA[tri_at(i, r)];
-      const v4 qi = *(const v4*)&sQ[i * LDQ + c4];
-#pragma unroll
-      for (int z = 0; z < 4; ++z) dk[z] += da * (float)qi[z] * __expf(gsum(i, c4 + z) - gsum(r, c4 + z));
-    }
-    const v4 qr = *(const v4*)&sQ[r * LDQ + c4], kr = *(const v4*)&sK[r * LDQ + c4];
-    T *dqp = (T*)p.dq + baseK + r * strideK + c4, *dkp = (T*)p.dk + baseK + r * strideK + c4;
-    const v4 oq = *(const v4*)dqp, ok = *(const v4*)dkp;
-    v4 nq, nk;
-#pragma unroll
-    for (int z = 0; z < 4; ++z) {
-      nq[z] = (T)((float)oq[z] + dq[z]);
-      nk[z] = (T)((float)ok[z] + dk[z]);
-      x[n][z] = (float)qr[z] * dq[z] - (float)kr[z] * dk[z];
-    }
-    *(v4*)dqp = nq;
-    *(v4*)dkp = nk;
-  }
-  __syncthreads();   // the gates make room for x
-  if constexpr (PH) {
-    // one gate per (token, head): the channels of a row are added up in the K / 4 lanes that hold it
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      float sum = (x[n][0] + x[n][1]) + (x[n][2] + x[n][3]);
-#pragma unroll
-      for (int m = K / 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
-      const int e = tid + 256 * n;
-      if (e % (K / 4) == 0) sGam[e / (K / 4)] = sum;
-    }
-    __syncthreads();
-    if (tid < L) {
-      float run = 0.f;
-#pragma unroll 1
-      for (int t = L - 1; t >= tid; --t) run += sGam[t];
-      p.dg[(cl.row0 + tid) * H + hh] += run;
-    }
-  } else {
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      const int e = tid + 256 * n, r = e / (K / 4), c4 = (e % (K / 4)) * 4;
-#pragma unroll
-      for (int z = 0; z < 4; ++z) sG[r * LDG + c4 + z] = x[n][z];
+  __syncthreads();   // v and do make room for the gates
+  if constexpr (!PH) {
+#pragma unroll 4
+    for (int e = tid; e < BT * (K / 4); e += 256) {
+      const int row = e / (K / 4), c4 = (e % (K / 4)) * 4;
+      float gv[4] = {0.f, 0.f, 0.f, 0.f};
+      if (row < L) Load<GE>::x4((const GE*)p.g + baseK + row * strideK + c4, gv);
+      *(f32x4*)&sG[row * LDG + c4] = f32x4{finite_gate(gv[0]), finite_gate(gv[1]), finite_gate(gv[2]), finite_gate(gv[3])};
     }
     __syncthreads();
     if (tid < K) {
       float run = 0.f;
 #pragma unroll 1
-      for (int t = L - 1; t >= 0; --t) {
-        run += sG[t * LDG + tid];
-        p.dg[baseK + t * strideK + tid] += run;
+      for (int t0 = 0; t0 < BT; t0 += 16) {
+        float y[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) y[t] = sG[(t0 + t) * LDG + tid];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) sG[(t0 + t) * LDG + tid] = run += y[t];
       }
+    }
+    __syncthreads();
+  }
+  float a[10];   // A
+  blocks([&](int x, int, int) { a[x] = 0.f; });
+#pragma unroll 2
+  for (int ch = 0; ch < K; ch += 4) {
+    f32x4 qi[4], kj[4], gi[PH ? 1 : 4], gj[PH ? 1 : 4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      qi[m] = f4(*(const v4*)&sQ[(pa + 16 * m) * LDQ + ch]);
+      kj[m] = f4(*(const v4*)&sK[(pb + 16 * m) * LDQ + ch]);
+      if constexpr (!PH) {
+        gi[m] = *(const f32x4*)&sG[(pa + 16 * m) * LDG + ch];
+        gj[m] = *(const f32x4*)&sG[(pb + 16 * m) * LDG + ch];
+      }
+    }
+    blocks([&](int x, int m, int n) {
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        if constexpr (PH) a[x] = fmaf(qi[m][z], kj[n][z], a[x]);
+        else a[x] = fmaf(qi[m][z] * kj[n][z], __expf(gi[m][z] - gj[n][z]), a[x]);
+      }
+    });
+  }
+  // (per head the exponential is the pair's and goes onto dA as well)
+  blocks([&](int x, int m, int n) {
+    const int i = pa + 16 * m, j = pb + 16 * n;
+    const float e = PH ? __expf(sGam[i] - sGam[j]) : 1.f;
+    a[x] *= p.scale * e;
+    if (j <= i) sdA[tri_at(i, j)] = da[x] * p.scale * e;
+  });
+  __syncthreads();
+  float x[NR][4];    // q dq' - k dk', rows and channels as below
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    const int t = fresh_tid(tid0), r = t / (K / 4) + RP * n, c4 = (t % (K / 4)) * 4;
+    const int w0 = __builtin_amdgcn_readfirstlane(t >> 6) * (RP / 4) + RP * n;   // the wave's first row
+    const f32x4 gr = PH ? zero4() : *(const f32x4*)&sG[r * LDG + c4];
+    f32x4 dq = zero4(), dk = zero4();
+#pragma unroll 1
+    for (int j0 = 0; j0 < w0 + RP / 4; j0 += 4) {   // row r as the query row i
+      f32x4 kj[4], gj[4];
+      float w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        kj[u] = f4(*(const v4*)&sK[(j0 + u) * LDQ + c4]);
+        if constexpr (!PH) gj[u] = *(const f32x4*)&sG[(j0 + u) * LDG + c4];
+        w[u] = sdA[tri_at(r, j0 + u)];   // (past the diagonal: another element of the triangle, not used)
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+          const float y = PH ? w[u] * kj[u][z] : w[u] * kj[u][z] * __expf(gr[z] - gj[u][z]);
+          dq[z] += j0 + u <= r ? y : 0.f;
+        }
+    }
+#pragma unroll 1
+    for (int i0 = w0 & ~3; i0 < L; i0 += 4) {       // row r as the key row j
+      f32x4 qi[4], gi[4];
+      float w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        qi[u] = f4(*(const v4*)&sQ[(i0 + u) * LDQ + c4]);
+        if constexpr (!PH) gi[u] = *(const f32x4*)&sG[(i0 + u) * LDG + c4];
+        w[u] = sdA[tri_at(i0 + u, r)];   // (r > i0 + u: another element)
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+          const float y = PH ? w[u] * qi[u][z] : w[u] * qi[u][z] * __expf(gi[u][z] - gr[z]);
+          dk[z] += i0 + u >= r && i0 + u < L ? y : 0.f;
+        }
+    }
+#pragma unroll
+    for (int z = 0; z < 4; ++z) x[n][z] = 0.f;
+    if (r < L) {
+      const v4 qr = *(const v4*)&sQ[r * LDQ + c4], kr = *(const v4*)&sK[r * LDQ + c4];
+      T *dqp = (T*)p.dq + baseK + r * strideK + c4, *dkp = (T*)p.dk + baseK + r * strideK + c4;
+      const v4 oq = *(const v4*)dqp, ok = *(const v4*)dkp;
+      v4 nq, nk;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        nq[z] = (T)((float)oq[z] + dq[z]);
+        nk[z] = (T)((float)ok[z] + dk[z]);
+        x[n][z] = (float)qr[z] * dq[z] - (float)kr[z] * dk[z];
+      }
+      *(v4*)dqp = nq;
+      *(v4*)dkp = nk;
+    }
+  }
+  __syncthreads();   // the gates make room for x, q for do, k for A
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    const int r = tid / (K / 4) + RP * n, c4 = (tid % (K / 4)) * 4;
+    if constexpr (PH) {   // the channels of a row are added up in the K / 4 lanes that hold it
+      float sum = (x[n][0] + x[n][1]) + (x[n][2] + x[n][3]);
+#pragma unroll
+      for (int m = K / 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
+      if (c4 == 0) sGam[r] = sum;
+    } else {
+      *(f32x4*)&sX[r * LDG + c4] = f32x4{x[n][0], x[n][1], x[n][2], x[n][3]};
+    }
+  }
+  blocks([&](int y, int m, int n) {
+    const int i = pa + 16 * m, j = pb + 16 * n;
+    if (j <= i) sA[tri_at(i, j)] = a[y];
+  });
+#pragma unroll 4
+  for (int e = tid; e < BT * (V / 4); e += 256) {
+    const int row = e / (V / 4), c4 = (e % (V / 4)) * 4;
+    *(v4*)&sDo2[row * LDW + c4] = row < L ? *(const v4*)((const T*)p.dout + baseV + row * strideV + c4) : z4;
+  }
+  __syncthreads();
+  // dg: sums over the rows from the last one up
+  if constexpr (PH) {
+    if (tid < L) {
+      float run = 0.f;
+#pragma unroll 16
+      for (int t = BT - 1; t >= 0; --t) run += t >= tid ? sGam[t] : 0.f;
+      p.dg[(cl.row0 + tid) * H + hh] += run;
+    }
+  } else if (tid < K) {
+    float run = 0.f;
+    float* dg = p.dg + baseK + tid;
+#pragma unroll 1
+    for (int t0 = BT - 8; t0 >= 0; t0 -= 8) {
+      float old[8], y[8];
+#pragma unroll
+      for (int t = 7; t >= 0; --t) {
+        y[t] = sX[(t0 + t) * LDG + tid];
+        if (t0 + t < L) old[t] = dg[(t0 + t) * strideK];
+      }
+#pragma unroll
+      for (int t = 7; t >= 0; --t) {
+        run += y[t];
+        if (t0 + t < L) dg[(t0 + t) * strideK] = old[t] + run;
+      }
+    }
+  }
+  // dv_j += sum_{i>=j} A_ij do_i
+  constexpr int VP = 1024 / V;
+#pragma unroll 1
+  for (int n = 0; n < BT / VP; ++n) {
+    const int r = tid / (V / 4) + VP * n, c4 = (tid % (V / 4)) * 4;
+    const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6) * (VP / 4) + VP * n;
+    f32x4 acc = zero4();
+#pragma unroll 1
+    for (int i0 = w0 & ~3; i0 < L; i0 += 4) {
+      f32x4 y[4];
+      float w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        y[u] = f4(*(const v4*)&sDo2[(i0 + u) * LDW + c4]);
+        w[u] = sA[tri_at(i0 + u, r)];   // (r > i0 + u: another element)
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int z = 0; z < 4; ++z) acc[z] += i0 + u >= r && i0 + u < L ? w[u] * y[u][z] : 0.f;
+    }
+    if (r < L) {
+      T* dst = (T*)p.dv + baseV + r * strideV + c4;
+      const v4 old = *(const v4*)dst;
+      v4 nw;
+#pragma unroll
+      for (int z = 0; z < 4; ++z) nw[z] = (T)((float)old[z] + acc[z]);
+      *(v4*)dst = nw;
     }
   }
   __syncthreads();
@@ -355,8 +444,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_chunk_kernel(GlaChunkParams p,
   };
 
   // room for exact_scores()
-  static_assert(2 * BT * LDV * 2 <= AB && (PH || BT * (K + 1) * 4 <= AB) && BT * (K + 8) <= BT * (LDK > LDV ? LDK : LDV) &&
-                    kTriFloats * 4 <= BT * LDK * 2 && kTriFloats * 4 <= BT * LDT * 2,
+  static_assert(2 * BT * LDV * 2 <= AB && (PH || BT * LDG * 4 <= AB) && kTriFloats * 4 <= BT * LDK * 2 &&
+                    kTriFloats * 4 <= BT * LDT * 2,
                 "tiles of the pairwise score terms");
   bool any_flagged = false;
   const uint32_t it0 = xcd_remap(blockIdx.x, gridDim.x);

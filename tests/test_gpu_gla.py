@@ -367,6 +367,40 @@ def test_chunk_gla_backward_flagged_items_of_many(device, B, K, V, gates):
         assert_close(name, r.grad, x[:1, :2] if name == "dh0" else x[:1, :, :2], tol)
 
 
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (64, 128), (128, 64)])
+@pytest.mark.parametrize("head", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_chunk_gla_backward_flagged_lengths(device, K, V, head, dtype):
+    """The pairwise score terms at every remainder of four rows, of eight and of a block of sixteen: a packed batch whose chunks are all
+    flagged by one strong gate in their middle, the others weak, so that the pairs on either side of it count.  Tolerances of the
+    other tests of strong gates."""
+    from fla_amd.ops.gla import chunk_gla
+    from fla_amd.ops.simple_gla import chunk_simple_gla
+    from oracle.recurrent import naive_recurrent_gla
+    lens = (1, 2, 3, 4, 5, 8, 9, 15, 16, 17, 31, 33, 48, 63, 64, 64 + 7)
+    T, H = sum(lens), 2
+    q, k, v, g, h0 = gla_inputs(1, T, H, K, V, seed=98, normalizer=16.0, N=len(lens), dtype=dtype)
+    ends = [0]
+    for n in lens:
+        ends.append(ends[-1] + n)
+        for c in range(ends[-2], ends[-1], 64):
+            g[:, (c + min(c + 64, ends[-1])) // 2] = -90.0
+    g = g[..., 0].contiguous() if head else g
+    gen = torch.Generator().manual_seed(99)
+    do, dht = torch.randn(1, T, H, V, generator=gen).to(dtype), torch.randn(h0.shape, generator=gen)
+    print(f"chunk_gla backward, flagged chunks of {lens} K={K} V={V} head={head} {dtype}", flush=True)
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v, g, h0)]
+    op = chunk_simple_gla if head else chunk_gla
+    o, ht = op(*leaves[:4], initial_state=leaves[4], output_final_state=True, head_first=False, cu_seqlens=torch.tensor(ends, device=device))
+    torch.autograd.backward((o, ht), (do.to(device), dht.to(device)))
+    ref = [x.float().requires_grad_() for x in (q, k, v, g, h0)]
+    ro, rht = naive_recurrent_gla(*ref[:3], **{"g" if head else "gk": ref[3]}, initial_state=ref[4], output_final_state=True,
+                                  offsets=ends)
+    torch.autograd.backward((ro, rht), (do.float(), dht))
+    for name, r, x, tol in zip(("dq", "dk", "dv", "dg", "dh0"), ref, leaves, (1e-2, 1e-2, 1e-2, 2e-2, 5e-3)):
+        assert_close(name, r.grad, x.grad, tol)
+
+
 @pytest.mark.parametrize("keep", [True, False])
 @pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (64, 128), (128, 64)])
 @pytest.mark.parametrize("gates", ["float32", "bfloat16", "head"])
