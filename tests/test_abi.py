@@ -30,8 +30,9 @@ def test_library_exports_every_declared_symbol():
     assert be.lib().fla_abi_version() == be.ABI_VERSION
 
 
-# What a binding relies on, by version: a digest of the C declarations and of the argument counts of the host extension.
-INTERFACES = {15: "b7a4f7cfed6a371e", 16: "087cb7b8a1fcb11d"}
+# What a binding relies on, by version: a digest of the C declarations and of the names and argument counts of the host
+# extension's entries (15: without the names).
+INTERFACES = {15: "b7a4f7cfed6a371e", 16: "ecb9b6be8de7c997", 17: "8d259aba7a1ce02b"}
 
 
 def _interface():
@@ -40,7 +41,9 @@ def _interface():
     host = open(os.path.join(ROOT, "flash-linear-attention_amd", "csrc", "torch_host.cpp")).read()
     counts = re.findall(r"^PyObject\* (py_\w+)\(.*?expect\(n, (\d+)\)", host, flags=re.S | re.M)
     assert len(counts) >= 10
-    return hashlib.sha256(repr((text.split(), counts)).encode()).hexdigest()[:16]
+    entries = re.findall(r"^ +ENTRY\(\"(\w+)\"", host, flags=re.M)
+    assert len(entries) >= 10
+    return hashlib.sha256(repr((text.split(), counts, entries)).encode()).hexdigest()[:16]
 
 
 def test_version_moves_with_the_interface():
