@@ -62,21 +62,31 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 // Whether cutting pays is the longest sequence's chunk periods against those of a segment in the scan and in the first pass
 // and the launches ahead of the scan, fitted to the times below (K = V = 128, uncut / cut in us, launches replayed from a
 // graph; packed batches back to back).  The busier the CUs (triples of sequence, head and slab), the less a cut gains.
-// (The training steps of GLA were read with a forward that also wrote k^ and the score tiles and with per-key gates, those of the
-// delta rule with a forward that wrote w and a reverse scan of 162 us where today's takes 141: today's scans gain a little
-// less from a cut than these figures say.)
+// (The training steps of GLA were read with a forward that also wrote k^ and the score tiles and with per-key gates: today's gain
+// a little less from a cut than these figures say.)
 //   GLA: one sequence of 16 heads, 12 and 16 chunks 37.7 / 36.1 and 46.0 / 37.2; four, 16, 20 and 24 chunks 50.4 / 53.5,
 //     59.3 / 61.6 and 68.4 / 65.8, their training steps 145 / 162, 198 / 202 and 237 / 237.
-//   Delta rule: 4 and 8 heads, 24 chunks 45.9 / 44.0 and 46.3 / 45.7; 16 heads, 24, 28, 32 and 40 chunks 48.4 / 51.8, 54.1 /
-//     55.3, 59.9 / 58.9 and 70.6 / 63.0; 32 heads, 28, 40, 48 and 64 chunks 57.1 / 65.3, 75.1 / 77.2, 86.8 / 85.4 and 109.5 /
-//     100.9; packed, 16 heads, 54, 94 and 77 chunks 152 / 160, 80 and 171 chunks 253 / 174.
-//   Delta rule, a forward that keeps its intermediates and its backward: from five segments on (training step of two
-//     sequences of 64 chunks, 16 heads, in 4 462 / 472, three of 8 heads in 5 379 / 356); 8 heads, 24 chunks 123 / 116; 16
-//     heads, 24, 32 and 40 chunks 136 / 148, 168 / 172 and 203 / 193.
+//   Delta rule, forward: the uncut scan takes 1.1 us a chunk (64 key channels: 0.75), and a cut pays for: the chunks of a segment
+//     in the scan, more where its segments no longer fit in slabs of 32 columns; the same in the first pass, whose workgroups of
+//     128 of the K + V columns take as many rounds as 256 CUs need for them; the fold's steps; what the first pass loads and
+//     stores; the launches.  K = V = 128: 4 heads, 24, 28 and 32 chunks 35.7 / 37.3, 40.1 / 40.4 and 44.5 / 42.1; 8 heads 35.8 /
+//     38.6, 40.2 / 41.6 and 44.6 / 43.2; 12 heads, 36 and 40 chunks 51.0 / 53.5 and 55.7 / 53.8; 16 heads, 32, 36, 40 and 48
+//     47.6 / 52.1, 52.3 / 56.1, 57.0 / 56.7 and 65.5 / 60.0; 24 heads, 44 and 52 63.8 / 64.6 and 73.1 / 70.9; 32 heads, 56, 60 and
+//     68 80.3 / 83.6, 85.3 / 85.9 and 95.2 / 93.4; packed, 16 heads, 54, 94 and 77 chunks 132 / 146, 80 and 171 215 / 157.  128 keys,
+//     64 values (the first pass as long as with 128, the scan with half the slabs): 16 heads, 24, 32 and 36 chunks 37.0 / 41.3,
+//     46.8 / 47.0 and 52.0 / 50.1, 48 in two rounds 65.2 / 68.0; 32 heads, 32, 48 and 64 49.8 / 68.0, 69.3 / 80.2 and 89.0 / 91.7.
+//     64 keys, 128 values: 16 heads, 28 and 36 32.4 / 34.5 and 39.5 / 38.5.  K = V = 64: 8 heads, 20 and 24 24.3 / 25.4 and 27.3 /
+//     25.9; 16 heads, 24 28.7 / 28.3; 32 heads, 28, 36 and 40 35.3 / 37.2, 42.2 / 42.4 and 45.9 / 42.8; 64 heads, 64 73.1 / 76.3.
+//   Delta rule, a forward that keeps its intermediates and its backward (training steps): the same terms over both directions; a
+//     transition of every segment is formed.  K = V = 128: 4 heads, 23 and 24 chunks 87.0 / 89.0 and 89.3 / 88.5; 8 heads, 24 and
+//     28 92.1 / 92.3 and 102.9 / 97.9; 12 heads, 36 and 40 132.8 / 141.6 and 143.5 / 142.8; 16 heads, 40, 44, 48 and 56 162 / 169,
+//     172 / 178, 182 / 181 and 203 / 190; 24 heads, 72 and 80 311 / 323 and 350 / 340; 32 heads, 96 494 / 499; packed, 8 heads, 20, 63,
+//     49 and 26 chunks 243 / 250.  K = V = 64: 8 heads, 20 and 24 63.1 / 61.3 and 70.9 / 63.1; 32 heads, 48 152 / 135.
 //   The plain scan of chunk_simple_gla's forward takes half as long per chunk as the GLA kernel and fills the chip with half
-//     the pairs (slabs of 32 columns): 4 heads, 12 and 16 chunks 22.1 / 23.6 and 26.0 / 24.3; 16 heads, 12, 24 and 32 chunks
-//     22.9 / 27.7, 35.4 / 34.5 and 43.9 / 36.6, two sequences of them, 16, 32 and 64 chunks 28.2 / 34.8, 44.8 / 45.0 and 77.5 /
-//     64.8, four, 24 and 64 chunks 39.6 / 55.7 and 84.7 / 95.5; packed, 54, 94 and 77 chunks 103 / 94.
+//     the pairs (slabs of 32 columns).  K = V = 128: 4 heads, 12 and 16 chunks 16.5 / 18.1 and 20.6 / 18.8; 12 heads, 18 and 20 23.8
+//     / 24.2 and 25.8 / 24.6; 16 heads, 20, 22 and 24 25.1 / 27.1, 27.1 / 27.5 and 29.2 / 27.8; 32 heads, 32, 36 and 40 38.4 / 39.6,
+//     42.4 / 43.3 and 46.4 / 44.1; four sequences of 16, 64 and 128 76.8 / 87.9 and 159 / 164; packed, 16 heads, 54, 94 and 77
+//     chunks 101 / 89.  64 keys, 128 values: 16 heads, 24 and 28 22.3 / 22.6 and 25.2 / 23.3.
 //   The reverse scan of GLA's backward forms the state gradient alone, in half the time per chunk, and leaves every pass of the
 //     backward behind it alone, so only what it saves itself counts (whole training steps; per-key gates, K = V = 128): 4
 //     heads, 16, 24 and 32 chunks 63.5 / 67.3, 72.1 / 72.3 and 77.3 / 73.8; 8 heads, 24, 32 and 64 chunks 75.3 / 77.1, 84.0 /
@@ -87,9 +97,12 @@ extern "C" int fla_prepare_chunk_indices(const int64_t* offsets, int64_t n_seqs,
 extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                               int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base) {
   constexpr int64_t kCUs = 256, kChunk = 64, kPassWorkgroups = 256;
+  const bool keys64 = kind & FLA_SCAN_KEYS_64;
+  kind &= ~FLA_SCAN_KEYS_64;
   const bool delta = kind == FLA_SCAN_DELTA || kind == FLA_SCAN_DELTA_KEPT;
   int64_t min_seg = 4;
-  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_GLA_GRADIENT || N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
+  if (!out || kind < FLA_SCAN_GLA || kind > FLA_SCAN_GLA_GRADIENT || (keys64 && !delta)) return 0;
+  if (N <= 0 || H <= 0 || slabs <= 0 || N > 65536) return 0;
   auto chunks_of = [&](int64_t n) { return offsets ? fla_cdiv(offsets[n + 1] - offsets[n], kChunk) : fla_cdiv(T, kChunk); };
   int64_t longest = 0, total = 0;
   for (int64_t n = 0; n < N; ++n) {
@@ -114,17 +127,29 @@ extern "C" int fla_scan_split(const int64_t* offsets, int64_t N, int64_t T, int6
   seg = seg < min_seg ? min_seg : seg;
   while (segments(seg) > room) ++seg;
   const int64_t triples = fla_cdiv(total, longest) * H * slabs;   // sequences of other lengths: as many of the longest
-  const int64_t L = longest, steps = fla_cdiv(L, seg) - 1;
+  const int64_t L = longest, segs = segments(seg), steps = fla_cdiv(L, seg) - 1;
+  // the delta rule's first pass: workgroups of 128 of the K + V columns of a (segment, head); and the slabs its scan then has
+  const int64_t pass = H * (segs - (kind == FLA_SCAN_DELTA_KEPT ? 0 : N)) * fla_cdiv(slabs + (keys64 ? 1 : 2), 2);
+  const int64_t rounds = fla_cdiv(pass, kCUs), wide = 2 * segs * H * slabs > kCUs ? 1 : 0;
   bool pays;
-  switch (kind) {   // the scan of whole sequences against that of the segments and what stands ahead of it: see above
-    case FLA_SCAN_DELTA: pays = 4 * L >= 11 * seg + 7 * steps + (triples < 32 ? 7 + triples * 5 / 8 : 22 + triples * 5 / 32); break;
-    case FLA_SCAN_DELTA_KEPT: pays = steps >= 4 && L - seg >= 20 && L - seg >= 8 + triples * 3 / 4; break;
-    case FLA_SCAN_SIMPLE: pays = 5 * L >= 11 * seg + 28 + (triples < 64 ? triples : 64) * 3 / 4; break;
+  switch (kind) {   // the scan of whole sequences against that of the segments and what stands ahead of it, in twentieths of a chunk
+                    // of the former (the last two in fifths and elevenths): see above
+    case FLA_SCAN_DELTA:
+      pays = keys64 ? 20 * L >= seg * (3 + 50 * rounds + 12 * wide) + 12 * steps + pass * 189 / 256 + 140
+                    : 20 * L >= seg * (2 + 35 * rounds + 20 * wide) + 34 * steps + pass * 112 / 256 + 170;
+      break;
+    case FLA_SCAN_DELTA_KEPT:
+      pays = keys64 ? 20 * L >= seg * (1 + 54 * rounds + 29 * wide) + 23 * steps + 57
+                    : 20 * L >= seg * (6 * rounds + 55 * wide) + pass * 165 / 256 + 426;
+      break;
+    case FLA_SCAN_SIMPLE:
+      pays = 5 * L >= 9 * seg + (triples < 8 ? 28 : triples < 32 ? 12 + 2 * triples : 52 + (triples < 64 ? triples : 64) * 3 / 4);
+      break;
     case FLA_SCAN_GLA_GRADIENT: pays = 11 * (L - seg) >= 165 + 3 * triples; break;
     default: pays = 5 * L >= 7 * seg + 31;
   }
   if (steps == 0 || !pays) return 0;
-  const int64_t formed = H * (segments(seg) - N);   // (segment, head) pairs the first pass works on
+  const int64_t formed = H * (segs - N);   // (segment, head) pairs the first pass works on
   int64_t ratio = formed > 0 ? kPassWorkgroups / formed : 1;
   ratio = ratio > seg / 2 ? seg / 2 : ratio;
   if (delta) ratio = 1;

@@ -385,6 +385,11 @@ struct GdrKept {
   Tensor gc, AT, Aw, v_new, hT, Aqk, Mt;   // Mt: the segments' transposed transitions where the forward was cut
 };
 
+// the kind of a delta-rule scan as fla_scan_split takes it: the same for a forward that keeps its intermediates and its backward
+int delta_scan(const Dims& d, bool kept) {
+  return (kept ? FLA_SCAN_DELTA_KEPT : FLA_SCAN_DELTA) | (d.K == 64 ? FLA_SCAN_KEYS_64 : 0);
+}
+
 Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& h0,
                    const GdrArgs& a, Tensor* ht, GdrKept* kept) {
   const Dims& d = a.d;
@@ -395,7 +400,7 @@ Tensor gdr_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   if (a.want_ht) *ht = fresh({d.N, d.H, d.K, d.V}, q, at::kFloat);
   // sequences cut into segments: their K x K transitions take the place of the decays
   auto cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), false, q, d.K * d.V, d.K * d.K,
-                            kept ? FLA_SCAN_DELTA_KEPT : FLA_SCAN_DELTA);
+                      delta_scan(d, kept));
   auto scan_cut = [&](const Tensor& rstd, const GdrKept& x) {
     check(fla_chunk_gated_delta_rule_fwd_scan_split(ptr(q), ptr(k), ptr(v), ptr(AT), fptr(gc), fptr(rstd), fptr(h0), ptr(o),
                                                     fptr(*ht), ptr(x.v_new), ptr(x.hT), ptr(x.Aqk), offs(a.plan), coff(a.plan),
@@ -490,7 +495,7 @@ struct GdrNode : torch::autograd::Function<GdrNode> {
     Tensor dh0 = r.has_h0 ? fresh({d.N, d.H, d.K, d.V}, q, at::kFloat) : Tensor();
     std::optional<Cut> cut;
     if (Mt.defined())
-      cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), true, q, d.K * d.V, 0, FLA_SCAN_DELTA_KEPT);
+      cut = cut_scan(a.plan, d.N, d.T, d.H, (int)(d.V / 64), true, q, d.K * d.V, 0, delta_scan(d, true));
     if (cut) cut->s.decays = fptr(Mt);
     check(fla_chunk_gated_delta_rule_bwd_tiles(
               ptr(q), ptr(k), ptr(v), ptr(AT), ptr(v_new), fptr(beta), fptr(gc), ptr(Aw), ptr(dout), fptr(dht), ptr(hT),

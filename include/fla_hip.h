@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define FLA_ABI_VERSION 17
+#define FLA_ABI_VERSION 18
 
 enum fla_dtype { FLA_F32 = 0, FLA_BF16 = 1, FLA_F16 = 2 };
 
@@ -80,14 +80,15 @@ enum fla_scan_kind {
   FLA_SCAN_DELTA = 1,
   FLA_SCAN_DELTA_KEPT = 2, /* keeps its intermediates */
   FLA_SCAN_SIMPLE = 3,     /* the plain scan: AT == NULL in fla_chunk_gated_delta_rule_fwd_scan_split */
-  FLA_SCAN_GLA_GRADIENT = 4 /* the state gradient alone: fla_chunk_gla_bwd_split */
+  FLA_SCAN_GLA_GRADIENT = 4, /* the state gradient alone: fla_chunk_gla_bwd_split */
+  FLA_SCAN_KEYS_64 = 8 /* added to one of the delta rule's: 64 key channels, not 128 */
 };
 
 /* The plan for N sequences of T tokens (or, with offsets_host [N+1], of a packed batch) and H heads in `slabs` workgroups
  * per (sequence, head); reverse: for a scan from right to left; kind: the recurrence (the delta rule: segments of one
- * sub-block).  Fills the integer fields and returns 1, or returns 0 where
- * cutting would not pay (host arithmetic, host pointers).  A packed batch's tables are written on a second call with
- * seg_table / sub_table / sub_base given (2 x nseg, 2 x nsub and N+1 words). */
+ * sub-block; whether a cut pays also goes by the key channels, FLA_SCAN_KEYS_64).  Fills the integer fields and returns 1, or
+ * returns 0 where cutting would not pay (host arithmetic, host pointers).  A packed batch's tables are written on a second
+ * call with seg_table / sub_table / sub_base given (2 x nseg, 2 x nsub and N+1 words). */
 int fla_scan_split(const int64_t* offsets_host, int64_t N, int64_t T, int64_t H, int32_t slabs, int32_t reverse,
                    int32_t kind, fla_split* out, int32_t* seg_table, int32_t* sub_table, int32_t* sub_base);
 

@@ -14,6 +14,11 @@ from oracle.recurrent import naive_recurrent_gated_delta_rule, naive_recurrent_g
 pytestmark = pytest.mark.gpu
 
 
+def _delta(kind, K):
+    """The delta rule's kinds go by their key channels."""
+    return kind | (8 if K == 64 else 0)
+
+
 def _cut(N, T, H, slabs, reverse, bounds, kind=0):
     """Whether the launches cut this batch."""
     from fla_amd import _backend as be
@@ -81,8 +86,8 @@ def test_gla_cut_gate_logits_and_strong_gates(device):
 
 GDR_CASES = [
     (1, 1601, 1, 64, 64, None, torch.bfloat16),      # 26 chunks, the last of one token
-    (2, 1727, 2, 128, 128, None, torch.bfloat16),    # the last chunk of 63 tokens
-    (1, 1600, 3, 128, 64, None, torch.float16),
+    (2, 2047, 2, 128, 128, None, torch.bfloat16),    # the last chunk of 63 tokens
+    (1, 1856, 3, 128, 64, None, torch.float16),
     (1, 2500, 2, 64, 128, [0, 1, 1, 1900, 1964, 2500], torch.bfloat16),
     (1, 3200, 1, 128, 128, [0, 1790, 1854, 3200], torch.bfloat16),
 ]
@@ -96,7 +101,7 @@ def test_gdr_cut_sequences(device, B, T, H, K, V, bounds, dtype, gated):
     from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
+    assert _cut(N, T, H, V // 64, False, bounds, _delta(1, K)) and _cut(N, T, H, V // 64, True, bounds, _delta(2, K))
     print("cut delta rule", B, T, H, K, V, bounds, dtype, gated, flush=True)
     q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=2000.0, N=N)
     beta = beta * 0.02
@@ -131,7 +136,7 @@ def test_gdr_cut_l2norm_in_kernel(device, K, V):
     q, k, v, g, beta, h0 = gdr_inputs(1, 1700, 2, K, V, seed=3, normalizer=2000.0)
     k = torch.randn(k.shape).to(k.dtype) * 3
     beta = beta * 0.02
-    assert _cut(1, 1700, 2, V // 64, False, None, 1)
+    assert _cut(1, 1700, 2, V // 64, False, None, _delta(1, K))
     print("cut delta rule, raw q and k", K, V, flush=True)
     with torch.no_grad():
         o, ht = chunk_gated_delta_rule(*(t.to(device) for t in (q, k, v, g, beta)), initial_state=h0.to(device),
@@ -214,9 +219,9 @@ def test_gdr_cut_backward_that_reads_w(device, K, V, dtype, gated):
     chunks = AT.shape[0]
     new = lambda *shape: q.new_empty(*shape)
     o, ht, v_new, hT, Aqk = torch.empty_like(v), torch.empty_like(h0), torch.empty_like(v), new(chunks, H, K * V), torch.empty_like(AT)
-    sp, bufs = _split(q, B, T, H, V // 64, 2, K * V, K * K)
+    sp, bufs = _split(q, B, T, H, V // 64, _delta(2, K), K * V, K * K)
     back = be.Split()
-    assert lib.fla_scan_split(None, B, T, H, V // 64, 1, 2, ctypes.byref(back), None, None, None)
+    assert lib.fla_scan_split(None, B, T, H, V // 64, 1, _delta(2, K), ctypes.byref(back), None, None, None)
     assert (back.nseg, back.sub_chunks, back.ratio, back.slots) == (sp.nseg, sp.sub_chunks, 1, sp.slots) and sp.nseg > 1
     Mt = torch.empty_like(bufs[1])
     sp.transitions_t = Mt.data_ptr()
@@ -387,7 +392,7 @@ def test_gdr_cut_state_passes_in_fp32(device, K, V, dtype, bounds):
     from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
     T, H = 2500, 2
     N = 1 if bounds is None else len(bounds) - 1
-    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
+    assert _cut(N, T, H, V // 64, False, bounds, _delta(1, K)) and _cut(N, T, H, V // 64, True, bounds, _delta(2, K))
     q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, T, H, K, V, seed=6, dtype=dtype, N=N))
     kw = dict(output_final_state=True, head_first=False,
               cu_seqlens=None if bounds is None else torch.tensor(bounds, device=device))
@@ -437,7 +442,7 @@ def test_tables_of_a_cut_do_not_wait_for_the_device(device, delta):
     from fla_amd.ops.gla import chunk_gla
     from fla_amd.utils import VarlenPlan
     T, bounds = 3200, [0, 1790, 1854, 3200]
-    assert _cut(3, T, 1, 1, False, bounds, 2 * delta) and _cut(3, T, 1, 1, True, bounds, 2 if delta else 4)
+    assert _cut(3, T, 1, 1, False, bounds, _delta(2, 64) * delta) and _cut(3, T, 1, 1, True, bounds, _delta(2, 64) if delta else 4)
     q, k, v, g, beta, _ = (x.to(device) for x in gdr_inputs(1, T, 1, 64, 64, seed=2, normalizer=600.0))
     gk = g[..., None].expand(-1, -1, -1, 64).contiguous()
     q.requires_grad_()
@@ -504,7 +509,7 @@ def test_gdr_cut_ordinary_corrections(device, B, T, H, K, V, bounds, dtype, norm
     from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
     N = B if bounds is None else len(bounds) - 1
     offs = None if bounds is None else torch.tensor(bounds, device=device)
-    assert _cut(N, T, H, V // 64, False, bounds, 1) and _cut(N, T, H, V // 64, True, bounds, 2)
+    assert _cut(N, T, H, V // 64, False, bounds, _delta(1, K)) and _cut(N, T, H, V // 64, True, bounds, _delta(2, K))
     print("cut, ordinary beta", B, T, H, K, V, bounds, dtype, normalizer, states, flush=True)
     q, k, v, g, beta, h0 = gdr_inputs(B, T, H, K, V, seed=T, dtype=dtype, normalizer=normalizer, N=N, h0=states)
     kw = dict(output_final_state=states, cu_seqlens=offs, head_first=False)
@@ -552,7 +557,7 @@ def test_cut_entry_against_the_uncut_one(device, K, V, dtype, op):
     if not delta:
         g = gla_inputs(B, T, H, K, V, seed=3, normalizer=200.0)[3].to(device)
     lib, p, scale, st = be.lib(), be.ptr, K ** -0.5, be.stream_of(q)
-    sp, bufs = _split(q, B, T, H, V // 64, int(delta), K * V, K * K if delta else K)
+    sp, bufs = _split(q, B, T, H, V // 64, _delta(1, K) * delta, K * V, K * K if delta else K)
     assert sp.nseg > 1
     print("cut against uncut", op, K, V, dtype, sp.nseg, sp.sub_chunks, sp.ratio, flush=True)
     o, ht = [torch.empty_like(v) for _ in range(2)], [torch.empty_like(h0) for _ in range(2)]
@@ -590,7 +595,7 @@ def test_gdr_cut_forward_with_its_backward_under_capture(device, bounds):
     packed batch and runs uncut; for one sequence it needs none."""
     from fla_amd.ops.gated_delta_rule import chunk_gated_delta_rule
     T, N = 3200, 1 if bounds is None else 3
-    assert _cut(N, T, 1, 1, False, bounds, 2) and _cut(N, T, 1, 1, True, bounds, 2)
+    assert _cut(N, T, 1, 1, False, bounds, _delta(2, 64)) and _cut(N, T, 1, 1, True, bounds, _delta(2, 64))
     leaves = [x.to(device).requires_grad_() for x in gdr_inputs(1, T, 1, 64, 64, seed=2, normalizer=600.0, h0=False)[:5]]
     do = torch.randn(1, T, 1, 64, device=device).to(leaves[0].dtype)
     offs = None if bounds is None else torch.tensor(bounds, device=device)
@@ -632,7 +637,7 @@ def test_cut_states_at_any_float_address(device, op):
     from fla_amd.ops.simple_gla import chunk_simple_gla
     T, K = 2020, 64
     delta = op == "chunk_gated_delta_rule"
-    assert _cut(1, T, 2, 1, False, None, 2 * delta) and _cut(1, T, 2, 1, True, None, 2 if delta else 4)
+    assert _cut(1, T, 2, 1, False, None, _delta(2, K) * delta) and _cut(1, T, 2, 1, True, None, _delta(2, K) if delta else 4)
     q, k, v, g, beta, h0 = (x.to(device) for x in gdr_inputs(1, T, 2, K, K, seed=4, normalizer=200.0))
     do, dht = torch.randn(v.shape, device=device).to(v.dtype), torch.randn(h0.shape, device=device)
 
