@@ -36,11 +36,12 @@ struct ConvParams {
   void* y;             // [B,T,D]
   const void* dy;      // backward
   void* dx;
-  float* dw;           // [gridDim.y, D, W] fp32 partial sums
-  float* dbias;        // [gridDim.y, D] fp32 partial sums or NULL
+  float* dw;           // [conv_bwd_parts(B, T), D, W] fp32 partial sums
+  float* dbias;        // [conv_bwd_parts(B, T), D] fp32 partial sums or NULL
   int64_t B, T;
   int D;
   unsigned cblocks, tiles_per_seq, tiles;   // channel blocks of a row, tiles of a sequence and of all
+  unsigned tile0;                           // forward: the launch's first tile
 };
 
 FLA_DEVICE float silu_f(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
@@ -138,7 +139,7 @@ FLA_DEVICE void conv_fwd_tile(const ConvParams& p, int64_t b, int64_t t0, int d0
 template <typename T, int W, int TT, int CV, bool SILU>
 __global__ __launch_bounds__(256) void conv_fwd_kernel(ConvParams p) {
   const unsigned cb = blockIdx.x % p.cblocks;
-  const unsigned first = __builtin_amdgcn_readfirstlane(blockIdx.x / p.cblocks * 4 + threadIdx.y);
+  const unsigned first = __builtin_amdgcn_readfirstlane(p.tile0 + blockIdx.x / p.cblocks * 4 + threadIdx.y);
   const int d0 = (int)(cb * 64 + threadIdx.x) * CV;
   if (d0 >= p.D) return;
   float w[W][CV], bias[CV];   // (ahead of the rows: all of them are used with the first one)
@@ -308,26 +309,32 @@ int64_t conv_bwd_parts(int64_t B, int64_t T) {
   return g < 1 ? 1 : (g > 128 ? 128 : g);
 }
 
+// a launch has fewer than 2^32 threads in x: workgroups of 64 x 4
+constexpr int64_t kMostBlocks = (1LL << 26) - 1;
+
 template <typename T, int W, int TT, int CV, bool SILU>
 int launch_fwd(ConvParams p, hipStream_t st) {
   const int64_t per = fla_cdiv(p.T, TT), tiles = p.B * per, cb = fla_cdiv(p.D / CV, 64);
-  FLA_REQUIRE(tiles <= 0xffffffffLL - 0x100000 && cb <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
+  FLA_REQUIRE(tiles <= 0xffffffffLL - 0x100000 && cb <= kMostBlocks, FLA_E_UNSUPPORTED);
   p.cblocks = (unsigned)cb, p.tiles_per_seq = (unsigned)per, p.tiles = (unsigned)tiles;
   int64_t groups = fla_cdiv(tiles, 4);
   // fp32: a few tiles per wave, the weights loaded once (8 x 4096 x 2048: 96 - 98 us, a tile per wave up to 111); a tile per wave
   // in 16 bits (50 and 52 us)
   if (sizeof(T) == 4 && groups * cb > 4096) groups = fla_cdiv(4096, cb);
-  FLA_REQUIRE(groups * cb <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
-  const int64_t blocks = groups * cb;
-  hipLaunchKernelGGL((conv_fwd_kernel<T, W, TT, CV, SILU>), dim3((unsigned)blocks), dim3(64, 4), 0, st, p);
-  FLA_CHECK_LAUNCH();
+  const int64_t most = kMostBlocks / cb;   // rows of a few channels and 2^31 of them in 16 bits: the tiles of a launch after another's
+  for (int64_t g0 = 0; g0 < groups; g0 += most) {
+    p.tile0 = (unsigned)(4 * g0);
+    const int64_t blocks = (groups - g0 < most ? groups - g0 : most) * cb;
+    hipLaunchKernelGGL((conv_fwd_kernel<T, W, TT, CV, SILU>), dim3((unsigned)blocks), dim3(64, 4), 0, st, p);
+    FLA_CHECK_LAUNCH();
+  }
   return FLA_OK;
 }
 
 template <typename T, int W, int TT, int CV, bool SILU>
 int launch_bwd(ConvParams p, hipStream_t st) {
   const int64_t per = fla_cdiv(p.T, TT), tiles = p.B * per, cb = fla_cdiv(p.D / CV, 64), groups = conv_bwd_parts(p.B, p.T);
-  FLA_REQUIRE(tiles <= 0xffffffffLL - 0x10000 && groups * cb <= 0x7fffffffLL, FLA_E_UNSUPPORTED);
+  FLA_REQUIRE(tiles <= 0xffffffffLL - 0x10000 && groups * cb <= kMostBlocks, FLA_E_UNSUPPORTED);
   p.cblocks = (unsigned)cb, p.tiles_per_seq = (unsigned)per, p.tiles = (unsigned)tiles;
   const dim3 grid((unsigned)(groups * cb)), block(64, 4);   // a partial sum per workgroup of a channel block
   if (p.bias || p.dbias) hipLaunchKernelGGL((conv_bwd_kernel<T, W, TT, CV, SILU, true>), grid, block, 0, st, p);
@@ -390,7 +397,7 @@ extern "C" int fla_causal_conv1d_fwd(const void* x, const float* weight, const f
   FLA_REQUIRE(D % 8 == 0 && D < (1 << 30) && W >= 2 && W <= 4, FLA_E_UNSUPPORTED);   // (a row: 32-bit byte offsets)
   FLA_REQUIRE((((uintptr_t)x) | ((uintptr_t)y)) % 16 == 0, FLA_E_ALIGNMENT);
   if (B == 0 || T == 0) return FLA_OK;
-  ConvParams p{x, weight, bias, y, nullptr, nullptr, nullptr, nullptr, B, T, (int)D, 0, 0, 0};
+  ConvParams p{x, weight, bias, y, nullptr, nullptr, nullptr, nullptr, B, T, (int)D, 0, 0, 0, 0};
   hipStream_t st = (hipStream_t)stream;
   if (dtype == FLA_BF16) return dispatch_conv<bf16>(p, (int)W, silu, false, st);
   if (dtype == FLA_F16) return dispatch_conv<f16>(p, (int)W, silu, false, st);
@@ -409,7 +416,7 @@ extern "C" int fla_causal_conv1d_bwd(const void* x, const float* weight, const f
   FLA_REQUIRE(D % 8 == 0 && D < (1 << 30) && W >= 2 && W <= 4, FLA_E_UNSUPPORTED);   // (a row: 32-bit byte offsets)
   FLA_REQUIRE((((uintptr_t)x) | ((uintptr_t)dy) | ((uintptr_t)dx)) % 16 == 0, FLA_E_ALIGNMENT);
   if (B == 0 || T == 0) return FLA_OK;
-  ConvParams p{x, weight, bias, nullptr, dy, dx, dweight, dbias, B, T, (int)D, 0, 0, 0};
+  ConvParams p{x, weight, bias, nullptr, dy, dx, dweight, dbias, B, T, (int)D, 0, 0, 0, 0};
   hipStream_t st = (hipStream_t)stream;
   if (dtype == FLA_BF16) return dispatch_conv<bf16>(p, (int)W, silu, true, st);
   if (dtype == FLA_F16) return dispatch_conv<f16>(p, (int)W, silu, true, st);

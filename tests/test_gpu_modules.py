@@ -219,6 +219,27 @@ def test_causal_conv1d_at_tile_edges(device, dtype, B, T, D, bias, act):
             assert_close(name, r.grad, d.grad, tol)
 
 
+def test_causal_conv1d_of_more_tiles_than_a_launch_has(device):
+    """2^31 time steps and a few of 8 channels in 16 bits: 2^26 workgroups, more than one launch takes.  The same bits as from
+    pieces of it, each with the steps ahead of it."""
+    from fla_amd.modules.convolution import causal_conv1d
+    T, D, W, piece = 2 ** 31 + 77, 8, 4, 2 ** 28
+    if torch.cuda.mem_get_info()[0] < 90 * 2 ** 30:
+        pytest.skip("needs 90 GiB of free memory")
+    gen = torch.Generator().manual_seed(12)
+    w, b = (torch.rand(D, W, generator=gen) - 0.5).to(device), torch.randn(D, generator=gen).to(device)
+    print("short conv", T, D, flush=True)
+    x = torch.empty(1, T, D, dtype=torch.bfloat16, device=device).normal_()
+    with torch.no_grad():
+        y = causal_conv1d(x, w, b, "silu")
+        for t in range(0, T, piece):
+            lead = min(t, W - 1)
+            part = causal_conv1d(x[:, t - lead:t + piece], w, b, "silu")
+            assert torch.equal(y[:, t:t + piece], part[:, lead:]), t
+    del x, y, part
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W", [2, 3, 4])
 @pytest.mark.parametrize("T,D,bias,act", [(1, 64, False, "silu"), (5, 64, True, "silu"), (64, 200, False, None),
