@@ -192,19 +192,24 @@ def test_causal_conv1d_on_wide_tiles(device, dtype, B, T, D, W):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("B,T,D,bias,act", [(130, 15, 1032, True, "silu"), (130, 16, 1032, False, "silu"),
-                                            (130, 17, 1032, False, None), (130, 34, 1032, True, None),
-                                            (2, 2, 8, True, "silu"), (1, 16401, 2056, False, "silu")])
-def test_causal_conv1d_at_tile_edges(device, dtype, B, T, D, bias, act):
-    """Tiles of 16 and of 8 time steps that end with their sequence, one step before and behind its end; rows of channels
-    that end inside a workgroup; the last case takes the forward's 8 x 4 tiles in 16 bits."""
+@pytest.mark.parametrize("B,T,D,W,bias,act", [
+    # tiles of 8 steps: fewer than 2048 waves of 16 steps x 2 channels
+    (130, 7, 1032, 4, True, "silu"), (130, 8, 1032, 4, False, None), (130, 9, 1032, 3, True, None), (130, 15, 1032, 4, True, "silu"),
+    (130, 16, 1032, 4, False, "silu"), (2, 2, 8, 4, True, "silu"),
+    # tiles of 16 steps (the forward in 16 bits, the backward)
+    (260, 15, 1032, 4, True, "silu"), (260, 16, 1032, 4, False, "silu"), (260, 16, 1032, 2, True, None), (130, 17, 1032, 4, False, None),
+    (130, 31, 1032, 3, False, "silu"), (130, 32, 1032, 4, True, None), (130, 34, 1032, 4, True, None),
+    # the 16-bit forward in 8 steps x 4 channels: 16384 waves of these and more
+    (1, 16401, 2056, 4, False, "silu"), (1, 16400, 2056, 3, True, "silu"), (2, 8192, 2056, 2, True, None), (1, 16399, 2056, 4, True, None)])
+def test_causal_conv1d_at_tile_edges(device, dtype, B, T, D, W, bias, act):
+    """Sequences that end with a tile, one step ahead of its end and one or two behind it, in every shape of tile the forward and the
+    backward take; rows of channels that end inside a workgroup."""
     from fla_amd.modules.convolution import causal_conv1d as conv
     from oracle.modules import causal_conv1d
     gen = torch.Generator().manual_seed(T)
-    W = 4
     x, dy = (torch.randn(B, T, D, generator=gen).to(dtype) for _ in range(2))
     w, b = torch.rand(D, W, generator=gen) - 0.5, torch.randn(D, generator=gen) if bias else None
-    print("short conv at tile edges", dtype, B, T, D, bias, act, flush=True)
+    print("short conv at tile edges", dtype, B, T, D, W, bias, act, flush=True)
     leaves = [None if t is None else t.to(device).requires_grad_() for t in (x, w, b)]
     y = conv(*leaves, act)
     y.backward(dy.to(device))
