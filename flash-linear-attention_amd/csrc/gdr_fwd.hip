@@ -108,46 +108,53 @@ FLA_DEVICE void wy_stage_t(T* dstT, const typename Elem<T>::v4* reg, const float
   }
 }
 
-// One step of the forward substitution of wy_invert: x[c] += nm[J] * (x[c] of lane J of this DPP row), c <= J, each update one
+// One step of the forward substitution of wy_diagonal: x[c] += nm[J] * (x[c] of lane J of this DPP row), c <= J, each update one
 // instruction (the compiler makes a move and a multiply-add of it, and waits between them: 240 instructions and 110 waits
-// instead of 120 in all).  A register written by the vector ALU is read through DPP two instructions later at the earliest:
-// step J - 1 wrote x[c] J instructions ago, and the wait in front covers the first steps.
+// instead of 120 and 15 in all).  A register written by the vector ALU is read through DPP two wait states later at the
+// earliest, and no compiler check sees inside the asm: s_nop 1 is two wait states ahead of a step's first read, and within a
+// step an instruction reads through DPP only the register it writes itself, c ascending.
+#define FLA_UPDATE(c) "v_fmac_f32_dpp %" #c ", %" #c ", %[m] row_newbcast:%[j] row_mask:0xf bank_mask:0xf\n\t"
+// updates and operands of c = 0 .. J
+#define FLA_UPDATES_0 FLA_UPDATE(0)
+#define FLA_OPERANDS_0 "+v"(x[0])
+#define FLA_UPDATES_1 FLA_UPDATES_0 FLA_UPDATE(1)
+#define FLA_OPERANDS_1 FLA_OPERANDS_0, "+v"(x[1])
+#define FLA_UPDATES_2 FLA_UPDATES_1 FLA_UPDATE(2)
+#define FLA_OPERANDS_2 FLA_OPERANDS_1, "+v"(x[2])
+#define FLA_UPDATES_3 FLA_UPDATES_2 FLA_UPDATE(3)
+#define FLA_OPERANDS_3 FLA_OPERANDS_2, "+v"(x[3])
+#define FLA_UPDATES_4 FLA_UPDATES_3 FLA_UPDATE(4)
+#define FLA_OPERANDS_4 FLA_OPERANDS_3, "+v"(x[4])
+#define FLA_UPDATES_5 FLA_UPDATES_4 FLA_UPDATE(5)
+#define FLA_OPERANDS_5 FLA_OPERANDS_4, "+v"(x[5])
+#define FLA_UPDATES_6 FLA_UPDATES_5 FLA_UPDATE(6)
+#define FLA_OPERANDS_6 FLA_OPERANDS_5, "+v"(x[6])
+#define FLA_UPDATES_7 FLA_UPDATES_6 FLA_UPDATE(7)
+#define FLA_OPERANDS_7 FLA_OPERANDS_6, "+v"(x[7])
+#define FLA_UPDATES_8 FLA_UPDATES_7 FLA_UPDATE(8)
+#define FLA_OPERANDS_8 FLA_OPERANDS_7, "+v"(x[8])
+#define FLA_UPDATES_9 FLA_UPDATES_8 FLA_UPDATE(9)
+#define FLA_OPERANDS_9 FLA_OPERANDS_8, "+v"(x[9])
+#define FLA_UPDATES_10 FLA_UPDATES_9 FLA_UPDATE(10)
+#define FLA_OPERANDS_10 FLA_OPERANDS_9, "+v"(x[10])
+#define FLA_UPDATES_11 FLA_UPDATES_10 FLA_UPDATE(11)
+#define FLA_OPERANDS_11 FLA_OPERANDS_10, "+v"(x[11])
+#define FLA_UPDATES_12 FLA_UPDATES_11 FLA_UPDATE(12)
+#define FLA_OPERANDS_12 FLA_OPERANDS_11, "+v"(x[12])
+#define FLA_UPDATES_13 FLA_UPDATES_12 FLA_UPDATE(13)
+#define FLA_OPERANDS_13 FLA_OPERANDS_12, "+v"(x[13])
+#define FLA_UPDATES_14 FLA_UPDATES_13 FLA_UPDATE(14)
+#define FLA_OPERANDS_14 FLA_OPERANDS_13, "+v"(x[14])
 template <int J>
 FLA_DEVICE void wy_subst_step(float (&x)[16], const float (&nm)[16]) {
-#define FLA_STEP(c) "v_fmac_f32_dpp %" #c ", %" #c ", %[m] row_newbcast:%[j] row_mask:0xf bank_mask:0xf\n\t"
-  if constexpr (J == 0)
-    asm("s_nop 1\n\t" FLA_STEP(0) : "+v"(x[0]) : [m] "v"(nm[0]), [j] "i"(0));
-  if constexpr (J == 1)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) : "+v"(x[0]), "+v"(x[1]) : [m] "v"(nm[1]), [j] "i"(1));
-  if constexpr (J == 2)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]) : [m] "v"(nm[2]), [j] "i"(2));
-  if constexpr (J == 3)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]) : [m] "v"(nm[3]), [j] "i"(3));
-  if constexpr (J == 4)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]) : [m] "v"(nm[4]), [j] "i"(4));
-  if constexpr (J == 5)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]) : [m] "v"(nm[5]), [j] "i"(5));
-  if constexpr (J == 6)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]) : [m] "v"(nm[6]), [j] "i"(6));
-  if constexpr (J == 7)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]) : [m] "v"(nm[7]), [j] "i"(7));
-  if constexpr (J == 8)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]) : [m] "v"(nm[8]), [j] "i"(8));
-  if constexpr (J == 9)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]) : [m] "v"(nm[9]), [j] "i"(9));
-  if constexpr (J == 10)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]) : [m] "v"(nm[10]), [j] "i"(10));
-  if constexpr (J == 11)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]) : [m] "v"(nm[11]), [j] "i"(11));
-  if constexpr (J == 12)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]) : [m] "v"(nm[12]), [j] "i"(12));
-  if constexpr (J == 13)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) FLA_STEP(13) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]) : [m] "v"(nm[13]), [j] "i"(13));
-  if constexpr (J == 14)
-    asm("s_nop 1\n\t" FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7) FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) FLA_STEP(13) FLA_STEP(14) : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]), "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]) : [m] "v"(nm[14]), [j] "i"(14));
+#define FLA_STEP(N) \
+  if constexpr (J == N) asm("s_nop 1\n\t" FLA_UPDATES_##N : FLA_OPERANDS_##N : [m] "v"(nm[N]), [j] "i"(N));
+  FLA_STEP(0) FLA_STEP(1) FLA_STEP(2) FLA_STEP(3) FLA_STEP(4) FLA_STEP(5) FLA_STEP(6) FLA_STEP(7)
+  FLA_STEP(8) FLA_STEP(9) FLA_STEP(10) FLA_STEP(11) FLA_STEP(12) FLA_STEP(13) FLA_STEP(14)
 #undef FLA_STEP
   if constexpr (J < 14) wy_subst_step<J + 1>(x, nm);
 }
+#undef FLA_UPDATE
 
 // The 16x16 diagonal blocks of X = (I + M)^-1 for a strictly lower triangular fp32 M [64][LDM] in LDS, by forward
 // substitution, all four at once on one wave: DPP row b is block b, a lane holds row i of its block of M (zero on and above
