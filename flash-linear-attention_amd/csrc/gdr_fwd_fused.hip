@@ -271,7 +271,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           // (rows 4 further: another value of row bit 2, which moves the slot by 2)
           const v8 h = tr2(src + (hsrc ^ 32 * kt), src + ((hsrc ^ 32 * kt ^ 16) + 4 * K));
           // (non-temporal: the backward pass reads it much later.  4 x 4096 tokens, training step 518.6 -> 511.1 us; v_new as well
-          // 514.9, and 67 -> 72 us for the scan of 32 heads of 64)
+          // 514.9, and 67 -> 72 us for the scan of 32 heads of 64.  Steps whose states the last-level cache would hold, plain / so:
+          // 0.3 to 34 MB within 0.9 % of each other, but 32 heads of 64 of 2 x 2000 tokens, 17 MB, 136.6 / 138.6; 16 x 512 tokens, 32
+          // heads of 64, 34 MB, 238 / 233, 16 heads of 128, 67 MB, 247 / 241)
           __builtin_nontemporal_store(h, (v8*)(hbase + (n * KS + kt) * 2048 + x * 1024 + hlane));
         }
         hbase += (int64_t)H * K * V * 2;
@@ -577,8 +579,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int ci = 0; ci < nchunks; ++ci) {
         const int b = ci & 1;
         const T *Kr = sK[b3], *Tu = sTu[b];
-        // LDS reads are issued a group ahead of the matrix instructions that consume them (the fences keep them there: at most
-        // sixteen are outstanding)
+        // LDS reads are issued a group ahead of the matrix instructions that consume them (the fences keep that order; with 128
+        // key channels a group of k is sixteen reads, and two are on their way before the first is used)
         v8 fa[2][KS], fb[2][KS];
         auto read_k = [&](int t0, v8 (*f)[KS]) __attribute__((always_inline)) {   // two row tiles
 #pragma unroll

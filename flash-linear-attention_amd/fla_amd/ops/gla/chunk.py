@@ -450,7 +450,7 @@ def chunk_gla_bwd_device(q, k, v, g, scale, initial_state, do, dht, offsets, wid
     recomputes the per-chunk states as the reference does (``fla/ops/gla/chunk.py:1239-1253``).  ``qg``, ``decay``:
     the gated queries and chunk decays of ``fla_chunk_gla_fwd_fused_kept``, if the forward kept them.  ``wide``: the forward's
     gate-range flags (int32 ``[chunks, H]``); flagged chunks get their intra-chunk terms
-    from the exact kernel.  Without it the result is exact only while the chunk-cumulative
+    with pairwise exponents (``exact_scores`` in ``csrc/gla_bwd_chunk.hip``).  Without it the result is exact only while the chunk-cumulative
     log-gate stays within +-80.  ``head_gates``: ``g`` is one fp32 log-gate per (token, head), ``[B, T, H]``, and
     ``dg`` comes back in that shape (``fla_chunk_simple_gla_bwd`` when the forward kept its gated queries; otherwise
     the gates are broadcast over the key channels and the per-key gradient is summed afterwards).  ``kh``, ``scores``: what

@@ -345,8 +345,8 @@ def test_chunk_simple_gla_rows_outside_the_sequences(device, native, bounds, mon
 
 @pytest.mark.parametrize("varlen", [False, True])
 def test_chunk_simple_gla_strong_gates_backward_reproducible(device, varlen, monkeypatch):
-    """Gates strong enough that chunks leave the single-reference range (their intra-chunk terms come from the
-    exact kernel): the per-head gate gradient, which the backward kernels accumulate from their key slices, is
+    """Gates strong enough that chunks leave the single-reference range (their intra-chunk terms come with
+    pairwise exponents): the per-head gate gradient, which the backward kernels accumulate from their key slices, is
     the same bit for bit on a second run, agrees with the form that writes per-key gradients and sums them
     afterwards (the backward that recomputes the states), and both meet the fp32 recurrence."""
     import fla_amd.ops.gla.chunk as gla_mod
