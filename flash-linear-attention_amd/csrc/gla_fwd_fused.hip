@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256 + 64 * NSTG) void gla_fwd_fused_kernel(FusedPar
               // it reads first.  Training step of 4 x 4096 tokens, 16 heads of 128: 467 us, with whole stores 462.6 (the
               // forward 137.5 -> 131.2), non-temporal too 456; the gated queries as well 452.4, but 132.8 -> 139.5 for 2 x 2048
               // tokens, where they would still be in the last-level cache.  Steps with states of 0.3 to 67 MB, whole stores plain /
-              // non-temporal: within 0.8 % of each other (2 x 256 tokens, 4 heads of 64 28.7 / 28.8; 2 x 2048, 16 of 128 132.3 / 133.0,
+              // non-temporal: 0.8 % more at most, 2 % less at most (2 x 256 tokens, 4 heads of 64 28.7 / 28.8; 2 x 2048, 16 of 128 132.3 / 133.0,
               // per-head gates 109.5 / 108.4; 4 x 2048 240.8 / 240.5).
               typedef uint32_t u4 __attribute__((ext_vector_type(4)));
               u4 x = __builtin_bit_cast(u4, lo), y = __builtin_bit_cast(u4, hi);
